@@ -152,8 +152,8 @@ int  pimc_plan_rotor3d_split(int protmax, int nchains, int nrot, int blocks_per_
                           depend on it: every draw is addressed by (sweep, slice).
      "bisect_lanes_small", "bisect_lanes_medium", "bisect_lanes_large"
                           lanes (64, 128 or 256) per bisection segment for replicas of at most
-                          24, at most 64 and more atoms; defaults 64, 128, 256.  Results do not
-                          depend on them.
+                          24, at most 64 and more atoms; by default chosen from the number of
+                          segments.  Results do not depend on them.
      "delayed_acceptance" 1: the non-linear rotor move (MCRot3Dstep mc_piqmc.cc:938-1199) runs
                           its test as three Metropolis factors: the density, the surrogate
                           network, then the exact correction (see the surrogate section below);

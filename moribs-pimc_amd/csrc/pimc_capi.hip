@@ -91,6 +91,17 @@ std::vector<Part> xcd_order(const std::vector<Part>& parts, Work work) {
 // bisection size classes of the linear family: lanes per workgroup by atom count
 inline int bisect_class(int natoms) { return natoms <= 24 ? 0 : (natoms <= 64 ? 1 : 2); }
 
+// Lanes of a segment's group in size class k with segs segments in all.  With few segments a chain's
+// atoms in turn are the time, and four waves shorten a move; with many the device is full and one
+// wave a segment wastes least.  Bisection per pass at 256 and 64 lanes: 40 atoms 1.02 and 1.16 ms on
+// 512 segments, 1.28 and 1.24 on 1024; 100 atoms 3.38 and 3.96 ms on 1024, 6.44 and 4.70 on 2048.
+// Up to 24 atoms a wave holds the partners as it is (8 atoms: 0.30 and 0.32 ms on 512), and two
+// segments share one on a full device (0.445 against 0.470 ms on 4096).
+inline int bisect_group(int k, long long segs) {
+    if (k == 0) return segs >= 4096 ? 32 : 64;
+    return segs <= (k == 1 ? 768 : 1280) ? 256 : 64;
+}
+
 template <typename T>
 T* dalloc(size_t n) {
     T* p = nullptr;
@@ -199,20 +210,30 @@ struct pimc_ctx {
     int2* d_rows1 = nullptr;
     int nrows1 = 0;
     size_t lds_bisect1 = 0;
-    int2* d_work = nullptr;
-    int nwork = 0;
+    int2* d_work = nullptr;  // bisection blocks of the linear family: (replica, first segment)
     int* d_all = nullptr;
     int* d_rotreps = nullptr;
     int nrotreps = 0;
     double* d_est = nullptr;
-    size_t lds_bisect = 0, lds_rotor = 0;
+    size_t lds_rotor = 0;
     int Smax = 1, Pmax = 1, Nmax = 1, max_types = 1;
     int bisect_block = 64;
-    // linear-family bisection in three size classes (N <= 24, <= 64, larger) with 64, 128 and
-    // 256 lanes and their own LDS sizes, launched as parallel branches of the pass
-    int bw_n[3] = {0, 0, 0}, bw_off[3] = {0, 0, 0};
-    int bw_lanes[3] = {64, 128, 256};  // lanes per segment of each class
+    // linear-family bisection in three size classes (N <= 24, <= 64, larger), each with its own
+    // lanes per segment, block and LDS, launched as parallel branches of the pass
+    int bw_n[3] = {0, 0, 0}, bw_off[3] = {0, 0, 0};  // blocks of a class and their place in d_work
+    int bw_opt[3] = {0, 0, 0};      // lanes per segment asked for (64, 128, 256), 0: by load
+    int bw_gw[3] = {64, 64, 64};    // lanes per segment (32: two segments share a wave)
+    int bw_block[3] = {64, 64, 64}; // lanes per block
     size_t bw_lds[3] = {0, 0, 0};
+    bool bw_uniform[3] = {false, false, false};  // FP32 on uniform tables
+    // proposals of the next bisection launch: the layout of the beads
+    double4* d_prop = nullptr;
+    PathItem* d_paths = nullptr;  // batches of (atom, segment) pairs, grouped by type, four per block
+    int path_off[PIMC_MAX_TYPES] = {0, 0, 0, 0}, path_n[PIMC_MAX_TYPES] = {0, 0, 0, 0};  // blocks of a type
+    int path_ring_len = 0;
+    hipStream_t side_paths = nullptr;  // the proposals' launch beside the rotor sweep
+    hipEvent_t ev_paths[2] = {nullptr, nullptr};
+    bool paths_beside = false;
     hipStream_t side[2] = {nullptr, nullptr};
     hipEvent_t ev_fork = nullptr, ev_join[2] = {nullptr, nullptr};
     int2* d_rows = nullptr;     // (replica, tile) work of the estimator pair sum
@@ -341,7 +362,7 @@ void pimc_destroy(pimc_ctx* c) {
                     c->d_t1, c->d_v2f, c->d_v2c, c->d_v2d, c->d_g2d, c->d_g2f, c->d_t2, c->d_rk, c->d_re, c->d_tr,
                     c->d_work, c->d_all, c->d_rotreps, c->d_est, c->d_rows, c->d_rowbuf, c->d_parts, c->d_flags, c->d_xrec,
                     c->d_r3, c->d_v3d, c->d_v3f, c->d_t3, c->d_frames, c->d_work1, c->d_all0, c->d_all1, c->d_rot3, c->d_rows1, c->d_mlp,
-                    c->d_rcf, c->d_rcfreps, c->d_cparts0, c->d_cparts1, c->d_cflags, c->d_cslots,
+                    c->d_rcf, c->d_rcfreps, c->d_cparts0, c->d_cparts1, c->d_cflags, c->d_cslots, c->d_prop, c->d_paths,
                     c->d_parts3, c->d_flags3, c->d_pub3};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -350,6 +371,9 @@ void pimc_destroy(pimc_ctx* c) {
         if (c->ev_join[k]) (void)hipEventDestroy(c->ev_join[k]);
     }
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
+    if (c->side_paths) (void)hipStreamDestroy(c->side_paths);
+    for (hipEvent_t e : c->ev_paths)
+        if (e) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -687,7 +711,7 @@ int pimc_set_option(pimc_ctx* c, const char* name, long value) {
         if (std::strcmp(name, lanes_opt[k]) == 0) {
             if (value != 64 && value != 128 && value != 256)
                 return fail(c, std::string(name) + " is 64, 128 or 256");
-            c->bw_lanes[k] = (int)value;
+            c->bw_opt[k] = (int)value;
             return 0;
         }
     if (std::strcmp(name, "centroid_parts") == 0) {
@@ -842,6 +866,98 @@ static int plan_centroid_parts(pimc_ctx* c, int target_parts) {
     return 0;
 }
 
+// The bisection's blocks: per size class the lanes of a segment's group (want[k]: 64, 128 or 256,
+// or 0 for a choice by load), the block and its LDS, and the (replica, first segment) list.  Called
+// at commit and again by the autotuner.
+static int plan_bisect(pimc_ctx* c, const int want[3]) {
+    const int rsize = c->fp64 ? 8 : 4;
+    struct Item {
+        int2 wk;
+        long long cost;
+    };
+    std::vector<Item> items[3];
+    for (int k = 0; k < 3; ++k) {
+        long long segs = 0;
+        size_t knots = 0, seg_bytes = 0;
+        bool uniform = !c->fp64;
+        for (const Rep& p : c->rep) {
+            if (p.fam || bisect_class(p.natoms) != k) continue;
+            segs += c->ref_order ? 1 : p.P / p.S;
+            seg_bytes = std::max(seg_bytes, (size_t)bisect_seg_bytes(p.natoms, p.S, rsize));
+            if (p.pot1d_id >= 0) uniform &= c->t1[p.pot1d_id].uniform != 0;
+            if (p.pot2d_id >= 0) uniform &= c->t2[p.pot2d_id].uniform != 0;
+        }
+        for (const Rep& p : c->rep)  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
+            if (!p.fam && bisect_class(p.natoms) == k && p.pot1d_id >= 0)
+                knots = std::max(knots, (size_t)c->t1[p.pot1d_id].n *
+                                            (c->fp64 ? sizeof(double4) : (uniform ? sizeof(float2) : sizeof(float4))));
+        if (!segs) {
+            c->bw_n[k] = 0;
+            continue;
+        }
+        knots = (knots + 15) & ~(size_t)15;
+        int gw = want[k];
+        if (gw == 0) gw = bisect_group(k, segs);
+        // as many waves per block as share the knots in 64 KB, a single wave when there are few
+        // segments for the device's CUs
+        int block = std::max(gw, segs * gw >= 64 * 1024 ? 256 : 64);
+        while (block > std::max(gw, 64) && knots + (size_t)(block / gw) * seg_bytes > 64 * 1024) block /= 2;
+        if (gw < 64 && knots + (size_t)(block / gw) * seg_bytes > 64 * 1024) gw = 64;
+        const size_t lds = knots + (size_t)(block / gw) * seg_bytes;
+        if (lds > 160 * 1024) return fail(c, "segment window exceeds LDS (too many atoms for this segment size)");
+        c->bw_uniform[k] = uniform;
+        c->bw_gw[k] = gw;
+        c->bw_block[k] = block;
+        c->bw_lds[k] = lds;
+        for (int r = 0; r < c->nrep; ++r) {
+            const Rep& p = c->rep[r];
+            if (p.fam || bisect_class(p.natoms) != k) continue;
+            const int nseg = c->ref_order ? 1 : p.P / p.S;
+            for (int q = 0; q < nseg; q += block / gw)
+                items[k].push_back({make_int2(r, q), (long long)p.natoms * p.natoms * p.S});
+        }
+        // largest windows first: the longest atom sequences start while the grid fills
+        std::stable_sort(items[k].begin(), items[k].end(), [](const Item& a, const Item& b) { return a.cost > b.cost; });
+    }
+    std::vector<int2> work;
+    for (int k = 2; k >= 0; --k) {
+        c->bw_off[k] = (int)work.size();
+        c->bw_n[k] = (int)items[k].size();
+        for (const Item& i : items[k]) work.push_back(i.wk);
+    }
+    if (c->d_work) (void)hipFree(c->d_work);
+    c->d_work = dalloc<int2>(work.size());
+    if (!c->d_work) return fail(c, "hipMalloc failed");
+    if (!work.empty()) HIPCHECK(c, hipMemcpy(c->d_work, work.data(), sizeof(int2) * work.size(), hipMemcpyHostToDevice));
+    return 0;
+}
+
+// The proposals' batches: per type the (atom, segment) pairs of every replica, four batches (one a
+// wave) per block.
+static int plan_paths(pimc_ctx* c) {
+    std::vector<PathItem> items;
+    c->path_ring_len = 0;
+    for (int ty = 0; ty < PIMC_MAX_TYPES; ++ty) {
+        c->path_off[ty] = (int)items.size() / 4;
+        for (int r = 0; r < c->nrep; ++r) {
+            const Rep& p = c->rep[r];
+            if (ty >= p.ntypes) continue;
+            const int L = p.tlev[ty], nm = (1 << L) - 1;
+            c->path_ring_len = std::max(c->path_ring_len, path_ring(nm, L));
+            const int pairs = p.tnumb[ty] * (c->ref_order ? 1 : p.P / p.S);
+            for (int q = 0; q < pairs; q += path_batch(nm, L)) items.push_back(PathItem{r, ty, q, 0});
+        }
+        while (items.size() % 4) items.push_back(PathItem{-1, ty, 0, 0});
+        c->path_n[ty] = (int)items.size() / 4 - c->path_off[ty];
+    }
+    c->d_paths = dalloc<PathItem>(items.size());
+    if (!c->d_paths) return fail(c, "hipMalloc failed");
+    HIPCHECK(c, hipMemcpy(c->d_paths, items.data(), sizeof(PathItem) * items.size(), hipMemcpyHostToDevice));
+    HIPCHECK(c, hipStreamCreate(&c->side_paths));  // default priority, like the main stream
+    for (hipEvent_t& e : c->ev_paths) HIPCHECK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return 0;
+}
+
 int pimc_commit(pimc_ctx* c) {
     if (c->committed) return fail(c, "already committed");
     for (int r = 0; r < c->nrep; ++r)
@@ -850,11 +966,10 @@ int pimc_commit(pimc_ctx* c) {
     c->rep.resize(c->nrep);
     long long boff = 0, roff = 0, hoff = 0, rcfoff = 0;
     std::vector<int> rcfreps;
-    std::vector<int2> work, rows, work1, rows1;
+    std::vector<int2> rows, work1, rows1;
     std::vector<int> rotreps, all0, all1, rot3;
     size_t lds_b1 = 0;
     long long rowoff = 0;
-    size_t lds_b = 0;
     c->bead_moves_per_pass = 0;
     for (int r = 0; r < c->nrep; ++r) {
         const pimc_replica_desc& d = c->desc[r];
@@ -996,24 +1111,14 @@ int pimc_commit(pimc_ctx* c) {
         c->lds_est = std::max(c->lds_est, (size_t)(3 * p.natoms * (ts + 1) + 3 * ts) * sizeof(double) +
                                               (size_t)p.natoms * sizeof(int));
         int W = S + 1;
-        // (y, y'') pairs of uniform FP32 knots in the linear family, vec4 knots otherwise
-        size_t knots = 0;
-        if (p.pot1d_id >= 0) {
-            const Tab1D& t = c->t1[p.pot1d_id];
-            knots = (size_t)t.n * (c->fp64 ? sizeof(double4) : (p.fam == 0 && t.uniform ? sizeof(float2) : sizeof(float4)));
+        if (p.fam) {  // the non-linear family's bisection: the layout of k_bisect_nl
+            size_t knots = 0;
+            if (p.pot1d_id >= 0) knots = (size_t)c->t1[p.pot1d_id].n * (c->fp64 ? sizeof(double4) : sizeof(float4));
+            lds_b1 = std::max(lds_b1, 16 * sizeof(double) +
+                                          (size_t)(p.natoms + 1) * W * (c->fp64 ? sizeof(double4) : sizeof(float4)) +
+                                          (size_t)12 * p.nrot * W * sizeof(double) + knots);
+            for (int k = 0; k < (c->ref_order ? 1 : p.P / S); ++k) work1.push_back(make_int2(r, k));
         }
-        // bisection LDS: new positions and the draw ring (FP64), the window, the new midpoints
-        // and the rotor axes in the pair precision, frames, knots (the layout of bisect_body)
-        const size_t lds_w = (size_t)((3 * W + bisect_ring(W) + 3) & ~3) * sizeof(double) +
-                             (size_t)(p.natoms + 2) * W * (c->fp64 ? sizeof(double4) : sizeof(float4)) +
-                             (size_t)12 * p.nrot * W * sizeof(double) + knots;
-        (p.fam ? lds_b1 : lds_b) = std::max(p.fam ? lds_b1 : lds_b, lds_w);
-        if (!p.fam) {
-            const int k = bisect_class(p.natoms);
-            c->bw_lds[k] = std::max(c->bw_lds[k], lds_w);
-        }
-        int nseg = c->ref_order ? 1 : p.P / S;
-        for (int k = 0; k < nseg; ++k) (p.fam ? work1 : work).push_back(make_int2(r, k));
         c->Nmax = std::max(c->Nmax, p.natoms);
         c->Smax = std::max(c->Smax, S);
         c->Pmax = std::max(c->Pmax, p.P);
@@ -1028,10 +1133,9 @@ int pimc_commit(pimc_ctx* c) {
             return fail(c, c->ref_order ? "samples_per_pass must divide P"
                                         : "samples_per_pass must divide the segment size 2^levels");
     }
-    if (std::max(lds_b, lds_b1) > 160 * 1024)
+    if (lds_b1 > 160 * 1024)
         return fail(c, "segment window exceeds LDS (too many atoms for this segment size)");
     if (c->lds_est > 150 * 1024) return fail(c, "estimator tile exceeds LDS (too many atoms)");
-    c->lds_bisect = lds_b;
     c->lds_bisect1 = lds_b1;
     for (const Tab1D& t : c->t1)
         c->lds_knots = std::max(c->lds_knots, (size_t)t.n * (c->fp64 ? sizeof(double4) : sizeof(float4)));
@@ -1058,17 +1162,9 @@ int pimc_commit(pimc_ctx* c) {
         const Rep &a = c->rep[x.x], &b = c->rep[y.x];
         return (long long)a.natoms * a.natoms * a.S > (long long)b.natoms * b.natoms * b.S;
     };
-    std::stable_sort(work.begin(), work.end(), heavier);
     std::stable_sort(work1.begin(), work1.end(), heavier);
-    {  // size classes of the linear family, heaviest class first in the work array
-        std::vector<int2> byc[3];
-        for (const int2& w : work) byc[bisect_class(c->rep[w.x].natoms)].push_back(w);
-        work.clear();
-        for (int k = 2; k >= 0; --k) {
-            c->bw_off[k] = (int)work.size();
-            c->bw_n[k] = (int)byc[k].size();
-            work.insert(work.end(), byc[k].begin(), byc[k].end());
-        }
+    if (plan_bisect(c, c->bw_opt) || plan_paths(c)) return -1;
+    {
         int busy = 0;
         for (int k = 0; k < 3; ++k) busy += c->bw_n[k] > 0;
         if (busy > 1)
@@ -1147,7 +1243,6 @@ int pimc_commit(pimc_ctx* c) {
             HIPCHECK(c, hipMemset(c->d_pub3, 0, sizeof(unsigned long long) * nflags3 * c->pub3_stride));
         }
     }
-    c->nwork = (int)work.size();
     c->nwork1 = (int)work1.size();
     c->nall0 = (int)all0.size();
     c->nall1 = (int)all1.size();
@@ -1165,6 +1260,16 @@ int pimc_commit(pimc_ctx* c) {
     if (upv(c->d_work1, work1.data(), work1.size() * sizeof(int2)) || upv(c->d_all1, all1.data(), all1.size() * sizeof(int)) ||
         upv(c->d_rot3, rot3.data(), rot3.size() * sizeof(int)) || upv(c->d_rows1, rows1.data(), rows1.size() * sizeof(int2)))
         return fail(c, "upload failed");
+    {
+        // the proposals run beside a rotor sweep whose blocks leave half of the CUs free (8.0 against
+        // 8.6 ms per pass on 23 mixed replicas); beside one that fills the device they keep parts
+        // from being resident together, and their neighbours wait (226 against 145 ms on 128 pairs
+        // of water rotors)
+        hipDeviceProp_t prop;
+        HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
+        const int blocks = c->nparts + (int)rot3.size() + c->nparts3;
+        c->paths_beside = blocks > 0 && blocks <= prop.multiProcessorCount / 2;
+    }
     c->nrotreps = (int)rotreps.size();
     c->nrows = (int)rows.size();
     c->d_rows = dalloc<int2>(rows.size());
@@ -1175,22 +1280,21 @@ int pimc_commit(pimc_ctx* c) {
     c->d_rep = dalloc<Rep>(c->nrep);
     c->d_mut = dalloc<Mut>(c->nrep);
     c->d_beads = dalloc<double4>(boff);
+    c->d_prop = dalloc<double4>(boff);
     c->d_rotb = dalloc<RotBead>(roff);
     c->d_hist = dalloc<unsigned>(hoff);
-    c->d_work = dalloc<int2>(work.size());
     c->d_all = dalloc<int>(c->nrep);
     c->d_rotreps = dalloc<int>(rotreps.size());
     c->d_est = dalloc<double>(8 * (size_t)c->nrep);
     c->sample_cap = 4096;
     c->d_samples = dalloc<double>((size_t)8 * c->sample_cap * c->nrep);
     for (int r = 0; r < c->nrep; ++r) c->rep[r].sample_off = (long long)8 * c->sample_cap * r;
-    if (!c->d_rep || !c->d_mut || !c->d_beads || !c->d_rotb || !c->d_hist || !c->d_work || !c->d_all ||
+    if (!c->d_rep || !c->d_mut || !c->d_beads || !c->d_prop || !c->d_rotb || !c->d_hist || !c->d_all ||
         !c->d_rotreps || !c->d_est || !c->d_samples)
         return fail(c, "hipMalloc failed");
     HIPCHECK(c, hipMemcpy(c->d_rep, c->rep.data(), sizeof(Rep) * c->nrep, hipMemcpyHostToDevice));
     HIPCHECK(c, hipMemset(c->d_mut, 0, sizeof(Mut) * c->nrep));
     HIPCHECK(c, hipMemset(c->d_hist, 0, sizeof(unsigned) * std::max<long long>(hoff, 1)));
-    HIPCHECK(c, hipMemcpy(c->d_work, work.data(), sizeof(int2) * work.size(), hipMemcpyHostToDevice));
     std::vector<int> all(c->nrep);
     for (int r = 0; r < c->nrep; ++r) all[r] = r;
     HIPCHECK(c, hipMemcpy(c->d_all, all.data(), sizeof(int) * c->nrep, hipMemcpyHostToDevice));
@@ -1465,6 +1569,45 @@ void resolve_events(pimc_ctx* c) {
     c->pending.clear();
 }
 
+// the proposals of types [tb, te) for the bisection launch of start slice u, on stream s
+void launch_paths(pimc_ctx* c, hipStream_t s, int u, int tb, int te) {
+    const Run run{c->seed, u, c->ref_order ? 1 : 0, tb, te};
+    te = std::min(te, (int)PIMC_MAX_TYPES);
+    const int b0 = c->path_off[tb], n = c->path_off[te - 1] + c->path_n[te - 1] - b0;
+    if (n > 0)
+        hipLaunchKernelGGL(k_bisect_paths, dim3(n), dim3(256), sizeof(double) * 4 * c->path_ring_len, s, c->d_rep, c->d_mut,
+                           c->d_beads, c->d_prop, c->d_paths + 4 * (size_t)b0, c->path_ring_len, run);
+}
+
+// one bisection size class on stream s
+template <typename R>
+void launch_bisect_class(pimc_ctx* c, int k, hipStream_t s, const Run& run) {
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(c->bw_n[k]), dim3(c->bw_block[k]), c->bw_lds[k], s, c->d_rep, c->d_mut, c->d_beads,
+                           c->d_rotb, c->tables(), c->d_prop, c->d_work + c->bw_off[k], run);
+    };
+    auto group = [&](auto mi_c, auto ut_c) {
+        constexpr bool MI = decltype(mi_c)::value, UT = decltype(ut_c)::value;
+        switch (c->bw_gw[k]) {
+            case 32: launch(k_bisect<R, MI, UT, 32>); break;
+            case 64: launch(k_bisect<R, MI, UT, 64>); break;
+            case 128: launch(k_bisect<R, MI, UT, 128>); break;
+            default: launch(k_bisect<R, MI, UT, 256>);
+        }
+    };
+    auto tables = [&](auto ut_c) {
+        if (c->any_mi) group(std::true_type{}, ut_c);
+        else group(std::false_type{}, ut_c);
+    };
+    if constexpr (std::is_same<R, float>::value) {
+        if (c->bw_uniform[k]) {
+            tables(std::true_type{});
+            return;
+        }
+    }
+    tables(std::false_type{});
+}
+
 template <typename R>
 void launch_bisect(pimc_ctx* c, int u, int tb, int te) {
     Run run{c->seed, u, c->ref_order ? 1 : 0, tb, te};
@@ -1486,14 +1629,13 @@ void launch_bisect(pimc_ctx* c, int u, int tb, int te) {
             s = c->side[nside];
             (void)hipStreamWaitEvent(s, c->ev_fork, 0);
         }
-        hipLaunchKernelGGL((c->any_mi ? k_bisect<R, true> : k_bisect<R, false>), dim3(c->bw_n[k]), dim3(c->bw_lanes[k]), c->bw_lds[k], s, c->d_rep, c->d_mut,
-                           c->d_beads, c->d_rotb, c->tables(), c->d_work + c->bw_off[k], run);
+        launch_bisect_class<R>(c, k, s, run);
         if (k != top) (void)hipEventRecord(c->ev_join[nside++], s);
     }
     for (int i = 0; i < nside; ++i) (void)hipStreamWaitEvent(c->stream, c->ev_join[i], 0);
     if (c->nwork1)
         hipLaunchKernelGGL((c->any_mi ? k_bisect_nl<R, true> : k_bisect_nl<R, false>), dim3(c->nwork1), dim3(c->bisect_block), c->lds_bisect1, c->stream,
-                           c->d_rep, c->d_mut, c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_work1, run);
+                           c->d_rep, c->d_mut, c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_prop, c->d_work1, run);
 }
 
 template <typename R>
@@ -1556,13 +1698,6 @@ void launch_estimate(pimc_ctx* c, double* out) {
 // Autotuner launches: one bisection size class alone, and the linear-rotor sweep alone, over
 // the start slices of one pass as the context issues them.
 template <typename R>
-void launch_bisect_class(pimc_ctx* c, int k, int u) {
-    Run run{c->seed, u, c->ref_order ? 1 : 0, 0, c->max_types};
-    hipLaunchKernelGGL((c->any_mi ? k_bisect<R, true> : k_bisect<R, false>), dim3(c->bw_n[k]), dim3(c->bw_lanes[k]), c->bw_lds[k], c->stream, c->d_rep,
-                       c->d_mut, c->d_beads, c->d_rotb, c->tables(), c->d_work + c->bw_off[k], run);
-}
-
-template <typename R>
 void launch_centroid_all(pimc_ctx* c) {
     for (int ty = 0; ty < c->max_types; ++ty) {
         Run run{c->seed, 0, c->ref_order ? 1 : 0, ty, ty + 1};
@@ -1584,34 +1719,53 @@ void launch_rotor_linear(pimc_ctx* c, int u) {
                        c->d_beads, c->d_rotb, c->tables(), c->tables3(), c->d_parts, c->d_flags, c->d_xrec, run);
 }
 
+// Rotor sweep of start slice u and, beside it where it leaves CUs free, the proposals of the bisection of start slice u + 1
+// (of n start slices): they read the beads, which the sweep leaves alone.  Returns whether
+// join_paths has to follow before that bisection.
+template <typename R>
+bool launch_rotor_and_paths(pimc_ctx* c, int u, int n) {
+    const bool next = u + 1 < n;
+    const bool beside = next && !c->profile && c->paths_beside;
+    if (beside) {
+        (void)hipEventRecord(c->ev_paths[0], c->stream);
+        (void)hipStreamWaitEvent(c->side_paths, c->ev_paths[0], 0);
+        launch_paths(c, c->side_paths, u + 1, 0, PIMC_MAX_TYPES);
+        (void)hipEventRecord(c->ev_paths[1], c->side_paths);
+    }
+    launch_rotor<R>(c, u);
+    if (next && !beside) {
+        Timed t(c, "bisect");
+        launch_paths(c, c->stream, u + 1, 0, PIMC_MAX_TYPES);
+    }
+    return beside;
+}
+
 // one pass in the order described at the top of this file; with `sampled` and samples_per_pass
 // k > 1, an estimator sample after every P/k time steps (reference order) or every S/k phases
 // (segment order), as the reference samples every MCSKIP_AVERG time steps (mc_main.cc:383-386)
 template <typename R>
 void issue_pass(pimc_ctx* c, bool sampled) {
     const int k = sampled ? c->opt_samples_per_pass : 1;
-    if (c->ref_order) {
-        for (int t = 0; t < c->Pmax; ++t) {
+    const int n = c->ref_order ? c->Pmax : c->Smax;  // start slices
+    bool join = false;
+    for (int u = 0; u < n; ++u) {
+        if (join) (void)hipStreamWaitEvent(c->stream, c->ev_paths[1], 0);
+        if (u == 0) {
             for (int ty = 0; ty < c->max_types; ++ty) {
-                if (t == 0) launch_centroid<R>(c, ty);
-                launch_bisect<R>(c, t, ty, ty + 1);
-            }
-            launch_rotor<R>(c, t);
-            if (k > 1 && (t + 1) % (c->Pmax / k) == 0) launch_estimate<R>(c, nullptr);
-        }
-    } else {
-        for (int u = 0; u < c->Smax; ++u) {
-            if (u == 0) {
-                for (int ty = 0; ty < c->max_types; ++ty) {
-                    launch_centroid<R>(c, ty);
-                    launch_bisect<R>(c, 0, ty, ty + 1);
+                launch_centroid<R>(c, ty);
+                {
+                    Timed t(c, "bisect");
+                    launch_paths(c, c->stream, 0, ty, ty + 1);
                 }
-            } else {
-                launch_bisect<R>(c, u, 0, PIMC_MAX_TYPES);
+                launch_bisect<R>(c, 0, ty, ty + 1);
             }
-            launch_rotor<R>(c, u);
-            if (k > 1 && (u + 1) % (c->Smax / k) == 0) launch_estimate<R>(c, nullptr);
+        } else if (c->ref_order) {
+            for (int ty = 0; ty < c->max_types; ++ty) launch_bisect<R>(c, u, ty, ty + 1);
+        } else {
+            launch_bisect<R>(c, u, 0, PIMC_MAX_TYPES);
         }
+        join = launch_rotor_and_paths<R>(c, u, n);
+        if (k > 1 && (u + 1) % (n / k) == 0) launch_estimate<R>(c, nullptr);
     }
     hipLaunchKernelGGL(k_pass_end, dim3((c->nrep + 255) / 256), dim3(256), 0, c->stream, c->d_mut, c->nrep);
 }
@@ -1711,23 +1865,31 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
         rc = fail(c, "autotune: event or copy failed");
     } else {
         static const int lanes[3] = {64, 128, 256};
+        int chosen_lanes[3] = {c->bw_gw[0], c->bw_gw[1], c->bw_gw[2]};
         for (int k = 0; k < 3 && rc == 0; ++k) {
             if (!c->bw_n[k]) continue;
-            int best = c->bw_lanes[k];
+            int best = chosen_lanes[k];
             double tbest = -1.0;
             for (int L : lanes) {
-                c->bw_lanes[k] = L;
+                chosen_lanes[k] = L;
+                if (plan_bisect(c, chosen_lanes)) {
+                    rc = -1;
+                    break;
+                }
                 const double t = timed([&](int u) {
-                    if (c->fp64) launch_bisect_class<double>(c, k, u);
-                    else launch_bisect_class<float>(c, k, u);
+                    const Run run{c->seed, u, c->ref_order ? 1 : 0, 0, c->max_types};
+                    launch_paths(c, c->stream, u, 0, PIMC_MAX_TYPES);
+                    if (c->fp64) launch_bisect_class<double>(c, k, c->stream, run);
+                    else launch_bisect_class<float>(c, k, c->stream, run);
                 });
                 if (t >= 0.0 && (tbest < 0.0 || t < tbest)) {
                     tbest = t;
                     best = L;
                 }
             }
-            c->bw_lanes[k] = best;
+            chosen_lanes[k] = best;
         }
+        if (rc == 0 && plan_bisect(c, chosen_lanes)) rc = -1;
         if (rc == 0 && !c->rot_chains.empty()) {
             static const int budgets[4] = {40, 52, 64, 78};
             int best = c->rotor_lds_kb;
@@ -1781,7 +1943,7 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
             *gx = nullptr;
         }
     if (rc == 0 && chosen) {
-        for (int k = 0; k < 3; ++k) chosen[k] = c->bw_lanes[k];
+        for (int k = 0; k < 3; ++k) chosen[k] = std::max(64, c->bw_gw[k]);
         chosen[3] = c->rotor_lds_kb;
         chosen[4] = c->centroid_target;
     }

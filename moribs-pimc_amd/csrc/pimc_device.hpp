@@ -340,18 +340,49 @@ __device__ __forceinline__ R spot1d(const Lut1D<R>& L, const vec4_t<R>* __restri
     }
 }
 
+// FP32 products and sums of the move kernels in a fixed order of fused operations.  Which of two
+// products a sum fuses is otherwise the compiler's choice, made anew in every kernel, and a chain
+// depends on the last bit of its pair terms.
+__device__ __forceinline__ float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+__device__ __forceinline__ float dot3(float ax, float ay, float az, float bx, float by, float bz) {
+    return __builtin_fmaf(az, bz, __builtin_fmaf(ax, bx, rounded_product(ay, by)));
+}
+
 // SPot1D on uniform FP32 knots from (y, y'') pairs alone (x and the cell width follow from the
 // grid), for kernels that stage the knots in LDS at half the size; the same branchless form
-__device__ __forceinline__ float spot1d_u2(const Lut1D<float>& L, const float2* __restrict__ k2, float r) {
-    const float t = (r - L.x0) * L.inv_h;
-    float f = floor(t);
+__device__ __forceinline__ float spot1d_u2_cell(const Lut1D<float>& L, const float2* __restrict__ k2, float r) {
+    const float x = r - L.x0;
+    float f = floor(rounded_product(x, L.inv_h));
     f = fmin(fmax(f, 0.f), (float)(L.n - 2));
     const int i = (int)f;
     const float2 a = k2[i], b = k2[i + 1];
-    const float h = fast_div(1.0f, L.inv_h);
-    const float B = t - f, A = 1.0f - B;
-    const float v = A * a.x + B * b.x + ((A * A * A - A) * a.y + (B * B * B - B) * b.y) * (h * h) * (1.0f / 6.0f);
-    return spot1d_tails(L, r, v);
+    const float h = fast_div(1.0f, L.inv_h), h2 = rounded_product(h, h);
+    const float B = __builtin_fmaf(L.inv_h, x, -f), A = 1.0f - B;
+    const float ca = __builtin_fmaf(A, rounded_product(A, A), -A), cb = __builtin_fmaf(B, rounded_product(B, B), -B);
+    const float cub = __builtin_fmaf(ca, a.y, rounded_product(cb, b.y));
+    return __builtin_fmaf(1.0f / 6.0f, rounded_product(h2, cub), __builtin_fmaf(A, a.x, rounded_product(B, b.x)));
+}
+
+// SPot1D at n distances, the table part of all of them before any tail: the tails' wave-uniform
+// branches end the span in which independent look-ups interleave, so a move's new and old distances
+// (and several partners') go through one pair of branches together
+template <int n>
+__device__ __forceinline__ void spot1d_u2_many(const Lut1D<float>& L, const float2* __restrict__ k2, const float (&r)[n],
+                                               float (&v)[n]) {
+    float lo = r[0], hi = r[0];
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+        v[i] = spot1d_u2_cell(L, k2, r[i]);
+        lo = fminf(lo, r[i]);
+        hi = fmaxf(hi, r[i]);
+    }
+    if (__any(lo <= L.x0) || __any(hi >= L.xmax)) {
+#pragma unroll
+        for (int i = 0; i < n; ++i) v[i] = spot1d_tails(L, r[i], v[i]);
+    }
 }
 
 // LPot2D on a uniform FP32 grid in two steps, so that the loads of many look-ups can be in
@@ -396,6 +427,37 @@ __device__ __forceinline__ R lpot2d(const Lut2D<R>& L, R r, R c) {
     R dr = (r - r1) / (r2 - r1);
     R dc = (c - c1) / (c2 - c1);
     return ((R)1 - dr) * ((R)1 - dc) * y1 + dr * ((R)1 - dc) * y2 + dr * dc * y3 + ((R)1 - dr) * dc * y4;
+}
+
+// The pair of the linear rotor and an atom (pair_d with rot_a or rot_j) in two steps, so that table
+// loads of many pairs fly together: the distance and its cell, then the value.  rot_a: the mover is
+// the rotor, which turns the separation and so the cosine's sign.  On uniform FP32 tables the cosine
+// is rounded to FP32 before its weight is formed, and for an atom's move the cell takes it unrounded;
+// chains depend on that last bit, so it is written out rather than left to contraction.
+struct RotorCell {
+    float4 q;
+    float wr, wc;
+};
+
+__device__ __forceinline__ RotorCell rotor_pair_load(const Lut2D<float>& L, bool rot_a, float dx, float dy, float dz,
+                                                     float nx, float ny, float nz) {
+    const float r = fast_sqrt(dot3(dx, dy, dz, dx, dy, dz));
+    const float dot = dot3(nx, ny, nz, dx, dy, dz), ir = __builtin_amdgcn_rcpf(r);
+    float c = rounded_product(dot, ir);
+    if (rot_a) c = -c;
+    const float above = rot_a ? c - L.cmin : __builtin_fmaf(ir, dot, -L.cmin);
+    float fr = floor((r - L.rmin) * L.inv_dr), fc = floor(above * L.inv_dc);
+    fr = fmin(fmax(fr, 0.f), (float)(L.nr - 2));
+    fc = fmin(fmax(fc, 0.f), (float)(L.nc - 2));
+    RotorCell k;
+    k.q = L.vc[(int)fr * (L.nc - 1) + (int)fc];
+    k.wr = (r - (L.rmin + fr * L.gdr)) * L.inv_gdr;
+    k.wc = (c - (L.cmin + fc * L.gdc)) * L.inv_gdc;
+    return k;
+}
+
+__device__ __forceinline__ float rotor_pair_value(const RotorCell& k) {
+    return lpot2d_u_lerp(k.q.x, k.q.y, k.q.z, k.q.w, k.wr, k.wc);
 }
 
 // SRotDens (mc_poten.cc:548-570) with the table descriptor already resolved: the last value
@@ -523,10 +585,9 @@ __device__ __forceinline__ double rot_spline(const Tables& T, int tid, double g,
 // mc_piqmc.cc:1847-1958, for one atom type and one linear-molecule type per system,
 // mc_input.cc:386-387).  rot_a / rot_j: the mover / partner is the linear molecule; (nx,ny,nz)
 // is its axis at that slice.
-// ... on the separation (dx, dy, dz) = mover - partner.  HALF: k1 points to (y, y'') pairs of
-// uniform FP32 knots (spot1d_u2), otherwise to vec4 knots.
-template <typename R, bool HALF = false>
-__device__ __forceinline__ R pair_d(const Lut1D<R>& l1, const void* __restrict__ k1, const Lut2D<R>& l2,
+// ... on the separation (dx, dy, dz) = mover - partner.
+template <typename R>
+__device__ __forceinline__ R pair_d(const Lut1D<R>& l1, const vec4_t<R>* __restrict__ k1, const Lut2D<R>& l2,
                                     bool rot_a, bool rot_j, R dx, R dy, R dz, double nx, double ny, double nz) {
     const R r = fast_sqrt(dx * dx + dy * dy + dz * dz);
     if (rot_a || rot_j) {
@@ -534,8 +595,7 @@ __device__ __forceinline__ R pair_d(const Lut1D<R>& l1, const void* __restrict__
         if (rot_a) cost = -cost;
         return lpot2d<R>(l2, r, cost);
     }
-    if constexpr (HALF && is_fp32<R>()) return spot1d_u2(l1, static_cast<const float2*>(k1), r);
-    else return spot1d<R>(l1, static_cast<const vec4_t<R>*>(k1), r);
+    return spot1d<R>(l1, k1, r);
 }
 
 // MINIMAGE (mc_piqmc.cc:1239-1240,1832-1833; mc_estim.cc:536-537,916-917): component id of a
@@ -555,15 +615,6 @@ __device__ __forceinline__ R pair_v(const Lut1D<R>& l1, const vec4_t<R>* __restr
                                     double zj, double nx, double ny, double nz, const double* box = nullptr) {
     return pair_d<R>(l1, k1, l2, rot_a, rot_j, (R)nearest_image(xa - xj, box, 0), (R)nearest_image(ya - yj, box, 1),
                      (R)nearest_image(za - zj, box, 2), nx, ny, nz);
-}
-
-// positions already in the pair precision (the bisection window)
-template <typename R, bool HALF = false>
-__device__ __forceinline__ R pair_vr(const Lut1D<R>& l1, const void* __restrict__ k1, const Lut2D<R>& l2,
-                                     bool rot_a, bool rot_j, R xa, R ya, R za, R xj, R yj, R zj, double nx, double ny,
-                                     double nz, const double* box = nullptr) {
-    return pair_d<R, HALF>(l1, k1, l2, rot_a, rot_j, nearest_image(xa - xj, box, 0), nearest_image(ya - yj, box, 1),
-                           nearest_image(za - zj, box, 2), nx, ny, nz);
 }
 
 // One DPP lane move within rows of 16 lanes (ctrl: quad_perm 0x00-0xff, row_mirror 0x140,

@@ -1,10 +1,11 @@
 // pimc_kernels.hpp -- gfx950 kernels of the sampling hot path.
 //
-//   k_bisect     one workgroup per (replica, imaginary-time segment).  The segment window
-//                (all atoms' beads on the S+1 slices of the segment, plus the linear rotor's
-//                axis there) is staged in LDS once and every atom of the selected types is
-//                moved in turn, as MCBisectionMove does (mc_piqmc.cc:194-294).  Segments of
-//                one offset share only fixed end points, so they run concurrently.
+//   k_bisect     linear family: a group of 16 to 256 lanes per (replica, imaginary-time segment).
+//                All atoms' beads on the segment's inner slices, plus the linear rotor's axis
+//                there, are staged in LDS once and every atom of the selected types is moved in
+//                turn, as MCBisectionMove does (mc_piqmc.cc:194-294).  Segments of one offset
+//                share only fixed end points, so they run concurrently.
+//   k_bisect_nl  the same for the non-linear family, one workgroup per segment.
 //   k_centroid_parts  a replica's slices split over workgroups; atoms in turn, Delta V over the
 //                part's slices x partners, partials exchanged as numbered words in memory
 //                (MCMolecularMove mc_piqmc.cc:54-102).
@@ -96,22 +97,450 @@ __device__ __forceinline__ const Frame& frame_at(const Frame* __restrict__ frame
 }
 
 // ------------------------------------------------------------------------- bisection
-constexpr int BIS_RING = 128;  // doubles of draws staged for a batch of atoms
+// A workgroup barrier that orders LDS only.  __syncthreads also waits for every global access in
+// flight, which here are a prefetch and the stores of an accepted move that no lane reads again.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
-// doubles of the draw ring for a window of W slots: a batch of atoms, or one atom's draws
-__host__ __device__ constexpr int bisect_ring(int W) { return BIS_RING > 3 * W + 16 ? BIS_RING : 3 * W + 16; }
+// block_sum with those barriers
+__device__ __forceinline__ double block_sum_lds(double v, double* red) {
+    v = wave_sum(v);
+    const int wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    lds_barrier();
+    if ((threadIdx.x & 63) == 0) red[wid] = v;
+    lds_barrier();
+    double s = 0;
+    for (int i = 0; i < nw; ++i) s += red[i];
+    return s;
+}
 
+// LDS written by some lanes of a wave and read by others: a wave's LDS operations complete in
+// order, so only the compiler has to keep theirs
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the same among the GW lanes of a group, which may span waves
+template <int GW>
+__device__ __forceinline__ void group_sync() {
+    if constexpr (GW > 64) lds_barrier();
+    else wave_sync();
+}
+
+// The proposals of one launch of the bisection, ahead of it.  An atom's new midpoints depend on its
+// draws and on its segment's end points alone, which no move of the launch changes, so every move's
+// are formed here with all lanes busy; inside the moves' chain of dependent steps the generator, the
+// logarithm and the cosine were a fifth of the time.  prop has the layout of beads: the midpoint of
+// an inner slot at that bead's place, and in .w of slot l + 1 the acceptance draw of level l.  The
+// launch runs beside the rotor sweep of the phase before, which leaves most issue slots idle.
+// A wave takes a batch of (atom, segment) pairs, so that all its lanes draw.
+struct PathItem {
+    int r, ty, first, pad;  // pairs first, first + 1, ... of type ty; pair = atom * segments + segment
+};
+
+// doubles of a batch's draws; pairs of a batch whose moves have nm midpoints and L levels
+__host__ __device__ constexpr int path_ring(int nm, int L) { return 192 > 3 * nm + L ? 192 : 3 * nm + L; }
+__host__ __device__ constexpr int path_batch(int nm, int L) { return 192 > 3 * nm + L ? 192 / (3 * nm + L) : 1; }
+
+__global__ __launch_bounds__(256) void k_bisect_paths(const Rep* __restrict__ reps, const Mut* __restrict__ mut,
+                                                      const double4* __restrict__ beads, double4* __restrict__ prop,
+                                                      const PathItem* __restrict__ items, int ring, Run run) {
+    extern __shared__ double smem[];
+    const int l = threadIdx.x & 63;
+    double* gw = smem + (threadIdx.x >> 6) * ring;  // the batch's draws: per pair 3 per midpoint, then one per level
+    const PathItem item = items[blockIdx.x * 4 + (threadIdx.x >> 6)];
+    if (item.r < 0) return;  // padding of the list
+    const Rep& rp = reps[item.r];
+    const int S = rp.S, P = rp.P;
+    if (run.u >= (run.ref_order ? P : S)) return;
+    const int ty = item.ty, L = rp.tlev[ty], St = 1 << L, nm = St - 1, per = 3 * nm + L;
+    const int nseg = run.ref_order ? 1 : P / S;
+    const int left = rp.tnumb[ty] * nseg - item.first;
+    const int nk = left < path_batch(nm, L) ? left : path_batch(nm, L);
+    const int ia0 = item.first / nseg, seg0 = item.first - ia0 * nseg;
+    const uint32_t pass = mut[item.r].pass;
+    const float inv_per = 1.0f / (float)per, inv_nm3 = 1.0f / (float)(3 * nm);
+    const double gscale = sqrt(rp.lambda[ty] * rp.tau);  // Gaussian width at the last level
+    auto pair_at = [&](int k, int& a, int& s0) {
+        int seg = seg0 + k, ia = ia0;
+        while (seg >= nseg) {
+            seg -= nseg;
+            ++ia;
+        }
+        a = rp.tbegin[ty] + ia;
+        s0 = run.ref_order ? run.u : run.u + seg * S;
+    };
+    // Gaussians of midpoint m (level-major order) and the level acceptance uniforms u, kept as
+    // -log(u): the level test exp(-dV) > u (mc_piqmc.cc:265-273) is then dV < -log(u), a comparison.
+    // Both kinds take one generator call and one logarithm, on one path
+    for (int i = l; i < nk * per; i += 64) {
+        const int k = (int)(((float)i + 0.5f) * inv_per), d = i - k * per;
+        int a, s0;
+        pair_at(k, a, s0);
+        const bool gauss = d < 3 * nm;
+        const int m = d / 3, id = d - 3 * m;
+        const int level = gauss ? 31 - __clz(m + 1) : d - 3 * nm;
+        const int q = m + 1 - (1 << level);
+        const uint4 w4 = draw(run.seed, rp.key, pass, K_BISECT, 0, (uint32_t)a, (uint32_t)s0,
+                              ((uint32_t)level << 24) | (gauss ? ((uint32_t)q << 8) | (uint32_t)id : 0xFFFFu << 8));
+        const double u = u53(w4.x, w4.y);
+        double v = -log(gauss ? 1.0 - u : u);
+        if (gauss) {  // Box-Muller of density exp(-alpha x^2), alpha = 1 / (lambda tau 2^(L - level))
+            const int ex = L - level;
+            v = sqrt(v) * cospi(2.0 * u53(w4.z, w4.w)) * ((ex & 1 ? 1.4142135623730951 : 1.0) * (double)(1 << (ex >> 1)) * gscale);
+            gw[i] = v;
+        } else {
+            const int it = s0 + 1 + level < P ? s0 + 1 + level : s0 + 1 + level - P;
+            prop[rp.bead_off + (long long)a * P + it].w = v;
+        }
+    }
+    wave_sync();
+    // coordinate id of slot s: a lane follows its slot down the bisection tree (the midpoints above
+    // it are formed again with the same operands)
+    for (int i = l; i < nk * 3 * nm; i += 64) {
+        const int k = (int)(((float)i + 0.5f) * inv_nm3), c = i - k * 3 * nm;
+        const int s = c / 3 + 1, id = c - 3 * (s - 1);
+        int a, s0;
+        pair_at(k, a, s0);
+        const long long b0 = rp.bead_off + (long long)a * P;
+        double lo = reinterpret_cast<const double*>(beads + b0 + s0)[id];
+        double hi = reinterpret_cast<const double*>(beads + b0 + (s0 + St < P ? s0 + St : s0 + St - P))[id];
+        const double* g = gw + k * per;
+        double v;
+        for (int level = 0;; ++level) {
+            const int q = s >> (L - level), mid = (q << (L - level)) + (1 << (L - level - 1));
+            v = 0.5 * (lo + hi) + g[3 * ((1 << level) - 1 + q) + id];
+            if (s == mid) break;
+            if (s < mid) hi = v;
+            else lo = v;
+        }
+        reinterpret_cast<double*>(prop + b0 + (s0 + s < P ? s0 + s : s0 + s - P))[id] = v;
+    }
+}
+
+// The linear family (atoms and at most one linear rotor): a group of GW lanes per segment.  GW of 32
+// or 64 keeps a segment within a wave (two share one), so that nothing waits on a barrier and what
+// does not grow with the partners (level sums, tests) costs one wave; GW of 128 or 256 spreads one
+// segment over waves, for the few segments of a single chain.  Per segment LDS holds the mover's
+// midpoints, the rotor terms and, in the pair precision, the S-1 inner slots of every atom: 12 bytes
+// a bead in FP32.  A move sums Delta V of its levels in chunks, each one pass over (midpoint,
+// partner) and one reduction: a chunk's midpoints share the group, GW over a power of two lanes each.
+
+// bytes of one segment in LDS (nwf, nhf, part, th, rt, win of k_bisect, in that order)
+__host__ __device__ constexpr int bisect_seg_bytes(int N, int S, int rsize) {
+    return (8 * rsize * (S - 1) + 8 * (16 + 16) + rsize * (2 * (S - 1) + 3 * N * (S - 1)) + 15) & ~15;
+}
+
+// Sum of V(new) - V(old) over U partners of an atom at one slot, from the separations
+// d[0 .. U-1] (new position) and d[U .. 2U-1] (old); the first `ok` partners count
+template <typename R, bool UT, int U>
+__device__ __forceinline__ double atom_terms(const Lut1D<R>& l1, const void* kn, const R (&d)[2 * U][3], int ok) {
+    R r[2 * U], v[2 * U];
+#pragma unroll
+    for (int i = 0; i < 2 * U; ++i) {
+        if constexpr (UT) r[i] = fast_sqrt(dot3(d[i][0], d[i][1], d[i][2], d[i][0], d[i][1], d[i][2]));
+        else r[i] = fast_sqrt(d[i][0] * d[i][0] + d[i][1] * d[i][1] + d[i][2] * d[i][2]);
+    }
+    if constexpr (UT) {
+        spot1d_u2_many<2 * U>(l1, static_cast<const float2*>(kn), r, v);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2 * U; ++i) v[i] = spot1d<R>(l1, static_cast<const vec4_t<R>*>(kn), r[i]);
+    }
+    double acc = 0.0;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const double t = (double)v[i] - (double)v[U + i];
+        acc += i < ok ? t : 0.0;
+    }
+    return acc;
+}
+
+// MI: built for contexts that hold a replica under the minimum image (its pairs then take their
+// nearest image); without it the kernels carry no trace of it.  UT: FP32 on uniform 1D and 2D
+// tables, knots staged as (y, y'') pairs.
+template <typename R, bool MI, bool UT, int GW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bisect(
+    const Rep* __restrict__ reps, Mut* __restrict__ mut, double4* __restrict__ beads, const RotBead* __restrict__ rotb,
+    Tables T, const double4* __restrict__ prop, const int2* __restrict__ work, Run run) {
+    extern __shared__ double smem[];
+    using P4 = vec4_t<R>;
+    const int2 wk = work[blockIdx.x];
+    const Rep& rp = reps[wk.x];
+    const int S = rp.S, P = rp.P, N = rp.natoms, lgS = 31 - __clz(S), S1 = S - 1;
+    if (run.u >= (run.ref_order ? P : S)) return;
+    const int gl = (int)threadIdx.x & (GW - 1);
+    const Lut1D<R> l1 = lut1d<R>(T, rp.pot1d_id);
+    const Lut2D<R> l2 = lut2d<R>(T, rp.pot2d_id);
+    const double* box = MI && rp.minimage ? rp.box : nullptr;  // MINIMAGE (not with a rotating linear rotor)
+    // the 1D knots, shared by the block's segments
+    P4* kn = reinterpret_cast<P4*>(smem);
+    int kbytes = l1.n * (int)sizeof(P4);
+    if constexpr (UT) {
+        float2* k2 = reinterpret_cast<float2*>(kn);
+        for (int i = threadIdx.x; i < l1.n; i += blockDim.x) k2[i] = make_float2((float)l1.k[i].y, (float)l1.k[i].z);
+        kbytes = (l1.n * (int)sizeof(float2) + 15) & ~15;
+    } else {
+        for (int i = threadIdx.x; i < l1.n; i += blockDim.x) kn[i] = l1.k[i];
+    }
+    __syncthreads();
+    const int seg = wk.y + (int)threadIdx.x / GW;
+    if (seg >= (run.ref_order ? 1 : P / S)) return;  // no segment for this group: it leaves whole
+    const int s0 = run.ref_order ? run.u : run.u + seg * S;
+    char* mem = reinterpret_cast<char*>(smem) + kbytes +
+                ((int)threadIdx.x / GW) * bisect_seg_bytes(N, S, (int)sizeof(R));
+    P4* nwf = reinterpret_cast<P4*>(mem);                // the move's new midpoints, pair precision
+    P4* nhf = nwf + S1;                                  // rotor axes
+    double* part = reinterpret_cast<double*>(nhf + S1);  // partial sums of a chunk, two buffers of 8
+    double* th = part + 16;                              // level tests of this move and the next, 8 each
+    R* rt = reinterpret_cast<R*>(th + 16);               // rotor terms (new, old) of every midpoint
+    R* win = rt + 2 * S1;                                // [slot - 1][atom][3]
+    for (int i = gl; i < N << lgS; i += GW) {
+        const int w = i & S1, a = i >> lgS;
+        if (w == 0) continue;
+        const int it = s0 + w < P ? s0 + w : s0 + w - P;
+        const double4 b = bead(beads, rp, a, it);
+        R* d = win + ((w - 1) * N + a) * 3;
+        d[0] = (R)b.x;
+        d[1] = (R)b.y;
+        d[2] = (R)b.z;
+    }
+    for (int w = gl; w < S1; w += GW) {
+        double x, y, z;
+        rotor_axis(rotb, rp, s0 + 1 + w < P ? s0 + 1 + w : s0 + 1 + w - P, x, y, z);
+        P4 q;
+        q.x = (R)x;  // the pair functions take the axis in the pair precision
+        q.y = (R)y;
+        q.z = (R)z;
+        q.w = (R)0;
+        nhf[w] = q;
+    }
+
+    const bool has_rotor = rp.lin_atom >= 0;  // then the last atom
+    const int nat = has_rotor ? N - 1 : N;    // atoms
+    const double tau = rp.tau;
+    unsigned long long evals = 0;
+    int pb = 0;  // buffer of the next partial sums
+    const int tend = run.type_end < rp.ntypes ? run.type_end : rp.ntypes;
+
+    for (int ty = run.type_begin; ty < tend; ++ty) {
+        const int L = rp.tlev[ty];
+        const int nm = (1 << L) - 1;
+        unsigned acc_n = 0;
+        // slot gl + 1 of the mover on lane gl: its proposal in registers from one move ahead until
+        // it is accepted.  (Moves of more midpoints than lanes read the others where they need them.)
+        const int itl = s0 + 1 + gl < P ? s0 + 1 + gl : s0 + 1 + gl - P;
+        long long ib = rp.bead_off + (long long)rp.tbegin[ty] * P;
+        auto proposal = [&](int i) { return prop[ib + (s0 + 1 + i < P ? s0 + 1 + i : s0 + 1 + i - P)]; };
+        auto put = [&](int i, const double4& v, int buf) {
+            P4 q;
+            q.x = (R)v.x;
+            q.y = (R)v.y;
+            q.z = (R)v.z;
+            q.w = (R)0;
+            nwf[i] = q;
+            if (i < L) th[8 * buf + i] = v.w;
+        };
+        double4 cur = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (gl < nm) cur = prop[ib + itl];
+        group_sync<GW>();
+        for (int i = gl; i < nm; i += GW) put(i, i == gl ? cur : proposal(i), 0);
+        group_sync<GW>();
+        for (int ia = 0; ia < rp.tnumb[ty]; ++ia) {
+            const int a = rp.tbegin[ty] + ia;
+            const double* tst = th + 8 * (ia & 1);  // this move's level tests
+            double4 nxt = cur;
+            if (gl < nm && ia + 1 < rp.tnumb[ty]) nxt = prop[ib + P + itl];
+            auto level_sums = [&](auto mi_c) -> bool {
+                // the minimum image as its own instance of the loops, so the plain one is unchanged
+                const double* bx = decltype(mi_c)::value ? box : nullptr;
+                const bool rot_a = a == rp.lin_atom;
+                // the terms with the rotor of every midpoint, new and old on neighbouring lanes: one
+                // pass of that code per move.  On uniform FP32 tables the table loads fly while the
+                // first chunk's atom terms run
+                const bool rterms = has_rotor && !rot_a;
+                auto slot_of = [&](int m) {  // of midpoint m, level-major order
+                    const int level = 31 - __clz(m + 1), q = m + 1 - (1 << level);
+                    return (q << (L - level)) + (1 << (L - level - 1)) - 1;
+                };
+                // separation from the rotor at midpoint i / 2, of the new (even i) or old position
+                auto to_rotor = [&](int i, R (&d)[3], P4& ax) {
+                    const int slot = slot_of(i >> 1);
+                    const R* pr = win + (slot * N + N - 1) * 3;
+                    const R* po = win + (slot * N + a) * 3;
+                    const P4 pn = nwf[slot];
+                    ax = nhf[slot];
+                    d[0] = nearest_image((i & 1 ? po[0] : pn.x) - pr[0], bx, 0);
+                    d[1] = nearest_image((i & 1 ? po[1] : pn.y) - pr[1], bx, 1);
+                    d[2] = nearest_image((i & 1 ? po[2] : pn.z) - pr[2], bx, 2);
+                };
+                RotorCell rc{};
+                const bool early = UT && 2 * nm <= GW;
+                if (rterms)
+                    for (int i = gl; i < 2 * nm; i += GW) {
+                        R d[3];
+                        P4 ax;
+                        to_rotor(i, d, ax);
+                        if constexpr (UT) {
+                            rc = rotor_pair_load(l2, false, d[0], d[1], d[2], ax.x, ax.y, ax.z);
+                            if (!early) rt[i] = rotor_pair_value(rc);
+                        } else {
+                            rt[i] = pair_d<R>(l1, kn, l2, false, true, d[0], d[1], d[2], (double)ax.x, (double)ax.y,
+                                              (double)ax.z);
+                        }
+                    }
+                double cum = 0.0;
+                bool alive = true;
+                for (int l0 = 0; l0 < L;) {
+                    // levels [l0, l1) in this pass: the first three together, then one at a time.
+                    // Terms of levels behind a rejection are a fifth of all on the 256-replica scan
+                    // (half on 8 atoms) and cost less than a pass and a reduction per level: 5.5
+                    // against 6.2 ms per pass there, 1.31 against 1.55 on a single 64-atom chain
+                    const int l1e = l0 > 0 ? l0 + 1 : (L < 3 ? L : 3);
+                    const int m0 = (1 << l0) - 1, nmc = (1 << l1e) - 1 - m0;
+                    // lanes per midpoint: the chunk's midpoints rounded up to a power of two
+                    const int lgn = l0 > 0 ? l0 : (l1e == 1 ? 0 : l1e);
+                    const int G = GW >> lgn > 0 ? GW >> lgn : 1;
+                    if (alive) {
+                        const int lgG = 31 - __clz(G);
+                        const int jl = gl & (G - 1);
+                        double acc = 0.0;
+                        for (int mc = gl >> lgG; mc < nmc; mc += GW >> lgG) {
+                            const int slot = slot_of(m0 + mc);
+                            const P4 pn = nwf[slot];
+                            const R* po = win + (slot * N + a) * 3;
+                            const R xa = po[0], ya = po[1], za = po[2];
+                            const R* ws = win + slot * N * 3;
+                            if (rot_a) {  // the rotor's partners are the atoms before it
+                                const P4 ax = nhf[slot];
+                                for (int j = jl; j < nat; j += G) {
+                                    const R* pj = ws + 3 * j;
+                                    const R dx = nearest_image(pn.x - pj[0], bx, 0), dy = nearest_image(pn.y - pj[1], bx, 1),
+                                            dz = nearest_image(pn.z - pj[2], bx, 2);
+                                    const R ex = nearest_image(xa - pj[0], bx, 0), ey = nearest_image(ya - pj[1], bx, 1),
+                                            ez = nearest_image(za - pj[2], bx, 2);
+                                    R vn, vo;
+                                    if constexpr (UT) {
+                                        const RotorCell kn_ = rotor_pair_load(l2, true, dx, dy, dz, ax.x, ax.y, ax.z);
+                                        const RotorCell ko_ = rotor_pair_load(l2, true, ex, ey, ez, ax.x, ax.y, ax.z);
+                                        vn = rotor_pair_value(kn_);
+                                        vo = rotor_pair_value(ko_);
+                                    } else {
+                                        const double nx = ax.x, ny = ax.y, nz = ax.z;
+                                        vn = pair_d<R>(l1, kn, l2, true, false, dx, dy, dz, nx, ny, nz);
+                                        vo = pair_d<R>(l1, kn, l2, true, false, ex, ey, ez, nx, ny, nz);
+                                    }
+                                    acc += (double)vn - (double)vo;
+                                }
+                            } else {
+                                auto partners = [&](auto u_c) {
+                                    constexpr int U = decltype(u_c)::value;
+                                    for (int jp = jl; jp < nat - 1; jp += U * G) {
+                                        R d[2 * U][3];
+#pragma unroll
+                                        for (int i = 0; i < U; ++i) {
+                                            const int jn = i == 0 || jp + i * G < nat - 1 ? jp + i * G : jp;
+                                            const R* pj = ws + 3 * (jn + (jn >= a));
+                                            const R x = pj[0], y = pj[1], z = pj[2];
+                                            d[i][0] = nearest_image(pn.x - x, bx, 0);
+                                            d[i][1] = nearest_image(pn.y - y, bx, 1);
+                                            d[i][2] = nearest_image(pn.z - z, bx, 2);
+                                            d[U + i][0] = nearest_image(xa - x, bx, 0);
+                                            d[U + i][1] = nearest_image(ya - y, bx, 1);
+                                            d[U + i][2] = nearest_image(za - z, bx, 2);
+                                        }
+                                        acc += atom_terms<R, UT, U>(l1, kn, d, U == 1 || jp + G < nat - 1 ? U : 1);
+                                    }
+                                };
+                                // partners in pairs, so that four look-ups of a lane interleave,
+                                // where most lanes have two or more
+                                if (UT && 2 * (nat - 1) > 3 * G) partners(std::integral_constant<int, 2>{});
+                                else partners(std::integral_constant<int, 1>{});
+                            }
+                        }
+                        if (rterms) {
+                            if constexpr (UT)
+                                if (l0 == 0 && early && gl < 2 * nm)
+                                    rt[gl] = rotor_pair_value(rc);
+                            if (l0 == 0) group_sync<GW>();
+                            // a midpoint's rotor terms on one of its lanes
+                            if (jl == 0)
+                                for (int mc = gl >> lgG; mc < nmc; mc += GW >> lgG)
+                                    acc += (double)rt[2 * (m0 + mc)] - (double)rt[2 * (m0 + mc) + 1];
+                        }
+                        // partial sums of up to 64 lanes of one midpoint (of the whole group when it
+                        // has more midpoints than lanes), added in order by every lane
+                        const int Gr = lgn > 3 ? (GW < 64 ? GW : 64) : (G < 64 ? G : 64);
+                        acc = group_sum(acc, Gr);
+                        double* pt = part + 8 * pb;
+                        pb ^= 1;
+                        if ((gl & (Gr - 1)) == 0) pt[gl / Gr] = acc;
+                        group_sync<GW>();
+                        evals += 2ull * (unsigned)(nmc * (N - 1));
+                        // sum over all points up to a level; level acceptance of mc_piqmc.cc:263-273
+                        const int per_m = G / Gr > 0 ? G / Gr : 1, np_all = GW / Gr;
+                        for (int level = l0, i = 0; level < l1e; ++level) {
+                            const double prev = cum;
+                            const int i1 = l0 > 0 ? np_all : i + (per_m << level);
+                            for (; i < i1; ++i) cum += pt[i];
+                            const double deltav = (cum - 2.0 * prev) * (tau * (double)(1 << (L - level - 1)));
+                            alive = alive && (deltav < 0.0 || deltav < tst[level]);
+                        }
+                    }
+                    if (GW >= 64 ? !alive : !__any(alive)) break;
+                    l0 = l1e;
+                }
+                return alive;
+            };
+            bool accepted;
+            if constexpr (MI) accepted = box ? level_sums(std::true_type{}) : level_sums(std::false_type{});
+            else accepted = level_sums(std::false_type{});
+            // the next move's midpoints and level tests; its loads are waited for here, before an
+            // accepted move's stores, which share the wait counter
+            if (ia + 1 < rp.tnumb[ty] && gl < nm) put(gl, nxt, (ia + 1) & 1);
+            if (accepted) {  // the new midpoints into the window and, in FP64, to HBM
+                acc_n += 1;
+                for (int i = gl; i < nm; i += GW) {
+                    const double4 v = i == gl ? cur : proposal(i);
+                    R* d = win + (i * N + a) * 3;
+                    d[0] = (R)v.x;
+                    d[1] = (R)v.y;
+                    d[2] = (R)v.z;
+                    beads[ib + (s0 + 1 + i < P ? s0 + 1 + i : s0 + 1 + i - P)] = make_double4(v.x, v.y, v.z, 0.0);
+                }
+            }
+            ib += P;
+            if (ia + 1 < rp.tnumb[ty])
+                for (int i = gl + GW; i < nm; i += GW) put(i, proposal(i), (ia + 1) & 1);
+            cur = nxt;
+            group_sync<GW>();
+        }
+        if (gl == 0) {
+            atomicAdd(&mut[wk.x].total[ty][1], (unsigned long long)rp.tnumb[ty]);
+            atomicAdd(&mut[wk.x].accep[ty][1], (unsigned long long)acc_n);
+        }
+    }
+    if (gl == 0) atomicAdd(&mut[wk.x].pair_evals[0], evals);
+}
+
+// Non-linear rotors: one workgroup per segment, its window of all atoms' beads and of the rotors'
+// frames in LDS, every level's items (midpoint, partner) over the block.
 // The window of all atoms' positions on the segment's S+1 slots is held in the pair precision
-// (float4 in FP32 runs, double4 in FP64 runs); new positions are built in FP64 from FP64 end
-// points, and accepted ones go to HBM in FP64 at once.  blockDim a multiple of 64.
-// FAM 1 (non-linear rotors) adds the rotors' frames at the window's slots: fr [nrot*(S+1)].
+// (float4 in FP32 runs, double4 in FP64 runs); new positions come from prop, one atom ahead, and
+// accepted ones go to HBM in FP64 at once.  blockDim a multiple of 64.  The rotors' frames at the
+// window's slots: fr [nrot*(S+1)].
 // MI: built for contexts that hold a replica under the minimum image (its pairs then take their
 // nearest image); without it the kernels carry no trace of it
-template <typename R, int FAM, bool MI>
-__device__ __forceinline__ void bisect_body(const Rep* __restrict__ reps, Mut* __restrict__ mut,
-                                            double4* __restrict__ beads, const RotBead* __restrict__ rotb,
-                                            const Frame* __restrict__ frames, Tables T, Tables3 T3,
-                                            const int2* __restrict__ work, Run run) {
+template <typename R, bool MI>
+__global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps, Mut* __restrict__ mut,
+                                                   double4* __restrict__ beads, const RotBead* __restrict__ rotb,
+                                                   const Frame* __restrict__ frames, Tables T, Tables3 T3,
+                                                   const double4* __restrict__ prop, const int2* __restrict__ work, Run run) {
     extern __shared__ double smem[];
     __shared__ double red[16];
     const int2 wk = work[blockIdx.x];
@@ -128,34 +557,23 @@ __device__ __forceinline__ void bisect_body(const Rep* __restrict__ reps, Mut* _
     }
     const int W = S + 1;
     using P4 = vec4_t<R>;
-    // LDS: the moving atom's new positions and its draws (FP64), then in the pair precision the
-    // window of all atoms' positions (x, y, z, -), the new midpoints again (one read per item)
-    // and the rotor axes at the window's slices, then rotor frames (FAM 1) and the 1D spline
-    // knots: (y, y'') pairs of uniform FP32 knots (linear family), vec4 knots otherwise
-    double* nw = smem;
-    double* gw = nw + 3 * W;  // draws of a batch of atoms: per atom 3 per midpoint, then one per level
-    P4* win = reinterpret_cast<P4*>(smem + ((3 * W + bisect_ring(W) + 3) & ~3));
+    // LDS: the level tests of this move and the next, then in the pair precision the window of all
+    // atoms' positions (x, y, z, -) and the mover's new midpoints, then the rotor frames and the 1D
+    // spline knots
+    double* th = smem;
+    P4* win = reinterpret_cast<P4*>(smem + 16);
     P4* nwf = win + N * W;
-    P4* nhf = nwf + W;
-    Frame* fr = reinterpret_cast<Frame*>(nhf + W);
-    const int nfr = FAM == 1 ? rp.nrot * W : 0;
+    Frame* fr = reinterpret_cast<Frame*>(nwf + W);
+    const int nfr = rp.nrot * W;
     P4* kn = reinterpret_cast<P4*>(fr + nfr);
     const Lut1D<R> l1 = lut1d<R>(T, rp.pot1d_id);
-    const Lut2D<R> l2 = lut2d<R>(T, rp.pot2d_id);
-    const Lut3D<R> l3 = lut3d<R>(T3, FAM == 1 ? rp.pot3d_id : -1);
-    const bool half_knots = FAM == 0 && is_fp32<R>() && l1.uniform;
-    const double* box = MI && rp.minimage ? rp.box : nullptr;  // MINIMAGE (not with a rotating linear rotor)
-    if (half_knots) {
-        float2* k2 = reinterpret_cast<float2*>(kn);
-        for (int i = tid; i < l1.n; i += nth) k2[i] = make_float2((float)l1.k[i].y, (float)l1.k[i].z);
-    } else {
-        for (int i = tid; i < l1.n; i += nth) kn[i] = l1.k[i];
+    const Lut3D<R> l3 = lut3d<R>(T3, rp.pot3d_id);
+    const double* box = MI && rp.minimage ? rp.box : nullptr;  // MINIMAGE
+    for (int i = tid; i < l1.n; i += nth) kn[i] = l1.k[i];
+    for (int i = tid; i < nfr; i += nth) {
+        const int q = i / W, w = i - q * W;
+        fr[i] = frame_at(frames, rp, rp.nl_atom + q, (s0 + w) % P);
     }
-    if constexpr (FAM == 1)
-        for (int i = tid; i < nfr; i += nth) {
-            const int q = i / W, w = i - q * W;
-            fr[i] = frame_at(frames, rp, rp.nl_atom + q, (s0 + w) % P);
-        }
     for (int i = tid; i < N * W; i += nth) {
         const int a = i / W, w = i - a * W;
         const double4 b = bead(beads, rp, a, (s0 + w) % P);
@@ -166,19 +584,8 @@ __device__ __forceinline__ void bisect_body(const Rep* __restrict__ reps, Mut* _
         q.w = (R)0;
         win[i] = q;
     }
-    for (int w = tid; w < W; w += nth) {
-        double x, y, z;
-        rotor_axis(rotb, rp, (s0 + w) % P, x, y, z);
-        P4 q;
-        q.x = (R)x;  // the pair functions take the axis in the pair precision
-        q.y = (R)y;
-        q.z = (R)z;
-        q.w = (R)0;
-        nhf[w] = q;
-    }
     __syncthreads();
 
-    const uint32_t pass = mut[wk.x].pass;
     unsigned long long evals = 0;
     unsigned long long tot[MAXT] = {0, 0, 0, 0}, acc_n[MAXT] = {0, 0, 0, 0};
     const int tend = run.type_end < rp.ntypes ? run.type_end : rp.ntypes;
@@ -186,175 +593,103 @@ __device__ __forceinline__ void bisect_body(const Rep* __restrict__ reps, Mut* _
     for (int ty = run.type_begin; ty < tend; ++ty) {
         const int L = rp.tlev[ty];
         const int St = 1 << L;
-        const double bnorm = 1.0 / (rp.lambda[ty] * rp.tau);
         const int nm = St - 1;
-        const int per = 3 * nm + L;  // draws of one atom's move
-        const int K = per <= BIS_RING ? (nth < BIS_RING ? nth : BIS_RING) / per : 1;  // atoms per draw batch
-        // end points of an atom's segment (slots 0 and St) in FP64 from HBM (no move of this launch
-        // changes them), loaded one atom ahead on the three coordinate lanes
-        double e0 = 0.0, e1 = 0.0;
-        if (tid < 3 && rp.tnumb[ty] > 0) {
-            const int a = rp.tbegin[ty];
-            const double4 b0 = bead(beads, rp, a, s0 % P), b1 = bead(beads, rp, a, (s0 + St) % P);
-            e0 = tid == 0 ? b0.x : (tid == 1 ? b0.y : b0.z);
-            e1 = tid == 0 ? b1.x : (tid == 1 ? b1.y : b1.z);
-        }
+        // slot tid + 1 of the mover on lane tid: its proposal in registers from one move ahead until
+        // it is accepted
+        long long ib = rp.bead_off + (long long)rp.tbegin[ty] * P;
+        auto put = [&](int i, const double4& v, int buf) {
+            P4 q;
+            q.x = (R)v.x;
+            q.y = (R)v.y;
+            q.z = (R)v.z;
+            q.w = (R)0;
+            nwf[i + 1] = q;
+            if (i < L) th[8 * buf + i] = v.w;
+        };
+        auto proposal = [&](int i) { return prop[ib + (s0 + 1 + i) % P]; };
+        double4 cur = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (tid < nm) cur = proposal(tid);
+        for (int i = tid; i < nm; i += nth) put(i, i == tid ? cur : proposal(i), 0);
+        lds_barrier();
         for (int ia = 0; ia < rp.tnumb[ty]; ++ia) {
             const int a = rp.tbegin[ty] + ia;
-            const int kk = ia % K;
-            if (kk == 0) {
-                // every draw of the next K moves at once: Gaussians of midpoint m (level-major
-                // order) and the level acceptance uniforms u, kept as -log(u): the level test
-                // exp(-dV) > u (mc_piqmc.cc:265-273) is then dV < -log(u), a comparison
-                const int nk = rp.tnumb[ty] - ia < K ? rp.tnumb[ty] - ia : K;
-                for (int i = tid; i < nk * per; i += nth) {
-                    const int k = i / per, d = i - k * per;
-                    const uint32_t ab = (uint32_t)(a + k);
-                    if (d < 3 * nm) {
-                        int m = d / 3, id = d - 3 * m;
-                        int level = 31 - __clz(m + 1);
-                        int q = m + 1 - (1 << level);
-                        uint4 w4 = draw(run.seed, rp.key, pass, K_BISECT, 0, ab, (uint32_t)s0,
-                                        ((uint32_t)level << 24) | ((uint32_t)q << 8) | (uint32_t)id);
-                        gw[i] = gauss_from(w4, bnorm / (double)(1 << (L - level)));
-                    } else {
-                        int level = d - 3 * nm;
-                        uint4 w4 = draw(run.seed, rp.key, pass, K_BISECT, 0, ab, (uint32_t)s0,
-                                        ((uint32_t)level << 24) | (0xFFFFu << 8));
-                        gw[i] = -log(u53(w4.x, w4.y));
-                    }
-                }
-            }
-            const double* g = gw + kk * per;  // this move's draws
-            if (tid < 3) {
-                nw[tid] = e0;
-                nw[3 * St + tid] = e1;
-                if (ia + 1 < rp.tnumb[ty]) {  // the next atom's end points, used one move later
-                    const double4 b0 = bead(beads, rp, a + 1, s0 % P), b1 = bead(beads, rp, a + 1, (s0 + St) % P);
-                    e0 = tid == 0 ? b0.x : (tid == 1 ? b0.y : b0.z);
-                    e1 = tid == 0 ? b1.x : (tid == 1 ? b1.y : b1.z);
-                }
-            }
-            if (kk == 0) __syncthreads();  // the batch's draws are visible to every lane
+            const double* tst = th + 8 * (ia & 1);  // this move's level tests
+            double4 nxt = cur;
+            if (tid < nm && ia + 1 < rp.tnumb[ty]) nxt = prop[ib + P + (s0 + 1 + tid) % P];
             double cum = 0.0;
             bool accepted = false;
             for (int level = 0; level < L; ++level) {
                 const int lss = 1 << (L - level);
                 const int half = lss >> 1;
                 const int nmid = 1 << level;
-                // new midpoints: slot = half + q*lss, from the current new end points
-                for (int i = tid; i < 3 * nmid; i += nth) {
-                    int q = i / 3, id = i - 3 * q;
-                    int slot = half + q * lss;
-                    const double v = 0.5 * (nw[3 * (slot - half) + id] + nw[3 * (slot + half) + id]) +
-                                     g[3 * (nmid - 1 + q) + id];
-                    nw[3 * slot + id] = v;
-                    reinterpret_cast<R*>(nwf + slot)[id] = (R)v;
-                }
-                __syncthreads();
                 // Delta V at the new midpoints: items (midpoint, partner)
                 const int np = N - 1;
                 const int items = nmid * np;
-                const bool rot_a = FAM == 1 ? (rp.nl_atom >= 0 && a >= rp.nl_atom) : (a == rp.lin_atom);
-                // an atom with the linear rotor last among its partners: the atom-atom terms and
-                // the rotor terms in one index space, rotor terms last, so a wave runs one
-                // table's code except at the seam
-                const bool split = FAM == 0 && !rot_a && rp.lin_atom == N - 1;
-                auto item_sum = [&](auto half_c, auto mi_c) -> double {
-                    constexpr bool H = decltype(half_c)::value;
+                const bool rot_a = a >= rp.nl_atom;
+                auto item_sum = [&](auto mi_c) -> double {
                     // the minimum image as its own instance of the loop, so the plain one is unchanged
                     const double* bx = decltype(mi_c)::value ? box : nullptr;
-                    // (that instance takes every pair through the general branch)
-                    const bool spl = !decltype(mi_c)::value && split;
                     double acc = 0.0;
-                    // item i = (midpoint qa, partner index jp) with den partners per midpoint in
-                    // the atom range; a lane's items advance by nth, so (qa, jp) is carried
-                    // along with one division per level
-                    const int den = spl ? np - 1 : np;
-                    const int n1 = spl ? nmid * den : items;  // items of the atom range
-                    const int dd = den > 0 ? den : 1;
+                    // item i = (midpoint q, partner index jp); a lane's items advance by nth, so
+                    // (q, jp) is carried along with one division per level
+                    const int dd = np > 0 ? np : 1;
                     const int dq = nth / dd, dj = nth - dq * dd;
-                    int qa = tid / dd, jp = tid - qa * dd;
+                    int q = tid / dd, jp = tid - q * dd;
                     for (int i = tid; i < items; i += nth) {
-                        int q, j;
-                        bool rj;
-                        if (i >= n1) {  // the rotor terms after the atom range (split)
-                            rj = true;
-                            q = i - n1;
-                            j = N - 1;
-                        } else {
-                            q = qa;
-                            j = jp + (jp >= a);
-                            rj = spl ? false
-                                       : (FAM == 1 ? (rp.nl_atom >= 0 && j >= rp.nl_atom) : (j == rp.lin_atom));
-                        }
+                        const int j = jp + (jp >= a);
+                        const bool rj = j >= rp.nl_atom;
+                        const int slot = half + q * lss;
+                        const P4 pj = win[j * W + slot], pa = win[a * W + slot], pn = nwf[slot];
+                        const Frame& fa = fr[(rot_a ? a - rp.nl_atom : 0) * W + slot];
+                        const Frame& fj = fr[(rj ? j - rp.nl_atom : 0) * W + slot];
+                        acc += pair_nl<R>(l1, kn, l3, rot_a, rj, pn.x, pn.y, pn.z, pj.x, pj.y, pj.z, fa, fj, bx) -
+                               pair_nl<R>(l1, kn, l3, rot_a, rj, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, fa, fj, bx);
                         jp += dj;
-                        qa += dq;
+                        q += dq;
                         if (jp >= dd) {
                             jp -= dd;
-                            ++qa;
-                        }
-                        const int slot = half + q * lss;
-                        const P4 pj = win[j * W + slot], pa = win[a * W + slot];
-                        const P4 pn = nwf[slot];
-                        const R xn = pn.x, yn = pn.y, zn = pn.z;
-                        if constexpr (FAM == 1) {
-                            const Frame& fa = fr[(rot_a ? a - rp.nl_atom : 0) * W + slot];
-                            const Frame& fj = fr[(rj ? j - rp.nl_atom : 0) * W + slot];
-                            acc += pair_nl<R>(l1, kn, l3, rot_a, rj, xn, yn, zn, pj.x, pj.y, pj.z, fa, fj, bx) -
-                                   pair_nl<R>(l1, kn, l3, rot_a, rj, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, fa, fj, bx);
-                        } else if (spl) {
-                            if (rj) {
-                                const P4 ax = nhf[slot];
-                                const double nx = ax.x, ny = ax.y, nz = ax.z;
-                                acc += (double)pair_vr<R, H>(l1, kn, l2, false, true, xn, yn, zn, pj.x, pj.y, pj.z, nx, ny, nz, bx) -
-                                       (double)pair_vr<R, H>(l1, kn, l2, false, true, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, nx, ny, nz, bx);
-                            } else {
-                                acc += (double)pair_vr<R, H>(l1, kn, l2, false, false, xn, yn, zn, pj.x, pj.y, pj.z, 0.0, 0.0, 1.0, bx) -
-                                       (double)pair_vr<R, H>(l1, kn, l2, false, false, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, 0.0, 0.0, 1.0, bx);
-                            }
-                        } else {
-                            const P4 ax = nhf[slot];
-                            const double nx = ax.x, ny = ax.y, nz = ax.z;
-                            acc += (double)pair_vr<R, H>(l1, kn, l2, rot_a, rj, xn, yn, zn, pj.x, pj.y, pj.z, nx, ny, nz, bx) -
-                                   (double)pair_vr<R, H>(l1, kn, l2, rot_a, rj, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, nx, ny, nz, bx);
+                            ++q;
                         }
                     }
                     return acc;
                 };
-                using T1 = std::integral_constant<bool, true>;
-                using F1 = std::integral_constant<bool, false>;
                 double acc;
                 if constexpr (MI)
-                    acc = half_knots ? (box ? item_sum(T1{}, T1{}) : item_sum(T1{}, F1{}))
-                                     : (box ? item_sum(F1{}, T1{}) : item_sum(F1{}, F1{}));
+                    acc = box ? item_sum(std::integral_constant<bool, true>{}) : item_sum(std::integral_constant<bool, false>{});
                 else
-                    acc = half_knots ? item_sum(T1{}, F1{}) : item_sum(F1{}, F1{});
-                acc = block_sum(acc, red);
+                    acc = item_sum(std::integral_constant<bool, false>{});
+                acc = block_sum_lds(acc, red);
                 evals += 2ull * (unsigned long long)items;
                 // sum over all points up to this level; level acceptance of mc_piqmc.cc:263-273
                 const double prev = cum;
                 cum += acc;
                 double deltav = (cum - 2.0 * prev) * (rp.tau * (double)half);
-                accepted = deltav < 0.0 || deltav < g[3 * nm + level];
+                accepted = deltav < 0.0 || deltav < tst[level];
                 if (!accepted) break;
             }
             tot[ty] += 1;
+            // the next move's midpoints and level tests; its loads are waited for here, before an
+            // accepted move's stores, which share the wait counter
+            if (ia + 1 < rp.tnumb[ty] && tid < nm) put(tid, nxt, (ia + 1) & 1);
             if (accepted) {  // the new midpoints into the window and, in FP64, to HBM
                 acc_n[ty] += 1;
-                for (int i = tid; i < St - 1; i += nth) {
+                for (int i = tid; i < nm; i += nth) {
                     const int slot = 1 + i;
-                    const double x = nw[3 * slot], y = nw[3 * slot + 1], z = nw[3 * slot + 2];
+                    const double4 v = i == tid ? cur : proposal(i);
                     P4 q;
-                    q.x = (R)x;
-                    q.y = (R)y;
-                    q.z = (R)z;
+                    q.x = (R)v.x;
+                    q.y = (R)v.y;
+                    q.z = (R)v.z;
                     q.w = (R)0;
                     win[a * W + slot] = q;
-                    beads[rp.bead_off + (long long)a * P + (s0 + slot) % P] = make_double4(x, y, z, 0.0);
+                    beads[ib + (s0 + slot) % P] = make_double4(v.x, v.y, v.z, 0.0);
                 }
             }
-            __syncthreads();
+            ib += P;
+            if (ia + 1 < rp.tnumb[ty])
+                for (int i = tid + nth; i < nm; i += nth) put(i, proposal(i), (ia + 1) & 1);
+            cur = nxt;
+            lds_barrier();
         }
     }
     if (tid == 0) {
@@ -364,22 +699,6 @@ __device__ __forceinline__ void bisect_body(const Rep* __restrict__ reps, Mut* _
         }
         atomicAdd(&mut[wk.x].pair_evals[0], evals);
     }
-}
-
-// the linear family keeps four waves per SIMD; the non-linear family needs more registers
-template <typename R, bool MI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bisect(
-    const Rep* __restrict__ reps, Mut* __restrict__ mut, double4* __restrict__ beads, const RotBead* __restrict__ rotb,
-    Tables T, const int2* __restrict__ work, Run run) {
-    bisect_body<R, 0, MI>(reps, mut, beads, rotb, nullptr, T, Tables3{}, work, run);
-}
-
-template <typename R, bool MI>
-__global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps, Mut* __restrict__ mut,
-                                                   double4* __restrict__ beads, const RotBead* __restrict__ rotb,
-                                                   const Frame* __restrict__ frames, Tables T, Tables3 T3,
-                                                   const int2* __restrict__ work, Run run) {
-    bisect_body<R, 1, MI>(reps, mut, beads, rotb, frames, T, T3, work, run);
 }
 
 // ------------------------------------------------------------------------- linear rotor
