@@ -246,10 +246,13 @@ struct pimc_ctx {
     unsigned long long* d_xrec = nullptr;  // per part, its two boundary records (8 words each) as last published
     int nparts = 0, nflags = 0;
     int opt_rotor_part_slices = 0;  // most rotor slices per part, 0: from the LDS budget
-    int opt_rotor_lds_kb = 52;      // LDS budget of a rotor part (52 KB: three parts per CU)
+    int opt_rotor_lds_kb = 0;       // LDS budget of a rotor part, 0: by load
     int opt_centroid_parts = 0;     // target number of centroid parts, 0: from the capacity
     int centroid_target = 0;        // target the current centroid parts were planned with
     int rotor_lds_kb = 52;          // budget the current parts were planned with
+    int rotor_resident = 0;         // parts the device holds at once
+    bool rotor_uniform = false;     // the sweep's tables are uniform FP32 ones
+    bool rotor_long = false;        // a part has more than ROTOR_SLICES_MAX slices
     std::vector<int> rot_chains;    // replicas with a linear rotor, heaviest first
     RotPart* d_parts3 = nullptr;     // non-linear chains split by slice range
     unsigned* d_flags3 = nullptr;
@@ -317,6 +320,13 @@ static int fail(pimc_ctx* c, const std::string& m) {
         hipError_t e_ = (x);                                                               \
         if (e_ != hipSuccess) return fail(ctx, std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
+
+template <typename F>
+static void rotor_kernel(const pimc_ctx* c, F&& f) {  // the linear sweep's instance for this context
+    if (c->fp64) c->rotor_long ? f(k_rotor<double, false, ROTOR_MPL_LONG>) : f(k_rotor<double, false, 1>);
+    else if (c->rotor_long) f(k_rotor<float, false, ROTOR_MPL_LONG>);
+    else c->rotor_uniform ? f(k_rotor<float, true, 1>) : f(k_rotor<float, false, 1>);
+}
 
 extern "C" {
 
@@ -453,8 +463,15 @@ int pimc_add_rotdens(pimc_ctx* c, int n, const double* x, const double* rho, con
     t.x0 = gx[0];
     t.xmax = gx[n - 1];
     t.inv_h = (double)(n - 1) / (gx[n - 1] - gx[0]);
+    // the knots that the sweep stages: the last ROTOR_KNOTS, or fewer where the density has fallen to a
+    // millionth of its largest value
+    double top = 0.0;
+    for (double v : yr) top = std::max(top, std::fabs(v));
+    t.hot = n - 2;
+    while (t.hot > 0 && n - t.hot < ROTOR_KNOTS && std::fabs(yr[t.hot]) > 1e-6 * top) --t.hot;
+    t.pad = 0;
     for (int i = 0; i < n; ++i) {
-        c->rk.push_back(make_double4(gx[i], yr[i], s0[i], 0.0));
+        c->rk.push_back(make_double4(gx[i], yr[i], s0[i], i + 1 < n ? 1.0 / (gx[i + 1] - gx[i]) : 0.0));
         c->re.push_back(make_double4(ye[i], s1[i], ys[i], s2[i]));
     }
     c->tr.push_back(t);
@@ -747,19 +764,38 @@ static int plan_rotor_parts(pimc_ctx* c, int lds_kb) {
     HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
     constexpr int NXCD = 8;
     std::vector<RotorChain> chains;
+    c->rotor_uniform = !c->fp64;  // FP32 on uniform tables
+    for (int r : c->rot_chains)
+        if (c->rep[r].pot2d_id >= 0) c->rotor_uniform &= c->t2[c->rep[r].pot2d_id].uniform != 0;
     for (int r : c->rot_chains) chains.push_back(RotorChain{r, c->rep[r].Prot, c->rep[r].RotRatio, c->rep[r].natoms});
     // resident parts per CU at a launch's LDS size, as the runtime computes it for k_rotor
     auto occupancy = [&](size_t lds) {
         int occ = 0;
-        hipError_t e = c->fp64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_rotor<double>, 256, lds)
-                               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_rotor<float>, 256, lds);
+        hipError_t e = hipErrorUnknown;
+        rotor_kernel(c, [&](auto kernel) { e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, 256, lds); });
         return e == hipSuccess ? occ : 0;
     };
     std::vector<RotPart> parts;
     size_t lds_r = 0;
     std::string err;
-    if (plan_linear_rotor(chains, geo_bytes, lds_kb, c->opt_rotor_part_slices, prop.multiProcessorCount / NXCD, occupancy,
-                          parts, lds_r, err))
+    // parts of at most ROTOR_SLICES_MAX slices, or, where the option asks for more or a chain of those
+    // cannot be resident, as large as they have to be; the budget holds the kernel's own 9 KB too
+    auto plan = [&](int most) {
+        return plan_linear_rotor(chains, geo_bytes, std::max(1, lds_kb - 9), most, prop.multiProcessorCount / NXCD, occupancy,
+                                 parts, lds_r, err);
+    };
+    auto too_long = [&]() {
+        for (const RotPart& p : parts)
+            if (p.k1 - p.k0 > ROTOR_SLICES_MAX) return true;
+        return false;
+    };
+    c->rotor_long = false;
+    int rc = plan(c->opt_rotor_part_slices > 0 ? c->opt_rotor_part_slices : ROTOR_SLICES_MAX);
+    if (rc || too_long()) {
+        c->rotor_long = true;
+        rc = plan(c->opt_rotor_part_slices);
+    }
+    if (rc)
         return fail(c, err);
     const int nflags = (int)parts.size();
     parts = xcd_order(parts, [&](int r) {
@@ -777,6 +813,7 @@ static int plan_rotor_parts(pimc_ctx* c, int lds_kb) {
     c->nparts = (int)parts.size();
     c->rotor_lds_kb = lds_kb;
     if (parts.empty()) return 0;
+    c->rotor_resident = prop.multiProcessorCount * occupancy(lds_r);
     c->d_parts = dalloc<RotPart>(parts.size());
     c->d_flags = dalloc<unsigned>(nflags);
     c->d_xrec = dalloc<unsigned long long>(16 * (size_t)nflags);
@@ -1144,7 +1181,12 @@ int pimc_commit(pimc_ctx* c) {
         return (long long)a.P * a.Prot * a.natoms > (long long)b.P * b.Prot * b.natoms;
     });
     c->rot_chains = rotreps;
-    if (plan_rotor_parts(c, c->opt_rotor_lds_kb)) return -1;
+    // A part's share of LDS by load: 52 KB, or 78 KB when the parts of 52 KB are more than the device
+    // holds at once.  A chain's time is its half-sweeps in turn, and smaller parts shorten a half; but
+    // parts that wait for a CU lengthen the launch by whole sweeps.  Sweep per pass at 52 and 78 KB:
+    // 1.83 and 2.40 ms on one chain of 64 atoms, 1.15 and 1.45 on 23 mixed replicas, 5.3 and 4.8 on 256
+    if (plan_rotor_parts(c, c->opt_rotor_lds_kb ? c->opt_rotor_lds_kb : 52)) return -1;
+    if (!c->opt_rotor_lds_kb && c->rotor_resident < c->nflags && plan_rotor_parts(c, 78)) return -1;
     if (plan_centroid_parts(c, c->opt_centroid_parts)) return -1;
     c->nbeads = boff;
     c->nrotb = roff;
@@ -1652,14 +1694,20 @@ void launch_centroid(pimc_ctx* c, int type) {
                            c->d_cslots, c->ncflags, run);
 }
 
+void launch_rotor_parts(pimc_ctx* c, const Run& run) {
+    rotor_kernel(c, [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(c->nparts), dim3(256), c->lds_rotor, c->stream, c->d_rep, c->d_mut, c->d_beads,
+                           c->d_rotb, c->tables(), c->d_parts, c->d_flags, c->d_xrec, run);
+    });
+}
+
 template <typename R>
 void launch_rotor(pimc_ctx* c, int u) {
     if (c->nparts == 0 && c->nrot3 == 0 && c->nparts3 == 0) return;
     Run run{c->seed, u, c->ref_order ? 1 : 0, 0, 0};
     Timed t(c, "rotor");
     if (c->nparts)
-        hipLaunchKernelGGL(k_rotor<R>, dim3(c->nparts), dim3(256), c->lds_rotor, c->stream, c->d_rep, c->d_mut,
-                           c->d_beads, c->d_rotb, c->tables(), c->tables3(), c->d_parts, c->d_flags, c->d_xrec, run);
+        launch_rotor_parts(c, run);
     if (c->nparts3 && c->opt_da)
         hipLaunchKernelGGL(k_rotor3d_da<R>, dim3(c->nparts3), dim3(256), c->lds_parts3, c->stream, c->d_rep, c->d_mut,
                            c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_parts3, c->d_flags3,
@@ -1710,13 +1758,6 @@ void launch_centroid_all(pimc_ctx* c) {
                                c->d_mut, c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_cparts1,
                                c->d_cflags, c->d_cslots, c->ncflags, run);
     }
-}
-
-template <typename R>
-void launch_rotor_linear(pimc_ctx* c, int u) {
-    Run run{c->seed, u, c->ref_order ? 1 : 0, 0, 0};
-    hipLaunchKernelGGL(k_rotor<R>, dim3(c->nparts), dim3(256), c->lds_rotor, c->stream, c->d_rep, c->d_mut,
-                       c->d_beads, c->d_rotb, c->tables(), c->tables3(), c->d_parts, c->d_flags, c->d_xrec, run);
 }
 
 // Rotor sweep of start slice u and, beside it where it leaves CUs free, the proposals of the bisection of start slice u + 1
@@ -1900,8 +1941,7 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
                     break;
                 }
                 const double t = timed([&](int u) {
-                    if (c->fp64) launch_rotor_linear<double>(c, u);
-                    else launch_rotor_linear<float>(c, u);
+                    launch_rotor_parts(c, Run{c->seed, u, c->ref_order ? 1 : 0, 0, 0});
                 });
                 if (t >= 0.0 && (tbest < 0.0 || t < tbest)) {
                     tbest = t;

@@ -84,6 +84,7 @@ struct Tab2D {
 };
 struct TabRot {
     int n, off;
+    int hot, pad;  // knots from here to the end hold the links a chain meets (see rot_rho_hot)
     double x0, xmax, inv_h;
 };
 
@@ -104,7 +105,7 @@ struct Tables {
     const double* g2d;
     const float* g2f;
     const Tab2D* t2;
-    const double4* rk;  // x, rho, rho'', -
+    const double4* rk;  // x, rho, rho'', 1/(x[i+1]-x[i])
     const double4* re;  // erot, erot'', esq, esq''
     const TabRot* tr;
 };
@@ -460,6 +461,19 @@ __device__ __forceinline__ float rotor_pair_value(const RotorCell& k) {
     return lpot2d_u_lerp(k.q.x, k.q.y, k.q.z, k.q.w, k.wr, k.wc);
 }
 
+// the spline of SRotDens between knots a and b
+__device__ __forceinline__ double rho_between(const double4& a, const double4& b, double g) {
+    const double h = b.x - a.x;
+    const double A = (b.x - g) * a.w, B = (g - a.x) * a.w;
+    return A * a.y + B * b.y + ((A * A * A - A) * a.z + (B * B * B - B) * b.z) * (h * h) * (1.0 / 6.0);
+}
+
+__device__ __forceinline__ int rho_cell(const TabRot& t, double g) {
+    double f = floor((g - t.x0) * t.inv_h);
+    f = fmin(fmax(f, 0.0), (double)(t.n - 2));
+    return (int)f;
+}
+
 // SRotDens (mc_poten.cc:548-570) with the table descriptor already resolved: the last value
 // above the grid, the line through the first two knots below it, the spline inside.
 __device__ __forceinline__ double rot_rho(const Tables& T, const TabRot& t, double g) {
@@ -471,9 +485,7 @@ __device__ __forceinline__ double rot_rho(const Tables& T, const TabRot& t, doub
         double sb = (k0.y * k1.x - k1.y * k0.x) / (k1.x - k0.x);
         return sa * g + sb;
     }
-    double f = floor((g - t.x0) * t.inv_h);
-    f = fmin(fmax(f, 0.0), (double)(t.n - 2));
-    int i = (int)f;
+    int i = rho_cell(t, g);
     double4 a = k[i], b = k[i + 1];
     while (i > 0 && a.x > g) {
         --i;
@@ -485,53 +497,26 @@ __device__ __forceinline__ double rot_rho(const Tables& T, const TabRot& t, doub
         a = b;
         b = k[i + 1];
     }
-    double h = b.x - a.x;
-    double A = (b.x - g) / h, B = (g - a.x) / h;
-    return A * a.y + B * b.y + ((A * A * A - A) * a.z + (B * B * B - B) * b.z) * (h * h) / 6.;
+    return rho_between(a, b, g);
 }
 
-// rot_rho in two steps, so that its knot loads can be in flight with other loads: the knots of
-// the cell the grid arithmetic guesses, then the value (with the cell corrected if needed).
-struct RhoCell {
-    double4 a, b;
-    int i;
-};
-
-__device__ __forceinline__ RhoCell rot_rho_load(const Tables& T, const TabRot& t, double g) {
-    const double4* k = T.rk + t.off;
-    double f = floor((g - t.x0) * t.inv_h);
-    f = fmin(fmax(f, 0.0), (double)(t.n - 2));
-    RhoCell c;
-    c.i = (int)f;
-    c.a = k[c.i];
-    c.b = k[c.i + 1];
-    return c;
-}
-
-__device__ __forceinline__ double rot_rho_eval(const Tables& T, const TabRot& t, double g, RhoCell c) {
-    const double4* k = T.rk + t.off;
-    if (g > t.xmax) return k[t.n - 1].y;
-    if (g < t.x0) {
-        double4 k0 = k[0], k1 = k[1];
-        double sa = (k1.y - k0.y) / (k1.x - k0.x);
-        double sb = (k0.y * k1.x - k1.y * k0.x) / (k1.x - k0.x);
-        return sa * g + sb;
+// rot_rho at the two links of a move, with the table's knots t.hot .. n-1 staged in LDS (hk): the
+// density falls off within a few tenths of a radian, so the links of a chain stay among the knots
+// near cos(gamma) = 1, and a look-up there costs an LDS access instead of a trip to L2.  A wave with
+// a lane elsewhere (below the staged knots, or where the guessed cell is not the knots' own) takes
+// the general form.
+__device__ __forceinline__ void rot_rho_hot(const Tables& T, const TabRot& t, const double4* hk, double g0, double g1,
+                                            double& r0, double& r1) {
+    const int i0 = rho_cell(t, g0) - t.hot, i1 = rho_cell(t, g1) - t.hot;
+    const int j0 = i0 > 0 ? i0 : 0, j1 = i1 > 0 ? i1 : 0;
+    const double4 a0 = hk[j0], b0 = hk[j0 + 1], a1 = hk[j1], b1 = hk[j1 + 1];
+    const bool in0 = i0 >= 0 && a0.x <= g0 && g0 < b0.x, in1 = i1 >= 0 && a1.x <= g1 && g1 < b1.x;
+    r0 = rho_between(a0, b0, g0);
+    r1 = rho_between(a1, b1, g1);
+    if (!__all(in0 && in1)) {
+        if (!in0) r0 = rot_rho(T, t, g0);
+        if (!in1) r1 = rot_rho(T, t, g1);
     }
-    int i = c.i;
-    double4 a = c.a, b = c.b;
-    while (i > 0 && a.x > g) {
-        --i;
-        b = a;
-        a = k[i];
-    }
-    while (i < t.n - 2 && b.x <= g) {
-        ++i;
-        a = b;
-        b = k[i + 1];
-    }
-    double h = b.x - a.x;
-    double A = (b.x - g) / h, B = (g - a.x) / h;
-    return A * a.y + B * b.y + ((A * A * A - A) * a.z + (B * B * B - B) * b.z) * (h * h) / 6.;
 }
 
 // .rot spline in FP64 (x, f, f'') at column `col`: 0 rho, 1 erot, 2 esq.

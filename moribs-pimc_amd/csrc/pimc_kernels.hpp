@@ -10,12 +10,13 @@
 //                part's slices x partners, partials exchanged as numbered words in memory
 //                (MCMolecularMove mc_piqmc.cc:54-102).
 //   k_rotor      one workgroup per part of a linear rotor's chain (a range of slices): the part's
-//                orientations and its rotor-partner geometry live in LDS for all sweeps of a
+//                orientations and its rotor-partner geometry live on chip for all sweeps of a
 //                launch; each half of the even/odd checkerboard (mc_piqmc.cc:490-512) is a
-//                parallel step over slices, a lane group per slice sums Delta V over partners
-//                (MCRotLinStep :781-936); parts trade one boundary slice per half-sweep as a
-//                record of numbered words (each 64-bit word: the publishing half's number over
-//                32 bits of a double), so a poll of the record returns the data with its check.
+//                parallel step over slices (MCRotLinStep :781-936), tests on one or two waves
+//                and the partner energies of the next half's proposals on the others; parts
+//                trade one boundary slice per half-sweep as a record of numbered words (each
+//                64-bit word: the publishing half's number over 32 bits of a double), so a poll
+//                of the record returns the data with its check.
 //   k_est_tiles  one workgroup per (replica, tile of slices): the tile's part of the pair sum of
 //                GetPotEnergy_Densities (mc_estim.cc:500-687, every pair, with the g(r),
 //                g(r,theta) and (r,theta,chi) bins) and of GetKinEnergy (mc_estim.cc:876-937),
@@ -899,71 +900,92 @@ __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ 
     }
 }
 
-// Sum over a slice's partners of V(r, cos theta) with the rotor axis n: cos = -(n . dr)/r
-// (PotRotEnergy mc_piqmc.cc:1967-2044).  Items i = gl, gl+G, ... of the slice's geometry block,
-// loaded in batches of eight so their table lookups overlap.
-template <typename R>
-__device__ __forceinline__ double slice_energy(const Lut2D<R>& l2, const vec4_t<R>* pk, int items, int gl, int G,
-                                               double nx, double ny, double nz) {
-    constexpr int B = 8;  // partner look-ups in flight per lane
+// Sum over items i0, i0 + step, ... < items of a slice of V(r, cos theta) with the rotor axis n:
+// cos = -(n . dr)/r (PotRotEnergy mc_piqmc.cc:1967-2044), from the slice's geometry block g.  UT
+// (FP32 on a uniform table): g holds unit vectors and distances; the cells of a batch first, then
+// all its loads, then the lerps, so that the table look-ups of a lane fly together.
+template <typename R, bool UT, int B>
+__device__ __forceinline__ void pair_batch(const Lut2D<R>& l2, const vec4_t<R>* g, int i0, int step, int items, R fx, R fy,
+                                           R fz, double& acc) {
+    if constexpr (UT) {
+        int cell[B];
+        float wr[B], wc[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int i = i0 + b * step;
+            const float4 d = g[i < items ? i : i0];
+            const float c = -__builtin_fmaf(d.z, fz, __builtin_fmaf(d.y, fy, rounded_product(d.x, fx)));
+            lpot2d_u_cell(l2, d.w, c, cell[b], wr[b], wc[b]);
+        }
+        float4 q[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) q[b] = l2.vc[cell[b]];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const double v = (double)lpot2d_u_lerp(q[b].x, q[b].y, q[b].z, q[b].w, wr[b], wc[b]);
+            acc += i0 + b * step < items ? v : 0.0;
+        }
+    } else {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int i = i0 + b * step;
+            const vec4_t<R> d = g[i < items ? i : i0];
+            R c;
+            if constexpr (is_fp32<R>()) c = -(fx * d.x + fy * d.y + fz * d.z);
+            else c = -((fx * d.x + fy * d.y + fz * d.z) / d.w);
+            const double v = (double)lpot2d<R>(l2, d.w, c);
+            acc += i < items ? v : 0.0;
+        }
+    }
+}
+
+template <typename R, bool UT>
+__device__ __forceinline__ double pair_terms(const Lut2D<R>& l2, const vec4_t<R>* g, int i0, int step, int items, double nx,
+                                             double ny, double nz) {
     double acc = 0.0;
     const R fx = (R)nx, fy = (R)ny, fz = (R)nz;
-    if constexpr (is_fp32<R>()) {
-        if (l2.uniform) {  // all cells of a batch first, then all loads, then the lerps
-            for (int base = gl; base < items; base += B * G) {
-                int cell[B];
-                float wr[B], wc[B];
-#pragma unroll
-                for (int b = 0; b < B; ++b) {
-                    const int i = base + b * G;
-                    const float4 d = i < items ? pk[i] : make_float4(0.f, 0.f, 1.f, 1.f);
-                    lpot2d_u_cell(l2, d.w, -(fx * d.x + fy * d.y + fz * d.z), cell[b], wr[b], wc[b]);
-                }
-                float4 q[B];
-#pragma unroll
-                for (int b = 0; b < B; ++b) q[b] = l2.vc[cell[b]];
-#pragma unroll
-                for (int b = 0; b < B; ++b)
-                    if (base + b * G < items) acc += (double)lpot2d_u_lerp(q[b].x, q[b].y, q[b].z, q[b].w, wr[b], wc[b]);
-            }
-            acc = group_sum(acc, G);
-            return acc;
-        }
-    }
-    for (int base = gl; base < items; base += B * G) {
-        vec4_t<R> d[B];
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-            int i = base + b * G;
-            if (i < items) d[b] = pk[i];
-            else { d[b].x = d[b].y = d[b].z = (R)0; d[b].w = (R)1; }
-        }
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-            R c;
-            if constexpr (is_fp32<R>()) c = -(fx * d[b].x + fy * d[b].y + fz * d[b].z);
-            else c = -((fx * d[b].x + fy * d[b].y + fz * d[b].z) / d[b].w);
-            R v = lpot2d<R>(l2, d[b].w, c);
-            if (base + b * G < items) acc += (double)v;
-        }
-    }
-    acc = group_sum(acc, G);
+    constexpr int B = UT ? 8 : 2;
+    int i = i0;
+    for (; i + (B / 2) * step < items; i += B * step) pair_batch<R, UT, B>(l2, g, i, step, items, fx, fy, fz, acc);
+    if (i < items) pair_batch<R, UT, B / 2>(l2, g, i, step, items, fx, fy, fz, acc);
     return acc;
 }
 
-// LDS (local index kl = k - k0 + 1; kl = 0 and ns+1 are the neighbours' boundary slices):
-// phi, cth, nv[3], E, Lk over ns+2 entries (double), then the geometry block
-// geo[(it - k0*RR) * np + jp] (vec4).  E[kl] is the partner energy of slice kl at its current
-// axis and Lk[kl] the density factor rho(n_kl . n_kl+1) of the link kl -> kl+1: the "old"
-// values of a move are the "new" values of the last accepted move that changed them (for a
-// link to a neighbour part, the value that part published with its slice).
-template <typename R>
+// One part of a linear rotor's chain: all sweeps of a launch.  The block's waves split the work: the
+// first one or two hold the chain of dependent steps, a lane per pair of slices (kl, kl + 1) -- link
+// densities, the test, the next proposal --; the others sum the partner energies of the proposals.
+// A proposal and its energy depend on the slice's own orientation alone, not on its neighbours, so
+// both are formed half a sweep ahead: while the chain waves test parity p, the energy waves work on
+// the proposals of parity 1 - p, which the chain waves made in the half before.  A half costs the
+// longer of the two instead of their sum, and what a move needs once runs on one lane instead of on
+// every lane of its group.
+// With every wave doing all of it in turn a half of a 512-slice chain took 5.0 us, now 1.8: bound by
+// the exchange with the neighbouring part (a store and a load at agent scope) on chains in several
+// parts, by the chain waves' FP64 steps on one part (8 atoms: 4.3 us, now 1.9), and on a full device
+// by how many parts are resident (two per CU for their registers; 168 registers spill and cost more
+// than the third part gives).  Sweep per pass, 256 replicas: 9.3 -> 4.8 ms.
+// LDS (local index kl = k - k0 + 1; kl = 0 and ns+1 are the neighbours' boundary slices): nv[3], Lk
+// and the proposals' axes np[3] over ns+2 entries (double), then the geometry block
+// geo[(it - k0*RR) * np + jp] (vec4).  Lk[kl] is the density factor rho(n_kl . n_kl+1) of the link
+// kl -> kl+1 and a lane's E its slices' partner energy: the "old" values of a move are the "new"
+// values of the last accepted move that changed them (for a link to a neighbour part, the value that
+// part published with its slice).
+constexpr int ROTOR_PARTIALS = 192;       // partial energies of a half: at most one per energy lane
+constexpr int ROTOR_KNOTS = 192;          // density knots staged in LDS
+constexpr int ROTOR_SLICES_MAX = 256;     // slices of a part where a chain lane holds two
+// Longer parts (chains of tens of thousands of slices with hardly any partners) take MPL pairs of
+// slices per chain lane: 2 * 128 * 12 slices are more than LDS holds.
+constexpr int ROTOR_MPL_LONG = 12;
+
+template <typename R, bool UT, int MPL>
 __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut* __restrict__ mut,
                                                const double4* __restrict__ beads, RotBead* __restrict__ rotb,
-                                               Tables T, Tables3 T3, const RotPart* __restrict__ parts,
+                                               Tables T, const RotPart* __restrict__ parts,
                                                unsigned* __restrict__ flags, unsigned long long* __restrict__ xrec, Run run) {
     extern __shared__ double smem[];
-    __shared__ unsigned long long red_acc[4];
+    __shared__ double pe[2][ROTOR_PARTIALS];
+    __shared__ double4 hk[ROTOR_KNOTS];
+    __shared__ unsigned s_acc[2];
     __shared__ int s_err;
     const RotPart pt = parts[blockIdx.x];
     if (pt.r < 0) return;  // padding of the XCD-ordered grid
@@ -982,27 +1004,25 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
     const int k0 = pt.k0, ns = pt.k1 - pt.k0, W = pt.W;
     const int np = N - 1;
     const int items = RR * np;
-    double* phi = smem;
-    double* cth = phi + (ns + 2);
-    double* nv = cth + (ns + 2);
-    double* E = nv + 3 * (ns + 2);
-    double* Lk = E + (ns + 2);
+    double* nv = smem;
+    double* Lk = nv + 3 * (ns + 2);
+    double* na = Lk + (ns + 2);  // axes of the proposals
     vec4_t<R>* geo = reinterpret_cast<vec4_t<R>*>(smem + ((7 * (ns + 2) + 3) & ~3));
     const int ar = rp.rot_atom;
     const long long rbase = rp.rot_off + (long long)(ar - rp.tbegin[rp.imtype]) * Prot;
     unsigned* myflag = flags + pt.fbase + pt.w;  // half-sweeps done by the launches before this one
     if (threadIdx.x == 0) s_err = 0;
-    // own slices and both neighbours' boundary slices
+    if (threadIdx.x < 2) s_acc[threadIdx.x] = 0;
+    // axes of the own slices and of both neighbours' boundary slices; the first energies are those of
+    // the current axes
     for (int kl = threadIdx.x; kl < ns + 2; kl += blockDim.x) {
         int k = k0 + kl - 1;
         if (k < 0) k += Prot;
         if (k >= Prot) k -= Prot;
-        RotBead b = rotb[rbase + k];
-        phi[kl] = b.phi;
-        cth[kl] = b.cth;
-        nv[3 * kl] = b.nx;
-        nv[3 * kl + 1] = b.ny;
-        nv[3 * kl + 2] = b.nz;
+        const RotBead b = rotb[rbase + k];
+        nv[3 * kl] = na[3 * kl] = b.nx;
+        nv[3 * kl + 1] = na[3 * kl + 1] = b.ny;
+        nv[3 * kl + 2] = na[3 * kl + 2] = b.nz;
     }
     // rotor-partner geometry of the part's translational slices (beads of one atom are
     // contiguous in slices, so consecutive lanes take consecutive slices)
@@ -1024,191 +1044,265 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
         geo[itl * np + jp] = v;
     }
     const uint32_t pass = mut[r].pass;
-    const int rtype = rp.imtype;
     const Lut2D<R> l2 = lut2d<R>(T, rp.pot2d_id);
     const TabRot trt = T.tr[rp.rotdens];
-    // lane groups of G lanes (power of two <= 64) per slice move
-    const int maxmoves = (ns + 1) / 2;
-    int G = 1;
-    while (G < 64 && G * 2 * maxmoves <= (int)blockDim.x) G *= 2;
-    const int groups = blockDim.x / G;
-    const int g = threadIdx.x / G, gl = threadIdx.x % G;
+    for (int i = threadIdx.x; i < trt.n - trt.hot; i += blockDim.x) hk[i] = T.rk[trt.off + trt.hot + i];
     const unsigned base = __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int nmoves = ns >> 1;                    // of either parity: k0 and ns are even
+    const int nchain = nmoves <= 64 ? 64 : 128;    // lanes of the chain waves
+    const bool chain = __builtin_amdgcn_readfirstlane((int)threadIdx.x) < nchain;  // a wave's role, scalar
+    // energy lanes: lpm per move, of which each quad or row of 16 leaves one partial sum in pe.  A
+    // long part's lanes take moves in turn and leave the sum in place of the proposal's axis
+    const int nen = (int)blockDim.x - nchain;
+    int lpm = MPL > 1 ? 1 : nen / nmoves;
+    const int gr = lpm >= 16 ? 16 : (lpm >= 4 ? 4 : 1);
+    lpm -= lpm % gr;
+    const int npart = lpm / gr;
+    const int le = (int)threadIdx.x - nchain, emv = le / lpm, eli = le - emv * lpm;
+    auto energies = [&](int parity) {  // of the proposals of one parity
+        for (int m = emv; m < nmoves; m += MPL > 1 ? nen : nmoves) {
+            const int kl = 2 * m + parity + 1;
+            double e = pair_terms<R, UT>(l2, geo + (long long)(kl - 1) * items, eli, lpm, items, na[3 * kl], na[3 * kl + 1],
+                                         na[3 * kl + 2]);
+            if constexpr (MPL > 1) {
+                na[3 * kl] = e;
+            } else {
+                e = group_sum(e, gr);
+                if ((eli & (gr - 1)) == 0) pe[parity][m * npart + eli / gr] = e;
+            }
+        }
+    };
+    auto energy_of = [&](int parity, int mv) {  // sum of the partials of a move
+        if constexpr (MPL > 1) return na[3 * (2 * mv + parity + 1)];
+        double e = 0.0;
+        for (int i = 0; i < npart; ++i) e += pe[parity][mv * npart + i];
+        return e;
+    };
     __syncthreads();
-    for (int kl = 1 + g; kl <= ns; kl += groups) {
-        double e = slice_energy<R>(l2, geo + (long long)(kl - 1) * items, items, gl, G, nv[3 * kl], nv[3 * kl + 1],
-                                   nv[3 * kl + 2]);
-        if (gl == 0) E[kl] = e;
+    if (!chain) {
+        energies(0);
+        energies(1);
     }
     for (int kl = threadIdx.x; kl <= ns; kl += blockDim.x) {
         double p = nv[3 * kl] * nv[3 * kl + 3] + nv[3 * kl + 1] * nv[3 * kl + 4] + nv[3 * kl + 2] * nv[3 * kl + 5];
         Lk[kl] = rot_rho(T, trt, p);
     }
     __syncthreads();
-    unsigned long long nacc = 0, nev = (threadIdx.x == 0) ? (unsigned long long)ns * items : 0ull;
+    // a chain lane's two slices, kl = 2 mv + 1 (even half) and 2 mv + 2 (odd half): the state, and the
+    // proposal in hand (its axis is in na)
+    struct Slice {
+        double phi, cth, E;      // now
+        double ph, cost, u;      // proposed, and the test's uniform
+        double nx, ny, nz;
+    };
+    Slice sl[MPL][2] = {};
+    auto move_of = [&](int q) { return q * nchain + (int)threadIdx.x; };
+    auto propose = [&](Slice& s, int mv, int parity, int sw) {
+        const int kl = 2 * mv + parity + 1;
+        const uint32_t jsweep = (uint32_t)(j0 + sw * jstride), k = (uint32_t)(k0 + kl - 1);
+        const uint4 w0 = draw(run.seed, rp.key, pass, K_ROTLIN, jsweep, (uint32_t)ar, k, 0);
+        const uint4 w1 = draw(run.seed, rp.key, pass, K_ROTLIN, jsweep, (uint32_t)ar, k, 1);
+        double cost = s.cth + rp.rtstep * (u53(w0.x, w0.y) - 0.5);
+        s.ph = s.phi + rp.rtstep * (u53(w0.z, w0.w) - 0.5);
+        if (cost > 1.0) cost = 2.0 - cost;
+        if (cost < -1.0) cost = -2.0 - cost;
+        s.cost = cost;
+        s.u = u53(w1.x, w1.y);
+        const double sint = sqrt(1.0 - cost * cost);
+        double sn, cs;
+        sincos(s.ph, &sn, &cs);
+        s.nx = sint * cs;
+        s.ny = sint * sn;
+        s.nz = cost;
+        na[3 * kl] = s.nx;
+        na[3 * kl + 1] = s.ny;
+        na[3 * kl + 2] = s.nz;
+    };
+    if (chain)
+        for (int q = 0; q < MPL; ++q) {
+            const int mv = move_of(q);
+            if (mv >= nmoves) break;
+#pragma unroll
+            for (int parity = 0; parity < 2; ++parity) {
+                const RotBead b = rotb[rbase + k0 + 2 * mv + parity];
+                sl[q][parity].phi = b.phi;
+                sl[q][parity].cth = b.cth;
+                sl[q][parity].E = energy_of(parity, mv);
+            }
+        }
+    __syncthreads();  // the current axes' energies are read; na and pe are the proposals' from here on
+    if (chain)
+        for (int q = 0; q < MPL; ++q) {
+            const int mv = move_of(q);
+            if (mv >= nmoves) break;
+            propose(sl[q][0], mv, 0, 0);
+            propose(sl[q][1], mv, 1, 0);
+        }
+    __syncthreads();
+    if (!chain) energies(0);
+    __syncthreads();
+    unsigned nacc = 0;
     int err = 0;
-    for (int sw = 0; sw < nsweep; ++sw) {
-        const uint32_t jsweep = (uint32_t)(j0 + sw * jstride);
-        for (int parity = 0; parity < 2; ++parity) {
-            const unsigned h = 2u * (unsigned)sw + (unsigned)parity;  // half-sweeps done before this one
-            // the neighbour's boundary slice this half reads: k0-1 (even half), k1 (odd half).
-            // Split parts receive it inside the boundary move below.  A single part is its own
-            // neighbour: local slices 0 and ns are one slice, as are 1 and ns + 1, and links 0 and
-            // ns one link, so the move that changes one copy writes the other (below)
-            const int nmoves = (ns - parity + 1) / 2;  // k0 is even, so local slice kl has parity (kl - 1) & 1
-            // the move that reads the neighbour's slice: kl = 1 (even half) or kl = ns (odd half)
-            const bool receive = W > 1 && !(sw == 0 && parity == 0);
-            const int kl_b = parity == 0 ? 1 : ns;
-            for (int mv = g; mv < nmoves; mv += groups) {
-                const int kl = 2 * mv + parity + 1;
-                const int k = k0 + kl - 1;
-                const bool bnd = receive && kl == kl_b;
-                // the lane whose link factor needs the neighbour's slice: rho(n_k-1 . n') on the
-                // lane of kl - 1 in the even half, rho(n' . n_k+1) on the lane of kl + 1 in the odd
-                const int dep = bnd ? (G == 1 ? 0 : parity) : -1;
-                // both draws of the move up front (independent, so they interleave)
-                const uint4 w0 = draw(run.seed, rp.key, pass, K_ROTLIN, jsweep, (uint32_t)ar, (uint32_t)k, 0);
-                const uint4 w1 = draw(run.seed, rp.key, pass, K_ROTLIN, jsweep, (uint32_t)ar, (uint32_t)k, 1);
-                double cost = cth[kl] + rp.rtstep * (u53(w0.x, w0.y) - 0.5);
-                double ph = phi[kl] + rp.rtstep * (u53(w0.z, w0.w) - 0.5);
-                if (cost > 1.0) cost = 2.0 - cost;
-                if (cost < -1.0) cost = -2.0 - cost;
-                double sint = sqrt(1.0 - cost * cost);
-                double nnx = sint * cos(ph), nny = sint * sin(ph), nnz = cost;
-                // new link factors rho(n_k-1 . n') and rho(n' . n_k+1), on two lanes when G >= 2;
-                // their knots are loaded before the partner gathers, so the loads overlap (the
-                // factor that needs the neighbour's slice waits for it, after the gathers)
-                double rho0 = 0.0, rho1 = 0.0, pa = 0.0, pb = 0.0;
-                RhoCell ca{}, cb{};
-                auto link_a = [&]() {
-                    const int kn = gl == 0 ? kl - 1 : kl + 1;
-                    pa = gl == 0 ? nv[3 * kn] * nnx + nv[3 * kn + 1] * nny + nv[3 * kn + 2] * nnz
-                                 : nnx * nv[3 * kn] + nny * nv[3 * kn + 1] + nnz * nv[3 * kn + 2];
-                    ca = rot_rho_load(T, trt, pa);
-                };
-                auto link_b = [&]() {
-                    pb = nnx * nv[3 * kl + 3] + nny * nv[3 * kl + 4] + nnz * nv[3 * kl + 5];
-                    cb = rot_rho_load(T, trt, pb);
-                };
-                if (gl < 2 && gl != dep) link_a();
-                if (G == 1 && !(bnd && parity == 1)) link_b();
-                double enew = slice_energy<R>(l2, geo + (long long)(kl - 1) * items, items, gl, G, nnx, nny, nnz);
-                if (bnd) {
-                    // The even half reads what the previous part published after its odd half of
-                    // the last sweep, the odd half what the next part published after its even
-                    // half of this sweep: the orientation and the density of the shared link (the
-                    // same product of the same operands this part would form), as eight words
-                    // that each carry the publishing half's number (base + h) above 32 bits of a
-                    // value.  Lanes of this move's group poll the words themselves, so the data
-                    // comes with its check; the neighbour cannot publish that record again before
-                    // this part's next half.  Only this move waits, after its partner gathers.
-                    const int nb = parity == 0 ? (pt.w + W - 1) % W : (pt.w + 1) % W;
-                    const unsigned long long* rec = xrec + ((size_t)(pt.fbase + nb) * 2 + (parity == 0 ? 1 : 0)) * 8;
-                    const unsigned want = base + h;
-                    const int klr = parity == 0 ? 0 : ns + 1;
-                    for (int w = gl; w < 8; w += G) {
-                        unsigned long long wv = 0;
-                        unsigned spins = 0;
-                        for (;;) {
-                            wv = __hip_atomic_load(rec + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            if ((unsigned)(wv >> 32) == want) break;
-                            if (++spins > ROT_SPIN_LIMIT) {
-                                s_err = 2;
-                                break;
-                            }
-                            __builtin_amdgcn_s_sleep(2);
-                        }
-                        const int i = w >> 1;  // doubles: the orientation, then the link density
-                        double* dst = i < 3 ? &nv[3 * klr + i] : &Lk[parity == 0 ? 0 : ns];
-                        reinterpret_cast<unsigned*>(dst)[w & 1] = (unsigned)wv;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    if (gl == dep) link_a();
-                    if (G == 1 && parity == 1) link_b();
+    // The neighbour's boundary slice that half h of the next parity reads: k0-1 before an even half
+    // (published by the previous part after its odd half), k1 before an odd half (by the next part
+    // after its even half): the orientation and the density of the shared link (the same product of
+    // the same operands this part would form), as eight words that each carry the publishing half's
+    // number (base + h) above 32 bits of a value.  Eight lanes poll the words themselves, so the data
+    // comes with its check; the neighbour cannot publish that record again before this part's next
+    // half.  A single part is its own neighbour: local slices 0 and ns are one slice, as are 1 and
+    // ns + 1, and links 0 and ns one link, so the move that changes one copy writes the other.
+    auto record = [&](int parity) {
+        const int nb = parity == 0 ? (pt.w + W - 1) % W : (pt.w + 1) % W;
+        return xrec + ((size_t)(pt.fbase + nb) * 2 + (parity == 0 ? 1 : 0)) * 8;
+    };
+    auto receive = [&](int parity, unsigned h, unsigned long long wv) {
+        const int lane = threadIdx.x & 63;
+        const unsigned long long* rec = record(parity);
+        const unsigned want = base + h;
+        const int klr = parity == 0 ? 0 : ns + 1;
+        if (lane < 8) {
+            unsigned spins = 0;
+            while ((unsigned)(wv >> 32) != want) {
+                if (++spins > ROT_SPIN_LIMIT) {
+                    s_err = 2;
+                    break;
                 }
-                if (gl < 2) {
-                    if (gl == 0) rho0 = rot_rho_eval(T, trt, pa, ca);
-                    else rho1 = rot_rho_eval(T, trt, pa, ca);
-                }
-                if (G == 1) rho1 = rot_rho_eval(T, trt, pb, cb);
-                if (G > 1) rho1 = __shfl_xor(rho1, 1, G);
-                if (gl == 0) {
-                    nev += (unsigned long long)items;
-                    double dold = Lk[kl - 1] * Lk[kl];
-                    if (fabs(dold) < RZERO) dold = 0.0;
-                    double dnew = rho0 * rho1;
-                    if (fabs(dnew) < RZERO) dnew = 0.0;
-                    if (dold < 0.0 || dnew < 0.0) {
-                        err = 1;  // "Negative rot density" (mc_piqmc.cc:850,886): the move is not taken
-                    } else {
-                        double rd = (dold > RZERO) ? dnew / dold : 1.0;
-                        rd *= exp(-rp.tau * (enew - E[kl]));
-                        const bool accepted = rd > 1.0 || rd > u53(w1.x, w1.y);
-                        if (accepted) {
-                            ++nacc;
-                            cth[kl] = cost;
-                            phi[kl] = ph;
-                            nv[3 * kl] = nnx;
-                            nv[3 * kl + 1] = nny;
-                            nv[3 * kl + 2] = nnz;
-                            E[kl] = enew;
-                            Lk[kl - 1] = rho0;
-                            Lk[kl] = rho1;
-                            if (W == 1 && (kl == 1 || kl == ns)) {  // the other copy of the slice and link
-                                const int km = kl == 1 ? ns + 1 : 0;
-                                nv[3 * km] = nnx;
-                                nv[3 * km + 1] = nny;
-                                nv[3 * km + 2] = nnz;
-                                Lk[kl == 1 ? ns : 0] = kl == 1 ? rho0 : rho1;
-                            }
-                        }
+                __builtin_amdgcn_s_sleep(1);
+                wv = __hip_atomic_load(rec + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            const int i = lane >> 1;  // doubles: the orientation, then the link density
+            double* dst = i < 3 ? &nv[3 * klr + i] : &Lk[parity == 0 ? 0 : ns];
+            reinterpret_cast<unsigned*>(dst)[lane & 1] = (unsigned)wv;
+        }
+    };
+    // parity p of sweep sw on the chain waves: test, update, publish, the proposal of the next sweep,
+    // and what the next half needs of the neighbour, which has published it about when this part did:
+    // the record is asked for before the proposal and checked after it, while the energy waves work
+    auto move = [&](auto p_c, int sw, int q) {
+        constexpr int parity = decltype(p_c)::value;
+        Slice& s = sl[q][parity];
+        const int mv = move_of(q);
+        const bool mine = mv < nmoves;
+        const int kl = 2 * mv + parity + 1;
+        const unsigned h = 2u * (unsigned)sw + (unsigned)parity;  // half-sweeps done before this one
+        const int bnd_mv = parity == 0 ? 0 : nmoves - 1;  // the move at the slice that is published
+        const int lane = threadIdx.x & 63;
+        if (mine) {
+            const double p0 = nv[3 * kl - 3] * s.nx + nv[3 * kl - 2] * s.ny + nv[3 * kl - 1] * s.nz;  // n_k-1 . n'
+            const double p1 = s.nx * nv[3 * kl + 3] + s.ny * nv[3 * kl + 4] + s.nz * nv[3 * kl + 5];  // n' . n_k+1
+            double rho0, rho1;
+            rot_rho_hot(T, trt, hk, p0, p1, rho0, rho1);
+            const double enew = energy_of(parity, mv);
+            double dold = Lk[kl - 1] * Lk[kl];
+            if (fabs(dold) < RZERO) dold = 0.0;
+            double dnew = rho0 * rho1;
+            if (fabs(dnew) < RZERO) dnew = 0.0;
+            if (dold < 0.0 || dnew < 0.0) {
+                err = 1;  // "Negative rot density" (mc_piqmc.cc:850,886): the move is not taken
+            } else {
+                // dnew / dold exp(-tau dV) > u (the reference's ratio counts as 1 where dold is zero)
+                const double x = exp(-rp.tau * (enew - s.E));
+                const bool accepted = dold > RZERO ? dnew * x > s.u * dold : x > s.u;
+                if (accepted) {
+                    ++nacc;
+                    s.cth = s.cost;
+                    s.phi = s.ph;
+                    s.E = enew;
+                    nv[3 * kl] = s.nx;
+                    nv[3 * kl + 1] = s.ny;
+                    nv[3 * kl + 2] = s.nz;
+                    Lk[kl - 1] = rho0;
+                    Lk[kl] = rho1;
+                    if (W == 1 && (kl == 1 || kl == ns)) {  // the other copy of the slice and link
+                        const int km = kl == 1 ? ns + 1 : 0;
+                        nv[3 * km] = s.nx;
+                        nv[3 * km + 1] = s.ny;
+                        nv[3 * km + 2] = s.nz;
+                        Lk[kl == 1 ? ns : 0] = kl == 1 ? rho0 : rho1;
                     }
                 }
             }
-            __syncthreads();
-            // a wait that gave up: leave at once instead of waiting again at every later half
-            // (every lane reads s_err after the barrier; it is written again only in the next half)
-            if (s_err) {
-                sw = nsweep;
-                break;
-            }
-            // publish the boundary slice this half moved (k0 after the even half, k1-1 after
-            // the odd half), then the count of half-sweeps done
-            if (W > 1 && threadIdx.x < 8) {
-                // orientation and the density of the link to the neighbour's adjacent slice
-                // (Lk[0] after the even half, for the previous part; Lk[ns] after the odd half,
-                // for the next), two words per double; no wait for the stores, the reader
-                // checks every word's number
-                const int kl = parity == 0 ? 1 : ns;
-                const int i = threadIdx.x >> 1;
-                const double v = i < 3 ? nv[3 * kl + i] : Lk[parity == 0 ? 0 : ns];
+        }
+        // publish the boundary slice this half moved (k0 after the even half, k1-1 after the odd)
+        const bool publisher = W > 1 && bnd_mv / nchain == q && (bnd_mv % nchain) >> 6 == (int)threadIdx.x >> 6;
+        const bool more = !(parity == 1 && sw + 1 == nsweep);  // a half follows in this launch
+        unsigned long long wv = 0;
+        if (publisher) {
+            wave_sync();
+            if (lane < 8) {
+                // orientation and the density of the link to the neighbour's adjacent slice (Lk[0]
+                // after the even half, for the previous part; Lk[ns] after the odd half, for the
+                // next), two words per double; no wait for the stores, the reader checks every
+                // word's number
+                const int kb = parity == 0 ? 1 : ns;
+                const int i = lane >> 1;
+                const double v = i < 3 ? nv[3 * kb + i] : Lk[parity == 0 ? 0 : ns];
                 const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-                const unsigned half = (threadIdx.x & 1) ? (unsigned)(bits >> 32) : (unsigned)bits;
-                __hip_atomic_store(xrec + ((size_t)(pt.fbase + pt.w) * 2 + parity) * 8 + threadIdx.x,
-                                   ((unsigned long long)(base + h + 1u) << 32) | half, __ATOMIC_RELAXED,
+                const unsigned word = (lane & 1) ? (unsigned)(bits >> 32) : (unsigned)bits;
+                __hip_atomic_store(xrec + ((size_t)(pt.fbase + pt.w) * 2 + parity) * 8 + lane,
+                                   ((unsigned long long)(base + h + 1u) << 32) | word, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
+                if (more) wv = __hip_atomic_load(record(1 - parity) + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+        }
+        if (mine && sw + 1 < nsweep) propose(s, mv, parity, sw + 1);
+        if (publisher && more) receive(1 - parity, h + 1u, wv);
+    };
+    auto half = [&](auto p_c, int sw) {
+        for (int q = 0; q < MPL; ++q)
+            if (MPL == 1 || q * nchain < nmoves) move(p_c, sw, q);
+    };
+    // the two roles in loops of their own, barrier for barrier, so that neither holds the other's
+    // registers.  A wait that gave up: leave at once instead of waiting again at every later half
+    // (every lane reads s_err after the barrier; it is written again only in the next half)
+    if (chain) {
+        for (int sw = 0; sw < nsweep; ++sw) {
+            half(std::integral_constant<int, 0>{}, sw);
+            lds_barrier();
+            if (s_err) break;
+            half(std::integral_constant<int, 1>{}, sw);
+            lds_barrier();
+            if (s_err) break;
+        }
+    } else {
+        for (int sw = 0; sw < nsweep; ++sw) {
+            energies(1);
+            lds_barrier();
+            if (s_err) break;
+            if (sw + 1 < nsweep) energies(0);
+            lds_barrier();
+            if (s_err) break;
         }
     }
     if (W > 1 && threadIdx.x == 0)  // every part of the chain ran the same halves
         __hip_atomic_store(myflag, base + 2u * (unsigned)nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int kl = 1 + threadIdx.x; kl <= ns; kl += blockDim.x) {
-        RotBead b = rotb[rbase + k0 + kl - 1];
-        b.phi = phi[kl];
-        b.cth = cth[kl];
-        b.nx = nv[3 * kl];
-        b.ny = nv[3 * kl + 1];
-        b.nz = nv[3 * kl + 2];
-        rotb[rbase + k0 + kl - 1] = b;
+    if (chain)
+        for (int q = 0; q < MPL; ++q) {
+            const int mv = move_of(q);
+            if (mv >= nmoves) break;
+#pragma unroll
+            for (int parity = 0; parity < 2; ++parity) {
+                const int kl = 2 * mv + parity + 1;
+                RotBead& b = rotb[rbase + k0 + kl - 1];
+                b.phi = sl[q][parity].phi;
+                b.cth = sl[q][parity].cth;
+                b.nx = nv[3 * kl];
+                b.ny = nv[3 * kl + 1];
+                b.nz = nv[3 * kl + 2];
+            }
+        }
+    if (chain) {
+        const unsigned s = wave_sum(nacc);
+        if ((threadIdx.x & 63) == 0) s_acc[threadIdx.x >> 6] = s;
     }
-    unsigned long long s = block_sum(nacc, red_acc);
-    unsigned long long ne = block_sum(nev, red_acc);
+    __syncthreads();
     if (err) atomicOr(&mut[r].err, 1);
     if (threadIdx.x == 0) {
         if (s_err) atomicOr(&mut[r].err, s_err);
-        atomicAdd(&mut[r].total[rtype][2], (unsigned long long)nsweep * ns);
-        atomicAdd(&mut[r].accep[rtype][2], s);
-        atomicAdd(&mut[r].pair_evals[2], ne);
+        atomicAdd(&mut[r].total[rp.imtype][2], (unsigned long long)nsweep * ns);
+        atomicAdd(&mut[r].accep[rp.imtype][2], (unsigned long long)(s_acc[0] + s_acc[1]));
+        // the current axes once per launch, then every proposal
+        atomicAdd(&mut[r].pair_evals[2], (unsigned long long)(nsweep + 1) * ns * items);
     }
 }
 
