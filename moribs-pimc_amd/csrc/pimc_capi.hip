@@ -2204,75 +2204,63 @@ int pimc_kernel_time(pimc_ctx* c, const char* family, double* ms, long* launches
 // ------------------------------------------------------------------------------ surrogate
 namespace {
 
+// Device memory of a training run (rows, weights, what a batch leaves for its gradients) in one
+// allocation, freed with the object.
 struct MlpBuffers {
-    float *x = nullptr, *y = nullptr, *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Z3 = nullptr,
-          *H3 = nullptr, *out = nullptr, *dout = nullptr, *dA = nullptr, *dB = nullptr;
-    double* loss = nullptr;
-    int cap = 0;
-    bool alloc(int B) {
-        cap = B;
-        const size_t h = (size_t)B * MLP_H;
-        x = dalloc<float>((size_t)B * MLP_IN);
-        y = dalloc<float>(B);
-        Z1 = dalloc<float>(h); H1 = dalloc<float>(h);
-        Z2 = dalloc<float>(h); H2 = dalloc<float>(h);
-        Z3 = dalloc<float>(h); H3 = dalloc<float>(h);
-        out = dalloc<float>(B); dout = dalloc<float>(B);
-        dA = dalloc<float>(h); dB = dalloc<float>(h);
-        loss = dalloc<double>(1);
-        return x && y && Z1 && H1 && Z2 && H2 && Z3 && H3 && out && dout && dA && dB && loss;
+    MlpTrain t{};
+    float *X = nullptr, *Y = nullptr;
+    int* perm = nullptr;
+    double* loss = nullptr;  // one partial per block of rows of every step of an epoch
+    void* mem = nullptr;
+    bool alloc(int n, int batch, bool adam, size_t nloss) {
+        const size_t pad = ((size_t)batch + 31) / 32 * 32;
+        size_t at = 0;
+        auto lay = [&](bool place) {
+            at = 0;
+            auto take = [&](auto*& p, size_t count) {
+                if (place) p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(static_cast<char*>(mem) + at);
+                at += (count * sizeof(*p) + 255) / 256 * 256;
+            };
+            take(X, (size_t)n * MLP_IN);
+            take(Y, n);
+            take(perm, n);
+            take(loss, nloss);
+            take(t.ops, 6 * pad * MLP_H);
+            take(t.opx, pad * 32);
+            take(t.opd, pad * 32);
+            take(t.dz, 3 * pad * MLP_H);
+            take(t.dout, pad);
+            take(t.pw, 4 * (size_t)MLP_H * MLP_H);
+            take(t.th, MLP_NW);
+            take(t.m, MLP_NW);
+            take(t.v, MLP_NW);
+            if (!adam) take(t.g, MLP_NW);
+        };
+        lay(false);
+        if (hipMalloc(&mem, at) != hipSuccess) {
+            mem = nullptr;
+            return false;
+        }
+        lay(true);
+        t.X = X;
+        t.Y = Y;
+        t.B = batch;
+        t.pad = (int)pad;
+        return true;
     }
     ~MlpBuffers() {
-        void* p[] = {x, y, Z1, H1, Z2, H2, Z3, H3, out, dout, dA, dB, loss};
-        for (void* q : p)
-            if (q) (void)hipFree(q);
+        if (mem) (void)hipFree(mem);
     }
 };
 
-void mlp_gemm(hipStream_t s, int M, int N, int K, const float* A, int lda, int ta, const float* B, int ldb, int tb,
-              float* C, int ldc) {
-    hipLaunchKernelGGL(k_mlp_gemm, dim3((N + 31) / 32, (M + 31) / 32), dim3(64), 0, s, M, N, K, A, lda, ta, B, ldb,
-                       tb, C, ldc, 0);
+void mlp_pack_weights(hipStream_t s, const MlpTrain& t) {
+    hipLaunchKernelGGL(k_mlp_train_pack, dim3(2 * MLP_H * MLP_H / 256), dim3(256), 0, s, t.th, t.pw);
 }
 
-void mlp_bias(hipStream_t s, float* Z, float* H, const float* b, int rows, int cols, int act) {
-    const long long n = (long long)rows * cols;
-    hipLaunchKernelGGL(k_mlp_bias_act, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, Z, H, b, rows, cols, act);
-}
-
-void mlp_back(hipStream_t s, float* dH, const float* Z, int rows) {
-    const long long n = (long long)rows * MLP_H;
-    hipLaunchKernelGGL(k_mlp_act_back, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dH, Z, n);
-}
-
-// Loss and gradient of the batch in m.x / m.y (B rows, normalised) at weights th; g gets the
-// gradient, m.loss accumulates the loss.
-void mlp_forward_backward(hipStream_t s, const float* th, float* g, MlpBuffers& m, int B) {
-    // forward: Z = H_prev W^T + b, H = SiLU(Z)
-    mlp_gemm(s, B, MLP_H, MLP_IN, m.x, MLP_IN, 0, th + MLP_OFF_W1, MLP_IN, 1, m.Z1, MLP_H);
-    mlp_bias(s, m.Z1, m.H1, th + MLP_OFF_B1, B, MLP_H, 1);
-    mlp_gemm(s, B, MLP_H, MLP_H, m.H1, MLP_H, 0, th + MLP_OFF_W2, MLP_H, 1, m.Z2, MLP_H);
-    mlp_bias(s, m.Z2, m.H2, th + MLP_OFF_B2, B, MLP_H, 1);
-    mlp_gemm(s, B, MLP_H, MLP_H, m.H2, MLP_H, 0, th + MLP_OFF_W3, MLP_H, 1, m.Z3, MLP_H);
-    mlp_bias(s, m.Z3, m.H3, th + MLP_OFF_B3, B, MLP_H, 1);
-    mlp_gemm(s, B, 1, MLP_H, m.H3, MLP_H, 0, th + MLP_OFF_W4, 1, 0, m.out, 1);
-    mlp_bias(s, m.out, m.out, th + MLP_OFF_B4, B, 1, 0);
-    hipLaunchKernelGGL(k_mlp_mse, dim3((B + 255) / 256), dim3(256), 0, s, m.out, m.y, B, m.dout, m.loss);
-    // backward
-    mlp_gemm(s, MLP_H, 1, B, m.H3, MLP_H, 1, m.dout, 1, 0, g + MLP_OFF_W4, 1);
-    hipLaunchKernelGGL(k_mlp_colsum, dim3(1), dim3(256), 0, s, m.dout, B, 1, g + MLP_OFF_B4);
-    mlp_gemm(s, B, MLP_H, 1, m.dout, 1, 0, th + MLP_OFF_W4, MLP_H, 0, m.dA, MLP_H);  // dH3
-    mlp_back(s, m.dA, m.Z3, B);                                                      // dZ3
-    mlp_gemm(s, MLP_H, MLP_H, B, m.dA, MLP_H, 1, m.H2, MLP_H, 0, g + MLP_OFF_W3, MLP_H);
-    hipLaunchKernelGGL(k_mlp_colsum, dim3(MLP_H), dim3(256), 0, s, m.dA, B, MLP_H, g + MLP_OFF_B3);
-    mlp_gemm(s, B, MLP_H, MLP_H, m.dA, MLP_H, 0, th + MLP_OFF_W3, MLP_H, 0, m.dB, MLP_H);  // dH2
-    mlp_back(s, m.dB, m.Z2, B);
-    mlp_gemm(s, MLP_H, MLP_H, B, m.dB, MLP_H, 1, m.H1, MLP_H, 0, g + MLP_OFF_W2, MLP_H);
-    hipLaunchKernelGGL(k_mlp_colsum, dim3(MLP_H), dim3(256), 0, s, m.dB, B, MLP_H, g + MLP_OFF_B2);
-    mlp_gemm(s, B, MLP_H, MLP_H, m.dB, MLP_H, 0, th + MLP_OFF_W2, MLP_H, 0, m.dA, MLP_H);  // dH1
-    mlp_back(s, m.dA, m.Z1, B);
-    mlp_gemm(s, MLP_H, MLP_IN, B, m.dA, MLP_H, 1, m.x, MLP_IN, 0, g + MLP_OFF_W1, MLP_IN);
-    hipLaunchKernelGGL(k_mlp_colsum, dim3(MLP_H), dim3(256), 0, s, m.dA, B, MLP_H, g + MLP_OFF_B1);
+// Loss partials and weight gradients of a batch; then, without t.g, the step on the weights
+void mlp_step(hipStream_t s, const MlpTrain& t, const MlpAdam& ad) {
+    hipLaunchKernelGGL(k_mlp_rows, dim3(t.pad / 32), dim3(256), 0, s, t);
+    hipLaunchKernelGGL(k_mlp_grads, dim3(MLP_GRAD_JOBS), dim3(256), MLP_GRAD_LDS, s, t, ad);
 }
 
 int mlp_upload(pimc_ctx* c) {
@@ -2330,26 +2318,28 @@ int pimc_surrogate_grad(pimc_ctx* c, const float* theta, const float* x, const f
                         double* loss) {
     if (!theta || !x || !y || !grad || !loss || n < 1 || n > (1 << 20)) return fail(c, "surrogate_grad: bad arguments");
     MlpBuffers m;
-    float *th = dalloc<float>(MLP_NW), *g = dalloc<float>(MLP_NW);
-    int rc = 0;
-    hipError_t e0 = hipSuccess;
-    auto ck = [&](hipError_t x) { if (e0 == hipSuccess) e0 = x; };
-    if (!m.alloc(n) || !th || !g) rc = fail(c, "surrogate_grad: out of device memory");
-    if (rc == 0) {
-        ck(hipMemcpy(th, theta, sizeof(float) * MLP_NW, hipMemcpyHostToDevice));
-        ck(hipMemcpy(m.x, x, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice));
-        ck(hipMemcpy(m.y, y, sizeof(float) * n, hipMemcpyHostToDevice));
-        ck(hipMemset(m.loss, 0, sizeof(double)));
-        mlp_forward_backward(c->stream, th, g, m, n);
-        ck(hipGetLastError());
-        hipError_t e = e0 != hipSuccess ? e0 : hipStreamSynchronize(c->stream);
-        if (e == hipSuccess) e = hipMemcpy(grad, g, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(loss, m.loss, sizeof(double), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) rc = fail(c, std::string("surrogate_grad: ") + hipGetErrorString(e));
+    const int nblock = (n + 31) / 32;
+    if (!m.alloc(n, n, false, nblock)) return fail(c, "surrogate_grad: out of device memory");
+    hipError_t e = hipSuccess;
+    auto ck = [&](hipError_t x) { if (e == hipSuccess) e = x; };
+    std::vector<double> part(nblock);
+    m.t.loss = m.loss;
+    ck(hipMemcpyAsync(m.t.th, theta, sizeof(float) * MLP_NW, hipMemcpyHostToDevice, c->stream));
+    ck(hipMemcpyAsync(m.X, x, sizeof(float) * MLP_IN * n, hipMemcpyHostToDevice, c->stream));
+    ck(hipMemcpyAsync(m.Y, y, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
+    if (e == hipSuccess) {
+        mlp_pack_weights(c->stream, m.t);
+        mlp_step(c->stream, m.t, MlpAdam{});
     }
-    if (th) (void)hipFree(th);
-    if (g) (void)hipFree(g);
-    return rc;
+    ck(hipGetLastError());
+    ck(hipMemcpyAsync(grad, m.t.g, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost, c->stream));
+    ck(hipMemcpyAsync(part.data(), m.loss, sizeof(double) * nblock, hipMemcpyDeviceToHost, c->stream));
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    ck(es);
+    if (e != hipSuccess) return fail(c, std::string("surrogate_grad: ") + hipGetErrorString(e));
+    *loss = 0.0;
+    for (double v : part) *loss += v;
+    return 0;
 }
 
 int pimc_surrogate_train(pimc_ctx* c, const float* x, const float* v, int n, int epochs, int batch, double lr,
@@ -2404,51 +2394,46 @@ int pimc_surrogate_train(pimc_ctx* c, const float* x, const float* v, int n, int
     fill(MLP_OFF_W3, MLP_H, MLP_H);
     fill(MLP_OFF_W4, 1, MLP_H);
     MlpBuffers m;
-    float *dX = dalloc<float>((size_t)n * MLP_IN), *dY = dalloc<float>(n), *dth = dalloc<float>(MLP_NW),
-          *dg = dalloc<float>(MLP_NW), *dm = dalloc<float>(MLP_NW), *dv = dalloc<float>(MLP_NW);
-    int* dperm = dalloc<int>(n);
-    int rc = 0;
-    hipError_t e0 = hipSuccess;
-    auto ck = [&](hipError_t x) { if (e0 == hipSuccess) e0 = x; };
-    if (!m.alloc(batch) || !dX || !dY || !dth || !dg || !dm || !dv || !dperm) rc = fail(c, "surrogate_train: out of device memory");
-    if (rc == 0) {
-        ck(hipMemcpy(dX, xn.data(), sizeof(float) * xn.size(), hipMemcpyHostToDevice));
-        ck(hipMemcpy(dY, yn.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-        ck(hipMemcpy(dth, th.data(), sizeof(float) * MLP_NW, hipMemcpyHostToDevice));
-        ck(hipMemset(dm, 0, sizeof(float) * MLP_NW));
-        ck(hipMemset(dv, 0, sizeof(float) * MLP_NW));
-        std::vector<int> perm(n);
-        for (int i = 0; i < n; ++i) perm[i] = i;
-        const int steps = n / batch;
-        long t = 0;
-        for (int ep = 0; ep < epochs && rc == 0; ++ep) {
-            for (int i = n - 1; i > 0; --i) std::swap(perm[i], perm[(int)(unif() * (i + 1))]);
-            ck(hipMemcpy(dperm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-            ck(hipMemset(m.loss, 0, sizeof(double)));
-            const float lr_ep = (float)(lr * std::pow(0.1, (double)ep / epochs));  // decays tenfold over the run
-            for (int s = 0; s < steps; ++s) {
-                hipLaunchKernelGGL(k_mlp_gather, dim3((batch + 255) / 256), dim3(256), 0, c->stream, dX, dY, dperm,
-                                   s * batch, batch, m.x, m.y);
-                mlp_forward_backward(c->stream, dth, dg, m, batch);
-                ++t;
-                const float c1 = (float)(1.0 - std::pow(0.9, (double)t)), c2 = (float)(1.0 - std::pow(0.999, (double)t));
-                hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NW + 255) / 256), dim3(256), 0, c->stream, dth, dg, dm, dv,
-                                   MLP_NW, lr_ep, c1, c2);
-            }
-            double l = 0.0;
-            ck(hipGetLastError());
-            hipError_t e = e0 != hipSuccess ? e0 : hipStreamSynchronize(c->stream);
-            if (e == hipSuccess) e = hipMemcpy(&l, m.loss, sizeof(double), hipMemcpyDeviceToHost);
-            if (e != hipSuccess) rc = fail(c, std::string("surrogate_train: ") + hipGetErrorString(e));
-            if (loss) loss[ep] = l / steps;
+    const int steps = n / batch, nblock = (batch + 31) / 32;
+    if (!m.alloc(n, batch, true, (size_t)steps * nblock)) return fail(c, "surrogate_train: out of device memory");
+    hipError_t e = hipSuccess;
+    auto ck = [&](hipError_t x) { if (e == hipSuccess) e = x; };
+    ck(hipMemcpyAsync(m.X, xn.data(), sizeof(float) * xn.size(), hipMemcpyHostToDevice, c->stream));
+    ck(hipMemcpyAsync(m.Y, yn.data(), sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
+    ck(hipMemcpyAsync(m.t.th, th.data(), sizeof(float) * MLP_NW, hipMemcpyHostToDevice, c->stream));
+    ck(hipMemsetAsync(m.t.m, 0, sizeof(float) * MLP_NW, c->stream));
+    ck(hipMemsetAsync(m.t.v, 0, sizeof(float) * MLP_NW, c->stream));
+    mlp_pack_weights(c->stream, m.t);
+    std::vector<int> perm(n), sent;
+    for (int i = 0; i < n; ++i) perm[i] = i;
+    auto shuffle = [&]() {
+        for (int i = n - 1; i > 0; --i) std::swap(perm[i], perm[(int)(unif() * (i + 1))]);
+    };
+    std::vector<double> part((size_t)steps * nblock);
+    shuffle();
+    long t = 0;
+    for (int ep = 0; ep < epochs && e == hipSuccess; ++ep) {
+        sent = perm;
+        ck(hipMemcpyAsync(m.perm, sent.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+        const float lr_ep = (float)(lr * std::pow(0.1, (double)ep / epochs));  // decays tenfold over the run
+        for (int s = 0; s < steps; ++s) {
+            ++t;
+            m.t.perm = m.perm + (size_t)s * batch;
+            m.t.loss = m.loss + (size_t)s * nblock;
+            mlp_step(c->stream, m.t, MlpAdam{lr_ep, (float)(1.0 - std::pow(0.9, (double)t)), (float)(1.0 - std::pow(0.999, (double)t))});
         }
-        if (rc == 0 && hipMemcpy(th.data(), dth, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost) != hipSuccess)
-            rc = fail(c, "surrogate_train: copy back");
+        ck(hipGetLastError());
+        if (ep + 1 < epochs) shuffle();  // the next epoch's order while this one runs
+        ck(hipMemcpyAsync(part.data(), m.loss, sizeof(double) * part.size(), hipMemcpyDeviceToHost, c->stream));
+        ck(hipStreamSynchronize(c->stream));
+        double l = 0.0;
+        for (double v : part) l += v;
+        if (loss && e == hipSuccess) loss[ep] = l / steps;
     }
-    void* ptrs[] = {dX, dY, dth, dg, dm, dv, dperm};
-    for (void* q : ptrs)
-        if (q) (void)hipFree(q);
-    if (rc) return rc;
+    ck(hipMemcpyAsync(th.data(), m.t.th, sizeof(float) * MLP_NW, hipMemcpyDeviceToHost, c->stream));
+    const hipError_t es = hipStreamSynchronize(c->stream);  // also after an error: the memory goes with m
+    ck(es);
+    if (e != hipSuccess) return fail(c, std::string("surrogate_train: ") + hipGetErrorString(e));
     c->theta = th;
     c->norm = norm;
     return mlp_upload(c);
