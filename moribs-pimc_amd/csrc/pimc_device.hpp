@@ -665,4 +665,12 @@ __device__ __forceinline__ T wave_sum(T v) {
     return group_sum(v, 64);
 }
 
+// A workgroup barrier that orders LDS only.  __syncthreads also waits for every global access in
+// flight, such as a prefetch or the stores of results that no lane of the block reads again.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 }  // namespace pimc

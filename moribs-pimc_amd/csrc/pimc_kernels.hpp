@@ -98,15 +98,7 @@ __device__ __forceinline__ const Frame& frame_at(const Frame* __restrict__ frame
 }
 
 // ------------------------------------------------------------------------- bisection
-// A workgroup barrier that orders LDS only.  __syncthreads also waits for every global access in
-// flight, which here are a prefetch and the stores of an accepted move that no lane reads again.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// block_sum with those barriers
+// block_sum with barriers that order LDS only
 __device__ __forceinline__ double block_sum_lds(double v, double* red) {
     v = wave_sum(v);
     const int wid = threadIdx.x >> 6, nw = blockDim.x >> 6;

@@ -22,6 +22,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "pimc_device.hpp"
 
 constexpr int MLP_IN = 4;
 constexpr int MLP_H = 128;
@@ -174,12 +175,12 @@ __device__ __forceinline__ void mlp_pair_features(const double m[9], double zn, 
 // order of the sums is part of the result.
 //
 // What bounds a step is that order: a weight gradient sums over the batch, 512 dependent matrix
-// instructions for 4096 rows (9 us), on 40 tiles of 32x32.  Everything else is arranged around that
+// instructions for 4096 rows (20 us), on 40 tiles of 32x32.  Everything else is arranged around that
 // chain: activations stay in registers and LDS from the gather to dZ1, operands are written once in
 // the lane order in which the chain reads them and staged ahead of it by the block's four waves,
 // and the step on the weights, with their operands for the next step, is the chain's last act.
 // A launch per product and per elementwise operation, a wave per tile reading FP32 operands one by
-// one, took 1.56 ms a step of 4096 rows.
+// one, took 1.56 ms a step of 4096 rows; the two kernels now take 19 and 22 us.
 
 // Operand order of a 32x32x8 product whose contraction runs over rows: [rows / 16][tile][lane][8],
 // value 4 s + j of lane l is row 8 s + 4 (l / 32) + j of the sixteen, unit l % 32 of the tile.  The
@@ -249,6 +250,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(MlpTrain t) {
     __shared__ alignas(16) uint16_t ex[5][32 * MLP_XS];
     __shared__ float4 xs[32];
     __shared__ float ys[32], ds[32];
+    __shared__ alignas(8) uint16_t w4s[MLP_H];
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, hi = l >> 5, u = l & 31, unit = 32 * w + u;
     const int row0 = blockIdx.x * 32;
     const size_t opn = (size_t)t.pad * MLP_H;  // values of one operand array
@@ -271,8 +273,10 @@ __global__ __launch_bounds__(256) void k_mlp_rows(MlpTrain t) {
     }
     const float4 w1 = *reinterpret_cast<const float4*>(t.th + MLP_OFF_W1 + unit * MLP_IN);
     const float b1 = t.th[MLP_OFF_B1 + unit], b2 = t.th[MLP_OFF_B2 + unit], b3 = t.th[MLP_OFF_B3 + unit],
-                b4 = t.th[MLP_OFF_B4], w4 = t.th[MLP_OFF_W4 + unit];
-    __syncthreads();
+                b4 = t.th[MLP_OFF_B4];
+    const uint16_t w4 = f2bf(t.th[MLP_OFF_W4 + unit]);
+    if (hi == 0) w4s[unit] = w4;
+    pimc::lds_barrier();
     auto row_of = [&](int i) { return 8 * (i >> 2) + 4 * hi + (i & 3); };
     // a tile's values to LDS for the next product and to memory as operands of the gradient
     auto put = [&](int x, const float (&h)[16], int a) {
@@ -319,23 +323,21 @@ __global__ __launch_bounds__(256) void k_mlp_rows(MlpTrain t) {
         activate(mlp_mfma(a, b, acc), b1, z1);
     }
     put(0, h, 0);
-    __syncthreads();
+    pimc::lds_barrier();
     activate(product(0, wt[0]), b2, z2);
     put(1, h, 1);
-    __syncthreads();
+    pimc::lds_barrier();
     activate(product(1, wt[1]), b3, z3);
     put(2, h, 2);
-    __syncthreads();
+    pimc::lds_barrier();
     // the output row by row, in every wave: column 0 of H3 w4
     mlp_f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    for (int kb = 0; kb < 16; ++kb) {
-        mlp_bf16x4 b = {0, 0, 0, 0};
-        if (u == 0)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = (short)f2bf(t.th[MLP_OFF_W4 + 8 * kb + 4 * hi + j]);
-        acc = mlp_mfma(operand(2, kb), b, acc);
+    for (int kb = 0; kb < 16; ++kb) {
+        const mlp_bf16x4 none = {0, 0, 0, 0}, b = mlp_load4(&w4s[8 * kb + 4 * hi]);
+        acc = mlp_mfma(operand(2, kb), u == 0 ? b : none, acc);
     }
     float dout[16], d[16];
     uint16_t eo[16];
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(MlpTrain t) {
         if (w == 3 && u == 0) ds[row_of(i)] = in ? e : 0.0f;
     }
     // dZ3 = (dout w4) SiLU'(Z3): the product of two BF16 values is exact
-    const float w4b = bf2f(f2bf(w4));
+    const float w4b = bf2f(w4);
     auto back = [&](float dh, float z) {
         const float s = mlp_sigmoid(z);
         dh *= s * (1.0f + z * (1.0f - s));
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(MlpTrain t) {
     if (w == 2 && u == 0)
 #pragma unroll
         for (int i = 0; i < 16; ++i) t.dout[row0 + row_of(i)] = dout[i];
-    __syncthreads();
+    pimc::lds_barrier();
     if (w == 3) {  // loss: (1/2n) sum (out - y)^2
         const float e = u == l ? ds[u] : 0.0f;
         double s = 0.5 * (double)e * (double)e / (double)t.B;
@@ -381,7 +383,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(MlpTrain t) {
     for (int i = 0; i < 16; ++i) d[i] = back(acc[i], z2[i]);
     put(4, d, 4);
     put_dz(1, d);
-    __syncthreads();
+    pimc::lds_barrier();
     acc = product(4, wt[2]);
     uint16_t e[16];
 #pragma unroll
@@ -409,13 +411,13 @@ __device__ __forceinline__ float mlp_adam(float th, float gi, float& m, float& v
 
 // Weight gradients of a batch and the step on the weights.  Blocks 0..39 take a 32x32 tile of dW3,
 // dW2, dW4 and dW1 = dZ^T H each: one wave runs the chain of products over the batch from LDS while
-// all four bring in the chunks after it, the next in LDS's other half and the one after that in
-// registers.  The other blocks sum biases: 16 columns of a dZ each, and dout.
+// the other three bring in the chunks after it, the next in LDS's other half and the one after that
+// in registers.  The other blocks sum biases: 16 columns of a dZ each, and dout.
 constexpr int MLP_TILE_JOBS = 40, MLP_COL = 16, MLP_COL_JOBS = 3 * MLP_H / MLP_COL;
 constexpr int MLP_GRAD_JOBS = MLP_TILE_JOBS + MLP_COL_JOBS + 1;
-constexpr int MLP_CHUNK = 16;                           // groups of 16 rows staged at a time
+constexpr int MLP_CHUNK = 24;                           // groups of 16 rows staged at a time
 constexpr int MLP_CHUNK_Q = MLP_CHUNK * 64;             // 16-byte words of one operand of a chunk
-constexpr int MLP_CHUNK_T = MLP_CHUNK_Q / 256;          // of them per lane
+constexpr int MLP_CHUNK_T = MLP_CHUNK_Q / 192;          // of them per lane of three waves
 constexpr int MLP_GRAD_LDS = 4 * MLP_CHUNK_Q * 16;      // two operands, two buffers
 
 __global__ __launch_bounds__(256) void k_mlp_grads(MlpTrain t, MlpAdam ad) {
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(256) void k_mlp_grads(MlpTrain t, MlpAdam ad) {
     auto fetch = [&](int c, Words& r) {
 #pragma unroll
         for (int k = 0; k < MLP_CHUNK_T; ++k) {
-            const int q = tid + 256 * k, grp = c * MLP_CHUNK + (q >> 6);
+            const int q = tid - 64 + 192 * k, grp = c * MLP_CHUNK + (q >> 6);
             r.a[k] = r.b[k] = make_uint4(0, 0, 0, 0);
             if (grp < ng) {
                 r.a[k] = A[(size_t)grp * 256 + (q & 63)];
@@ -507,16 +509,18 @@ __global__ __launch_bounds__(256) void k_mlp_grads(MlpTrain t, MlpAdam ad) {
         uint4* d = mlp_lds + (c & 1) * 2 * MLP_CHUNK_Q;
 #pragma unroll
         for (int k = 0; k < MLP_CHUNK_T; ++k) {
-            d[tid + 256 * k] = r.a[k];
-            d[MLP_CHUNK_Q + tid + 256 * k] = r.b[k];
+            d[tid - 64 + 192 * k] = r.a[k];
+            d[MLP_CHUNK_Q + tid - 64 + 192 * k] = r.b[k];
         }
     };
     mlp_f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
     auto step = [&](int c, Words& next, Words& after) {
-        if (c + 2 < nchunk) fetch(c + 2, after);
-        if (chain) {
+        if (!chain) {
+            if (c + 2 < nchunk) fetch(c + 2, after);
+            if (c + 1 < nchunk) stage(c + 1, next);
+        } else {
             const uint4* s = mlp_lds + (c & 1) * 2 * MLP_CHUNK_Q;
 #pragma unroll
             for (int k = 0; k < MLP_CHUNK; ++k) {
@@ -525,14 +529,15 @@ __global__ __launch_bounds__(256) void k_mlp_grads(MlpTrain t, MlpAdam ad) {
                 acc = mlp_mfma(mlp_half(a, 1), mlp_half(b, 1), acc);
             }
         }
-        if (c + 1 < nchunk) stage(c + 1, next);
-        __syncthreads();
+        pimc::lds_barrier();
     };
     Words w0, w1;
-    fetch(0, w0);
-    if (nchunk > 1) fetch(1, w1);
-    stage(0, w0);
-    __syncthreads();
+    if (!chain) {
+        fetch(0, w0);
+        if (nchunk > 1) fetch(1, w1);
+        stage(0, w0);
+    }
+    pimc::lds_barrier();
     for (int c = 0; c < nchunk; c += 2) {
         step(c, w1, w0);
         if (c + 1 < nchunk) step(c + 1, w0, w1);
