@@ -1218,8 +1218,8 @@ int pimc_commit(pimc_ctx* c) {
     }
     // Non-linear chains split by slice range when whole chains would leave CUs idle: as many
     // parts (powers of two, at least 16 slices each) as the device holds resident at once, since
-    // the parts of a chain wait for one another.  With delayed acceptance every chain runs as
-    // parts of k_rotor3d_da, a short chain as one part.
+    // the parts of a chain wait for one another.  A short chain is one part, a long one that is not
+    // split goes to k_rotor3d; with delayed acceptance every chain runs as parts of k_rotor3d_da.
     if (!rot3.empty()) {
         hipDeviceProp_t prop;
         HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
@@ -1244,7 +1244,7 @@ int pimc_commit(pimc_ctx* c) {
         };
         const int W = plan_rotor3d_split(protmax, (int)rot3.size(), prop.multiProcessorCount,
                                          prop.multiProcessorCount / 8, lds_for, occupancy);
-        if (W > 1 || da) {
+        {
             std::vector<RotPart> p3;
             std::vector<int> whole;
             for (int r : rot3) {
@@ -1252,7 +1252,7 @@ int pimc_commit(pimc_ctx* c) {
                 int ns = ((p.Prot + W - 1) / W + 1) & ~1;
                 if (ns > p.Prot) ns = p.Prot;
                 const int Wr = (p.Prot + ns - 1) / ns;
-                if (Wr < 2 && !da) {
+                if (Wr < 2 && !da && p.nrot * p.Prot > ROT3D_AHEAD) {
                     whole.push_back(r);
                     continue;
                 }

@@ -1380,8 +1380,8 @@ __global__ __launch_bounds__(BLOCK) void k_rotor3d(const Rep* __restrict__ reps,
                     double chi = cur.chi + twopi * (rp.rtstep * (rand3 - 0.5));
                     if (phi < 0.0) phi = twopi + phi;
                     if (chi < 0.0) chi = twopi + chi;
-                    phi = fmod(phi, twopi);
-                    chi = fmod(chi, twopi);
+                    phi = fmod_near(phi, twopi);
+                    chi = fmod_near(chi, twopi);
                     if (cost > 1.0) cost = 2.0 - cost;
                     if (cost < -1.0) cost = -2.0 - cost;
                     if (gl == 0) gf[nrot] = make_frame(phi, cost, chi);
@@ -1453,26 +1453,578 @@ __global__ __launch_bounds__(BLOCK) void k_rotor3d(const Rep* __restrict__ reps,
     }
 }
 
-// MCRotations3D with a chain split over W >= 2 workgroups by slice range [k0, k1) (even
-// length), as k_rotor splits linear chains: a half-sweep is a parallel step over the part's
-// slices with the moves of k_rotor3d.  Before its even half a part needs the frames of slice
-// k0-1 (the previous part's last, odd) and before its odd half those of slice k1 (the next
-// part's first, even).  After its even half a part publishes its first slice's frames, after its
-// odd half its last slice's, each with the density of its link to the neighbour, as a record of
-// 64-bit words that each carry the publishing half's number above 32 bits of a double; the
-// receiver's lanes poll the words themselves, so the data arrives with its check, and write the
-// halves into LDS.  A record is rewritten only after the neighbour has read it (its next half
-// needs this part's).  Bounded waits set error bit 2.
+// MCRotations3D by parts: a chain split over W workgroups by slice range [k0, k1) (even length), or
+// a short chain as one part.  A half-sweep is a parallel step over the part's slices.  Before its
+// even half a part needs the frames of slice k0-1 (the previous part's last, odd) and before its
+// odd half those of slice k1 (the next part's first, even).  After its even half a part publishes
+// its first slice's frames, after its odd half its last slice's, each with the density of its link
+// to the neighbour, as a record of 64-bit words that each carry the publishing half's number above
+// 32 bits of a double; the receiver's lanes poll the words themselves, so the data arrives with its
+// check, and write the halves into LDS.  A record is rewritten only after the neighbour has read it
+// (its next half needs this part's).  Bounded waits set error bit 2.
 // Record (part, parity) at pub + part * pub_stride + parity * pub_stride / 2: 2 words per double
 // of the nrot frames, then of the nrot link densities.
-// LDS: Lk[q][kl], kl = 0..ns (link kl joins local slices kl and kl+1; local slice 0 is k0-1 and
-// ns+1 is k1), the neighbours' frames fnb[2][nrot] (k0-1, then k1), then the groups' frames.
+// Link kl joins local slices kl and kl+1; local slice 0 is k0-1 and ns+1 is k1.  A link's density,
+// a rotor's sum over atoms and the pair energy of two rotors are kept as the last accepted move (or
+// the launch's start) left them, so a move evaluates its proposal alone.
+//
+// Two bodies, by the part's length.  Short parts (nrot ns <= ROT3D_AHEAD: few chains, many parts)
+// are bound by the chain of half-sweeps and take a group of lanes per move; what depends on the
+// slice alone is formed a sweep ahead (rotor3d_ahead).  Long parts (many chains: the device is full)
+// are bound by the FP64 instructions of a move and take a lane per move (rotor3d_long).
+constexpr int FRAME_D = (int)(sizeof(Frame) / sizeof(double));
+
+struct Rot3dEnv {
+    const Rep& rp;
+    const double4* beads;
+    RotBead* rotb;
+    Frame* frames;
+    const double4* tab;
+    unsigned seed;
+    uint32_t pass;
+    int nsweep, j0, jstride;
+    unsigned base;                    // half-sweeps done by the launches before this one
+    unsigned long long* mypub;        // + parity * half_rec
+    const unsigned long long* from[2];  // the records an even and an odd half wait for
+    int half_rec;
+    __device__ __forceinline__ uint32_t sweep(int sw) const { return (uint32_t)(j0 + sw * jstride); }
+    __device__ __forceinline__ long long at(int q, int k) const { return rp.rot_off + (long long)q * rp.Prot + k; }
+};
+
+struct Prop3 {
+    double phi, cth, chi, u;
+};
+
+// MCRot3Dstep's proposal for rotor q at slice k (mc_piqmc.cc:966-1010)
+__device__ __forceinline__ Prop3 rot3d_propose(const Rot3dEnv& e, int q, int k, uint32_t jsweep, double phi, double cth,
+                                               double chi) {
+    const double twopi = 2.0 * PI_D;
+    const uint32_t atom = (uint32_t)(e.rp.nl_atom + q);
+    const uint4 w0 = draw(e.seed, e.rp.key, e.pass, K_ROT3D, jsweep, atom, (uint32_t)k, 0);
+    const uint4 w1 = draw(e.seed, e.rp.key, e.pass, K_ROT3D, jsweep, atom, (uint32_t)k, 1);
+    const double rand1 = u53(w0.x, w0.y), rand2 = u53(w0.z, w0.w), rand3 = u53(w1.x, w1.y);
+    Prop3 p;
+    p.u = u53(w1.z, w1.w);
+    p.cth = cth + e.rp.rtstep * (rand1 - 0.5);
+    p.phi = phi + twopi * (e.rp.rtstep * (rand2 - 0.5));
+    p.chi = chi + twopi * (e.rp.rtstep * (rand3 - 0.5));
+    if (p.phi < 0.0) p.phi = twopi + p.phi;
+    if (p.chi < 0.0) p.chi = twopi + p.chi;
+    p.phi = fmod_near(p.phi, twopi);
+    p.chi = fmod_near(p.chi, twopi);
+    if (p.cth > 1.0) p.cth = 2.0 - p.cth;
+    if (p.cth < -1.0) p.cth = -2.0 - p.cth;
+    return p;
+}
+
+// the test of MCRot3Dstep (mc_piqmc.cc:1134-1178): link densities d0 d1 (now) and d2 d3 (proposed)
+__device__ __forceinline__ bool rot3d_accept(double d0, double d1, double d2, double d3, double taudv, double u) {
+    double dold = d0 * d1;
+    if (fabs(dold) < RZERO) dold = 0.0;
+    if (dold < 0.0) dold = fabs(dold);
+    double dnew = d2 * d3;
+    if (fabs(dnew) < RZERO) dnew = 0.0;
+    if (dnew < 0.0) dnew = fabs(dnew);
+    double rd = (dold > RZERO) ? dnew / dold : 1.0;
+    rd *= exp(-taudv);
+    return rd > 1.0 || rd > u;
+}
+
+__device__ __forceinline__ void rot3d_store(const Rot3dEnv& e, long long i, double phi, double cth, double chi, const Frame& f) {
+    RotBead b;
+    b.phi = phi;
+    b.cth = cth;
+    b.chi = chi;
+    b.pad0 = 0.0;
+    b.nx = f.m[6];  // the axis is the frame's third column
+    b.ny = f.m[7];
+    b.nz = f.m[8];
+    b.pad1 = 0.0;
+    e.rotb[i] = b;
+    e.frames[i] = f;
+}
+
+// one word of the neighbour's record, polled until it carries the half's number
+__device__ __forceinline__ unsigned rot3d_word(const unsigned long long* src, unsigned want, int* s_err) {
+    unsigned long long w = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned spins = 0;
+    while ((unsigned)(w >> 32) != want) {
+        if (++spins > ROT_SPIN_LIMIT) {
+            *s_err = 2;
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        w = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return (unsigned)w;
+}
+
+__device__ __forceinline__ unsigned long long rot3d_pack(double v, int word, unsigned tag) {
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    return (unsigned long long)tag << 32 | (word ? bits >> 32 : bits & 0xffffffffull);
+}
+
+// Short parts.  A half-sweep of a part is a chain: the neighbour's record, the link densities (angles
+// of two frames, a gather from a table of 750 MB), the test, the record for the neighbour.  All else
+// of a move depends on its slice alone: the draws, the proposal's frame, its energies with the atoms
+// and (two rotors) with the other rotor, moved or not; these are formed right after the slice's
+// previous move, while the records travel.  Frames, proposals and energies live in LDS for the
+// launch, a group's lanes read a move's alike, one lane per new link evaluates its density, and only
+// the waves with a boundary slice trade records, without a barrier of the block.
+// With everything formed inside the half and the state in memory, a half of 16 slices and 32 atoms
+// took 9.3 us.
+// LDS: Lk[q][ns+1], then frames fr[q][ns+2] and proposals' frames fp[q][ns], then sl[q][ns] and, with
+// two rotors, pr[ns].
+template <typename R, int NROT>
+__device__ __forceinline__ void rotor3d_ahead(const Rot3dEnv& e, const RotPart& pt, const Lut3D<R>& l3, double* smem, int* s_err,
+                                              unsigned long long& nacc, int& err) {
+    struct Slice {
+        double phi, cth, chi, E;  // now; E the sum over atoms
+        double Enew;
+        Prop3 p;
+    };
+    struct Pair {
+        double E, v[3];  // now; of (q0', q1), (q0, q1') and (q0', q1')
+    };
+    static_assert(sizeof(Slice) == 9 * sizeof(double) && sizeof(Pair) == 4 * sizeof(double), "rotor3d_part_lds");
+    const Rep& rp = e.rp;
+    const int k0 = pt.k0, ns = pt.k1 - pt.k0, W = pt.W, L = ns + 1, Prot = rp.Prot, RR = rp.RotRatio, nat = rp.nl_atom;
+    double* Lk = smem;
+    Frame* fr = reinterpret_cast<Frame*>(smem + ((NROT * L + 1) & ~1));
+    Frame* fp = fr + NROT * (ns + 2);
+    Slice* sl = reinterpret_cast<Slice*>(fp + NROT * ns);
+    Pair* pr = reinterpret_cast<Pair*>(sl + NROT * ns);
+    const int nmoves = ns >> 1;  // of either parity: k0 and ns are even
+    int G = 1;
+    while (G < 64 && G * 2 * nmoves <= (int)blockDim.x) G *= 2;
+    const int mv = (int)threadIdx.x / G, gl = (int)threadIdx.x & (G - 1), lane = threadIdx.x & 63, gbase = lane & ~(G - 1);
+    const bool mine = mv < nmoves;
+    const int items_a = RR * nat;
+    for (int i = threadIdx.x; i < NROT * (ns + 2); i += blockDim.x) {
+        const int q = i / (ns + 2);
+        int k = k0 + i - q * (ns + 2) - 1;
+        if (k < 0) k += Prot;
+        if (k >= Prot) k -= Prot;
+        fr[i] = e.frames[e.at(q, k)];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < NROT * L; i += blockDim.x) {
+        const int q = i / L, kl = i - q * L;
+        if (rotden_rho(fr[q * (ns + 2) + kl], fr[q * (ns + 2) + kl + 1], e.tab, Lk[i])) err = 1;
+    }
+    // separations of the lane's first atom of the sums at its even and odd slice: atoms stay during the launch
+    R sep[2][NROT][3];
+    auto atom_sum = [&](int parity, int q, int k, const Frame& f) -> double {
+        double v = 0.0;
+        if (gl < items_a)
+            v = (double)vcord_sep<R>(l3, f, parity ? sep[1][q][0] : sep[0][q][0], parity ? sep[1][q][1] : sep[0][q][1],
+                                     parity ? sep[1][q][2] : sep[0][q][2]);
+        for (int i = gl + G; i < items_a; i += G) {
+            const int it = k * RR + i / nat, a = i % nat;
+            const double4 xa = bead(e.beads, rp, nat + q, it), xj = bead(e.beads, rp, a, it);
+            v += (double)vcord_v<R>(l3, f, xa.x, xa.y, xa.z, xj.x, xj.y, xj.z);
+        }
+        return group_sum(v, G);
+    };
+    auto pair = [&](int k, int s, const Frame& f0, const Frame& f1) -> double {
+        const double4 x0 = bead(e.beads, rp, nat, k * RR + s), x1 = bead(e.beads, rp, nat + 1, k * RR + s);
+        return caleng_v(x0.x, x0.y, x0.z, x1.x, x1.y, x1.z, f0, f1);
+    };
+    auto ahead = [&](int parity, int sw) {
+        const int kl = 2 * mv + parity + 1, k = k0 + kl - 1;
+#pragma unroll
+        for (int q = 0; q < NROT; ++q) {
+            Slice& s = sl[q * ns + kl - 1];
+            const Prop3 p = rot3d_propose(e, q, k, e.sweep(sw), s.phi, s.cth, s.chi);
+            const Frame f = make_frame(p.phi, p.cth, p.chi);
+            double ea = 0.0;
+            if (nat > 0) ea = atom_sum(parity, q, k, f);
+            if (gl == 0) {
+                fp[q * ns + kl - 1] = f;
+                s.p = p;
+                s.Enew = ea;
+            }
+        }
+        wave_sync();
+        if constexpr (NROT == 2) {
+            double v0 = 0.0, v1 = 0.0, v2 = 0.0;
+#pragma unroll 1
+            for (int i = gl; i < 3 * RR; i += G) {
+                const int s = i / 3, c = i - 3 * s;
+                const double v = pair(k, s, c == 1 ? fr[kl] : fp[kl - 1], c == 0 ? fr[ns + 2 + kl] : fp[ns + kl - 1]);
+                v0 += c == 0 ? v : 0.0;
+                v1 += c == 1 ? v : 0.0;
+                v2 += c == 2 ? v : 0.0;
+            }
+            v0 = group_sum(v0, G);
+            v1 = group_sum(v1, G);
+            v2 = group_sum(v2, G);
+            if (gl == 0) {
+                pr[kl - 1].v[0] = v0;
+                pr[kl - 1].v[1] = v1;
+                pr[kl - 1].v[2] = v2;
+            }
+        }
+    };
+    unsigned moved = 0;  // bit parity * NROT + q: the slice's rotor q was moved in this launch
+    if (mine) {
+#pragma unroll
+        for (int parity = 0; parity < 2; ++parity)
+#pragma unroll
+            for (int q = 0; q < NROT; ++q) {
+                sep[parity][q][0] = sep[parity][q][1] = sep[parity][q][2] = (R)0;
+                if (gl < items_a) {
+                    const int it = (k0 + 2 * mv + parity) * RR + gl / nat, a = gl % nat;
+                    const double4 xa = bead(e.beads, rp, nat + q, it), xj = bead(e.beads, rp, a, it);
+                    sep[parity][q][0] = (R)(xj.x - xa.x);
+                    sep[parity][q][1] = (R)(xj.y - xa.y);
+                    sep[parity][q][2] = (R)(xj.z - xa.z);
+                }
+            }
+#pragma unroll 1
+        for (int parity = 0; parity < 2; ++parity) {
+            const int kl = 2 * mv + parity + 1, k = k0 + kl - 1;
+#pragma unroll
+            for (int q = 0; q < NROT; ++q) {
+                const RotBead& b = e.rotb[e.at(q, k)];
+                double ea = 0.0;
+                if (nat > 0) ea = atom_sum(parity, q, k, fr[q * (ns + 2) + kl]);
+                if (gl == 0) {
+                    Slice& s = sl[q * ns + kl - 1];
+                    s.phi = b.phi;
+                    s.cth = b.cth;
+                    s.chi = b.chi;
+                    s.E = ea;
+                }
+            }
+            if constexpr (NROT == 2) {
+                double v = 0.0;
+#pragma unroll 1
+                for (int s = gl; s < RR; s += G) v += pair(k, s, fr[kl], fr[ns + 2 + kl]);
+                v = group_sum(v, G);
+                if (gl == 0) pr[kl - 1].E = v;
+            }
+            wave_sync();
+            ahead(parity, 0);
+        }
+    }
+    __syncthreads();  // Lk
+    const int nwords = 2 * NROT * (FRAME_D + 1);
+#pragma unroll 1
+    for (int h = 0; h < 2 * e.nsweep; ++h) {
+        const int parity = h & 1, sw = h >> 1;
+        const int kl = 2 * mv + parity + 1;
+        const int bnd = parity == 0 ? 0 : nmoves - 1;  // the move beside the neighbour this half trades with
+        const bool trader = W > 1 && (bnd * G) >> 6 == (int)threadIdx.x >> 6;
+        if (trader && h > 0) {
+            const int kn = parity == 0 ? 0 : ns + 1, ln = parity == 0 ? 0 : ns;
+            for (int w = lane; w < nwords; w += 64) {
+                const unsigned v = rot3d_word(e.from[parity] + w, e.base + (unsigned)h, s_err);
+                const int i = w >> 1;  // the double: frames first, then link densities
+                double* d = i < NROT * FRAME_D ? reinterpret_cast<double*>(fr + (i / FRAME_D) * (ns + 2) + kn) + i % FRAME_D
+                                               : Lk + (i - NROT * FRAME_D) * L + ln;
+                reinterpret_cast<unsigned*>(d)[w & 1] = v;
+            }
+            wave_sync();
+        }
+        if (mine) {
+            const int c = gl & (2 * NROT - 1), lq = c >> 1, side = c & 1;
+            double rho;
+            if (rotden_link(fr[lq * (ns + 2) + kl - 1 + 2 * side], fp[lq * ns + kl - 1], side, e.tab, rho)) err = 1;
+            bool acc0 = false;
+#pragma unroll
+            for (int q = 0; q < NROT; ++q) {
+                Slice& s = sl[q * ns + kl - 1];
+                const double d2 = __shfl(rho, gbase + 2 * q), d3 = __shfl(rho, gbase + 2 * q + 1);
+                double dv = s.Enew - s.E, pe = 0.0;
+                if constexpr (NROT == 2) {
+                    const Pair& p = pr[kl - 1];
+                    pe = q == 0 ? p.v[0] : (acc0 ? p.v[2] : p.v[1]);
+                    dv = (s.Enew + pe) - (s.E + p.E);
+                }
+                const bool accepted = rot3d_accept(Lk[q * L + kl - 1], Lk[q * L + kl], d2, d3, rp.tau * dv, s.p.u);
+                wave_sync();  // every lane has read the old state
+                if (accepted) {
+                    if (q == 0) acc0 = true;
+                    moved |= 1u << (parity * NROT + q);
+                    const double* src = reinterpret_cast<const double*>(fp + q * ns + kl - 1);
+                    double* dst = reinterpret_cast<double*>(fr + q * (ns + 2) + kl);
+                    // a chain in one part is its own neighbour: slices 0 and ns are one, ns + 1 and 1,
+                    // links 0 and ns; the other copy of a boundary slice
+                    const bool twin = W == 1 && (kl == 1 || kl == ns);
+                    double* dst2 = reinterpret_cast<double*>(fr + q * (ns + 2) + (kl == 1 ? ns + 1 : 0));
+                    for (int i = gl; i < FRAME_D; i += G) {
+                        dst[i] = src[i];
+                        if (twin) dst2[i] = src[i];
+                    }
+                    if (gl == 0) {
+                        ++nacc;
+                        s.phi = s.p.phi;
+                        s.cth = s.p.cth;
+                        s.chi = s.p.chi;
+                        s.E = s.Enew;
+                        if constexpr (NROT == 2) pr[kl - 1].E = pe;
+                        Lk[q * L + kl - 1] = d2;
+                        Lk[q * L + kl] = d3;
+                        if (twin) Lk[q * L + (kl == 1 ? ns : 0)] = kl == 1 ? d2 : d3;
+                    }
+                }
+                wave_sync();
+            }
+        }
+        if (trader) {  // publish the boundary slice; no wait for the stores, the reader checks every word
+            wave_sync();
+            const int kb = parity == 0 ? 1 : ns, lb = parity == 0 ? 0 : ns;
+            for (int w = lane; w < nwords; w += 64) {
+                const int i = w >> 1;
+                const double v = i < NROT * FRAME_D ? reinterpret_cast<const double*>(fr + (i / FRAME_D) * (ns + 2) + kb)[i % FRAME_D]
+                                                    : Lk[(i - NROT * FRAME_D) * L + lb];
+                __hip_atomic_store(e.mypub + parity * e.half_rec + w, rot3d_pack(v, w & 1, e.base + (unsigned)h + 1u), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if (mine && sw + 1 < e.nsweep) ahead(parity, sw + 1);
+        lds_barrier();
+        // a wait that gave up: no later wait of this launch can succeed either, so the part leaves
+        // at once (every lane reads s_err after the barrier; it is written again in the next half)
+        if (*s_err) break;
+    }
+    if (mine && gl == 0)
+#pragma unroll
+        for (int parity = 0; parity < 2; ++parity) {
+            const int kl = 2 * mv + parity + 1;
+#pragma unroll
+            for (int q = 0; q < NROT; ++q) {
+                const Slice& s = sl[q * ns + kl - 1];
+                if (moved >> (parity * NROT + q) & 1) rot3d_store(e, e.at(q, k0 + kl - 1), s.phi, s.cth, s.chi, fr[q * (ns + 2) + kl]);
+            }
+        }
+}
+
+// Long parts: a lane per move.  With many chains the device is full and the time is a move's FP64
+// instructions (two generator calls, the frame, six arc cosines, an energy) and what it reads: its
+// neighbours' and partner's frames, its angles, and two gathers for its links.  InLds keeps the chain's
+// state in LDS for the launch, which leaves the gathers and positions to memory: of a frame the x and
+// z axes (y is their cross product) and of the angles phi and chi (cos theta is the z axis' third
+// component), 72 bytes a rotor and slice with the link's density, so that two parts of 512 slices of
+// two rotors share a CU.  Even and odd slices lie apart: the lanes' accesses then meet no bank twice.
+// Otherwise (rotor3d_in_lds) state is read and written in memory.
+// LDS: Lk[q][ns+1], Ea[q][ns] (sum over atoms) with atoms, Er[ns] (pair energy) with two rotors, then
+// axes[q][ns+2] and angles[q][ns], or the neighbours' frames fnb[2][nrot] (k0-1, then k1).
+template <typename R, int NROT, bool InLds>
+__device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& pt, const Lut3D<R>& l3, double* smem, int* s_err,
+                                             unsigned long long& nacc, int& err) {
+    struct alignas(16) Axes {
+        double x[3], z[3];
+    };
+    struct alignas(16) Angles {
+        double phi, chi;
+    };
+    const Rep& rp = e.rp;
+    const int k0 = pt.k0, ns = pt.k1 - pt.k0, L = ns + 1, Prot = rp.Prot, RR = rp.RotRatio, nat = rp.nl_atom;
+    double* Lk = smem;
+    double* Ea = Lk + NROT * L;
+    double* Er = Ea + (nat > 0 ? NROT * ns : 0);
+    double* rest = smem + ((NROT * L + (nat > 0 ? NROT * ns : 0) + (NROT - 1) * ns + 1) & ~1);
+    Frame* fnb = reinterpret_cast<Frame*>(rest);
+    Axes* ax = reinterpret_cast<Axes*>(rest);
+    Angles* ang = reinterpret_cast<Angles*>(ax + NROT * (ns + 2));
+    const int half_ns = ns >> 1;
+    auto axes = [&](int q, int kl) -> Axes& { return ax[q * (ns + 2) + (kl & 1) * (half_ns + 1) + (kl >> 1)]; };
+    auto angles = [&](int q, int kl) -> Angles& { return ang[q * ns + ((kl - 1) & 1) * half_ns + ((kl - 1) >> 1)]; };
+    auto slice = [&](int kl) {  // of local slice kl
+        const int k = k0 + kl - 1;
+        return k < 0 ? k + Prot : (k >= Prot ? k - Prot : k);
+    };
+    // the frame of rotor q at local slice kl (zn left out: it is asked of proposals only)
+    auto frame = [&](int q, int kl) -> Frame {
+        if constexpr (InLds) {
+            const Axes& a = axes(q, kl);
+            Frame f;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                f.m[i] = a.x[i];
+                f.m[6 + i] = a.z[i];
+            }
+            f.m[3] = f.m[7] * f.m[2] - f.m[8] * f.m[1];
+            f.m[4] = f.m[8] * f.m[0] - f.m[6] * f.m[2];
+            f.m[5] = f.m[6] * f.m[1] - f.m[7] * f.m[0];
+            f.zn = 1.0;
+            return f;
+        } else {
+            return kl == 0 ? fnb[q] : (kl == ns + 1 ? fnb[NROT + q] : e.frames[e.at(q, k0 + kl - 1)]);
+        }
+    };
+    auto set_axes = [&](int q, int kl, const Frame& f) {
+        Axes& a = axes(q, kl);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            a.x[i] = f.m[i];
+            a.z[i] = f.m[6 + i];
+        }
+    };
+    // at launch start no neighbour has moved its boundary slice yet (its first move on it waits
+    // for this part), so the boundary frames come straight from memory
+    if constexpr (InLds) {
+        for (int i = threadIdx.x; i < NROT * (ns + 2); i += blockDim.x) {
+            const int q = i / (ns + 2), kl = i - q * (ns + 2);
+            set_axes(q, kl, e.frames[e.at(q, slice(kl))]);
+            if (kl > 0 && kl <= ns) {
+                const RotBead& b = e.rotb[e.at(q, slice(kl))];
+                angles(q, kl) = {b.phi, b.chi};
+                axes(q, kl).z[2] = b.cth;
+            }
+        }
+    } else {
+        for (int i = threadIdx.x; i < 2 * NROT; i += blockDim.x) {
+            const int side = i / NROT, q = i - side * NROT;
+            fnb[i] = e.frames[e.at(q, slice(side ? ns + 1 : 0))];
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < NROT * L; i += blockDim.x) {
+        const int q = i / L, kl = i - q * L;
+        if (rotden_rho(frame(q, kl), frame(q, kl + 1), e.tab, Lk[i])) err = 1;
+    }
+    auto atom_sum = [&](int q, int k, const Frame& f) -> double {
+        double v = 0.0;
+        for (int s = 0; s < RR; ++s) {
+            const double4 xa = bead(e.beads, rp, nat + q, k * RR + s);
+            for (int a = 0; a < nat; ++a) {
+                const double4 xj = bead(e.beads, rp, a, k * RR + s);
+                v += (double)vcord_v<R>(l3, f, xa.x, xa.y, xa.z, xj.x, xj.y, xj.z);
+            }
+        }
+        return v;
+    };
+    auto pair = [&](int k, int q, const Frame& f, const Frame& fo) -> double {  // rotor q at f, the other at fo
+        double v = 0.0;
+#pragma unroll 1
+        for (int s = 0; s < RR; ++s) {
+            const double4 x = bead(e.beads, rp, nat + q, k * RR + s), xo = bead(e.beads, rp, nat + 1 - q, k * RR + s);
+            v += caleng_v(x.x, x.y, x.z, xo.x, xo.y, xo.z, f, fo);
+        }
+        return v;
+    };
+    for (int i = threadIdx.x; i < ns; i += blockDim.x) {
+        if (nat > 0)
+#pragma unroll
+            for (int q = 0; q < NROT; ++q) Ea[q * ns + i] = atom_sum(q, k0 + i, e.frames[e.at(q, k0 + i)]);
+        if constexpr (NROT == 2) Er[i] = pair(k0 + i, 0, frame(0, i + 1), frame(1, i + 1));
+    }
+    __syncthreads();
+    const int nwords = 2 * NROT * (FRAME_D + 1);
+    unsigned moved = 0;  // InLds: bit (move / lanes) 2 NROT + parity NROT + q, the slices to write back
+#pragma unroll 1
+    for (int h = 0; h < 2 * e.nsweep; ++h) {
+        const int parity = h & 1, sw = h >> 1;
+        if (h > 0) {
+            const int kn = parity == 0 ? 0 : ns + 1, ln = parity == 0 ? 0 : ns;
+            for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
+                const unsigned v = rot3d_word(e.from[parity] + w, e.base + (unsigned)h, s_err);
+                const int i = w >> 1, q = i / FRAME_D, c = i - q * FRAME_D;  // the double: frames first, then link densities
+                if (q >= NROT) {
+                    reinterpret_cast<unsigned*>(&Lk[(i - NROT * FRAME_D) * L + ln])[w & 1] = v;
+                } else if constexpr (InLds) {
+                    if (c < 3) reinterpret_cast<unsigned*>(&axes(q, kn).x[c])[w & 1] = v;
+                    else if (c >= 6 && c < 9) reinterpret_cast<unsigned*>(&axes(q, kn).z[c - 6])[w & 1] = v;
+                } else {
+                    reinterpret_cast<unsigned*>(fnb + (parity == 0 ? 0 : NROT))[w] = v;
+                }
+            }
+            __syncthreads();
+            if (*s_err) break;  // as in rotor3d_ahead
+        }
+        unsigned bit = parity * NROT;
+#pragma unroll 1
+        for (int mv = threadIdx.x; mv < half_ns; mv += blockDim.x, bit += 2 * NROT) {
+            const int kl = 2 * mv + parity + 1, k = k0 + kl - 1;
+#pragma unroll 1
+            for (int q = 0; q < NROT; ++q) {
+                const long long ik = e.at(q, k);
+                double phi, cth, chi;
+                if constexpr (InLds) {
+                    phi = angles(q, kl).phi;
+                    chi = angles(q, kl).chi;
+                    cth = axes(q, kl).z[2];
+                } else {
+                    const RotBead& cur = e.rotb[ik];
+                    phi = cur.phi;
+                    cth = cur.cth;
+                    chi = cur.chi;
+                }
+                const Prop3 p = rot3d_propose(e, q, k, e.sweep(sw), phi, cth, chi);
+                const Frame f = make_frame(p.phi, p.cth, p.chi);
+                RhoCell left, right;  // the gathers are asked for before the energy and read after it
+                if (rotden_cell(frame(q, kl - 1), f, 0, e.tab, left)) err = 1;
+                if (rotden_cell(frame(q, kl + 1), f, 1, e.tab, right)) err = 1;
+                double ea = 0.0, pe = 0.0, dv = 0.0;
+                if (nat > 0) {
+                    ea = atom_sum(q, k, f);
+                    dv = ea - Ea[q * ns + kl - 1];
+                }
+                if constexpr (NROT == 2) {  // rotor 1 sees rotor 0's move
+                    pe = pair(k, q, f, frame(1 - q, kl));
+                    dv = (ea + pe) - ((nat > 0 ? Ea[q * ns + kl - 1] : 0.0) + Er[kl - 1]);
+                }
+                const double d2 = rho_value(left), d3 = rho_value(right);
+                if (rot3d_accept(Lk[q * L + kl - 1], Lk[q * L + kl], d2, d3, rp.tau * dv, p.u)) {
+                    ++nacc;
+                    if constexpr (InLds) {
+                        set_axes(q, kl, f);
+                        angles(q, kl) = {p.phi, p.chi};
+                        moved |= 1u << (bit + q);
+                    } else {
+                        rot3d_store(e, ik, p.phi, p.cth, p.chi, f);
+                    }
+                    Lk[q * L + kl - 1] = d2;
+                    Lk[q * L + kl] = d3;
+                    if (nat > 0) Ea[q * ns + kl - 1] = ea;
+                    if constexpr (NROT == 2) Er[kl - 1] = pe;
+                }
+            }
+        }
+        __syncthreads();
+        // publish the boundary slice this half moved; no wait for the stores, the reader checks every word
+        const int kb = parity == 0 ? 1 : ns;
+        for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
+            const int i = w >> 1, q = i / FRAME_D;
+            double v;
+            if (q >= NROT) {
+                v = Lk[(i - NROT * FRAME_D) * L + (parity == 0 ? 0 : ns)];
+            } else {
+                const Frame f = frame(q, kb);
+                v = f.zn;
+#pragma unroll
+                for (int c = 0; c < 9; ++c)
+                    if (c == i - q * FRAME_D) v = f.m[c];
+            }
+            __hip_atomic_store(e.mypub + parity * e.half_rec + w, rot3d_pack(v, w & 1, e.base + (unsigned)h + 1u), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if constexpr (InLds) {
+#pragma unroll 1
+        for (int parity = 0; parity < 2; ++parity) {
+            unsigned bit = parity * NROT;
+            for (int mv = threadIdx.x; mv < half_ns; mv += blockDim.x, bit += 2 * NROT)
+#pragma unroll 1
+                for (int q = 0; q < NROT; ++q) {
+                    if (!(moved >> (bit + q) & 1)) continue;
+                    const int kl = 2 * mv + parity + 1;
+                    const double phi = angles(q, kl).phi, chi = angles(q, kl).chi, cth = axes(q, kl).z[2];
+                    rot3d_store(e, e.at(q, k0 + kl - 1), phi, cth, chi, make_frame(phi, cth, chi));
+                }
+        }
+    }
+}
+
 template <typename R>
-__global__ __launch_bounds__(256) void k_rotor3d_parts(const Rep* __restrict__ reps, Mut* __restrict__ mut,
-                                                       const double4* __restrict__ beads, RotBead* __restrict__ rotb,
-                                                       Frame* __restrict__ frames, Tables T, Tables3 T3,
-                                                       const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
-                                                       unsigned long long* __restrict__ pub, int pub_stride, Run run) {
+__global__ __launch_bounds__(256, 2) void k_rotor3d_parts(const Rep* __restrict__ reps, Mut* __restrict__ mut,
+                                                          const double4* __restrict__ beads, RotBead* __restrict__ rotb,
+                                                          Frame* __restrict__ frames, Tables T, Tables3 T3,
+                                                          const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
+                                                          unsigned long long* __restrict__ pub, int pub_stride, Run run) {
     extern __shared__ double smem[];
     __shared__ unsigned long long red_acc[4];
     __shared__ int s_err;
@@ -1481,245 +2033,48 @@ __global__ __launch_bounds__(256) void k_rotor3d_parts(const Rep* __restrict__ r
     const int r = pt.r;
     const Rep& rp = reps[r];
     if (rp.rotkind != 2 || rp.rot3d_id < 0) return;
-    const int Prot = rp.Prot, RR = rp.RotRatio, P = rp.P, N = rp.natoms, nrot = rp.nrot;
     int nsweep, j0, jstride;
     if (run.ref_order) {
-        if (run.u >= P) return;
+        if (run.u >= rp.P) return;
         nsweep = 1; j0 = run.u; jstride = 0;
     } else {
         if (run.u >= rp.S) return;
-        nsweep = P / rp.S; j0 = run.u; jstride = rp.S;
+        nsweep = rp.P / rp.S; j0 = run.u; jstride = rp.S;
     }
-    const int k0 = pt.k0, ns = pt.k1 - pt.k0, W = pt.W;
-    const int L = ns + 1;  // links per rotor
-    const int np = N - 1;
-    const int items = RR * np;
-    const long long rb0 = rp.rot_off;
-    const double4* tab = T3.r3 + (long long)rp.rot3d_id * 3 * ROT3D_SIZE;
-    const Lut1D<R> l1 = lut1d<R>(T, rp.pot1d_id);
-    const Lut3D<R> l3 = lut3d<R>(T3, rp.pot3d_id);
-    const int maxmoves = (ns + 1) / 2;
-    int G = 1;
-    while (G < 64 && G * 2 * maxmoves <= (int)blockDim.x) G *= 2;
-    const int groups = blockDim.x / G;
-    const int g = threadIdx.x / G, gl = threadIdx.x % G;
-    const int nat = rp.nl_atom;  // atoms come first: 0 .. nat-1
-    const int items_a = RR * nat, items_r = RR * (nrot - 1);
-    double* Lk = smem;
-    double* Ea = Lk + nrot * L;  // rotor-atom energy of every own slice at its current orientation
-    Frame* fnb = reinterpret_cast<Frame*>(smem + ((nrot * L + nrot * ns + 1) & ~1));
-    Frame* gf = fnb + 2 * nrot + (long long)g * (nrot + 1);
-    unsigned* myflag = flags + pt.fbase + pt.w;  // half-sweeps done by the launches before this one
-    constexpr int FD = (int)(sizeof(Frame) / sizeof(double));  // doubles per frame
-    const int nwords = 2 * nrot * (FD + 1);                      // words of one record
+    const int ns = pt.k1 - pt.k0, W = pt.W, nrot = rp.nrot;
+    unsigned* myflag = flags + pt.fbase + pt.w;
     const int half_rec = pub_stride / 2;
-    unsigned long long* mypub = pub + (long long)(pt.fbase + pt.w) * pub_stride;   // + parity * half_rec
-    const unsigned long long* prevlast = pub + (long long)(pt.fbase + (pt.w + W - 1) % W) * pub_stride + half_rec;
-    const unsigned long long* nextfirst = pub + (long long)(pt.fbase + (pt.w + 1) % W) * pub_stride;
-    const unsigned base = __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t pass = mut[r].pass;
-    const int rtype = rp.imtype;
-    const double twopi = 2.0 * PI_D;
-    auto own = [&](int q, int k) -> const Frame& { return frames[rb0 + (long long)q * Prot + k]; };
+    auto record = [&](int w, int parity) { return pub + (long long)(pt.fbase + w) * pub_stride + parity * half_rec; };
+    const Rot3dEnv e{rp, beads, rotb, frames, T3.r3 + (long long)rp.rot3d_id * 3 * ROT3D_SIZE, run.seed, mut[r].pass,
+                     nsweep, j0, jstride, __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                     record(pt.w, 0), {record((pt.w + W - 1) % W, 1), record((pt.w + 1) % W, 0)}, half_rec};
+    const Lut3D<R> l3 = lut3d<R>(T3, rp.pot3d_id);
     if (threadIdx.x == 0) s_err = 0;
     unsigned long long nacc = 0;
     int err = 0;
-    // at launch start no neighbour has moved its boundary slice yet (its first move on it waits
-    // for this part), so the boundary frames come straight from memory
-    for (int i = threadIdx.x; i < 2 * nrot; i += blockDim.x) {
-        const int side = i / nrot, q = i - side * nrot;
-        int k = side ? k0 + ns : k0 - 1;
-        if (k < 0) k += Prot;
-        if (k >= Prot) k -= Prot;
-        fnb[i] = own(q, k);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < nrot * L; i += blockDim.x) {
-        const int q = i / L, kl = i - q * L;
-        const Frame& fa = kl == 0 ? fnb[q] : own(q, k0 + kl - 1);
-        const Frame& fb = kl == ns ? fnb[nrot + q] : own(q, k0 + kl);
-        if (rotden_rho(fa, fb, tab, Lk[i])) err = 1;
-    }
-    // rotor-atom sums at the current orientations: atoms do not move during the sweep, so a
-    // move's old sum is this one or the new sum of the last move accepted at the slice (the same
-    // lanes add the same terms in the same order either way)
-    for (int kl = 1 + g; kl <= ns; kl += groups) {
-        const int k = k0 + kl - 1;
-        for (int q = 0; q < nrot; ++q) {
-            const int gatom = rp.nl_atom + q;
-            const Frame& fq = own(q, k);
-            double e = 0.0;
-            for (int i = gl; i < items_a; i += G) {
-                const int it = k * RR + i / nat, a = i % nat;
-                const double4 xa = bead(beads, rp, gatom, it), xj = bead(beads, rp, a, it);
-                e += (double)vcord_v<R>(l3, fq, xa.x, xa.y, xa.z, xj.x, xj.y, xj.z);
-            }
-            e = group_sum(e, G);
-            if (gl == 0) Ea[q * ns + kl - 1] = e;
-        }
-    }
-    __syncthreads();
-    for (int sw = 0; sw < nsweep; ++sw) {
-        const uint32_t jsweep = (uint32_t)(j0 + sw * jstride);
-        for (int parity = 0; parity < 2; ++parity) {
-            const unsigned h = 2u * (unsigned)sw + (unsigned)parity;  // half-sweeps done before this one
-            if (!(sw == 0 && parity == 0)) {
-                // even half: the previous part's record of its odd half of the last sweep; odd
-                // half: the next part's record of its even half of this sweep.  The neighbour's
-                // boundary frames, and the densities of the shared links that it evaluated from
-                // the same frames in the same order; each lane polls its own words.
-                const unsigned long long* src = parity == 0 ? prevlast : nextfirst;
-                unsigned* dstf = reinterpret_cast<unsigned*>(fnb + (parity == 0 ? 0 : nrot));
-                const unsigned want = base + h;
-                for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
-                    unsigned long long wv;
-                    unsigned spins = 0;
-                    for (;;) {
-                        wv = __hip_atomic_load(src + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        if ((unsigned)(wv >> 32) == want) break;
-                        if (++spins > ROT_SPIN_LIMIT) {
-                            s_err = 2;
-                            break;
-                        }
-                        __builtin_amdgcn_s_sleep(2);
-                    }
-                    const int i = w >> 1;  // the double: frames first, then link densities
-                    if (i < nrot * FD) dstf[w] = (unsigned)wv;
-                    else reinterpret_cast<unsigned*>(&Lk[(i - nrot * FD) * L + (parity == 0 ? 0 : ns)])[w & 1] = (unsigned)wv;
-                }
-                __syncthreads();
-                // a wait that gave up: no later wait of this launch can succeed either, so the
-                // part leaves at once (s_err is read by every lane after the barrier, and no lane
-                // writes it again before the barrier that closes this half)
-                if (s_err) {
-                    sw = nsweep;
-                    break;
-                }
-            }
-            const int nmoves = (ns - parity + 1) / 2;  // k0 is even: local slice kl has parity (kl - 1) & 1
-            for (int mv = g; mv < nmoves; mv += groups) {
-                const int kl = 2 * mv + parity + 1;
-                const int k = k0 + kl - 1;
-                for (int q = gl; q < nrot; q += G) gf[q] = own(q, k);
-                __builtin_amdgcn_wave_barrier();
-                for (int q = 0; q < nrot; ++q) {
-                    const int gatom = rp.nl_atom + q;
-                    const long long ik = rb0 + (long long)q * Prot + k;
-                    const RotBead cur = rotb[ik];
-                    const uint4 w0 = draw(run.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gatom, (uint32_t)k, 0);
-                    const uint4 w1 = draw(run.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gatom, (uint32_t)k, 1);
-                    const double rand1 = u53(w0.x, w0.y), rand2 = u53(w0.z, w0.w);
-                    const double rand3 = u53(w1.x, w1.y), rand4 = u53(w1.z, w1.w);
-                    double cost = cur.cth + rp.rtstep * (rand1 - 0.5);
-                    double phi = cur.phi + twopi * (rp.rtstep * (rand2 - 0.5));
-                    double chi = cur.chi + twopi * (rp.rtstep * (rand3 - 0.5));
-                    if (phi < 0.0) phi = twopi + phi;
-                    if (chi < 0.0) chi = twopi + chi;
-                    phi = fmod(phi, twopi);
-                    chi = fmod(chi, twopi);
-                    if (cost > 1.0) cost = 2.0 - cost;
-                    if (cost < -1.0) cost = -2.0 - cost;
-                    if (gl == 0) gf[nrot] = make_frame(phi, cost, chi);
-                    __builtin_amdgcn_wave_barrier();
-                    double d[4] = {Lk[q * L + kl - 1], Lk[q * L + kl], 0.0, 0.0};
-                    for (int c = 2 + gl; c < 4; c += G) {
-                        const Frame& fa = (c == 3) ? gf[nrot] : (kl == 1 ? fnb[q] : own(q, k - 1));
-                        const Frame& fb = (c == 2) ? gf[nrot] : (kl == ns ? fnb[nrot + q] : own(q, k + 1));
-                        if (rotden_rho(fa, fb, tab, d[c])) err = 1;
-                    }
-                    if (G > 1)
-                        for (int c = 2; c < 4; ++c) d[c] = __shfl(d[c], (c - 2) % G, G);
-                    // rotor-atom terms at the proposal (the old sum is cached), then the terms of
-                    // the other rotors at both orientations (a partner rotor may have moved)
-                    double ea = 0.0, eo = 0.0, en = 0.0;
-                    for (int i = gl; i < items_a; i += G) {
-                        const int it = k * RR + i / nat, a = i % nat;
-                        const double4 xa = bead(beads, rp, gatom, it), xj = bead(beads, rp, a, it);
-                        ea += (double)vcord_v<R>(l3, gf[nrot], xa.x, xa.y, xa.z, xj.x, xj.y, xj.z);
-                    }
-                    for (int i = gl; i < items_r; i += G) {
-                        const int it = k * RR + i / (nrot - 1), pp = i % (nrot - 1);
-                        const int p = pp + (pp >= q);
-                        const double4 xa = bead(beads, rp, gatom, it), xj = bead(beads, rp, rp.nl_atom + p, it);
-                        // the two orientations in turn, not interleaved: one caleng's sites
-                        // live at a time, which keeps the kernel within 256 registers (two
-                        // waves per SIMD, so two parts of a water chain share a CU)
-#pragma unroll 1
-                        for (int o = 0; o < 2; ++o) {
-                            const double e = caleng_v(xa.x, xa.y, xa.z, xj.x, xj.y, xj.z, gf[o ? nrot : q], gf[p]);
-                            if (o) en += e;
-                            else eo += e;
-                        }
-                    }
-                    for (int o = G >> 1; o > 0; o >>= 1) {  // the sums' shuffles interleave
-                        ea += __shfl_xor(ea, o, G);
-                        eo += __shfl_xor(eo, o, G);
-                        en += __shfl_xor(en, o, G);
-                    }
-                    const double ea_old = Ea[q * ns + kl - 1];
-                    eo += ea_old;
-                    en += ea;
-                    double dold = d[0] * d[1];
-                    if (fabs(dold) < RZERO) dold = 0.0;
-                    if (dold < 0.0) dold = fabs(dold);
-                    double dnew = d[2] * d[3];
-                    if (fabs(dnew) < RZERO) dnew = 0.0;
-                    if (dnew < 0.0) dnew = fabs(dnew);
-                    double rd = (dold > RZERO) ? dnew / dold : 1.0;
-                    rd *= exp(-rp.tau * (en - eo));
-                    const bool accepted = rd > 1.0 || rd > rand4;
-                    if (accepted && gl == 0) {
-                        ++nacc;
-                        const double sint = sqrt(1.0 - cost * cost);
-                        RotBead b = cur;
-                        b.cth = cost;
-                        b.phi = phi;
-                        b.chi = chi;
-                        b.nx = sint * cos(phi);
-                        b.ny = sint * sin(phi);
-                        b.nz = cost;
-                        rotb[ik] = b;
-                        frames[ik] = gf[nrot];
-                        gf[q] = gf[nrot];
-                        Lk[q * L + kl - 1] = d[2];
-                        Lk[q * L + kl] = d[3];
-                        Ea[q * ns + kl - 1] = ea;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                }
-            }
-            __syncthreads();
-            // publish the boundary slice this half moved: its frames and the boundary link
-            // densities (Lk[q][0] after the even half, Lk[q][ns] after the odd), two words per
-            // double numbered base + h + 1; no wait for the stores, the reader checks every word
-            {
-                const int ks = parity == 0 ? k0 : k0 + ns - 1;
-                unsigned long long* dst = mypub + (parity == 0 ? 0 : half_rec);
-                const unsigned long long tag = (unsigned long long)(base + h + 1u) << 32;
-                for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
-                    const int i = w >> 1;
-                    const double v = i < nrot * FD ? reinterpret_cast<const double*>(&own(i / FD, ks))[i % FD]
-                                                   : Lk[(i - nrot * FD) * L + (parity == 0 ? 0 : ns)];
-                    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-                    __hip_atomic_store(dst + w, tag | ((w & 1) ? (bits >> 32) : (bits & 0xffffffffull)), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-        }
-    }
-    if (threadIdx.x == 0)  // every part of the chain ran the same halves
-        __hip_atomic_store(myflag, base + 2u * (unsigned)nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool ahead = nrot * ns <= ROT3D_AHEAD;  // a longer part is one of several (W > 1)
+    const bool in_lds = rotor3d_in_lds(ns, nrot, rp.nl_atom > 0);
+    auto sweep = [&](auto n_c) {
+        constexpr int NROT = decltype(n_c)::value;
+        if (ahead) rotor3d_ahead<R, NROT>(e, pt, l3, smem, &s_err, nacc, err);
+        else if (in_lds) rotor3d_long<R, NROT, true>(e, pt, l3, smem, &s_err, nacc, err);
+        else rotor3d_long<R, NROT, false>(e, pt, l3, smem, &s_err, nacc, err);
+    };
+    if (nrot == 1) sweep(std::integral_constant<int, 1>{});
+    else sweep(std::integral_constant<int, 2>{});
+    if (W > 1 && threadIdx.x == 0)  // every part of the chain ran the same halves
+        __hip_atomic_store(myflag, e.base + 2u * (unsigned)nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (err) atomicOr(&mut[r].err, 4);
     unsigned long long sacc = block_sum(nacc, red_acc);
     if (threadIdx.x == 0) {
         if (s_err) atomicOr(&mut[r].err, s_err);
-        const unsigned long long moves = (unsigned long long)nsweep * ns * nrot;
-        atomicAdd(&mut[r].total[rtype][2], moves);
-        atomicAdd(&mut[r].accep[rtype][2], sacc);
-        // per move the proposal's rotor-atom terms and both orientations' rotor-rotor terms, and
-        // the cached sums once per launch
-        atomicAdd(&mut[r].pair_evals[2], moves * (unsigned long long)(items_a + 2 * items_r) +
-                                             (unsigned long long)ns * nrot * items_a);
+        const unsigned long long slices = (unsigned long long)nsweep * ns, items_a = (unsigned long long)(rp.RotRatio * rp.nl_atom);
+        atomicAdd(&mut[r].total[rp.imtype][2], slices * nrot);
+        atomicAdd(&mut[r].accep[rp.imtype][2], sacc);
+        // the atoms' terms of every proposal, the pair terms (two rotors: one per move, and with the
+        // energies ahead the one of both moved), and the current orientations' once per launch
+        const unsigned long long pairs = nrot < 2 ? 0 : (unsigned long long)rp.RotRatio;
+        atomicAdd(&mut[r].pair_evals[2], (slices + ns) * nrot * items_a + (slices * (ahead ? 3 : 2) + ns) * pairs);
     }
 }
 
@@ -2042,8 +2397,8 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
                         chi = cur.chi + twopi * (rp.rtstep * (rand3 - 0.5));
                         if (phi < 0.0) phi = twopi + phi;
                         if (chi < 0.0) chi = twopi + chi;
-                        phi = fmod(phi, twopi);
-                        chi = fmod(chi, twopi);
+                        phi = fmod_near(phi, twopi);
+                        chi = fmod_near(chi, twopi);
                         if (cost > 1.0) cost = 2.0 - cost;
                         if (cost < -1.0) cost = -2.0 - cost;
                         const Frame fn = make_frame(phi, cost, chi);

@@ -11,12 +11,31 @@
 namespace pimc {
 
 constexpr double PI_D = 3.14159265358979323846;
+constexpr double DEG_D = 180.0 / PI_D;
+
+// 1/sqrt(x) for x > 0: the hardware's estimate (2^-23) and one third-order step, within an ulp or
+// so; a square root and a division are four times the instructions.
+__device__ __forceinline__ double rsqrt_fast(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// fmod(x, y) for y > 0: exact by one subtraction below 2 y, which is where a proposal's angle lies
+__device__ __forceinline__ double fmod_near(double x, double y) {
+    const double a = fabs(x);
+    if (a >= 2.0 * y) return fmod(x, y);
+    return a >= y ? copysign(a - y, x) : x;
+}
 
 // matpre (rotden.f:136-163) of (phi, theta = acos(cos theta), chi), as MCRot3Dstep passes the
-// angles (mc_piqmc.cc:1019-1024).  Host and device build frames with the same expressions.
+// angles (mc_piqmc.cc:1019-1024); sin theta from (1 - cos)(1 + cos), whose factors are exact near
+// the poles.  Host and device build frames with the same expressions.
 __host__ __device__ inline Frame make_frame(double phi, double cth, double chi) {
-    const double theta = acos(cth);
-    const double cp = cos(phi), sp = sin(phi), ct = cos(theta), st = sin(theta), ck = cos(chi), sk = sin(chi);
+    double cp, sp, ck, sk;
+    sincos(phi, &sp, &cp);
+    sincos(chi, &sk, &ck);
+    const double ct = cth, st = sqrt((1.0 - cth) * (1.0 + cth));
     Frame f;
     f.m[0] = cp * ct * ck - sp * sk;   // (1,1)
     f.m[1] = sp * ct * ck + cp * sk;   // (2,1)
@@ -41,54 +60,90 @@ __device__ __forceinline__ double within1(double v) {  // rotden.f:208-216
     return v;
 }
 
-// deleul (rotden.f:32-134): Euler angles of R(e1)^T R(e2), radians
-__device__ inline void deleul_frames(const Frame& f1, const Frame& f2, double& phi2, double& theta2, double& chi2) {
+// deleul (rotden.f:32-134): Euler angles, in radians, of the rotation whose elements r2(i, j) gives
+template <typename M>
+__device__ __forceinline__ void deleul(M r2, double& phi2, double& theta2, double& chi2) {
     const double small = 1.0e-08;
-    double r2[9];
-    for (int i = 1; i <= 3; ++i)
-        for (int j = 1; j <= 3; ++j) {
-            double v = 0.0;
-            for (int k = 1; k <= 3; ++k) v = v + fm(f1, k, i) * fm(f2, k, j);
-            r2[(j - 1) * 3 + (i - 1)] = v;
-        }
-#define R2(i, j) r2[((j) - 1) * 3 + ((i) - 1)]
-    const double cost = within1(R2(3, 3));
+    const double cost = within1(r2(3, 3));
     theta2 = acos(cost);
-    const double sint = sin(theta2);
+    double cchi;
+    bool chi_up, phi_up = true;  // whether the sine is positive
+    phi2 = 0.0;
     if (fabs(1.0 - cost) < small) {
-        phi2 = 0.0;
-        const double cchi = within1(R2(1, 1)), schi = within1(R2(2, 1));
-        chi2 = (schi > 0.0) ? acos(cchi) : 2.0 * PI_D - acos(cchi);
+        cchi = r2(1, 1);
+        chi_up = r2(2, 1) > 0.0;
     } else if (fabs(1.0 + cost) < small) {
-        phi2 = 0.0;
-        const double cchi = within1(R2(2, 2)), schi = within1(R2(1, 2));
-        chi2 = (schi > 0.0) ? acos(cchi) : 2.0 * PI_D - acos(cchi);
+        cchi = r2(2, 2);
+        chi_up = r2(1, 2) > 0.0;
     } else {
-        const double cphi = within1(R2(1, 3) / sint), sphi = within1(R2(2, 3) / sint);
-        const double cchi = within1(-R2(3, 1) / sint), schi = within1(R2(3, 2) / sint);
-        phi2 = (sphi > 0.0) ? acos(cphi) : 2.0 * PI_D - acos(cphi);
-        chi2 = (schi > 0.0) ? acos(cchi) : 2.0 * PI_D - acos(cchi);
+        const double inv = rsqrt_fast((1.0 - cost) * (1.0 + cost));  // 1 / sin theta: positive in this branch
+        phi_up = r2(2, 3) > 0.0;
+        phi2 = acos(within1(r2(1, 3) * inv));
+        cchi = -r2(3, 1) * inv;
+        chi_up = r2(3, 2) > 0.0;
     }
-#undef R2
+    chi2 = acos(within1(cchi));
+    if (!phi_up) phi2 = 2.0 * PI_D - phi2;
+    if (!chi_up) chi2 = 2.0 * PI_D - chi2;
+}
+
+// element (i, j) of R(f1)^T R(f2)
+__device__ __forceinline__ double rel_element(const Frame& f1, const Frame& f2, int i, int j) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 1; k <= 3; ++k) v = v + fm(f1, k, i) * fm(f2, k, j);
+    return v;
 }
 
 // rotden (rotden.f:1-31) with rotpro (rotpro_sub.f:1-64): corner value plus one forward
 // difference per axis on the 1-degree grid, index (itheta*361 + iphi)*361 + ichi; E and E^2
 // converted from cm^-1 to Kelvin.  Returns 1 for an out-of-range angle (the reference's istop).
-// rho alone, for the moves: one 32-byte gather instead of three
-__device__ inline int rotden_rho(const Frame& f1, const Frame& f2, const double4* __restrict__ tab, double& rho) {
+// rho alone, for the moves: one 32-byte gather instead of three.  rotden_cell asks for a link's cell
+// and leaves the rest to rho_value, so that a move can do other work while the gather is under way.
+struct RhoCell {
+    double4 r;
+    double xc, xp, xt;
+};
+
+__device__ __forceinline__ double rho_value(const RhoCell& c) { return c.r.x + c.r.y * c.xc + c.r.z * c.xp + c.r.w * c.xt; }
+
+template <typename M>
+__device__ __forceinline__ int rotden_cell_of(M r2, const double4* __restrict__ tab, RhoCell& c) {
     double p2, t2, c2;
-    deleul_frames(f1, f2, p2, t2, c2);
-    const double phi = p2 * 180.0 / PI_D, theta = t2 * 180.0 / PI_D, chi = c2 * 180.0 / PI_D;
+    deleul(r2, p2, t2, c2);
+    const double phi = p2 * DEG_D, theta = t2 * DEG_D, chi = c2 * DEG_D;
     int stop = 0;
     int ichi = (int)chi, iphi = (int)phi, ith = (int)theta;
     if (ichi > 360 || ichi < 0) { ichi = 0; stop = 1; }
     if (iphi > 360 || iphi < 0) { iphi = 0; stop = 1; }
     if (ith > 180 || ith < 0) { ith = 0; stop = 1; }
-    const long long i0 = ((long long)ith * 361 + iphi) * 361 + ichi;
-    const double xc = chi - (double)ichi, xp = phi - (double)iphi, xt = theta - (double)ith;
-    const double4 r = tab[i0];
-    rho = r.x + r.y * xc + r.z * xp + r.w * xt;
+    c.r = tab[((long long)ith * 361 + iphi) * 361 + ichi];
+    c.xc = chi - (double)ichi;
+    c.xp = phi - (double)iphi;
+    c.xt = theta - (double)ith;
+    return stop;
+}
+
+// the link of a moved slice's frame f with the slice before it (side 0: f1 = other, f2 = f) or after
+// it (side 1: f1 = f, f2 = other); the two rotations are each other's transposes
+__device__ __forceinline__ int rotden_cell(const Frame& other, const Frame& f, int side, const double4* __restrict__ tab, RhoCell& c) {
+    return rotden_cell_of([&](int i, int j) {
+        const double a = rel_element(other, f, i, j), b = i == j ? a : rel_element(other, f, j, i);
+        return side ? b : a;
+    }, tab, c);
+}
+
+__device__ __forceinline__ int rotden_link(const Frame& other, const Frame& f, int side, const double4* __restrict__ tab, double& rho) {
+    RhoCell c;
+    const int stop = rotden_cell(other, f, side, tab, c);
+    rho = rho_value(c);
+    return stop;
+}
+
+__device__ inline int rotden_rho(const Frame& f1, const Frame& f2, const double4* __restrict__ tab, double& rho) {
+    RhoCell c;
+    const int stop = rotden_cell_of([&](int i, int j) { return rel_element(f1, f2, i, j); }, tab, c);
+    rho = rho_value(c);
     return stop;
 }
 
@@ -97,13 +152,13 @@ __device__ inline int rotden_frames(const Frame& f1, const Frame& f2, const doub
                                     double& erot, double& esq, double* rel = nullptr) {
     const double wno2k = 0.6950356;
     double p2, t2, c2;
-    deleul_frames(f1, f2, p2, t2, c2);
+    deleul([&](int i, int j) { return rel_element(f1, f2, i, j); }, p2, t2, c2);
     if (rel) {
         rel[0] = p2;
         rel[1] = t2;
         rel[2] = c2;
     }
-    const double phi = p2 * 180.0 / PI_D, theta = t2 * 180.0 / PI_D, chi = c2 * 180.0 / PI_D;
+    const double phi = p2 * DEG_D, theta = t2 * DEG_D, chi = c2 * DEG_D;
     int stop = 0;
     int ichi = (int)chi, iphi = (int)phi, ith = (int)theta;
     if (ichi > 360 || ichi < 0) { ichi = 0; stop = 1; }
@@ -171,12 +226,10 @@ __device__ __forceinline__ R vcalc(const Lut3D<R>& L, R r, R theta, R chi) {
     return q.x + (q.y / L.rstep) * (r - (L.rmin + (R)ir * L.rstep)) + q.z * (theta - (R)ith) + q.w * (chi - (R)ich);
 }
 
-// vcord (vcord.f:1-98): partner at rpt around the rotor centre rcom with body frame f
+// vcord (vcord.f:1-98): partner at the separation (rx, ry, rz) from the rotor centre with body frame f
 template <typename R>
-__device__ __forceinline__ R vcord_v(const Lut3D<R>& L, const Frame& f, double cx, double cy, double cz, double px,
-                                     double py, double pz) {
+__device__ __forceinline__ R vcord_sep(const Lut3D<R>& L, const Frame& f, R rx, R ry, R rz) {
     const R pi = (R)PI_D;
-    const R rx = (R)(px - cx), ry = (R)(py - cy), rz = (R)(pz - cz);
     const R hx0 = (R)f.m[0], hx1 = (R)f.m[1], hx2 = (R)f.m[2];
     const R hy0 = (R)f.m[3], hy1 = (R)f.m[4], hy2 = (R)f.m[5];
     const R hz0 = (R)f.m[6], hz1 = (R)f.m[7], hz2 = (R)f.m[8];
@@ -218,6 +271,13 @@ __device__ __forceinline__ R vcord_v(const Lut3D<R>& L, const Frame& f, double c
     return vcalc<R>(L, rad, the * (R)180 / pi, chiw * (R)180 / pi);
 }
 
+// the same with partner and centre at their positions
+template <typename R>
+__device__ __forceinline__ R vcord_v(const Lut3D<R>& L, const Frame& f, double cx, double cy, double cz, double px,
+                                     double py, double pz) {
+    return vcord_sep<R>(L, f, (R)(px - cx), (R)(py - cy), (R)(pz - cz));
+}
+
 // vcord's geometry for the density bins (vcord.f:40-75), FP64: radret = |rpt - rcom| in
 // Angstrom, theret = angle to the body z axis, chiret = azimuth about it in [0, 2 pi)
 __device__ inline void vcord_geometry(const Frame& f, double cx, double cy, double cz, double px, double py, double pz,
@@ -253,47 +313,36 @@ __device__ inline void vcord_geometry(const Frame& f, double cx, double cy, doub
 __device__ inline double caleng_v(double c1x, double c1y, double c1z, double c2x, double c2y, double c2z,
                                   const Frame& f1, const Frame& f2) {
     const double qm = -1.04, qh = 0.520, br2ang = 0.52917721092, hr2k = 3.1577465e5, kcal2k = 503.0;
-    const double site[4][3] = {{0.0, 0.0, 0.06562}, {0.0, 0.0, -0.08438}, {0.7557, 0.0, -0.5223},
-                               {-0.7557, 0.0, -0.5223}};  // O, M, H1, H2
-    double s1[4][3], s2[4][3];
-    const double c1[3] = {c1x, c1y, c1z}, c2[3] = {c2x, c2y, c2z};
-    for (int a = 0; a < 4; ++a)
-        for (int i = 1; i <= 3; ++i) {
-            double v = c1[i - 1], w = c2[i - 1];
-            for (int j = 1; j <= 3; ++j) {
-                v = v + fm(f1, i, j) * site[a][j - 1];
-                w = w + fm(f2, i, j) * site[a][j - 1];
-            }
-            s1[a][i - 1] = v;
-            s2[a][i - 1] = w;
+    const double zo = 0.06562, zm = -0.08438, xh = 0.7557, zh = -0.5223;  // O and M on the z axis, H at (+-xh, 0, zh)
+    double s1[4][3], s2[4][3];  // O, M, H1, H2
+    auto sites = [&](double cx, double cy, double cz, const Frame& f, double (&s)[4][3]) {
+        const double c[3] = {cx, cy, cz};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double x = f.m[i], z = f.m[6 + i];
+            s[0][i] = fma(z, zo, c[i]);
+            s[1][i] = fma(z, zm, c[i]);
+            s[2][i] = fma(z, zh, fma(x, xh, c[i]));
+            s[3][i] = fma(z, zh, fma(x, -xh, c[i]));
         }
-    double roo = 0.0, rmm = 0.0;
-    for (int i = 0; i < 3; ++i) {
-        roo = roo + (s1[0][i] - s2[0][i]) * (s1[0][i] - s2[0][i]);
-        rmm = rmm + (s1[1][i] - s2[1][i]) * (s1[1][i] - s2[1][i]);
-    }
-    rmm = sqrt(rmm);
-    const double roo4 = roo * roo, roo6 = roo4 * roo, roo12 = roo6 * roo6;
-    const double vlj = 6.e5 / roo12 - 610.0 / roo6;
-    double rhm[4] = {0, 0, 0, 0}, rhh[4] = {0, 0, 0, 0};
-    for (int i = 0; i < 3; ++i) {
-        rhm[0] = rhm[0] + (s1[1][i] - s2[2][i]) * (s1[1][i] - s2[2][i]);
-        rhm[1] = rhm[1] + (s1[1][i] - s2[3][i]) * (s1[1][i] - s2[3][i]);
-        rhm[2] = rhm[2] + (s2[1][i] - s1[2][i]) * (s2[1][i] - s1[2][i]);
-        rhm[3] = rhm[3] + (s2[1][i] - s1[3][i]) * (s2[1][i] - s1[3][i]);
-        rhh[0] = rhh[0] + (s1[2][i] - s2[2][i]) * (s1[2][i] - s2[2][i]);
-        rhh[1] = rhh[1] + (s1[2][i] - s2[3][i]) * (s1[2][i] - s2[3][i]);
-        rhh[2] = rhh[2] + (s1[3][i] - s2[2][i]) * (s1[3][i] - s2[2][i]);
-        rhh[3] = rhh[3] + (s1[3][i] - s2[3][i]) * (s1[3][i] - s2[3][i]);
-    }
-    for (int k = 0; k < 4; ++k) {
-        rhm[k] = sqrt(rhm[k]);
-        rhh[k] = sqrt(rhh[k]);
-    }
-    const double vmh = qm * qh * (1.0 / rhm[0] + 1.0 / rhm[1] + 1.0 / rhm[2] + 1.0 / rhm[3]);
-    const double vhh = qh * qh * (1.0 / rhh[0] + 1.0 / rhh[1] + 1.0 / rhh[2] + 1.0 / rhh[3]);
-    const double vmm = qm * qm * (1.0 / rmm);
-    return vlj * kcal2k + (vmh + vmm + vhh) * hr2k * br2ang;
+    };
+    sites(c1x, c1y, c1z, f1, s1);
+    sites(c2x, c2y, c2z, f2, s2);
+    auto sq = [&](int a, int b) {
+        const double x = s1[a][0] - s2[b][0], y = s1[a][1] - s2[b][1], z = s1[a][2] - s2[b][2];
+        return fma(z, z, fma(y, y, x * x));
+    };
+    const double roo = sq(0, 0);
+    const double roo4 = roo * roo, roo6 = 1.0 / (roo4 * roo);
+    const double vlj = 6.e5 * (roo6 * roo6) - 610.0 * roo6;
+    auto coulomb = [&](auto inverse) {  // of the inverse distance as a function of the squared one
+        const double vmh = qm * qh * (inverse(sq(1, 2)) + inverse(sq(1, 3)) + inverse(sq(2, 1)) + inverse(sq(3, 1)));
+        const double vhh = qh * qh * (inverse(sq(2, 2)) + inverse(sq(2, 3)) + inverse(sq(3, 2)) + inverse(sq(3, 3)));
+        return vmh + vhh + qm * qm * inverse(sq(1, 1));
+    };
+    double v = coulomb([](double x) { return rsqrt_fast(x); });
+    if (!(v == v)) v = coulomb([](double x) { return 1.0 / sqrt(x); });  // sites that coincide, or infinitely far
+    return vlj * kcal2k + v * hr2k * br2ang;
 }
 
 }  // namespace pimc

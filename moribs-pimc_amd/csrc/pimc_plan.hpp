@@ -143,16 +143,37 @@ inline int plan_linear_rotor(const std::vector<RotorChain>& chains, size_t geo_b
     return 0;
 }
 
-// LDS of a part of ns slices of k_rotor3d_parts with nrot rotors: the link densities and the
-// cached rotor-atom sums (nrot x (2 ns + 1) doubles, padded to two), the neighbours' boundary
-// frames (2 nrot), then per lane group of G lanes the frames of every rotor at its slice plus
-// the proposal's.  frame_bytes is sizeof(Frame); G follows the kernel's rule for 256 lanes.
+// A part of k_rotor3d_parts with nrot ns up to this takes a group of lanes per move and forms
+// proposals ahead.  Two per lane of 256: each move then has the lanes for its new links (two per
+// rotor) and the frames fit LDS beside those of other parts.
+constexpr int ROT3D_AHEAD = 256;
+
+// A longer part keeps its state in LDS where two parts of its size then share a CU (rotor3d_long):
+// energies and link densities, and 64 bytes a rotor and slice of axes and angles.
+constexpr size_t ROT3D_HALF_CU = 80 * 1024 - 256;
+constexpr size_t rotor3d_sums_lds(int ns, int nrot, bool atoms) {
+    return (size_t)((nrot * (ns + 1) + (atoms ? nrot * ns : 0) + (nrot - 1) * ns + 1) & ~1) * sizeof(double);
+}
+constexpr size_t rotor3d_state_lds(int ns, int nrot, bool atoms) {
+    return rotor3d_sums_lds(ns, nrot, atoms) + (size_t)nrot * (ns + 2) * 48 + (size_t)nrot * ns * 16;
+}
+constexpr bool rotor3d_in_lds(int ns, int nrot, bool atoms) { return rotor3d_state_lds(ns, nrot, atoms) <= ROT3D_HALF_CU; }
+
+// LDS that parts of up to ns slices of k_rotor3d_parts take with up to nrot rotors.  Short ones: the
+// link densities, then the frames of all slices (two neighbours' included) and of the proposals, nine
+// doubles a slice and rotor and four a slice with two rotors (rotor3d_ahead).
 inline size_t rotor3d_part_lds(int ns, int nrot, size_t frame_bytes) {
-    const int maxmoves = (ns + 1) / 2;
-    int G = 1;
-    while (G < 64 && G * 2 * maxmoves <= 256) G *= 2;
-    return (size_t)((nrot * (2 * ns + 1) + 1) & ~1) * sizeof(double) + (size_t)2 * nrot * frame_bytes +
-           (size_t)(256 / G) * (nrot + 1) * frame_bytes;
+    size_t lds = 0;
+    for (int nr = 1; nr <= nrot; ++nr) {
+        const int na = std::min(ns, ROT3D_AHEAD / nr);
+        lds = std::max(lds, (size_t)((nr * (na + 1) + 1) & ~1) * sizeof(double) + (size_t)nr * (2 * na + 2) * frame_bytes +
+                                (size_t)na * (9 * nr + (nr > 1 ? 4 : 0)) * sizeof(double));
+        if (nr * ns > ROT3D_AHEAD) {
+            lds = std::max(lds, rotor3d_sums_lds(ns, nr, true) + (size_t)2 * nr * frame_bytes);
+            lds = std::max(lds, std::min(rotor3d_state_lds(ns, nr, true), ROT3D_HALF_CU));
+        }
+    }
+    return lds;
 }
 
 // LDS of a part of ns slices of k_rotor3d_da (delayed acceptance, 256 lanes = 4 waves): the
