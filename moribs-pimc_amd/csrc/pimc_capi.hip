@@ -1243,7 +1243,7 @@ int pimc_commit(pimc_ctx* c) {
             return e == hipSuccess ? occ : 0;
         };
         const int W = plan_rotor3d_split(protmax, (int)rot3.size(), prop.multiProcessorCount,
-                                         prop.multiProcessorCount / 8, lds_for, occupancy);
+                                         prop.multiProcessorCount / 8, lds_for, occupancy, da ? 8 : 16);
         {
             std::vector<RotPart> p3;
             std::vector<int> whole;

@@ -1485,11 +1485,28 @@ struct Rot3dEnv {
     int nsweep, j0, jstride;
     unsigned base;                    // half-sweeps done by the launches before this one
     unsigned long long* mypub;        // + parity * half_rec
-    const unsigned long long* from[2];  // the records an even and an odd half wait for
+    const unsigned long long *from_prev, *from_next;  // the records an even and an odd half wait for
     int half_rec;
+    __device__ __forceinline__ const unsigned long long* from(int parity) const { return parity == 0 ? from_prev : from_next; }
     __device__ __forceinline__ uint32_t sweep(int sw) const { return (uint32_t)(j0 + sw * jstride); }
     __device__ __forceinline__ long long at(int q, int k) const { return rp.rot_off + (long long)q * rp.Prot + k; }
 };
+
+// whether the launch has a sweep for this replica
+__device__ __forceinline__ bool rotor3d_turn(const Rep& rp, const Run& run) {
+    return rp.rotkind == 2 && rp.rot3d_id >= 0 && run.u < (run.ref_order ? rp.P : rp.S);
+}
+
+__device__ __forceinline__ Rot3dEnv rotor3d_env(const Rep& rp, uint32_t pass, const double4* beads, RotBead* rotb, Frame* frames,
+                                                const Tables3& T3, const RotPart& pt, const unsigned* flags,
+                                                unsigned long long* pub, int pub_stride, const Run& run) {
+    const int half_rec = pub_stride / 2, W = pt.W;
+    auto record = [&](int w, int parity) { return pub + (long long)(pt.fbase + w) * pub_stride + parity * half_rec; };
+    return {rp, beads, rotb, frames, T3.r3 + (long long)rp.rot3d_id * 3 * ROT3D_SIZE, run.seed, pass,
+            run.ref_order ? 1 : rp.P / rp.S, run.u, run.ref_order ? 0 : rp.S,
+            __hip_atomic_load(flags + pt.fbase + pt.w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+            record(pt.w, 0), record((pt.w + W - 1) % W, 1), record((pt.w + 1) % W, 0), half_rec};
+}
 
 struct Prop3 {
     double phi, cth, chi, u;
@@ -1719,7 +1736,7 @@ __device__ __forceinline__ void rotor3d_ahead(const Rot3dEnv& e, const RotPart& 
         if (trader && h > 0) {
             const int kn = parity == 0 ? 0 : ns + 1, ln = parity == 0 ? 0 : ns;
             for (int w = lane; w < nwords; w += 64) {
-                const unsigned v = rot3d_word(e.from[parity] + w, e.base + (unsigned)h, s_err);
+                const unsigned v = rot3d_word(e.from(parity) + w, e.base + (unsigned)h, s_err);
                 const int i = w >> 1;  // the double: frames first, then link densities
                 double* d = i < NROT * FRAME_D ? reinterpret_cast<double*>(fr + (i / FRAME_D) * (ns + 2) + kn) + i % FRAME_D
                                                : Lk + (i - NROT * FRAME_D) * L + ln;
@@ -1921,7 +1938,7 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
         if (h > 0) {
             const int kn = parity == 0 ? 0 : ns + 1, ln = parity == 0 ? 0 : ns;
             for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
-                const unsigned v = rot3d_word(e.from[parity] + w, e.base + (unsigned)h, s_err);
+                const unsigned v = rot3d_word(e.from(parity) + w, e.base + (unsigned)h, s_err);
                 const int i = w >> 1, q = i / FRAME_D, c = i - q * FRAME_D;  // the double: frames first, then link densities
                 if (q >= NROT) {
                     reinterpret_cast<unsigned*>(&Lk[(i - NROT * FRAME_D) * L + ln])[w & 1] = v;
@@ -2032,22 +2049,9 @@ __global__ __launch_bounds__(256, 2) void k_rotor3d_parts(const Rep* __restrict_
     if (pt.r < 0) return;  // padding of the XCD-ordered grid
     const int r = pt.r;
     const Rep& rp = reps[r];
-    if (rp.rotkind != 2 || rp.rot3d_id < 0) return;
-    int nsweep, j0, jstride;
-    if (run.ref_order) {
-        if (run.u >= rp.P) return;
-        nsweep = 1; j0 = run.u; jstride = 0;
-    } else {
-        if (run.u >= rp.S) return;
-        nsweep = rp.P / rp.S; j0 = run.u; jstride = rp.S;
-    }
+    if (!rotor3d_turn(rp, run)) return;
     const int ns = pt.k1 - pt.k0, W = pt.W, nrot = rp.nrot;
-    unsigned* myflag = flags + pt.fbase + pt.w;
-    const int half_rec = pub_stride / 2;
-    auto record = [&](int w, int parity) { return pub + (long long)(pt.fbase + w) * pub_stride + parity * half_rec; };
-    const Rot3dEnv e{rp, beads, rotb, frames, T3.r3 + (long long)rp.rot3d_id * 3 * ROT3D_SIZE, run.seed, mut[r].pass,
-                     nsweep, j0, jstride, __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                     record(pt.w, 0), {record((pt.w + W - 1) % W, 1), record((pt.w + 1) % W, 0)}, half_rec};
+    const Rot3dEnv e = rotor3d_env(rp, mut[r].pass, beads, rotb, frames, T3, pt, flags, pub, pub_stride, run);
     const Lut3D<R> l3 = lut3d<R>(T3, rp.pot3d_id);
     if (threadIdx.x == 0) s_err = 0;
     unsigned long long nacc = 0;
@@ -2063,12 +2067,12 @@ __global__ __launch_bounds__(256, 2) void k_rotor3d_parts(const Rep* __restrict_
     if (nrot == 1) sweep(std::integral_constant<int, 1>{});
     else sweep(std::integral_constant<int, 2>{});
     if (W > 1 && threadIdx.x == 0)  // every part of the chain ran the same halves
-        __hip_atomic_store(myflag, e.base + 2u * (unsigned)nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(flags + pt.fbase + pt.w, e.base + 2u * (unsigned)e.nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (err) atomicOr(&mut[r].err, 4);
     unsigned long long sacc = block_sum(nacc, red_acc);
     if (threadIdx.x == 0) {
         if (s_err) atomicOr(&mut[r].err, s_err);
-        const unsigned long long slices = (unsigned long long)nsweep * ns, items_a = (unsigned long long)(rp.RotRatio * rp.nl_atom);
+        const unsigned long long slices = (unsigned long long)e.nsweep * ns, items_a = (unsigned long long)(rp.RotRatio * rp.nl_atom);
         atomicAdd(&mut[r].total[rp.imtype][2], slices * nrot);
         atomicAdd(&mut[r].accep[rp.imtype][2], sacc);
         // the atoms' terms of every proposal, the pair terms (two rotors: one per move, and with the
@@ -2168,39 +2172,322 @@ __device__ __forceinline__ void mlp_rotor_pair_features(const Frame& fq, const F
     out[3] = (float)(fq.m[6] * fp.m[6] + fq.m[7] * fp.m[7] + fq.m[8] * fp.m[8]);
 }
 
+// Short parts of the delayed-acceptance sweep (nrot ns <= ROT3D_AHEAD), where a half-sweep is a chain
+// of dependent steps: the neighbour's record, the links' densities, the network's layers, the exact
+// sums, the record for the neighbour.  As in rotor3d_ahead the state lives in LDS, proposals are
+// formed right after the slice's last move while the records travel, and only the waves with a
+// boundary slice trade records.  A wave takes its moves DA_SHORT at a time, lanes j and j + 32 of
+// move j one new link each; with at most 32 exact terms a half wave sums a move's.
+// With state in memory, both links on one lane and 16 slices a part, a half of 256 slices and 32 atoms
+// took 29 us, now 17, of which the network's three layers on a wave are about 5.
+// LDS: the network, Lk[q][ns+1], frames fr[q][ns+2] and proposals' frames fp[q][ns], sl[q][ns], then
+// 32 row outputs per wave.
+constexpr int DA_SHORT = 32;
+
 template <typename R>
-__global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps, Mut* __restrict__ mut,
-                                                    const double4* __restrict__ beads, RotBead* __restrict__ rotb,
-                                                    Frame* __restrict__ frames, Tables T, Tables3 T3,
-                                                    const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
-                                                    unsigned long long* __restrict__ pub, int pub_stride, Run run,
-                                                    const MlpPacked* __restrict__ Wg) {
-    extern __shared__ uint4 mlp_lds[];
-    MlpPacked* W = reinterpret_cast<MlpPacked*>(mlp_lds);
-    __shared__ unsigned long long red_a[4], red_p[4], red_n[4];
-    __shared__ int s_err;
-    const RotPart pt = parts[blockIdx.x];
-    if (pt.r < 0) return;  // padding of the XCD-ordered grid
-    const int r = pt.r;
-    const Rep& rp = reps[r];
-    if (rp.rotkind != 2 || rp.rot3d_id < 0) return;
-    const int Prot = rp.Prot, RR = rp.RotRatio, P = rp.P, nrot = rp.nrot;
+__device__ __forceinline__ void rotor3d_da_short(const Rot3dEnv& e, const RotPart& pt, const Lut3D<R>& l3, MlpPacked* W, int* s_err,
+                                                 unsigned long long& nacc, unsigned long long& npass, unsigned long long& nnet,
+                                                 int& err) {
+    struct Slice {
+        double phi, cth, chi, V, E;  // now; the network's and the exact sums over atoms
+        Prop3 p;
+        double u0, u2;               // uniforms of stages 0 and 2 (p.u: stage 1)
+    };
+    static_assert(sizeof(Slice) == 11 * sizeof(double), "rotor3d_da_part_lds");
+    const Rep& rp = e.rp;
+    const int k0 = pt.k0, ns = pt.k1 - pt.k0, NP = pt.W, L = ns + 1, Prot = rp.Prot, RR = rp.RotRatio, nrot = rp.nrot, nat = rp.nl_atom;
+    const bool net_atoms = nat > 0;  // network pairs: rotor-atom, else rotor-rotor
+    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, nw = blockDim.x >> 6, j = l & 31, side = l >> 5;
+    double* Lk = reinterpret_cast<double*>(W + 1);
+    Frame* fr = reinterpret_cast<Frame*>(Lk + ((nrot * L + 1) & ~1));
+    Frame* fp = fr + nrot * (ns + 2);
+    Slice* sl = reinterpret_cast<Slice*>(fp + nrot * ns);
+    float* rowo = reinterpret_cast<float*>(sl + nrot * ns) + wv * 32;
+    const double ys = (double)W->ys;
+    const int rpm = net_atoms ? RR * nat : RR * (nrot - 1) * 2;  // network rows per move
+    const int items_x = RR * nat;                                // exact rotor-atom pairs of a slice
+    for (int i = threadIdx.x; i < nrot * (ns + 2); i += blockDim.x) {
+        const int q = i / (ns + 2), kl = i - q * (ns + 2);
+        int k = k0 + kl - 1;
+        if (k < 0) k += Prot;
+        if (k >= Prot) k -= Prot;
+        fr[i] = e.frames[e.at(q, k)];
+        if (kl > 0 && kl <= ns) {
+            const RotBead& b = e.rotb[e.at(q, k)];
+            Slice& s = sl[q * ns + kl - 1];
+            s.phi = b.phi;
+            s.cth = b.cth;
+            s.chi = b.chi;
+            s.V = s.E = 0.0;
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nrot * L; i += blockDim.x) {
+        const int q = i / L, kl = i - q * L;
+        if (rotden_rho(fr[q * (ns + 2) + kl], fr[q * (ns + 2) + kl + 1], e.tab, Lk[i])) err = 1;
+    }
+    // the network's rows for slices of rotor q, summed per slice: entry i < nm of the list
+    // is the slice kl_j of lane src (src_j on lane i); sums of (old, new) rows return in so/sn on lane i
+    auto net_rows = [&](int q, int nm, int kl_j, int src_j, bool proposal, double& so, double& sn) {
+        so = 0.0;
+        sn = 0.0;
+        const int total = nm * rpm;
+        for (int b = 0; b < total; b += 32) {
+            const int row = b + j;
+            const int jj = min(row, total - 1) / rpm, jb = __shfl(jj, 0);
+            const int klr = __shfl(kl_j, __shfl(src_j, jj));
+            float f[MLP_IN] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (row < total) {
+                const int idx = row - jj * rpm, k = k0 + klr - 1, gq = nat + q;
+                const Frame& now = fr[q * (ns + 2) + klr];
+                const Frame& moved = fp[q * ns + klr - 1];
+                if (net_atoms) {
+                    const int s = idx / nat, a = idx - s * nat, it = k * RR + s;
+                    const double4 xa = bead(e.beads, rp, gq, it), xj = bead(e.beads, rp, a, it);
+                    const Frame& fq = proposal ? moved : now;
+                    mlp_pair_features(fq.m, fq.zn, xa.x, xa.y, xa.z, xj.x, xj.y, xj.z, f);
+                } else {
+                    const int s = (idx >> 1) / (nrot - 1), pp = (idx >> 1) - s * (nrot - 1), p = pp + (pp >= q), it = k * RR + s;
+                    const double4 xq = bead(e.beads, rp, gq, it), xp = bead(e.beads, rp, nat + p, it);
+                    mlp_rotor_pair_features(proposal && (idx & 1) ? moved : now, fr[p * (ns + 2) + klr], xq.x, xq.y, xq.z, xp.x,
+                                            xp.y, xp.z, f);
+                }
+#pragma unroll
+                for (int c = 0; c < MLP_IN; ++c) f[c] = (f[c] - W->xm[c]) * W->xinv[c];
+            }
+            // an opaque zero offset keeps the weight reads inside the loop (hoisted out they
+            // would hold ~130 registers of weights per lane)
+            int z = 0;
+            __asm__ volatile("" : "+s"(z));
+            const float o = mlp_rows32(reinterpret_cast<const MlpPacked*>(reinterpret_cast<const char*>(W) + z), f);
+            if (rpm >= 8) {  // entry by entry over the lanes that hold its rows
+                for (int i = jb; i * rpm < min(b + 32, total); ++i) {
+                    const bool in = l < 32 && row >= i * rpm && row < min((i + 1) * rpm, total);
+                    const bool moved = net_atoms || ((row - i * rpm) & 1);
+                    const double vn = wave_sum(in && moved ? (double)o : 0.0);
+                    if (l == i) sn += vn;
+                    if (!net_atoms) {
+                        const double vo = wave_sum(in && !moved ? (double)o : 0.0);
+                        if (l == i) so += vo;
+                    }
+                }
+                continue;
+            }
+            if (l < 32) rowo[l] = o;
+            wave_sync();
+            if (l < nm) {  // the rows of entry l that fall in this batch
+                const int r0 = max(l * rpm, b), r1 = min((l + 1) * rpm, b + 32);
+                for (int rr = r0; rr < r1; ++rr) {
+                    const double v = (double)rowo[rr - b];
+                    const bool moved = net_atoms || ((rr - l * rpm) & 1);
+                    sn += moved ? v : 0.0;
+                    so += moved ? 0.0 : v;
+                }
+            }
+            wave_sync();
+        }
+    };
+    // exact rotor-atom sums of rotor q with frame f at local slice kl, over GL lanes from this one's group
+    auto exact_atoms = [&](int q, int kl, const Frame& f, int GL) -> double {
+        const int k = k0 + kl - 1, gq = nat + q;
+        double v = 0.0;
+        for (int i = l & (GL - 1); i < items_x; i += GL) {
+            const int s = i / nat, a = i - s * nat, it = k * RR + s;
+            const double4 xa = bead(e.beads, rp, gq, it), xj = bead(e.beads, rp, a, it);
+            v += (double)vcord_v<R>(l3, f, xa.x, xa.y, xa.z, xj.x, xj.y, xj.z);
+        }
+        return group_sum(v, GL);
+    };
+    // exact rotor-rotor terms of rotor q moved, less those of it as it is: the half waves take one each
+    auto pair_change = [&](int q, int kl) -> double {
+        const int k = k0 + kl - 1;
+        const Frame& f = side == 0 ? fp[q * ns + kl - 1] : fr[q * (ns + 2) + kl];
+        double v = 0.0;
+        for (int p = 0; p < nrot; ++p) {
+            if (p == q) continue;
+            for (int s = 0; s < RR; ++s) {
+                const double4 xa = bead(e.beads, rp, nat + q, k * RR + s), xp = bead(e.beads, rp, nat + p, k * RR + s);
+                v += caleng_v(xa.x, xa.y, xa.z, xp.x, xp.y, xp.z, f, fr[p * (ns + 2) + kl]);
+            }
+        }
+        return v;
+    };
+    auto moves_of_wave = [&](int nmoves) { return nmoves > wv ? (nmoves - wv + nw - 1) / nw : 0; };  // wv, wv + nw, ...
+    auto ahead = [&](int parity, int sw) {  // the half waves take a rotor each
+        const int mine = moves_of_wave(ns >> 1);
+        for (int c0 = 0; c0 < mine; c0 += DA_SHORT) {
+            if (c0 + j >= mine || side >= nrot) continue;
+            const int kl = 2 * (wv + (c0 + j) * nw) + parity + 1, k = k0 + kl - 1, q = side;
+            Slice& s = sl[q * ns + kl - 1];
+            s.p = rot3d_propose(e, q, k, e.sweep(sw), s.phi, s.cth, s.chi);
+            const uint4 w2 = draw(e.seed, rp.key, e.pass, K_ROT3D, e.sweep(sw), (uint32_t)(nat + q), (uint32_t)k, 2);
+            s.u2 = u53(w2.x, w2.y);
+            s.u0 = u53(w2.z, w2.w);
+            fp[q * ns + kl - 1] = make_frame(s.p.phi, s.p.cth, s.p.chi);
+        }
+    };
+    if (net_atoms) {  // the sums of every own slice at its current orientation
+        for (int q = 0; q < nrot; ++q)
+            for (int c0 = wv * DA_SHORT; c0 < ns; c0 += nw * DA_SHORT) {
+                const int nm = min(DA_SHORT, ns - c0);
+                double so, sn;
+                net_rows(q, nm, c0 + l + 1, l, false, so, sn);
+                if (l < nm) sl[q * ns + c0 + l].V = sn;
+                for (int i = 0; i < nm; ++i) {
+                    const double v = exact_atoms(q, c0 + i + 1, fr[q * (ns + 2) + c0 + i + 1], 64);
+                    if (l == 0) sl[q * ns + c0 + i].E = v;
+                }
+            }
+    }
+    __syncthreads();
+    ahead(0, 0);
+    ahead(1, 0);
+    __syncthreads();
+    const int nwords = 2 * nrot * (FRAME_D + 1);
+#pragma unroll 1
+    for (int h = 0; h < 2 * e.nsweep; ++h) {
+        const int parity = h & 1, sw = h >> 1;
+        const int nmoves = ns >> 1, mine = moves_of_wave(nmoves);  // of either parity: k0 and ns are even
+        const bool trader = NP > 1 && (parity == 0 ? 0 : (nmoves - 1) % nw) == wv;  // has the move beside the neighbour
+        if (trader && h > 0) {
+            const int kn = parity == 0 ? 0 : ns + 1, ln = parity == 0 ? 0 : ns;
+            for (int w = l; w < nwords; w += 64) {
+                const unsigned v = rot3d_word(e.from(parity) + w, e.base + (unsigned)h, s_err);
+                const int i = w >> 1;  // the double: frames first, then link densities
+                double* d = i < nrot * FRAME_D ? reinterpret_cast<double*>(fr + (i / FRAME_D) * (ns + 2) + kn) + i % FRAME_D
+                                               : Lk + (i - nrot * FRAME_D) * L + ln;
+                reinterpret_cast<unsigned*>(d)[w & 1] = v;
+            }
+            wave_sync();
+        }
+#pragma unroll 1
+        for (int q = 0; q < nrot; ++q) {  // rotor 1 sees rotor 0's move at its slice: the same wave's
+#pragma unroll 1
+            for (int c0 = 0; c0 < mine; c0 += DA_SHORT) {
+                const int nm = min(DA_SHORT, mine - c0);
+                const int kl = 2 * (wv + (c0 + min(j, nm - 1)) * nw) + parity + 1;
+                Slice& s = sl[q * ns + kl - 1];
+                // (1) the new links, and the exact stage-1 terms
+                double rho;
+                if (rotden_link(fr[q * (ns + 2) + kl - 1 + 2 * side], fp[q * ns + kl - 1], side, e.tab, rho)) err = 1;
+                const double d2 = __shfl(rho, j), d3 = __shfl(rho, j + 32);
+                double dvx = 0.0;
+                if (net_atoms && nrot > 1) {
+                    const double v = pair_change(q, kl);
+                    dvx = __shfl(v, j) - __shfl(v, j + 32);
+                }
+                double dold = Lk[q * L + kl - 1] * Lk[q * L + kl];
+                if (fabs(dold) < RZERO) dold = 0.0;
+                if (dold < 0.0) dold = fabs(dold);
+                double dnew = d2 * d3;
+                if (fabs(dnew) < RZERO) dnew = 0.0;
+                if (dnew < 0.0) dnew = fabs(dnew);
+                const double ratio = (dold > RZERO) ? dnew / dold : 1.0;
+                // (2) stage 0, then the network rows of the moves that passed it, listed first in lane
+                // order (slot: a lane's place in that order, src: the lane whose move fills this place)
+                const bool pass0 = l < nm && (ratio > 1.0 || ratio > s.u0);
+                const unsigned long long m0 = __ballot(pass0);
+                const int n0 = __popcll(m0), below = __popcll(m0 & ((1ull << l) - 1ull));
+                const int slot = pass0 ? below : n0 + (l - below);
+                const int src = __builtin_amdgcn_ds_permute(slot << 2, l);
+                double so = 0.0, sn = 0.0;
+                if (n0) {
+                    net_rows(q, n0, kl, src, true, so, sn);
+                    so = __shfl(so, slot);
+                    sn = __shfl(sn, slot);
+                }
+                // (3) stage 1, the surrogate factor
+                bool pass1 = false;
+                double dvs = 0.0;
+                if (pass0) {
+                    if (net_atoms) so = s.V;
+                    dvs = ys * (sn - so);
+                    const double rd1 = exp(-rp.tau * (dvs + dvx));
+                    pass1 = rd1 > 1.0 || rd1 > s.p.u;
+                }
+                // (4) stage 2: exact network-pair sums of the moves that passed
+                double dve = 0.0, ex_new = 0.0;
+                unsigned long long todo = __ballot(pass1);
+                if (net_atoms) {
+                    const int GL = items_x <= 32 ? 32 : 64;
+                    while (todo) {
+                        const int ja = __ffsll((long long)todo) - 1;
+                        todo &= todo - 1;
+                        const bool two = GL == 32 && todo;
+                        const int jb = two ? __ffsll((long long)todo) - 1 : ja;
+                        if (two) todo &= todo - 1;
+                        const int klj = __shfl(kl, GL == 32 && side ? jb : ja);
+                        const double v = exact_atoms(q, klj, fp[q * ns + klj - 1], GL);
+                        const double va = __shfl(v, 0), vb = __shfl(v, 32);
+                        if (l == ja || l == jb) {
+                            ex_new = l == ja ? va : vb;
+                            dve = ex_new - s.E;
+                        }
+                    }
+                } else if (todo) {
+                    const double v = pair_change(q, kl);
+                    dve = __shfl(v, j) - __shfl(v, j + 32);
+                }
+                // (5) stage 2 and the update
+                if (pass0) {
+                    nnet += (unsigned long long)rpm;
+                    if (pass1) {
+                        ++npass;
+                        const double rd2 = exp(-rp.tau * (dve - dvs));
+                        if (rd2 > 1.0 || rd2 > s.u2) {
+                            ++nacc;
+                            const Frame& f = fp[q * ns + kl - 1];
+                            fr[q * (ns + 2) + kl] = f;
+                            s.phi = s.p.phi;
+                            s.cth = s.p.cth;
+                            s.chi = s.p.chi;
+                            s.V = sn;
+                            s.E = ex_new;
+                            Lk[q * L + kl - 1] = d2;
+                            Lk[q * L + kl] = d3;
+                            if (NP == 1 && (kl == 1 || kl == ns)) {  // its own neighbour, as in rotor3d_ahead
+                                fr[q * (ns + 2) + (kl == 1 ? ns + 1 : 0)] = f;
+                                Lk[q * L + (kl == 1 ? ns : 0)] = kl == 1 ? d2 : d3;
+                            }
+                            rot3d_store(e, e.at(q, k0 + kl - 1), s.phi, s.cth, s.chi, f);
+                        }
+                    }
+                }
+                wave_sync();
+            }
+        }
+        if (trader) {  // publish the boundary slice; no wait for the stores, the reader checks every word
+            const int kb = parity == 0 ? 1 : ns, lb = parity == 0 ? 0 : ns;
+            for (int w = l; w < nwords; w += 64) {
+                const int i = w >> 1;
+                const double v = i < nrot * FRAME_D ? reinterpret_cast<const double*>(fr + (i / FRAME_D) * (ns + 2) + kb)[i % FRAME_D]
+                                                    : Lk[(i - nrot * FRAME_D) * L + lb];
+                __hip_atomic_store(e.mypub + parity * e.half_rec + w, rot3d_pack(v, w & 1, e.base + (unsigned)h + 1u), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if (sw + 1 < e.nsweep) ahead(parity, sw + 1);
+        lds_barrier();
+        if (*s_err) break;  // as in rotor3d_ahead
+    }
+}
+
+// Longer parts: state in memory, everything of a move inside its half-sweep.
+template <typename R>
+__device__ __forceinline__ void rotor3d_da_long(const Rot3dEnv& e, const RotPart& pt, const Lut3D<R>& l3, MlpPacked* W, int* s_err,
+                                                unsigned long long& nacc, unsigned long long& npass, unsigned long long& nnet,
+                                                int& err) {
+    const Rep& rp = e.rp;
+    const int Prot = rp.Prot, RR = rp.RotRatio, nrot = rp.nrot;
     const int nat = rp.nl_atom;              // atoms come first: 0 .. nat-1
     const bool net_atoms = nat > 0;          // network pairs: rotor-atom, else rotor-rotor
-    int nsweep, j0, jstride;
-    if (run.ref_order) {
-        if (run.u >= P) return;
-        nsweep = 1; j0 = run.u; jstride = 0;
-    } else {
-        if (run.u >= rp.S) return;
-        nsweep = P / rp.S; j0 = run.u; jstride = rp.S;
-    }
     const int k0 = pt.k0, ns = pt.k1 - pt.k0, NP = pt.W;
     const int L = ns + 1;
     const long long rb0 = rp.rot_off;
-    const double4* tab = T3.r3 + (long long)rp.rot3d_id * 3 * ROT3D_SIZE;
-    const Lut1D<R> l1 = lut1d<R>(T, rp.pot1d_id);
-    const Lut3D<R> l3 = lut3d<R>(T3, rp.pot3d_id);
+    const double4* tab = e.tab;
+    const double4* beads = e.beads;
+    RotBead* rotb = e.rotb;
+    Frame* frames = e.frames;
     const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, nw = blockDim.x >> 6;
     double* Lk = reinterpret_cast<double*>(W + 1);
     double* Vs = Lk + nrot * L;   // cached surrogate sums (rotor-atom network)
@@ -2208,27 +2495,17 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
     Frame* fnb = reinterpret_cast<Frame*>(Lk + ((nrot * L + 2 * nrot * ns + 1) & ~1));
     Frame* prop = fnb + 2 * nrot + wv * DA_MV;
     float* rowo = reinterpret_cast<float*>(fnb + 2 * nrot + nw * DA_MV) + wv * 32;
-    unsigned* myflag = flags + pt.fbase + pt.w;
-    constexpr int FD = (int)(sizeof(Frame) / sizeof(double));
+    constexpr int FD = FRAME_D;
     const int nwords = 2 * nrot * (FD + 1);
-    const int half_rec = pub_stride / 2;
-    unsigned long long* mypub = pub + (long long)(pt.fbase + pt.w) * pub_stride;
-    const unsigned long long* prevlast = pub + (long long)(pt.fbase + (pt.w + NP - 1) % NP) * pub_stride + half_rec;
-    const unsigned long long* nextfirst = pub + (long long)(pt.fbase + (pt.w + 1) % NP) * pub_stride;
-    const unsigned base = __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t pass = mut[r].pass;
-    const int rtype = rp.imtype;
+    const unsigned base = e.base;
+    const uint32_t pass = e.pass;
     const double twopi = 2.0 * PI_D;
-    const double ys = (double)Wg->ys;
+    const double ys = (double)W->ys;
     // network rows per move: RR x atoms (proposal only; the old sum is cached), or RR x other
     // rotors x (old, new)
     const int rpm = net_atoms ? RR * nat : RR * (nrot - 1) * 2;
     const int items_x = RR * nat;  // exact rotor-atom pairs of a slice
     auto own = [&](int q, int k) -> const Frame& { return frames[rb0 + (long long)q * Prot + k]; };
-    if (threadIdx.x == 0) s_err = 0;
-    unsigned long long nacc = 0, npass = 0, nnet = 0;
-    int err = 0;
-    mlp_stage(Wg, W);
     for (int i = threadIdx.x; i < 2 * nrot; i += blockDim.x) {
         const int side = i / nrot, q = i - side * nrot;
         int k = side ? k0 + ns : k0 - 1;
@@ -2291,8 +2568,9 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
                 for (int rr = r0; rr < r1; ++rr) {
                     const int idx = rr - l * rpm;
                     const double v = (double)rowo[rr - b];
-                    if (net_atoms || (idx & 1)) sn += v;
-                    else so += v;
+                    const bool moved = net_atoms || (idx & 1);
+                    sn += moved ? v : 0.0;
+                    so += moved ? 0.0 : v;
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -2326,8 +2604,8 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
         }
     }
     __syncthreads();
-    for (int sw = 0; sw < nsweep; ++sw) {
-        const uint32_t jsweep = (uint32_t)(j0 + sw * jstride);
+    for (int sw = 0; sw < e.nsweep; ++sw) {
+        const uint32_t jsweep = e.sweep(sw);
         for (int parity = 0; parity < 2; ++parity) {
             const unsigned h = 2u * (unsigned)sw + (unsigned)parity;
             if (!(sw == 0 && parity == 0)) {
@@ -2344,29 +2622,17 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
                         }
                     }
                 } else {
-                    const unsigned long long* src = parity == 0 ? prevlast : nextfirst;
                     unsigned* dstf = reinterpret_cast<unsigned*>(fnb + (parity == 0 ? 0 : nrot));
-                    const unsigned want = base + h;
                     for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
-                        unsigned long long wvv;
-                        unsigned spins = 0;
-                        for (;;) {
-                            wvv = __hip_atomic_load(src + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            if ((unsigned)(wvv >> 32) == want) break;
-                            if (++spins > ROT_SPIN_LIMIT) {
-                                s_err = 2;
-                                break;
-                            }
-                            __builtin_amdgcn_s_sleep(2);
-                        }
+                        const unsigned v = rot3d_word(e.from(parity) + w, base + h, s_err);
                         const int i = w >> 1;
-                        if (i < nrot * FD) dstf[w] = (unsigned)wvv;
-                        else reinterpret_cast<unsigned*>(&Lk[(i - nrot * FD) * L + (parity == 0 ? 0 : ns)])[w & 1] = (unsigned)wvv;
+                        if (i < nrot * FD) dstf[w] = v;
+                        else reinterpret_cast<unsigned*>(&Lk[(i - nrot * FD) * L + (parity == 0 ? 0 : ns)])[w & 1] = v;
                     }
                 }
                 __syncthreads();
-                if (s_err) {  // a wait gave up: leave at once (see k_rotor3d_parts)
-                    sw = nsweep;
+                if (*s_err) {  // a wait gave up: leave at once (see rotor3d_ahead)
+                    sw = e.nsweep;
                     break;
                 }
             }
@@ -2385,9 +2651,9 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
                     RotBead cur{};
                     if (l < nm) {
                         cur = rotb[ik];
-                        const uint4 w0 = draw(run.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gq, (uint32_t)k, 0);
-                        const uint4 w1 = draw(run.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gq, (uint32_t)k, 1);
-                        const uint4 w2 = draw(run.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gq, (uint32_t)k, 2);
+                        const uint4 w0 = draw(e.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gq, (uint32_t)k, 0);
+                        const uint4 w1 = draw(e.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gq, (uint32_t)k, 1);
+                        const uint4 w2 = draw(e.seed, rp.key, pass, K_ROT3D, jsweep, (uint32_t)gq, (uint32_t)k, 2);
                         const double rand1 = u53(w0.x, w0.y), rand2 = u53(w0.z, w0.w), rand3 = u53(w1.x, w1.y);
                         rand4 = u53(w1.z, w1.w);
                         rand5 = u53(w2.x, w2.y);
@@ -2514,28 +2780,55 @@ __global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps
             // publish the boundary slice this half moved (k_rotor3d_parts' record)
             if (NP > 1) {
                 const int ks = parity == 0 ? k0 : k0 + ns - 1;
-                unsigned long long* dst = mypub + (parity == 0 ? 0 : half_rec);
-                const unsigned long long tag = (unsigned long long)(base + h + 1u) << 32;
                 for (int w = threadIdx.x; w < nwords; w += blockDim.x) {
                     const int i = w >> 1;
                     const double v = i < nrot * FD ? reinterpret_cast<const double*>(&own(i / FD, ks))[i % FD]
                                                    : Lk[(i - nrot * FD) * L + (parity == 0 ? 0 : ns)];
-                    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-                    __hip_atomic_store(dst + w, tag | ((w & 1) ? (bits >> 32) : (bits & 0xffffffffull)), __ATOMIC_RELAXED,
+                    __hip_atomic_store(e.mypub + parity * e.half_rec + w, rot3d_pack(v, w & 1, base + h + 1u), __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
         }
     }
+}
+
+template <typename R>
+__global__ __launch_bounds__(256) void k_rotor3d_da(const Rep* __restrict__ reps, Mut* __restrict__ mut,
+                                                    const double4* __restrict__ beads, RotBead* __restrict__ rotb,
+                                                    Frame* __restrict__ frames, Tables T, Tables3 T3,
+                                                    const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
+                                                    unsigned long long* __restrict__ pub, int pub_stride, Run run,
+                                                    const MlpPacked* __restrict__ Wg) {
+    extern __shared__ uint4 mlp_lds[];
+    MlpPacked* W = reinterpret_cast<MlpPacked*>(mlp_lds);
+    __shared__ unsigned long long red_a[4], red_p[4], red_n[4];
+    __shared__ int s_err;
+    const RotPart pt = parts[blockIdx.x];
+    if (pt.r < 0) return;  // padding of the XCD-ordered grid
+    const int r = pt.r;
+    const Rep& rp = reps[r];
+    if (!rotor3d_turn(rp, run)) return;
+    const int ns = pt.k1 - pt.k0, NP = pt.W, RR = rp.RotRatio, nrot = rp.nrot;
+    const bool net_atoms = rp.nl_atom > 0;
+    const Rot3dEnv e = rotor3d_env(rp, mut[r].pass, beads, rotb, frames, T3, pt, flags, pub, pub_stride, run);
+    const Lut3D<R> l3 = lut3d<R>(T3, rp.pot3d_id);
+    if (threadIdx.x == 0) s_err = 0;
+    unsigned long long nacc = 0, npass = 0, nnet = 0;
+    int err = 0;
+    mlp_stage(Wg, W);
+    __syncthreads();
+    if (nrot * ns <= ROT3D_AHEAD) rotor3d_da_short<R>(e, pt, l3, W, &s_err, nacc, npass, nnet, err);
+    else rotor3d_da_long<R>(e, pt, l3, W, &s_err, nacc, npass, nnet, err);
     if (threadIdx.x == 0 && NP > 1)  // every part of the chain ran the same halves
-        __hip_atomic_store(myflag, base + 2u * (unsigned)nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(flags + pt.fbase + pt.w, e.base + 2u * (unsigned)e.nsweep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (err) atomicOr(&mut[r].err, 4);
     const unsigned long long sa = block_sum(nacc, red_a);
     const unsigned long long sp = block_sum(npass, red_p);
     const unsigned long long sn_ = block_sum(nnet, red_n);
     if (threadIdx.x == 0) {
+        const int rtype = rp.imtype, items_x = RR * rp.nl_atom;
         if (s_err) atomicOr(&mut[r].err, s_err);
-        const unsigned long long moves = (unsigned long long)nsweep * ns * nrot;
+        const unsigned long long moves = (unsigned long long)e.nsweep * ns * nrot;
         atomicAdd(&mut[r].total[rtype][2], moves);
         atomicAdd(&mut[r].accep[rtype][2], sa);
         atomicAdd(&mut[r].da[0], moves);

@@ -51,7 +51,7 @@ static_assert(sizeof(MlpPacked) % 16 == 0, "staged with 16-byte copies");
 
 typedef short mlp_bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 mlp_bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned short mlp_u16x8 __attribute__((ext_vector_type(8)));
+typedef float mlp_f32x8 __attribute__((ext_vector_type(8)));
 typedef float mlp_f32x16 __attribute__((ext_vector_type(16)));
 
 __host__ __device__ inline uint16_t f2bf(float x) {  // round to nearest even
@@ -96,10 +96,10 @@ __device__ __forceinline__ void mlp_hidden(const uint16_t* __restrict__ w, const
     mlp_bf16x8 bin[8];
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) {
-        mlp_u16x8 t;
+        mlp_f32x8 t;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t[j] = f2bf(h[kb >> 1][8 * (kb & 1) + j]);
-        bin[kb] = __builtin_bit_cast(mlp_bf16x8, t);
+        for (int j = 0; j < 8; ++j) t[j] = h[kb >> 1][8 * (kb & 1) + j];
+        bin[kb] = __builtin_convertvector(t, mlp_bf16x8);  // to nearest even, two a instruction
     }
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {

@@ -176,29 +176,38 @@ inline size_t rotor3d_part_lds(int ns, int nrot, size_t frame_bytes) {
     return lds;
 }
 
-// LDS of a part of ns slices of k_rotor3d_da (delayed acceptance, 256 lanes = 4 waves): the
-// packed network (mlp_bytes), the link densities and the two cached sums per own slice
-// (nrot x (3 ns + 1) doubles, padded to two), the neighbours' boundary frames and DA_MV proposal
-// frames per wave, then 32 row outputs per wave.
-constexpr int DA_MV = 64;  // moves a wave takes at once in the delayed-acceptance sweep: one per lane
+// LDS of parts of up to ns slices of k_rotor3d_da (delayed acceptance, 256 lanes = 4 waves) with up to
+// nrot rotors: the packed network (mlp_bytes), then for short parts (nrot ns <= ROT3D_AHEAD) the link
+// densities, the frames of all slices and proposals and eleven doubles a slice and rotor; for longer
+// ones the link densities and the two cached sums per own slice, the neighbours' boundary frames and
+// DA_MV proposal frames per wave; and 32 row outputs per wave.
+constexpr int DA_MV = 64;  // moves a wave takes at once in the long parts: one per lane
 inline size_t rotor3d_da_part_lds(int ns, int nrot, size_t frame_bytes, size_t mlp_bytes) {
-    return mlp_bytes + (size_t)((nrot * (ns + 1) + 2 * nrot * ns + 1) & ~1) * sizeof(double) +
-           (size_t)(2 * nrot + 4 * DA_MV) * frame_bytes + (size_t)4 * 32 * sizeof(float);
+    size_t lds = 0;
+    for (int nr = 1; nr <= nrot; ++nr) {
+        const int na = std::min(ns, ROT3D_AHEAD / nr);
+        lds = std::max(lds, (size_t)((nr * (na + 1) + 1) & ~1) * sizeof(double) + (size_t)nr * (2 * na + 2) * frame_bytes +
+                                (size_t)nr * na * 11 * sizeof(double));
+        if (nr * ns > ROT3D_AHEAD)
+            lds = std::max(lds, (size_t)((nr * (ns + 1) + 2 * nr * ns + 1) & ~1) * sizeof(double) +
+                                    (size_t)(2 * nr + 4 * DA_MV) * frame_bytes);
+    }
+    return mlp_bytes + lds + (size_t)4 * 32 * sizeof(float);
 }
 
 // Split of the non-linear rotor chains: one count W for the launch, a power of two up to 64, the
-// largest whose parts hold at least 16 slices of the longest chain and fit LDS (lds_for(slices)),
+// largest whose parts hold at least min_slices slices of the longest chain and fit LDS (lds_for(slices)),
 // such that the parts of all chains are resident at once (ncu * blocks_per_cu) and the W parts
 // of one chain, which wait on one another on one XCD, fit that XCD (cus_per_xcd *
 // blocks_per_cu).  Returns 1 when whole chains are better left to one workgroup each.
 inline int plan_rotor3d_split(int protmax, int nchains, int ncu, int cus_per_xcd,
                               const std::function<size_t(int)>& lds_for,
-                              const std::function<int(size_t)>& blocks_per_cu) {
+                              const std::function<int(size_t)>& blocks_per_cu, int min_slices = 16) {
     int W = 1;
     for (int w = 2; w <= 64; w *= 2) {
         const int ns = ((protmax + w - 1) / w + 1) & ~1;
         const size_t lds = lds_for(ns);
-        if (ns < 16 || lds > ROTOR_LDS_MAX) break;
+        if (ns < min_slices || lds > ROTOR_LDS_MAX) break;
         const long long occ = std::max(0, blocks_per_cu(lds));
         if ((long long)w * nchains > occ * ncu || (long long)w > occ * cus_per_xcd) break;
         W = w;
