@@ -182,6 +182,14 @@ struct pimc_ctx {
     long long nrcfvals = 0;
     double* d_samples = nullptr;
     int sample_cap = 0;
+    // host memory that the device writes: every replica's Mut and its first back_samples samples as
+    // they are at the end of a run, then room for one replica's packed state
+    unsigned char* back = nullptr;
+    int back_samples = 0;
+    size_t back_state = 0, back_state_bytes = 0;
+    bool back_valid = false;  // nothing has changed the counters or samples since they were written there
+    Mut* back_mut() const { return reinterpret_cast<Mut*>(back); }
+    double* back_sample(int r) const { return reinterpret_cast<double*>(back + sizeof(Mut) * nrep) + (size_t)8 * back_samples * r; }
     float4* d_k1f = nullptr;
     double4* d_k1d = nullptr;
     Tab1D* d_t1 = nullptr;
@@ -376,6 +384,7 @@ void pimc_destroy(pimc_ctx* c) {
                     c->d_parts3, c->d_flags3, c->d_pub3};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (c->back) (void)hipHostFree(c->back);
     for (int k = 0; k < 2; ++k) {
         if (c->side[k]) (void)hipStreamDestroy(c->side[k]);
         if (c->ev_join[k]) (void)hipEventDestroy(c->ev_join[k]);
@@ -1334,6 +1343,17 @@ int pimc_commit(pimc_ctx* c) {
     if (!c->d_rep || !c->d_mut || !c->d_beads || !c->d_prop || !c->d_rotb || !c->d_hist || !c->d_all ||
         !c->d_rotreps || !c->d_est || !c->d_samples)
         return fail(c, "hipMalloc failed");
+    {
+        size_t state = 0;
+        for (const Rep& p : c->rep)
+            state = std::max(state, sizeof(double) * (3 * (size_t)p.natoms * p.P + 6 * (size_t)p.natoms * std::max(p.Prot, 0)));
+        c->back_samples = (int)std::min<size_t>(c->sample_cap, std::max<size_t>(1, 256 * 1024 / (64 * (size_t)c->nrep)));
+        c->back_state = sizeof(Mut) * c->nrep + (size_t)64 * c->back_samples * c->nrep;
+        c->back_state_bytes = std::min<size_t>(state, 4 << 20);  // a larger replica is copied and packed on the host
+        if (hipHostMalloc(reinterpret_cast<void**>(&c->back), c->back_state + c->back_state_bytes, hipHostMallocPortable | hipHostMallocMapped) !=
+            hipSuccess)
+            return fail(c, "hipHostMalloc failed");
+    }
     HIPCHECK(c, hipMemcpy(c->d_rep, c->rep.data(), sizeof(Rep) * c->nrep, hipMemcpyHostToDevice));
     HIPCHECK(c, hipMemset(c->d_mut, 0, sizeof(Mut) * c->nrep));
     HIPCHECK(c, hipMemset(c->d_hist, 0, sizeof(unsigned) * std::max<long long>(hoff, 1)));
@@ -1524,15 +1544,36 @@ int pimc_restore_state(pimc_ctx* c, int r, const double* coords, const double* a
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     HIPCHECK(c, hipMemcpy(&m, c->d_mut + r, sizeof(Mut), hipMemcpyDeviceToHost));
     m.pass = pass;
+    c->back_valid = false;
     HIPCHECK(c, hipMemcpy(c->d_mut + r, &m, sizeof(Mut), hipMemcpyHostToDevice));
     return 0;
 }
 
+}  // extern "C"
+
+namespace {
+
+// the host's copy of counters and samples, brought up to date where something changed them since the
+// last run's end wrote it; everything that does, clears back_valid
+int read_back(pimc_ctx* c) {
+    if (!c->back) return fail(c, "pimc_commit first");
+    if (c->back_valid) return 0;
+    hipLaunchKernelGGL(k_read_back, dim3(c->nrep), dim3(64), 0, c->stream, c->d_mut, c->d_rep, c->d_samples, c->back_samples,
+                       c->back_mut(), c->back_sample(0));
+    HIPCHECK(c, hipGetLastError());
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    c->back_valid = true;
+    return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
 int pimc_get_pass(pimc_ctx* c, int r, unsigned* pass) {
     if (!c->committed || r < 0 || r >= c->nrep || !pass) return fail(c, "bad replica");
-    Mut m;
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(&m, c->d_mut + r, sizeof(Mut), hipMemcpyDeviceToHost));
+    if (read_back(c)) return -1;
+    const Mut& m = c->back_mut()[r];
     *pass = m.pass;
     return 0;
 }
@@ -1540,10 +1581,21 @@ int pimc_get_pass(pimc_ctx* c, int r, unsigned* pass) {
 int pimc_get_state(pimc_ctx* c, int r, double* coords, double* angles, double* cosines) {
     if (!c->committed) return fail(c, "pimc_commit first");
     if (r < 0 || r >= c->nrep) return fail(c, "replica index out of range");
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
     const Rep& p = c->rep[r];
     const int n = p.natoms * p.P;
-    if (coords) {
+    const bool rotor = (angles || cosines) && (p.rotkind || p.fam == 1);
+    const int m = rotor ? p.tnumb[p.imtype] * p.Prot : 0;
+    const bool packed = sizeof(double) * (3 * (size_t)n + 6 * (size_t)m) <= c->back_state_bytes;
+    const double* st = reinterpret_cast<const double*>(c->back + c->back_state);
+    if (packed) {  // the device packs into host memory: 16 us for 1152 beads, two copies and the packing here 45
+        hipLaunchKernelGGL(k_pack_state, dim3(std::min((n + m + 255) / 256, 1024)), dim3(256), 0, c->stream,
+                           c->d_beads + p.bead_off, n, c->d_rotb + p.rot_off, m, reinterpret_cast<double*>(c->back + c->back_state));
+        HIPCHECK(c, hipGetLastError());
+    }
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    if (coords && packed) {
+        std::memcpy(coords, st, sizeof(double) * 3 * n);
+    } else if (coords) {
         std::vector<double4> b(n);
         HIPCHECK(c, hipMemcpy(b.data(), c->d_beads + p.bead_off, sizeof(double4) * n, hipMemcpyDeviceToHost));
         for (int i = 0; i < n; ++i) {
@@ -1553,11 +1605,20 @@ int pimc_get_state(pimc_ctx* c, int r, double* coords, double* angles, double* c
         }
     }
     if (angles || cosines) {
-        for (int i = 0; i < n; ++i) {  // non-rotor entries keep the initial values
-            if (angles) { angles[i] = 0; angles[n + i] = 1; angles[2 * n + i] = 0; }
-            if (cosines) { cosines[i] = 0; cosines[n + i] = 0; cosines[2 * n + i] = 1; }
-        }
-        if (p.rotkind || p.fam == 1) {
+        for (double* d : {angles, cosines})  // non-rotor entries keep the initial values
+            if (d) {
+                std::fill(d, d + 3 * (size_t)n, 0.0);
+                std::fill(d + (d == angles ? 1 : 2) * (size_t)n, d + (d == angles ? 2 : 3) * (size_t)n, 1.0);
+            }
+        if (rotor && packed) {
+            for (int a = 0; a < p.tnumb[p.imtype]; ++a)
+                for (int q = 0; q < 3; ++q) {
+                    const size_t to = (size_t)q * n + (size_t)(p.tbegin[p.imtype] + a) * p.P;
+                    const double* from = st + 3 * (size_t)n + (size_t)q * m + (size_t)a * p.Prot;
+                    if (angles) std::memcpy(angles + to, from, sizeof(double) * p.Prot);
+                    if (cosines) std::memcpy(cosines + to, from + 3 * (size_t)m, sizeof(double) * p.Prot);
+                }
+        } else if (rotor) {
             const int nr = p.tnumb[p.imtype];
             std::vector<RotBead> rb((size_t)nr * p.Prot);
             HIPCHECK(c, hipMemcpy(rb.data(), c->d_rotb + p.rot_off, sizeof(RotBead) * rb.size(), hipMemcpyDeviceToHost));
@@ -1812,9 +1873,8 @@ void issue_pass(pimc_ctx* c, bool sampled) {
 }
 
 int check_errors(pimc_ctx* c) {
-    std::vector<Mut> m(c->nrep);
-    HIPCHECK(c, hipMemcpyAsync(m.data(), c->d_mut, sizeof(Mut) * c->nrep, hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    if (read_back(c)) return -1;
+    const Mut* m = c->back_mut();
     for (int r = 0; r < c->nrep; ++r) {
         if (m[r].err & 2) return fail(c, "rotor sweep: a neighbouring part did not arrive (replica " + std::to_string(r) + ")");
         if (m[r].err & 4) return fail(c, "large matrix test error (relative Euler angle off the rotden grid, replica " + std::to_string(r) + ")");
@@ -1832,6 +1892,7 @@ int pimc_run(pimc_ctx* c, int n_passes, int sample_every) {
     if (!c->committed) return fail(c, "pimc_commit first");
     if (c->opt_da && c->nparts3 && !c->mlp_ready)
         return fail(c, "delayed acceptance needs a surrogate: pimc_surrogate_train or pimc_surrogate_set first");
+    c->back_valid = false;
     for (int p = 0; p < n_passes; ++p) {
         const bool sampled = sample_every > 0 && (p + 1) % sample_every == 0;
         const bool inside = sampled && c->opt_samples_per_pass > 1;  // samples within the pass
@@ -1863,6 +1924,7 @@ int pimc_run(pimc_ctx* c, int n_passes, int sample_every) {
 int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
     if (!c->committed) return fail(c, "pimc_commit first");
     if (passes < 1 || passes > 64) return fail(c, "autotune: passes is 1 to 64");
+    c->back_valid = false;
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     // every candidate starts from the same state; the chains get it back at the end
     double4* sb = dalloc<double4>((size_t)std::max<long long>(c->nbeads, 1));
@@ -1997,35 +2059,34 @@ int pimc_synchronize(pimc_ctx* c) {
 
 int pimc_get_samples(pimc_ctx* c, int r, double* out, int max_samples) {
     if (!c->committed || r < 0 || r >= c->nrep) return fail(c, "bad replica");
-    Mut m;
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(&m, c->d_mut + r, sizeof(Mut), hipMemcpyDeviceToHost));
+    if (read_back(c)) return -1;
+    const Mut& m = c->back_mut()[r];
     if ((long long)m.nsamples > c->sample_cap)
         return fail(c, "replica " + std::to_string(r) + " took " + std::to_string(m.nsamples) + " samples, more than the " +
                            std::to_string(c->sample_cap) + " its buffer holds: read and clear them (pimc_clear_samples) " +
                            "at least every " + std::to_string(c->sample_cap) + " samples");
     int n = std::min<int>(std::min<int>((int)m.nsamples, c->sample_cap), max_samples);
-    if (n > 0)
+    if (n > c->back_samples)
         HIPCHECK(c, hipMemcpy(out, c->d_samples + c->rep[r].sample_off, sizeof(double) * 8 * n, hipMemcpyDeviceToHost));
+    else if (n > 0)
+        std::memcpy(out, c->back_sample(r), sizeof(double) * 8 * n);
     return n;
 }
 
 int pimc_clear_samples(pimc_ctx* c) {
-    std::vector<Mut> m(c->nrep);
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(m.data(), c->d_mut, sizeof(Mut) * c->nrep, hipMemcpyDeviceToHost));
-    for (auto& x : m) x.nsamples = 0;
-    HIPCHECK(c, hipMemcpy(c->d_mut, m.data(), sizeof(Mut) * c->nrep, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemset(c->d_hist, 0, sizeof(unsigned) * std::max<long long>(c->nhist, 1)));
-    HIPCHECK(c, hipMemset(c->d_rcf, 0, sizeof(double) * std::max<long long>(c->nrcfvals, 1)));
+    if (!c->committed) return fail(c, "pimc_commit first");
+    c->back_valid = false;
+    hipLaunchKernelGGL(k_clear_samples, dim3((c->nrep + 255) / 256), dim3(256), 0, c->stream, c->d_mut, c->nrep);
+    HIPCHECK(c, hipGetLastError());
+    HIPCHECK(c, hipMemsetAsync(c->d_hist, 0, sizeof(unsigned) * std::max<long long>(c->nhist, 1), c->stream));
+    HIPCHECK(c, hipMemsetAsync(c->d_rcf, 0, sizeof(double) * std::max<long long>(c->nrcfvals, 1), c->stream));
     return 0;
 }
 
 int pimc_get_counters(pimc_ctx* c, int r, double* total, double* accep) {
     if (!c->committed || r < 0 || r >= c->nrep) return fail(c, "bad replica");
-    Mut m;
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(&m, c->d_mut + r, sizeof(Mut), hipMemcpyDeviceToHost));
+    if (read_back(c)) return -1;
+    const Mut& m = c->back_mut()[r];
     for (int t = 0; t < c->rep[r].ntypes; ++t)
         for (int k = 0; k < 3; ++k) {
             total[3 * t + k] = (double)m.total[t][k];
@@ -2082,12 +2143,10 @@ int pimc_get_rcf(pimc_ctx* c, int r, double* out, int max_values) {
 }
 
 int pimc_get_work(pimc_ctx* c, double* pair_evals, double* bead_moves) {
-    std::vector<Mut> m(c->nrep);
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(m.data(), c->d_mut, sizeof(Mut) * c->nrep, hipMemcpyDeviceToHost));
+    if (read_back(c)) return -1;
     double pe = 0;
-    for (auto& x : m)
-        for (int k = 0; k < 4; ++k) pe += (double)x.pair_evals[k];
+    for (int r = 0; r < c->nrep; ++r)
+        for (int k = 0; k < 4; ++k) pe += (double)c->back_mut()[r].pair_evals[k];
     if (pair_evals) *pair_evals = pe;
     if (bead_moves) *bead_moves = c->bead_moves;
     return 0;
@@ -2165,6 +2224,7 @@ int pimc_pot_energy_slice_noalloc(pimc_ctx* c, int nq, const int* qr, const int*
 
 int pimc_estimate(pimc_ctx* c, double* out) {
     if (!c->committed) return fail(c, "pimc_commit first");
+    c->back_valid = false;  // its pair evaluations are counted
     if (c->fp64) launch_estimate<double>(c, c->d_est);
     else launch_estimate<float>(c, c->d_est);
     HIPCHECK(c, hipGetLastError());
@@ -2179,11 +2239,9 @@ int pimc_family_evals(pimc_ctx* c, const char* family, double* evals) {
     for (int i = 0; i < 4; ++i)
         if (std::strcmp(names[i], family) == 0) k = i;
     if (k < 0) return fail(c, "unknown kernel family");
-    std::vector<Mut> m(c->nrep);
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(m.data(), c->d_mut, sizeof(Mut) * c->nrep, hipMemcpyDeviceToHost));
+    if (read_back(c)) return -1;
     double e = 0;
-    for (auto& x : m) e += (double)x.pair_evals[k];
+    for (int r = 0; r < c->nrep; ++r) e += (double)c->back_mut()[r].pair_evals[k];
     *evals = e;
     return 0;
 }
@@ -2480,9 +2538,8 @@ int pimc_surrogate_eval(pimc_ctx* c, const float* x, int n, float* out) {
 
 int pimc_get_da_counters(pimc_ctx* c, int r, double* out) {
     if (!c->committed || r < 0 || r >= c->nrep || !out) return fail(c, "bad replica");
-    Mut m;
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    HIPCHECK(c, hipMemcpy(&m, c->d_mut + r, sizeof(Mut), hipMemcpyDeviceToHost));
+    if (read_back(c)) return -1;
+    const Mut& m = c->back_mut()[r];
     for (int k = 0; k < 3; ++k) out[k] = (double)m.da[k];
     out[3] = (double)m.surrogate_evals;
     return 0;

@@ -2879,6 +2879,48 @@ __global__ void k_surrogate_collect(const Rep* __restrict__ reps, const double4*
     }
 }
 
+// ------------------------------------------------------------------------- read-back
+// Counters and the first `most` samples of every replica into host memory that the device writes:
+// one launch a run, instead of two copies a replica and getter at 10 to 15 us each.
+__global__ __launch_bounds__(64) void k_read_back(const Mut* __restrict__ mut, const Rep* __restrict__ reps,
+                                                  const double* __restrict__ samples, int most, Mut* __restrict__ hmut,
+                                                  double* __restrict__ hsamples) {
+    const int r = blockIdx.x;
+    static_assert(sizeof(Mut) % 8 == 0, "copied by words");
+    const unsigned long long* src = reinterpret_cast<const unsigned long long*>(mut + r);
+    unsigned long long* dst = reinterpret_cast<unsigned long long*>(hmut + r);
+    for (int i = threadIdx.x; i < (int)(sizeof(Mut) / 8); i += 64) dst[i] = src[i];
+    const int n = 8 * (int)min(mut[r].nsamples, (unsigned)most);
+    for (int i = threadIdx.x; i < n; i += 64) hsamples[(long long)r * most * 8 + i] = samples[reps[r].sample_off + i];
+}
+
+// A replica's n beads as [3][n] and its m rotor slices as [6][m] (phi, cos theta, chi, axis)
+__global__ __launch_bounds__(256) void k_pack_state(const double4* __restrict__ beads, int n, const RotBead* __restrict__ rotb,
+                                                    int m, double* __restrict__ out) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n + m; i += gridDim.x * 256) {
+        if (i < n) {
+            const double4 b = beads[i];
+            out[i] = b.x;
+            out[n + i] = b.y;
+            out[2 * n + i] = b.z;
+        } else {
+            const RotBead b = rotb[i - n];
+            double* o = out + 3 * n + (i - n);
+            o[0] = b.phi;
+            o[m] = b.cth;
+            o[2 * m] = b.chi;
+            o[3 * m] = b.nx;
+            o[4 * m] = b.ny;
+            o[5 * m] = b.nz;
+        }
+    }
+}
+
+__global__ void k_clear_samples(Mut* mut, int n) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < n) mut[r].nsamples = 0;
+}
+
 // ------------------------------------------------------------------------- end of pass
 __global__ void k_pass_end(Mut* mut, int n) {
     int r = blockIdx.x * blockDim.x + threadIdx.x;
