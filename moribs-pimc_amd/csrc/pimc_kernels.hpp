@@ -1822,9 +1822,10 @@ __device__ __forceinline__ void rotor3d_ahead(const Rot3dEnv& e, const RotPart& 
 // instructions (two generator calls, the frame, six arc cosines, an energy) and what it reads: its
 // neighbours' and partner's frames, its angles, and two gathers for its links.  InLds keeps the chain's
 // state in LDS for the launch, which leaves the gathers and positions to memory: of a frame the x and
-// z axes (y is their cross product) and of the angles phi and chi (cos theta is the z axis' third
-// component), 72 bytes a rotor and slice with the link's density, so that two parts of 512 slices of
-// two rotors share a CU.  Even and odd slices lie apart: the lanes' accesses then meet no bank twice.
+// z axes (y is their cross product) and of the angles phi and chi, 72 bytes a rotor and slice with
+// the link's density, so that two parts of 512 slices of two rotors share a CU; cos theta is on the
+// lane (at most one move a lane of either parity).  Even and odd slices lie apart: the lanes' accesses
+// then meet no bank twice.
 // Otherwise (rotor3d_in_lds) state is read and written in memory.
 // LDS: Lk[q][ns+1], Ea[q][ns] (sum over atoms) with atoms, Er[ns] (pair energy) with two rotors, then
 // axes[q][ns+2] and angles[q][ns], or the neighbours' frames fnb[2][nrot] (k0-1, then k1).
@@ -1889,7 +1890,6 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
             if (kl > 0 && kl <= ns) {
                 const RotBead& b = e.rotb[e.at(q, slice(kl))];
                 angles(q, kl) = {b.phi, b.chi};
-                axes(q, kl).z[2] = b.cth;
             }
         }
     } else {
@@ -1931,7 +1931,21 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
     }
     __syncthreads();
     const int nwords = 2 * NROT * (FRAME_D + 1);
-    unsigned moved = 0;  // InLds: bit (move / lanes) 2 NROT + parity NROT + q, the slices to write back
+    // InLds: cos theta of the lane's even and odd slice, and which of them were moved (bit parity NROT + q)
+    double cth_now[2][NROT];
+    unsigned moved = 0;
+    if constexpr (InLds) {
+#pragma unroll
+        for (int i = 0; i < 2 * NROT; ++i)
+            if ((int)threadIdx.x < half_ns)
+                cth_now[i / NROT][i % NROT] = e.rotb[e.at(i % NROT, k0 + 2 * (int)threadIdx.x + i / NROT)].cth;
+    }
+    auto cth_of = [&](int parity, int q) -> double {
+        const double c0 = parity ? cth_now[1][0] : cth_now[0][0];
+        if constexpr (NROT == 1) return c0;
+        const double c1 = parity ? cth_now[1][NROT - 1] : cth_now[0][NROT - 1];
+        return q ? c1 : c0;
+    };
 #pragma unroll 1
     for (int h = 0; h < 2 * e.nsweep; ++h) {
         const int parity = h & 1, sw = h >> 1;
@@ -1952,9 +1966,8 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
             __syncthreads();
             if (*s_err) break;  // as in rotor3d_ahead
         }
-        unsigned bit = parity * NROT;
 #pragma unroll 1
-        for (int mv = threadIdx.x; mv < half_ns; mv += blockDim.x, bit += 2 * NROT) {
+        for (int mv = threadIdx.x; mv < half_ns; mv += blockDim.x) {
             const int kl = 2 * mv + parity + 1, k = k0 + kl - 1;
 #pragma unroll 1
             for (int q = 0; q < NROT; ++q) {
@@ -1963,7 +1976,7 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
                 if constexpr (InLds) {
                     phi = angles(q, kl).phi;
                     chi = angles(q, kl).chi;
-                    cth = axes(q, kl).z[2];
+                    cth = cth_of(parity, q);
                 } else {
                     const RotBead& cur = e.rotb[ik];
                     phi = cur.phi;
@@ -1990,7 +2003,10 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
                     if constexpr (InLds) {
                         set_axes(q, kl, f);
                         angles(q, kl) = {p.phi, p.chi};
-                        moved |= 1u << (bit + q);
+#pragma unroll
+                        for (int i = 0; i < 2 * NROT; ++i)
+                            if (i == parity * NROT + q) cth_now[i / NROT][i % NROT] = p.cth;
+                        moved |= 1u << (parity * NROT + q);
                     } else {
                         rot3d_store(e, ik, p.phi, p.cth, p.chi, f);
                     }
@@ -2022,16 +2038,11 @@ __device__ __forceinline__ void rotor3d_long(const Rot3dEnv& e, const RotPart& p
     }
     if constexpr (InLds) {
 #pragma unroll 1
-        for (int parity = 0; parity < 2; ++parity) {
-            unsigned bit = parity * NROT;
-            for (int mv = threadIdx.x; mv < half_ns; mv += blockDim.x, bit += 2 * NROT)
-#pragma unroll 1
-                for (int q = 0; q < NROT; ++q) {
-                    if (!(moved >> (bit + q) & 1)) continue;
-                    const int kl = 2 * mv + parity + 1;
-                    const double phi = angles(q, kl).phi, chi = angles(q, kl).chi, cth = axes(q, kl).z[2];
-                    rot3d_store(e, e.at(q, k0 + kl - 1), phi, cth, chi, make_frame(phi, cth, chi));
-                }
+        for (int i = 0; i < 2 * NROT; ++i) {
+            if (!(moved >> i & 1)) continue;
+            const int parity = i / NROT, q = i - parity * NROT, kl = 2 * (int)threadIdx.x + parity + 1;
+            const double phi = angles(q, kl).phi, chi = angles(q, kl).chi, cth = cth_of(parity, q);
+            rot3d_store(e, e.at(q, k0 + kl - 1), phi, cth, chi, make_frame(phi, cth, chi));
         }
     }
 }

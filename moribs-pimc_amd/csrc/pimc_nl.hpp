@@ -11,7 +11,6 @@
 namespace pimc {
 
 constexpr double PI_D = 3.14159265358979323846;
-constexpr double DEG_D = 180.0 / PI_D;
 
 // 1/sqrt(x) for x > 0: the hardware's estimate (2^-23) and one third-order step, within an ulp or
 // so; a square root and a division are four times the instructions.
@@ -29,13 +28,15 @@ __device__ __forceinline__ double fmod_near(double x, double y) {
 }
 
 // matpre (rotden.f:136-163) of (phi, theta = acos(cos theta), chi), as MCRot3Dstep passes the
-// angles (mc_piqmc.cc:1019-1024); sin theta from (1 - cos)(1 + cos), whose factors are exact near
-// the poles.  Host and device build frames with the same expressions.
+// angles (mc_piqmc.cc:1019-1024).  Host and device build frames with the same expressions.
+// cos(acos(cth)) is not cth to the last bit, and it has to stay: a link between near frames divides
+// differences of products by the square of its small angle, and then meets the table's cells, whose
+// interpolation is not continuous, so that a last bit here decides a move of some runs differently.
 __host__ __device__ inline Frame make_frame(double phi, double cth, double chi) {
-    double cp, sp, ck, sk;
+    double cp, sp, ct, st, ck, sk;
     sincos(phi, &sp, &cp);
+    sincos(acos(cth), &st, &ct);
     sincos(chi, &sk, &ck);
-    const double ct = cth, st = sqrt((1.0 - cth) * (1.0 + cth));
     Frame f;
     f.m[0] = cp * ct * ck - sp * sk;   // (1,1)
     f.m[1] = sp * ct * ck + cp * sk;   // (2,1)
@@ -60,6 +61,13 @@ __device__ __forceinline__ double within1(double v) {  // rotden.f:208-216
     return v;
 }
 
+// a / b, correctly rounded, from the correctly rounded inverse of b: the product, and its remainder
+// (Markstein 1990); three instructions where a second division by the same b takes a dozen
+__device__ __forceinline__ double quotient(double a, double b, double inv) {
+    const double q = a * inv;
+    return fma(fma(-q, b, a), inv, q);
+}
+
 // deleul (rotden.f:32-134): Euler angles, in radians, of the rotation whose elements r2(i, j) gives
 template <typename M>
 __device__ __forceinline__ void deleul(M r2, double& phi2, double& theta2, double& chi2) {
@@ -76,10 +84,10 @@ __device__ __forceinline__ void deleul(M r2, double& phi2, double& theta2, doubl
         cchi = r2(2, 2);
         chi_up = r2(1, 2) > 0.0;
     } else {
-        const double inv = rsqrt_fast((1.0 - cost) * (1.0 + cost));  // 1 / sin theta: positive in this branch
+        const double sint = sin(theta2), inv = 1.0 / sint;  // positive in this branch
         phi_up = r2(2, 3) > 0.0;
-        phi2 = acos(within1(r2(1, 3) * inv));
-        cchi = -r2(3, 1) * inv;
+        phi2 = acos(within1(quotient(r2(1, 3), sint, inv)));
+        cchi = quotient(-r2(3, 1), sint, inv);
         chi_up = r2(3, 2) > 0.0;
     }
     chi2 = acos(within1(cchi));
@@ -94,6 +102,8 @@ __device__ __forceinline__ double rel_element(const Frame& f1, const Frame& f2, 
     for (int k = 1; k <= 3; ++k) v = v + fm(f1, k, i) * fm(f2, k, j);
     return v;
 }
+
+__device__ __forceinline__ double degrees(double x) { return quotient(x * 180.0, PI_D, 1.0 / PI_D); }
 
 // rotden (rotden.f:1-31) with rotpro (rotpro_sub.f:1-64): corner value plus one forward
 // difference per axis on the 1-degree grid, index (itheta*361 + iphi)*361 + ichi; E and E^2
@@ -111,7 +121,7 @@ template <typename M>
 __device__ __forceinline__ int rotden_cell_of(M r2, const double4* __restrict__ tab, RhoCell& c) {
     double p2, t2, c2;
     deleul(r2, p2, t2, c2);
-    const double phi = p2 * DEG_D, theta = t2 * DEG_D, chi = c2 * DEG_D;
+    const double phi = degrees(p2), theta = degrees(t2), chi = degrees(c2);
     int stop = 0;
     int ichi = (int)chi, iphi = (int)phi, ith = (int)theta;
     if (ichi > 360 || ichi < 0) { ichi = 0; stop = 1; }
@@ -158,7 +168,7 @@ __device__ inline int rotden_frames(const Frame& f1, const Frame& f2, const doub
         rel[1] = t2;
         rel[2] = c2;
     }
-    const double phi = p2 * DEG_D, theta = t2 * DEG_D, chi = c2 * DEG_D;
+    const double phi = degrees(p2), theta = degrees(t2), chi = degrees(c2);
     int stop = 0;
     int ichi = (int)chi, iphi = (int)phi, ith = (int)theta;
     if (ichi > 360 || ichi < 0) { ichi = 0; stop = 1; }

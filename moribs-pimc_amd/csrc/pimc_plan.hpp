@@ -148,8 +148,10 @@ inline int plan_linear_rotor(const std::vector<RotorChain>& chains, size_t geo_b
 // rotor) and the frames fit LDS beside those of other parts.
 constexpr int ROT3D_AHEAD = 256;
 
-// A longer part keeps its state in LDS where two parts of its size then share a CU (rotor3d_long):
-// energies and link densities, and 64 bytes a rotor and slice of axes and angles.
+// A longer part keeps its state in LDS where two parts of its size then share a CU and a lane has one
+// move of either parity (rotor3d_long): energies and link densities, and 64 bytes a rotor and slice
+// of axes and angles.
+constexpr int ROT3D_LANES = 512;
 constexpr size_t ROT3D_HALF_CU = 80 * 1024 - 256;
 constexpr size_t rotor3d_sums_lds(int ns, int nrot, bool atoms) {
     return (size_t)((nrot * (ns + 1) + (atoms ? nrot * ns : 0) + (nrot - 1) * ns + 1) & ~1) * sizeof(double);
@@ -157,7 +159,9 @@ constexpr size_t rotor3d_sums_lds(int ns, int nrot, bool atoms) {
 constexpr size_t rotor3d_state_lds(int ns, int nrot, bool atoms) {
     return rotor3d_sums_lds(ns, nrot, atoms) + (size_t)nrot * (ns + 2) * 48 + (size_t)nrot * ns * 16;
 }
-constexpr bool rotor3d_in_lds(int ns, int nrot, bool atoms) { return rotor3d_state_lds(ns, nrot, atoms) <= ROT3D_HALF_CU; }
+constexpr bool rotor3d_in_lds(int ns, int nrot, bool atoms) {
+    return ns <= ROT3D_LANES && rotor3d_state_lds(ns, nrot, atoms) <= ROT3D_HALF_CU;
+}
 
 // LDS that parts of up to ns slices of k_rotor3d_parts take with up to nrot rotors.  Short ones: the
 // link densities, then the frames of all slices (two neighbours' included) and of the proposals, nine
@@ -170,7 +174,7 @@ inline size_t rotor3d_part_lds(int ns, int nrot, size_t frame_bytes) {
                                 (size_t)na * (9 * nr + (nr > 1 ? 4 : 0)) * sizeof(double));
         if (nr * ns > ROT3D_AHEAD) {
             lds = std::max(lds, rotor3d_sums_lds(ns, nr, true) + (size_t)2 * nr * frame_bytes);
-            lds = std::max(lds, std::min(rotor3d_state_lds(ns, nr, true), ROT3D_HALF_CU));
+            lds = std::max(lds, std::min(rotor3d_state_lds(std::min(ns, ROT3D_LANES), nr, true), ROT3D_HALF_CU));
         }
     }
     return lds;
