@@ -1466,8 +1466,8 @@ int pimc_commit(pimc_ctx* c) {
         c->lds_rot3 = lds_for(c->rot3_block);
         if (!rot3.empty() && c->lds_rot3 > 160 * 1024) return fail(c, "non-linear rotor chain exceeds LDS");
     }
-    // bisection block: enough lanes for the widest level of the largest window
-    c->bisect_block = c->Nmax <= 24 ? 64 : (c->Nmax <= 64 ? 128 : 256);
+    // bisection block of the non-linear family: lanes for a pass over three levels of the largest window
+    c->bisect_block = c->Nmax <= 10 ? 64 : (c->Nmax <= 19 ? 128 : 256);
     c->committed = true;
     return 0;
 }
@@ -1797,7 +1797,7 @@ void launch_estimate(pimc_ctx* c, double* out) {
                            c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_rows1,
                            out ? nullptr : c->d_hist, c->d_rowbuf);
     if (!out && c->nrcf)
-        hipLaunchKernelGGL(k_rcf, dim3(c->nrcf, (c->rcf_protmax + 255) / 256), dim3(256), 0, c->stream, c->d_rep,
+        hipLaunchKernelGGL(k_rcf, dim3(c->nrcf, (c->rcf_protmax / 2 + RCF_OFFSETS) / RCF_OFFSETS), dim3(256), 0, c->stream, c->d_rep,
                            c->d_rotb, c->d_rcfreps, c->d_rcf);
     hipLaunchKernelGGL(k_est_final, dim3(c->nrep), dim3(256), 0, c->stream, c->d_rep, c->d_mut, c->d_rotb,
                        c->d_frames, c->tables(), c->tables3(),

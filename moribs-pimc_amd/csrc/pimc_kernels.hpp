@@ -98,18 +98,6 @@ __device__ __forceinline__ const Frame& frame_at(const Frame* __restrict__ frame
 }
 
 // ------------------------------------------------------------------------- bisection
-// block_sum with barriers that order LDS only
-__device__ __forceinline__ double block_sum_lds(double v, double* red) {
-    v = wave_sum(v);
-    const int wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    lds_barrier();
-    if ((threadIdx.x & 63) == 0) red[wid] = v;
-    lds_barrier();
-    double s = 0;
-    for (int i = 0; i < nw; ++i) s += red[i];
-    return s;
-}
-
 // LDS written by some lanes of a wave and read by others: a wave's LDS operations complete in
 // order, so only the compiler has to keep theirs
 __device__ __forceinline__ void wave_sync() {
@@ -522,7 +510,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 // Non-linear rotors: one workgroup per segment, its window of all atoms' beads and of the rotors'
-// frames in LDS, every level's items (midpoint, partner) over the block.
+// frames in LDS.  A move's first three levels are one pass over (midpoint, partner) with one
+// reduction, later levels one each: with few segments the barriers, reductions and idle lanes of a
+// pass per level were the time.  Partners that are rotors go to the last lanes, so that one wave and
+// not all of them takes the 3D table's path.  33 atoms on 32 segments: 163 us a launch with a pass
+// per level, now 128; two rotors on 32768 segments 214 us, now 139.
 // The window of all atoms' positions on the segment's S+1 slots is held in the pair precision
 // (float4 in FP32 runs, double4 in FP64 runs); new positions come from prop, one atom ahead, and
 // accepted ones go to HBM in FP64 at once.  blockDim a multiple of 64.  The rotors' frames at the
@@ -535,7 +527,7 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
                                                    const Frame* __restrict__ frames, Tables T, Tables3 T3,
                                                    const double4* __restrict__ prop, const int2* __restrict__ work, Run run) {
     extern __shared__ double smem[];
-    __shared__ double red[16];
+    __shared__ double red[2][4][3];  // a pass's level sums per wave, two buffers
     const int2 wk = work[blockIdx.x];
     const Rep& rp = reps[wk.x];
     const int tid = threadIdx.x, nth = blockDim.x;
@@ -580,6 +572,7 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
     __syncthreads();
 
     unsigned long long evals = 0;
+    int pb = 0;  // buffer of the next level sums
     unsigned long long tot[MAXT] = {0, 0, 0, 0}, acc_n[MAXT] = {0, 0, 0, 0};
     const int tend = run.type_end < rp.ntypes ? run.type_end : rp.ntypes;
 
@@ -611,32 +604,36 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
             if (tid < nm && ia + 1 < rp.tnumb[ty]) nxt = prop[ib + P + (s0 + 1 + tid) % P];
             double cum = 0.0;
             bool accepted = false;
-            for (int level = 0; level < L; ++level) {
-                const int lss = 1 << (L - level);
-                const int half = lss >> 1;
-                const int nmid = 1 << level;
-                // Delta V at the new midpoints: items (midpoint, partner)
-                const int np = N - 1;
-                const int items = nmid * np;
-                const bool rot_a = a >= rp.nl_atom;
-                auto item_sum = [&](auto mi_c) -> double {
+            const bool rot_a = a >= rp.nl_atom;
+            const int na = rp.nl_atom - (rot_a ? 0 : 1), nr = rp.nrot - (rot_a ? 1 : 0);  // partners by kind
+            for (int level = 0; level < L;) {
+                const int end = level == 0 ? min(3, L) : level + 1;  // levels of this pass
+                const int m0 = (1 << level) - 1, nmid = (1 << end) - 1 - m0;
+                double acc[3] = {0.0, 0.0, 0.0};
+                // Delta V at new midpoint m (level-major order) with partner j
+                auto item = [&](int m, int j, auto rj_c, const double* bx) {
+                    constexpr bool rj = decltype(rj_c)::value;
+                    const int lv = 31 - __clz(m + 1), half = 1 << (L - lv - 1);
+                    const int slot = half + ((m + 1 - (1 << lv)) << (L - lv));
+                    const P4 pj = win[j * W + slot], pa = win[a * W + slot], pn = nwf[slot];
+                    const Frame& fa = fr[(rot_a ? a - rp.nl_atom : 0) * W + slot];
+                    const Frame& fj = fr[(rj ? j - rp.nl_atom : 0) * W + slot];
+                    const double v = pair_nl<R>(l1, kn, l3, rot_a, rj, pn.x, pn.y, pn.z, pj.x, pj.y, pj.z, fa, fj, bx) -
+                                     pair_nl<R>(l1, kn, l3, rot_a, rj, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, fa, fj, bx);
+                    acc[0] += lv == level ? v : 0.0;
+                    acc[1] += lv == level + 1 ? v : 0.0;
+                    acc[2] += lv == level + 2 ? v : 0.0;
+                };
+                auto items = [&](auto mi_c) {
                     // the minimum image as its own instance of the loop, so the plain one is unchanged
                     const double* bx = decltype(mi_c)::value ? box : nullptr;
-                    double acc = 0.0;
-                    // item i = (midpoint q, partner index jp); a lane's items advance by nth, so
-                    // (q, jp) is carried along with one division per level
-                    const int dd = np > 0 ? np : 1;
+                    // item (m, jp) of the atoms: a lane's items advance by nth, so it is carried along
+                    // with one division per pass
+                    const int dd = na > 0 ? na : 1;
                     const int dq = nth / dd, dj = nth - dq * dd;
                     int q = tid / dd, jp = tid - q * dd;
-                    for (int i = tid; i < items; i += nth) {
-                        const int j = jp + (jp >= a);
-                        const bool rj = j >= rp.nl_atom;
-                        const int slot = half + q * lss;
-                        const P4 pj = win[j * W + slot], pa = win[a * W + slot], pn = nwf[slot];
-                        const Frame& fa = fr[(rot_a ? a - rp.nl_atom : 0) * W + slot];
-                        const Frame& fj = fr[(rj ? j - rp.nl_atom : 0) * W + slot];
-                        acc += pair_nl<R>(l1, kn, l3, rot_a, rj, pn.x, pn.y, pn.z, pj.x, pj.y, pj.z, fa, fj, bx) -
-                               pair_nl<R>(l1, kn, l3, rot_a, rj, pa.x, pa.y, pa.z, pj.x, pj.y, pj.z, fa, fj, bx);
+                    for (int i = tid; i < nmid * na; i += nth) {
+                        item(m0 + q, jp + (!rot_a && jp >= a), std::integral_constant<bool, false>{}, bx);
                         jp += dj;
                         q += dq;
                         if (jp >= dd) {
@@ -644,20 +641,34 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
                             ++q;
                         }
                     }
-                    return acc;
+                    for (int i = nth - 1 - tid; i < nmid * nr; i += nth) {
+                        const int m = i / nr, p = i - m * nr;
+                        item(m0 + m, rp.nl_atom + p + (rot_a && p >= a - rp.nl_atom), std::integral_constant<bool, true>{}, bx);
+                    }
                 };
-                double acc;
-                if constexpr (MI)
-                    acc = box ? item_sum(std::integral_constant<bool, true>{}) : item_sum(std::integral_constant<bool, false>{});
-                else
-                    acc = item_sum(std::integral_constant<bool, false>{});
-                acc = block_sum_lds(acc, red);
-                evals += 2ull * (unsigned long long)items;
-                // sum over all points up to this level; level acceptance of mc_piqmc.cc:263-273
-                const double prev = cum;
-                cum += acc;
-                double deltav = (cum - 2.0 * prev) * (rp.tau * (double)half);
-                accepted = deltav < 0.0 || deltav < tst[level];
+                if constexpr (MI) {
+                    if (box) items(std::integral_constant<bool, true>{});
+                    else items(std::integral_constant<bool, false>{});
+                } else {
+                    items(std::integral_constant<bool, false>{});
+                }
+                for (int k = 0; k < end - level; ++k) {
+                    const double v = wave_sum(k == 0 ? acc[0] : (k == 1 ? acc[1] : acc[2]));
+                    if ((tid & 63) == 0) red[pb][tid >> 6][k] = v;
+                }
+                lds_barrier();
+                evals += 2ull * (unsigned long long)(nmid * (N - 1));
+                // sum over all points up to each level; level acceptance of mc_piqmc.cc:263-273
+                for (int k = 0; level < end; ++level, ++k) {
+                    double sum = 0.0;
+                    for (int i = 0; i < nth >> 6; ++i) sum += red[pb][i][k];
+                    const double prev = cum;
+                    cum += sum;
+                    const double deltav = (cum - 2.0 * prev) * (rp.tau * (double)(1 << (L - level - 1)));
+                    accepted = deltav < 0.0 || deltav < tst[level];
+                    if (!accepted) break;
+                }
+                pb ^= 1;
                 if (!accepted) break;
             }
             tot[ty] += 1;
@@ -2110,31 +2121,53 @@ __global__ void k_frames_from_angles(const Rep* __restrict__ reps, const RotBead
 // first rotor of the rotating type, p = n(it0).n(it0+itc) with the unit axes of MCCosine;
 // rcf[0][itc] += p and rcf[l][itc] += P_l(p) for l = 1..9.  (The reference adds 1.0 for l >= 1:
 // its Legendre call is commented out; here P_l comes from the three-term recurrence.)
-// Grid (replica, offset block of 256): a lane per offset, accumulated in FP64.
+// The sum over origins is the same for an offset and its complement to Prot, so offsets up to Prot / 2
+// are summed.  Grid (replica, block of RCF_OFFSETS offsets): a block's lanes share the offsets by
+// ranges of origins, in FP64, the ranges' sums added in order.  A lane per offset over all origins,
+// dividing in the recurrence, took 1.91 ms for 128 chains of 2048 slices, now 0.76.
+constexpr int RCF_OFFSETS = 16, RCF_RANGES = 256 / RCF_OFFSETS;
 __global__ __launch_bounds__(256) void k_rcf(const Rep* __restrict__ reps, const RotBead* __restrict__ rotb,
                                              const int* __restrict__ list, double* __restrict__ rcf) {
+    __shared__ double part[RCF_RANGES][RCF_OFFSETS];
     const Rep& rp = reps[list[blockIdx.x]];
-    const int Prot = rp.Prot;
+    const int Prot = rp.Prot, last = Prot / 2;  // offsets 0 .. last
     const RotBead* b = rotb + rp.rot_off;
     double* out = rcf + rp.rcf_off;
-    for (int itc = blockIdx.y * blockDim.x + threadIdx.x; itc < Prot; itc += gridDim.y * blockDim.x) {
+    const int o = threadIdx.x % RCF_OFFSETS, g = threadIdx.x / RCF_OFFSETS;
+    const int from = (int)((long long)Prot * g / RCF_RANGES), end = (int)((long long)Prot * (g + 1) / RCF_RANGES);
+    for (int first = blockIdx.y * RCF_OFFSETS; first <= last; first += gridDim.y * RCF_OFFSETS) {
+        const int itc = first + o, to = itc <= last ? end : from;
         double acc[RCF_L];
+#pragma unroll
         for (int l = 0; l < RCF_L; ++l) acc[l] = 0.0;
-        int t1 = itc;
-        for (int it0 = 0; it0 < Prot; ++it0) {
+        int t1 = from + itc < Prot ? from + itc : from + itc - Prot;
+#pragma unroll 2
+        for (int it0 = from; it0 < to; ++it0) {
             const double p = b[it0].nx * b[t1].nx + b[it0].ny * b[t1].ny + b[it0].nz * b[t1].nz;
             acc[0] += p;
             double pm = 1.0, pc = p;  // P_0, P_1
             acc[1] += pc;
+#pragma unroll
             for (int l = 1; l + 1 < RCF_L; ++l) {
-                const double pn = ((2 * l + 1) * p * pc - l * pm) / (l + 1);
+                const double pn = ((2 * l + 1) / (double)(l + 1)) * (p * pc) - (l / (double)(l + 1)) * pm;
                 pm = pc;
                 pc = pn;
                 acc[l + 1] += pc;
             }
             if (++t1 == Prot) t1 = 0;
         }
-        for (int l = 0; l < RCF_L; ++l) out[(long long)l * Prot + itc] += acc[l];
+#pragma unroll
+        for (int l = 0; l < RCF_L; ++l) {
+            part[g][o] = acc[l];
+            __syncthreads();
+            if (g == l % RCF_RANGES && itc <= last) {
+                double v = 0.0;
+                for (int k = 0; k < RCF_RANGES; ++k) v += part[k][o];
+                out[(long long)l * Prot + itc] += v;
+                if (itc > 0 && 2 * itc != Prot) out[(long long)l * Prot + Prot - itc] += v;
+            }
+            __syncthreads();
+        }
     }
 }
 
