@@ -1345,9 +1345,11 @@ int pimc_commit(pimc_ctx* c) {
         return fail(c, "hipMalloc failed");
     {
         size_t state = 0;
-        for (const Rep& p : c->rep)
-            state = std::max(state, sizeof(double) * (3 * (size_t)p.natoms * p.P + 6 * (size_t)p.natoms * std::max(p.Prot, 0)));
-        c->back_samples = (int)std::min<size_t>(c->sample_cap, std::max<size_t>(1, 256 * 1024 / (64 * (size_t)c->nrep)));
+        for (const Rep& p : c->rep) {
+            const size_t m = p.rotkind || p.fam == 1 ? (size_t)p.tnumb[p.imtype] * p.Prot : 0;
+            state = std::max(state, sizeof(double) * (3 * (size_t)p.natoms * p.P + 6 * m));
+        }
+        c->back_samples = (int)std::min<size_t>(1024, std::max<size_t>(16, 128 * 1024 / (64 * (size_t)c->nrep)));
         c->back_state = sizeof(Mut) * c->nrep + (size_t)64 * c->back_samples * c->nrep;
         c->back_state_bytes = std::min<size_t>(state, 4 << 20);  // a larger replica is copied and packed on the host
         if (hipHostMalloc(reinterpret_cast<void**>(&c->back), c->back_state + c->back_state_bytes, hipHostMallocPortable | hipHostMallocMapped) !=

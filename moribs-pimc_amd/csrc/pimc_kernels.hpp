@@ -327,6 +327,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             nwf[i] = q;
             if (i < L) th[8 * buf + i] = v.w;
         };
+        const bool three = L >= 3;
+        const int m3 = gl / (GW / 8), lv3 = m3 < 7 ? 31 - __clz(m3 + 1) : 0;  // the lane's midpoint of the first three levels
+        const int slot3 = m3 < 7 && three ? ((m3 + 1 - (1 << lv3)) << (L - lv3)) + (1 << (L - lv3 - 1)) - 1 : 0;
+        const double tauh = tau * (double)(1 << (L - 1));
         double4 cur = make_double4(0.0, 0.0, 0.0, 0.0);
         if (gl < nm) cur = prop[ib + itl];
         group_sync<GW>();
@@ -375,9 +379,98 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                               (double)ax.z);
                         }
                     }
+                // V(new) - V(old) of the mover at a slot with partners jl, jl + G, ...
+                auto pairs = [&](int slot, int jl, int G) -> double {
+                    double acc = 0.0;
+                    const P4 pn = nwf[slot];
+                    const R* po = win + (slot * N + a) * 3;
+                    const R xa = po[0], ya = po[1], za = po[2];
+                    const R* ws = win + slot * N * 3;
+                    if (rot_a) {  // the rotor's partners are the atoms before it
+                        const P4 ax = nhf[slot];
+                        for (int j = jl; j < nat; j += G) {
+                            const R* pj = ws + 3 * j;
+                            const R dx = nearest_image(pn.x - pj[0], bx, 0), dy = nearest_image(pn.y - pj[1], bx, 1),
+                                    dz = nearest_image(pn.z - pj[2], bx, 2);
+                            const R ex = nearest_image(xa - pj[0], bx, 0), ey = nearest_image(ya - pj[1], bx, 1),
+                                    ez = nearest_image(za - pj[2], bx, 2);
+                            R vn, vo;
+                            if constexpr (UT) {
+                                const RotorCell kn_ = rotor_pair_load(l2, true, dx, dy, dz, ax.x, ax.y, ax.z);
+                                const RotorCell ko_ = rotor_pair_load(l2, true, ex, ey, ez, ax.x, ax.y, ax.z);
+                                vn = rotor_pair_value(kn_);
+                                vo = rotor_pair_value(ko_);
+                            } else {
+                                const double nx = ax.x, ny = ax.y, nz = ax.z;
+                                vn = pair_d<R>(l1, kn, l2, true, false, dx, dy, dz, nx, ny, nz);
+                                vo = pair_d<R>(l1, kn, l2, true, false, ex, ey, ez, nx, ny, nz);
+                            }
+                            acc += (double)vn - (double)vo;
+                        }
+                    } else {
+                        auto partners = [&](auto u_c) {
+                            constexpr int U = decltype(u_c)::value;
+                            for (int jp = jl; jp < nat - 1; jp += U * G) {
+                                R d[2 * U][3];
+#pragma unroll
+                                for (int i = 0; i < U; ++i) {
+                                    const int jn = i == 0 || jp + i * G < nat - 1 ? jp + i * G : jp;
+                                    const R* pj = ws + 3 * (jn + (jn >= a));
+                                    const R x = pj[0], y = pj[1], z = pj[2];
+                                    d[i][0] = nearest_image(pn.x - x, bx, 0);
+                                    d[i][1] = nearest_image(pn.y - y, bx, 1);
+                                    d[i][2] = nearest_image(pn.z - z, bx, 2);
+                                    d[U + i][0] = nearest_image(xa - x, bx, 0);
+                                    d[U + i][1] = nearest_image(ya - y, bx, 1);
+                                    d[U + i][2] = nearest_image(za - z, bx, 2);
+                                }
+                                acc += atom_terms<R, UT, U>(l1, kn, d, U == 1 || jp + G < nat - 1 ? U : 1);
+                            }
+                        };
+                        // partners in pairs, so that four look-ups of a lane interleave,
+                        // where most lanes have two or more
+                        if (UT && 2 * (nat - 1) > 3 * G) partners(std::integral_constant<int, 2>{});
+                        else partners(std::integral_constant<int, 1>{});
+                    }
+                    return acc;
+                };
                 double cum = 0.0;
                 bool alive = true;
-                for (int l0 = 0; l0 < L;) {
+                // The first three levels as one pass: an eighth of the group's lanes per midpoint, the
+                // sums of the seven midpoints added in their order.  With the general pass's loops and
+                // branches on L for them a move of 64 atoms issued 430 vector and 200 scalar
+                // instructions a wave and then read the partial sums one by one: a launch over 16
+                // boxes of 64 atoms 153 us, now 108; one chain of 64 145, now 107; the 256-replica
+                // scan 410, now 365.
+                if (three) {
+                    constexpr int G3 = GW / 8;
+                    double acc = 0.0;
+                    if (m3 < 7) acc = pairs(slot3, gl & (G3 - 1), G3);
+                    if (rterms) {
+                        if constexpr (UT)
+                            if (early && gl < 2 * nm) rt[gl] = rotor_pair_value(rc);
+                        group_sync<GW>();
+                        if (m3 < 7 && (gl & (G3 - 1)) == 0) acc += (double)rt[2 * m3] - (double)rt[2 * m3 + 1];
+                    }
+                    acc = group_sum(acc, G3);
+                    double* pt = part + 8 * pb;
+                    pb ^= 1;
+                    if ((gl & (G3 - 1)) == 0) pt[m3] = acc;
+                    group_sync<GW>();
+                    evals += 14ull * (unsigned)(N - 1);
+                    double p[7], t[3];
+#pragma unroll
+                    for (int i = 0; i < 7; ++i) p[i] = pt[i];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) t[i] = tst[i];
+                    // sum over all points up to a level; level acceptance of mc_piqmc.cc:263-273
+                    const double c0 = p[0], c1 = (c0 + p[1]) + p[2], c2 = (((c1 + p[3]) + p[4]) + p[5]) + p[6];
+                    const double dv0 = c0 * tauh, dv1 = (c1 - 2.0 * c0) * (0.5 * tauh), dv2 = (c2 - 2.0 * c1) * (0.25 * tauh);
+                    alive = (dv0 < 0.0 || dv0 < t[0]) && (dv1 < 0.0 || dv1 < t[1]) && (dv2 < 0.0 || dv2 < t[2]);
+                    cum = c2;
+                }
+                for (int l0 = three ? 3 : 0; l0 < L;) {
+                    if (GW >= 64 ? !alive : !__any(alive)) break;
                     // levels [l0, l1) in this pass: the first three together, then one at a time.
                     // Terms of levels behind a rejection are a fifth of all on the 256-replica scan
                     // (half on 8 atoms) and cost less than a pass and a reduction per level: 5.5
@@ -393,56 +486,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         double acc = 0.0;
                         for (int mc = gl >> lgG; mc < nmc; mc += GW >> lgG) {
                             const int slot = slot_of(m0 + mc);
-                            const P4 pn = nwf[slot];
-                            const R* po = win + (slot * N + a) * 3;
-                            const R xa = po[0], ya = po[1], za = po[2];
-                            const R* ws = win + slot * N * 3;
-                            if (rot_a) {  // the rotor's partners are the atoms before it
-                                const P4 ax = nhf[slot];
-                                for (int j = jl; j < nat; j += G) {
-                                    const R* pj = ws + 3 * j;
-                                    const R dx = nearest_image(pn.x - pj[0], bx, 0), dy = nearest_image(pn.y - pj[1], bx, 1),
-                                            dz = nearest_image(pn.z - pj[2], bx, 2);
-                                    const R ex = nearest_image(xa - pj[0], bx, 0), ey = nearest_image(ya - pj[1], bx, 1),
-                                            ez = nearest_image(za - pj[2], bx, 2);
-                                    R vn, vo;
-                                    if constexpr (UT) {
-                                        const RotorCell kn_ = rotor_pair_load(l2, true, dx, dy, dz, ax.x, ax.y, ax.z);
-                                        const RotorCell ko_ = rotor_pair_load(l2, true, ex, ey, ez, ax.x, ax.y, ax.z);
-                                        vn = rotor_pair_value(kn_);
-                                        vo = rotor_pair_value(ko_);
-                                    } else {
-                                        const double nx = ax.x, ny = ax.y, nz = ax.z;
-                                        vn = pair_d<R>(l1, kn, l2, true, false, dx, dy, dz, nx, ny, nz);
-                                        vo = pair_d<R>(l1, kn, l2, true, false, ex, ey, ez, nx, ny, nz);
-                                    }
-                                    acc += (double)vn - (double)vo;
-                                }
-                            } else {
-                                auto partners = [&](auto u_c) {
-                                    constexpr int U = decltype(u_c)::value;
-                                    for (int jp = jl; jp < nat - 1; jp += U * G) {
-                                        R d[2 * U][3];
-#pragma unroll
-                                        for (int i = 0; i < U; ++i) {
-                                            const int jn = i == 0 || jp + i * G < nat - 1 ? jp + i * G : jp;
-                                            const R* pj = ws + 3 * (jn + (jn >= a));
-                                            const R x = pj[0], y = pj[1], z = pj[2];
-                                            d[i][0] = nearest_image(pn.x - x, bx, 0);
-                                            d[i][1] = nearest_image(pn.y - y, bx, 1);
-                                            d[i][2] = nearest_image(pn.z - z, bx, 2);
-                                            d[U + i][0] = nearest_image(xa - x, bx, 0);
-                                            d[U + i][1] = nearest_image(ya - y, bx, 1);
-                                            d[U + i][2] = nearest_image(za - z, bx, 2);
-                                        }
-                                        acc += atom_terms<R, UT, U>(l1, kn, d, U == 1 || jp + G < nat - 1 ? U : 1);
-                                    }
-                                };
-                                // partners in pairs, so that four look-ups of a lane interleave,
-                                // where most lanes have two or more
-                                if (UT && 2 * (nat - 1) > 3 * G) partners(std::integral_constant<int, 2>{});
-                                else partners(std::integral_constant<int, 1>{});
-                            }
+                            acc += pairs(slot, jl, G);
                         }
                         if (rterms) {
                             if constexpr (UT)
@@ -473,7 +517,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                             alive = alive && (deltav < 0.0 || deltav < tst[level]);
                         }
                     }
-                    if (GW >= 64 ? !alive : !__any(alive)) break;
                     l0 = l1e;
                 }
                 return alive;
