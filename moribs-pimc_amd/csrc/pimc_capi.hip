@@ -270,6 +270,8 @@ struct pimc_ctx {
     RotPart* d_cparts0 = nullptr;    // centroid parts (slice ranges) of the linear family
     RotPart* d_cparts1 = nullptr;    // and of the non-linear family
     int ncp0 = 0, ncp1 = 0, ncflags = 0;
+    bool centroid_staged = false;    // every part keeps its beads in LDS
+    size_t lds_centroid = 0;
     unsigned* d_cflags = nullptr;    // atoms done per centroid part
     unsigned long long* d_cslots = nullptr;  // partial Delta V per part as two numbered words, two buffers
     // surrogate network of the delayed-acceptance rotor move
@@ -335,6 +337,17 @@ static void rotor_kernel(const pimc_ctx* c, F&& f) {  // the linear sweep's inst
     else if (c->rotor_long) f(k_rotor<float, false, ROTOR_MPL_LONG>);
     else c->rotor_uniform ? f(k_rotor<float, true, 1>) : f(k_rotor<float, false, 1>);
 }
+
+namespace {
+
+// the centroid move as the parts were planned
+template <typename R, int FAM>
+auto centroid_kernel(const pimc_ctx* c) {
+    if (c->centroid_staged) return c->any_mi ? k_centroid_parts<R, FAM, true, true> : k_centroid_parts<R, FAM, false, true>;
+    return c->any_mi ? k_centroid_parts<R, FAM, true, false> : k_centroid_parts<R, FAM, false, false>;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -843,21 +856,16 @@ static int plan_centroid_parts(pimc_ctx* c, int target_parts) {
     hipDeviceProp_t prop;
     HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
     const int ncu = prop.multiProcessorCount;
-    if (c->fp64) {
-        HIPCHECK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                        &occ0, (c->any_mi ? k_centroid_parts<double, 0, true> : k_centroid_parts<double, 0, false>), 256,
-                        c->lds_knots));
-        HIPCHECK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                        &occ1, (c->any_mi ? k_centroid_parts<double, 1, true> : k_centroid_parts<double, 1, false>), 256,
-                        c->lds_knots));
-    } else {
-        HIPCHECK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                        &occ0, (c->any_mi ? k_centroid_parts<float, 0, true> : k_centroid_parts<float, 0, false>), 256,
-                        c->lds_knots));
-        HIPCHECK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                        &occ1, (c->any_mi ? k_centroid_parts<float, 1, true> : k_centroid_parts<float, 1, false>), 256,
-                        c->lds_knots));
-    }
+    auto occupancy = [&](size_t lds) -> hipError_t {
+        auto both = [&](auto k0, auto k1) {
+            const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ0, k0, 256, lds);
+            return e != hipSuccess ? e : hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ1, k1, 256, lds);
+        };
+        return c->fp64 ? both(centroid_kernel<double, 0>(c), centroid_kernel<double, 1>(c))
+                       : both(centroid_kernel<float, 0>(c), centroid_kernel<float, 1>(c));
+    };
+    c->centroid_staged = false;
+    HIPCHECK(c, occupancy(c->lds_knots));
     const double capacity = (double)ncu * std::max(1, std::min(occ0, occ1));
     // the parts of a replica wait on one another on one XCD: at most what one XCD holds
     const int per_xcd = std::max(1, std::min(occ0, occ1)) * (ncu / 8);
@@ -888,6 +896,27 @@ static int plan_centroid_parts(pimc_ctx* c, int target_parts) {
             cp[p.fam].push_back(x);
         }
         fb += W;
+    }
+    // Beads in LDS where all parts' are within 24 KB and the parts stay resident at once, also the
+    // largest chain's on its XCD: single and few chains.  On a full device the larger parts read
+    // them from L2 (staged they would halve the parts a CU holds).
+    c->lds_centroid = c->lds_knots;
+    {
+        long long beads = 0;
+        int Wmax = 1;
+        for (const auto& list : cp)
+            for (const RotPart& q : list) {
+                beads = std::max(beads, (long long)(q.k1 - q.k0) * c->rep[q.r].natoms);
+                Wmax = std::max(Wmax, q.W);
+            }
+        const size_t lds = c->lds_knots + sizeof(double) * 3 * (size_t)beads;
+        if (beads <= 1024 && lds <= 64 * 1024) {
+            c->centroid_staged = true;
+            HIPCHECK(c, occupancy(lds));
+            const int occ = std::min(occ0, occ1);
+            c->centroid_staged = fb <= occ * ncu && Wmax <= occ * (ncu / 8);
+            if (c->centroid_staged) c->lds_centroid = lds;
+        }
     }
     auto cost = [&](int r) { return (double)c->rep[r].natoms * c->rep[r].natoms * c->rep[r].P; };
     for (int f = 0; f < 2; ++f)
@@ -1748,11 +1777,11 @@ void launch_centroid(pimc_ctx* c, int type) {
     Run run{c->seed, 0, c->ref_order ? 1 : 0, type, type + 1};
     Timed t(c, "centroid");
     if (c->ncp0)
-        hipLaunchKernelGGL((c->any_mi ? k_centroid_parts<R, 0, true> : k_centroid_parts<R, 0, false>), dim3(c->ncp0), dim3(256), c->lds_knots, c->stream, c->d_rep, c->d_mut,
+        hipLaunchKernelGGL((centroid_kernel<R, 0>(c)), dim3(c->ncp0), dim3(256), c->lds_centroid, c->stream, c->d_rep, c->d_mut,
                            c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_cparts0, c->d_cflags,
                            c->d_cslots, c->ncflags, run);
     if (c->ncp1)
-        hipLaunchKernelGGL((c->any_mi ? k_centroid_parts<R, 1, true> : k_centroid_parts<R, 1, false>), dim3(c->ncp1), dim3(256), c->lds_knots, c->stream, c->d_rep, c->d_mut,
+        hipLaunchKernelGGL((centroid_kernel<R, 1>(c)), dim3(c->ncp1), dim3(256), c->lds_centroid, c->stream, c->d_rep, c->d_mut,
                            c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_cparts1, c->d_cflags,
                            c->d_cslots, c->ncflags, run);
 }
@@ -1813,11 +1842,11 @@ void launch_centroid_all(pimc_ctx* c) {
     for (int ty = 0; ty < c->max_types; ++ty) {
         Run run{c->seed, 0, c->ref_order ? 1 : 0, ty, ty + 1};
         if (c->ncp0)
-            hipLaunchKernelGGL((c->any_mi ? k_centroid_parts<R, 0, true> : k_centroid_parts<R, 0, false>), dim3(c->ncp0), dim3(256), c->lds_knots, c->stream, c->d_rep,
+            hipLaunchKernelGGL((centroid_kernel<R, 0>(c)), dim3(c->ncp0), dim3(256), c->lds_centroid, c->stream, c->d_rep,
                                c->d_mut, c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_cparts0,
                                c->d_cflags, c->d_cslots, c->ncflags, run);
         if (c->ncp1)
-            hipLaunchKernelGGL((c->any_mi ? k_centroid_parts<R, 1, true> : k_centroid_parts<R, 1, false>), dim3(c->ncp1), dim3(256), c->lds_knots, c->stream, c->d_rep,
+            hipLaunchKernelGGL((centroid_kernel<R, 1>(c)), dim3(c->ncp1), dim3(256), c->lds_centroid, c->stream, c->d_rep,
                                c->d_mut, c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_cparts1,
                                c->d_cflags, c->d_cslots, c->ncflags, run);
     }
