@@ -2205,11 +2205,12 @@ int pot_slice_on(pimc_ctx* c, int nq, const int* qr, const int* qa, const int* q
     HIPCHECK(c, hipMemcpyAsync(d_a, qa, sizeof(int) * nq, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(d_i, qit, sizeof(int) * nq, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(d_p, qpos, sizeof(double) * 3 * nq, hipMemcpyHostToDevice, c->stream));
+    const dim3 grid((unsigned)std::min<long long>(((long long)nq * POT_LANES + 255) / 256, 1 << 20));
     if (c->fp64)
-        hipLaunchKernelGGL(k_pot_slice<double>, dim3((nq + 127) / 128), dim3(128), 0, c->stream, c->d_rep, c->d_beads,
+        hipLaunchKernelGGL(k_pot_slice<double>, grid, dim3(256), 0, c->stream, c->d_rep, c->d_beads,
                            c->d_rotb, c->d_frames, c->tables(), c->tables3(), nq, d_r, d_a, d_i, d_p, d_o);
     else
-        hipLaunchKernelGGL(k_pot_slice<float>, dim3((nq + 127) / 128), dim3(128), 0, c->stream, c->d_rep, c->d_beads,
+        hipLaunchKernelGGL(k_pot_slice<float>, grid, dim3(256), 0, c->stream, c->d_rep, c->d_beads,
                            c->d_rotb, c->d_frames, c->tables(), c->tables3(), nq, d_r, d_a, d_i, d_p, d_o);
     HIPCHECK(c, hipGetLastError());
     HIPCHECK(c, hipMemcpyAsync(out, d_o, sizeof(double) * nq, hipMemcpyDeviceToHost, c->stream));

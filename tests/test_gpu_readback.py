@@ -1,4 +1,4 @@
-"""What the getters return as the host's copy of counters and samples goes out of date, grows past its
+"""What queries and getters return: a batch of queries at the edges of its blocks, the getters as the host's copy of counters and samples goes out of date, grows past its
 room, and as a replica's state outgrows the packed read-back."""
 import numpy as np
 import pytest
@@ -55,4 +55,20 @@ def test_state_round_trip(atoms, P):
     assert np.array_equal(c, states[0])
     n = atoms * P
     assert np.array_equal(a, np.repeat([[0.0], [1.0], [0.0]], n, 1)) and np.array_equal(cs, np.repeat([[0.0], [0.0], [1.0]], n, 1))
+    ctx.close()
+
+
+@pytest.mark.parametrize("nq", [1, 31, 32, 33, 1000])
+def test_a_batch_of_queries_is_its_queries(nq):
+    """Whatever shares a query's block; the energies themselves are checked against the oracle with the
+    estimators.  One query's sum runs over the same lanes in any batch, so it is the same bits."""
+    ctx, states = box(3, 11, 16)
+    rng = np.random.default_rng(nq)
+    rep, atom, it = rng.integers(0, 3, nq), rng.integers(0, 11, nq), rng.integers(0, 16, nq)
+    pos = np.array([states[r][:, a * 16 + i] for r, a, i in zip(rep, atom, it)]) + rng.normal(0, 0.1, (nq, 3))
+    rep, atom, it = (x.astype(np.int32) for x in (rep, atom, it))
+    got = ctx.pot_energy_slice(rep, atom, it, pos)
+    for q in {0, nq // 2, nq - 1}:
+        one = ctx.pot_energy_slice(rep[q:q + 1], atom[q:q + 1], it[q:q + 1], pos[q:q + 1])
+        assert one[0] == got[q] and np.isfinite(got[q]) and got[q] != 0.0
     ctx.close()
