@@ -51,7 +51,7 @@ static_assert(sizeof(MlpPacked) % 16 == 0, "staged with 16-byte copies");
 
 typedef short mlp_bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 mlp_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float mlp_f32x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short mlp_u16x8 __attribute__((ext_vector_type(8)));
 typedef float mlp_f32x16 __attribute__((ext_vector_type(16)));
 
 __host__ __device__ inline uint16_t f2bf(float x) {  // round to nearest even
@@ -88,7 +88,9 @@ __device__ __forceinline__ mlp_bf16x4 mlp_load4(const uint16_t* p) {  // 4 BF16,
     return r;
 }
 
-// One hidden 128 -> 128 layer on D-layout activations h (in place): bias and SiLU applied.
+// One hidden 128 -> 128 layer on D-layout activations h (in place): bias and SiLU applied.  Operands
+// are rounded by integer operations: with the pair conversion instruction a delayed-acceptance pass
+// took 10 to 20 percent longer (200 passes of one top 2.05 against 1.85 s, waters 11.4 against 9.5).
 // w: the layer's packed A operands (in LDS).
 __device__ __forceinline__ void mlp_hidden(const uint16_t* __restrict__ w, const float* __restrict__ b,
                                            mlp_f32x16 h[4], int l) {
@@ -96,10 +98,10 @@ __device__ __forceinline__ void mlp_hidden(const uint16_t* __restrict__ w, const
     mlp_bf16x8 bin[8];
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) {
-        mlp_f32x8 t;
+        mlp_u16x8 t;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t[j] = h[kb >> 1][8 * (kb & 1) + j];
-        bin[kb] = __builtin_convertvector(t, mlp_bf16x8);  // to nearest even, two a instruction
+        for (int j = 0; j < 8; ++j) t[j] = f2bf(h[kb >> 1][8 * (kb & 1) + j]);
+        bin[kb] = __builtin_bit_cast(mlp_bf16x8, t);
     }
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
