@@ -227,13 +227,16 @@ struct pimc_ctx {
     int Smax = 1, Pmax = 1, Nmax = 1, max_types = 1;
     int bisect_block = 64;
     // linear-family bisection in three size classes (N <= 24, <= 64, larger), each with its own
-    // lanes per segment, block and LDS, launched as parallel branches of the pass
-    int bw_n[3] = {0, 0, 0}, bw_off[3] = {0, 0, 0};  // blocks of a class and their place in d_work
-    int bw_opt[3] = {0, 0, 0};      // lanes per segment asked for (64, 128, 256), 0: by load
-    int bw_gw[3] = {64, 64, 64};    // lanes per segment (32: two segments share a wave)
-    int bw_block[3] = {64, 64, 64}; // lanes per block
-    size_t bw_lds[3] = {0, 0, 0};
-    bool bw_uniform[3] = {false, false, false};  // FP32 on uniform tables
+    // lanes per segment, and in each the replicas on uniform FP32 tables and the others, with
+    // their own kernel, block and LDS; launched as parallel branches of the pass
+    struct BisectLaunch {
+        int n = 0, off = 0;  // blocks and their place in d_work
+        int block = 64;      // lanes per block
+        size_t lds = 0;
+    };
+    BisectLaunch bw[3][2];        // [class][uniform FP32 tables]
+    int bw_opt[3] = {0, 0, 0};    // lanes per segment asked for (64, 128, 256), 0: by load
+    int bw_gw[3] = {64, 64, 64};  // lanes per segment (32: two segments share a wave)
     // proposals of the next bisection launch: the layout of the beads
     double4* d_prop = nullptr;
     PathItem* d_paths = nullptr;  // batches of (atom, segment) pairs, grouped by type, four per block
@@ -242,8 +245,8 @@ struct pimc_ctx {
     hipStream_t side_paths = nullptr;  // the proposals' launch beside the rotor sweep
     hipEvent_t ev_paths[2] = {nullptr, nullptr};
     bool paths_beside = false;
-    hipStream_t side[2] = {nullptr, nullptr};
-    hipEvent_t ev_fork = nullptr, ev_join[2] = {nullptr, nullptr};
+    hipStream_t side[5] = {};  // for the bisection launches after the first
+    hipEvent_t ev_fork = nullptr, ev_join[5] = {};
     int2* d_rows = nullptr;     // (replica, tile) work of the estimator pair sum
     double2* d_rowbuf = nullptr;  // a (potential, kinetic) partial per tile
     int nrows = 0;
@@ -398,7 +401,7 @@ void pimc_destroy(pimc_ctx* c) {
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->back) (void)hipHostFree(c->back);
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < 5; ++k) {
         if (c->side[k]) (void)hipStreamDestroy(c->side[k]);
         if (c->ev_join[k]) (void)hipEventDestroy(c->ev_join[k]);
     }
@@ -941,65 +944,69 @@ static int plan_centroid_parts(pimc_ctx* c, int target_parts) {
     return 0;
 }
 
+// whether a replica's bisection runs on uniform FP32 tables: its own alone, so that its chain is
+// the same whatever the replicas beside it have
+static bool uniform_tables(const pimc_ctx* c, const Rep& p) {
+    return !c->fp64 && (p.pot1d_id < 0 || c->t1[p.pot1d_id].uniform) && (p.pot2d_id < 0 || c->t2[p.pot2d_id].uniform);
+}
+
 // The bisection's blocks: per size class the lanes of a segment's group (want[k]: 64, 128 or 256,
-// or 0 for a choice by load), the block and its LDS, and the (replica, first segment) list.  Called
-// at commit and again by the autotuner.
+// or 0 for a choice by load), and per launch of a class the block and its LDS, and the (replica,
+// first segment) list.  Called at commit and again by the autotuner.
 static int plan_bisect(pimc_ctx* c, const int want[3]) {
     const int rsize = c->fp64 ? 8 : 4;
     struct Item {
         int2 wk;
         long long cost;
     };
-    std::vector<Item> items[3];
+    std::vector<Item> items[3][2];
     for (int k = 0; k < 3; ++k) {
-        long long segs = 0;
-        size_t knots = 0, seg_bytes = 0;
-        bool uniform = !c->fp64;
+        long long segs = 0;  // of both launches: what the device has to hold
+        size_t knots[2] = {0, 0}, seg_bytes[2] = {0, 0};
         for (const Rep& p : c->rep) {
             if (p.fam || bisect_class(p.natoms) != k) continue;
             segs += c->ref_order ? 1 : p.P / p.S;
-            seg_bytes = std::max(seg_bytes, (size_t)bisect_seg_bytes(p.natoms, p.S, rsize));
-            if (p.pot1d_id >= 0) uniform &= c->t1[p.pot1d_id].uniform != 0;
-            if (p.pot2d_id >= 0) uniform &= c->t2[p.pot2d_id].uniform != 0;
+            const int u = uniform_tables(c, p);
+            seg_bytes[u] = std::max(seg_bytes[u], (size_t)bisect_seg_bytes(p.natoms, p.S, rsize));
+            if (p.pot1d_id >= 0) {  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
+                const Tab1D& t = c->t1[p.pot1d_id];
+                const size_t b = t.n * (c->fp64 ? sizeof(double4) : (t.uniform ? sizeof(float2) : sizeof(float4)));
+                knots[u] = std::max(knots[u], (b + 15) & ~(size_t)15);
+            }
         }
-        for (const Rep& p : c->rep)  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
-            if (!p.fam && bisect_class(p.natoms) == k && p.pot1d_id >= 0)
-                knots = std::max(knots, (size_t)c->t1[p.pot1d_id].n *
-                                            (c->fp64 ? sizeof(double4) : (uniform ? sizeof(float2) : sizeof(float4))));
-        if (!segs) {
-            c->bw_n[k] = 0;
-            continue;
-        }
-        knots = (knots + 15) & ~(size_t)15;
+        for (auto& b : c->bw[k]) b.n = 0;
+        if (!segs) continue;
         int gw = want[k];
         if (gw == 0) gw = bisect_group(k, segs);
         // as many waves per block as share the knots in 64 KB, a single wave when there are few
         // segments for the device's CUs
-        int block = std::max(gw, segs * gw >= 64 * 1024 ? 256 : 64);
-        while (block > std::max(gw, 64) && knots + (size_t)(block / gw) * seg_bytes > 64 * 1024) block /= 2;
-        if (gw < 64 && knots + (size_t)(block / gw) * seg_bytes > 64 * 1024) gw = 64;
-        const size_t lds = knots + (size_t)(block / gw) * seg_bytes;
-        if (lds > 160 * 1024) return fail(c, "segment window exceeds LDS (too many atoms for this segment size)");
-        c->bw_uniform[k] = uniform;
+        auto lds = [&](int u, int block) { return knots[u] + (size_t)(block / gw) * seg_bytes[u]; };
+        if (gw < 64 && std::max(lds(0, 64), lds(1, 64)) > 64 * 1024) gw = 64;
         c->bw_gw[k] = gw;
-        c->bw_block[k] = block;
-        c->bw_lds[k] = lds;
-        for (int r = 0; r < c->nrep; ++r) {
-            const Rep& p = c->rep[r];
-            if (p.fam || bisect_class(p.natoms) != k) continue;
-            const int nseg = c->ref_order ? 1 : p.P / p.S;
-            for (int q = 0; q < nseg; q += block / gw)
-                items[k].push_back({make_int2(r, q), (long long)p.natoms * p.natoms * p.S});
+        for (int u = 0; u < 2; ++u) {
+            pimc_ctx::BisectLaunch& b = c->bw[k][u];
+            b.block = std::max(gw, segs * gw >= 64 * 1024 ? 256 : 64);
+            while (b.block > std::max(gw, 64) && lds(u, b.block) > 64 * 1024) b.block /= 2;
+            b.lds = lds(u, b.block);
+            if (b.lds > 160 * 1024) return fail(c, "segment window exceeds LDS (too many atoms for this segment size)");
+            for (int r = 0; r < c->nrep; ++r) {
+                const Rep& p = c->rep[r];
+                if (p.fam || bisect_class(p.natoms) != k || uniform_tables(c, p) != (u == 1)) continue;
+                const int nseg = c->ref_order ? 1 : p.P / p.S;
+                for (int q = 0; q < nseg; q += b.block / gw)
+                    items[k][u].push_back({make_int2(r, q), (long long)p.natoms * p.natoms * p.S});
+            }
+            // largest windows first: the longest atom sequences start while the grid fills
+            std::stable_sort(items[k][u].begin(), items[k][u].end(), [](const Item& x, const Item& y) { return x.cost > y.cost; });
         }
-        // largest windows first: the longest atom sequences start while the grid fills
-        std::stable_sort(items[k].begin(), items[k].end(), [](const Item& a, const Item& b) { return a.cost > b.cost; });
     }
     std::vector<int2> work;
-    for (int k = 2; k >= 0; --k) {
-        c->bw_off[k] = (int)work.size();
-        c->bw_n[k] = (int)items[k].size();
-        for (const Item& i : items[k]) work.push_back(i.wk);
-    }
+    for (int k = 2; k >= 0; --k)
+        for (int u = 0; u < 2; ++u) {
+            c->bw[k][u].off = (int)work.size();
+            c->bw[k][u].n = (int)items[k][u].size();
+            for (const Item& i : items[k][u]) work.push_back(i.wk);
+        }
     if (c->d_work) (void)hipFree(c->d_work);
     c->d_work = dalloc<int2>(work.size());
     if (!c->d_work) return fail(c, "hipMalloc failed");
@@ -1246,9 +1253,10 @@ int pimc_commit(pimc_ctx* c) {
     if (plan_bisect(c, c->bw_opt) || plan_paths(c)) return -1;
     {
         int busy = 0;
-        for (int k = 0; k < 3; ++k) busy += c->bw_n[k] > 0;
+        for (const auto& cl : c->bw)
+            for (const auto& b : cl) busy += b.n > 0;
         if (busy > 1)
-            for (int k = 0; k < 2; ++k) {
+            for (int k = 0; k + 1 < busy; ++k) {
                 HIPCHECK(c, hipStreamCreate(&c->side[k]));  // default priority, like the main stream
                 HIPCHECK(c, hipEventCreateWithFlags(&c->ev_join[k], hipEventDisableTiming));
             }
@@ -1713,12 +1721,13 @@ void launch_paths(pimc_ctx* c, hipStream_t s, int u, int tb, int te) {
                            c->d_beads, c->d_prop, c->d_paths + 4 * (size_t)b0, c->path_ring_len, run);
 }
 
-// one bisection size class on stream s
+// one launch of a bisection size class on stream s: its replicas on uniform FP32 tables, or the others
 template <typename R>
-void launch_bisect_class(pimc_ctx* c, int k, hipStream_t s, const Run& run) {
+void launch_bisect_class(pimc_ctx* c, int k, int uniform, hipStream_t s, const Run& run) {
+    const pimc_ctx::BisectLaunch& b = c->bw[k][uniform];
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(c->bw_n[k]), dim3(c->bw_block[k]), c->bw_lds[k], s, c->d_rep, c->d_mut, c->d_beads,
-                           c->d_rotb, c->tables(), c->d_prop, c->d_work + c->bw_off[k], run);
+        hipLaunchKernelGGL(kernel, dim3(b.n), dim3(b.block), b.lds, s, c->d_rep, c->d_mut, c->d_beads, c->d_rotb, c->tables(),
+                           c->d_prop, c->d_work + b.off, run);
     };
     auto group = [&](auto mi_c, auto ut_c) {
         constexpr bool MI = decltype(mi_c)::value, UT = decltype(ut_c)::value;
@@ -1734,7 +1743,7 @@ void launch_bisect_class(pimc_ctx* c, int k, hipStream_t s, const Run& run) {
         else group(std::false_type{}, ut_c);
     };
     if constexpr (std::is_same<R, float>::value) {
-        if (c->bw_uniform[k]) {
+        if (uniform) {
             tables(std::true_type{});
             return;
         }
@@ -1748,25 +1757,20 @@ void launch_bisect(pimc_ctx* c, int u, int tb, int te) {
     Timed t(c, "bisect");
     // size classes: the heaviest present on the main stream, the others forked onto side
     // streams and joined again (parallel branches of the captured pass)
-    int busy = 0, top = -1;
-    for (int k = 2; k >= 0; --k)
-        if (c->bw_n[k]) {
-            ++busy;
-            if (top < 0) top = k;
-        }
+    int busy = 0, done = 0;
+    for (const auto& cl : c->bw)
+        for (const auto& b : cl) busy += b.n > 0;
     if (busy > 1) (void)hipEventRecord(c->ev_fork, c->stream);
-    int nside = 0;
-    for (int k = 2; k >= 0; --k) {
-        if (!c->bw_n[k]) continue;
-        hipStream_t s = c->stream;
-        if (k != top) {
-            s = c->side[nside];
-            (void)hipStreamWaitEvent(s, c->ev_fork, 0);
+    for (int k = 2; k >= 0; --k)
+        for (int v = 1; v >= 0; --v) {
+            if (!c->bw[k][v].n) continue;
+            hipStream_t s = done ? c->side[done - 1] : c->stream;
+            if (done) (void)hipStreamWaitEvent(s, c->ev_fork, 0);
+            launch_bisect_class<R>(c, k, v, s, run);
+            if (done) (void)hipEventRecord(c->ev_join[done - 1], s);
+            ++done;
         }
-        launch_bisect_class<R>(c, k, s, run);
-        if (k != top) (void)hipEventRecord(c->ev_join[nside++], s);
-    }
-    for (int i = 0; i < nside; ++i) (void)hipStreamWaitEvent(c->stream, c->ev_join[i], 0);
+    for (int i = 0; i + 1 < done; ++i) (void)hipStreamWaitEvent(c->stream, c->ev_join[i], 0);
     if (c->nwork1)
         hipLaunchKernelGGL((c->any_mi ? k_bisect_nl<R, true> : k_bisect_nl<R, false>), dim3(c->nwork1), dim3(c->bisect_block), c->lds_bisect1, c->stream,
                            c->d_rep, c->d_mut, c->d_beads, c->d_rotb, c->d_frames, c->tables(), c->tables3(), c->d_prop, c->d_work1, run);
@@ -2001,7 +2005,7 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
         static const int lanes[3] = {64, 128, 256};
         int chosen_lanes[3] = {c->bw_gw[0], c->bw_gw[1], c->bw_gw[2]};
         for (int k = 0; k < 3 && rc == 0; ++k) {
-            if (!c->bw_n[k]) continue;
+            if (c->bw[k][0].n + c->bw[k][1].n == 0) continue;
             int best = chosen_lanes[k];
             double tbest = -1.0;
             for (int L : lanes) {
@@ -2013,8 +2017,11 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
                 const double t = timed([&](int u) {
                     const Run run{c->seed, u, c->ref_order ? 1 : 0, 0, c->max_types};
                     launch_paths(c, c->stream, u, 0, PIMC_MAX_TYPES);
-                    if (c->fp64) launch_bisect_class<double>(c, k, c->stream, run);
-                    else launch_bisect_class<float>(c, k, c->stream, run);
+                    for (int v = 0; v < 2; ++v) {
+                        if (!c->bw[k][v].n) continue;
+                        if (c->fp64) launch_bisect_class<double>(c, k, v, c->stream, run);
+                        else launch_bisect_class<float>(c, k, v, c->stream, run);
+                    }
                 });
                 if (t >= 0.0 && (tbest < 0.0 || t < tbest)) {
                     tbest = t;

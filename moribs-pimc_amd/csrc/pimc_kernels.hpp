@@ -244,7 +244,8 @@ __device__ __forceinline__ double atom_terms(const Lut1D<R>& l1, const void* kn,
 
 // MI: built for contexts that hold a replica under the minimum image (its pairs then take their
 // nearest image); without it the kernels carry no trace of it.  UT: FP32 on uniform 1D and 2D
-// tables, knots staged as (y, y'') pairs.
+// tables, a launch of its own for the replicas that have them, so that a chain's arithmetic does
+// not depend on the replicas beside it.  Uniform FP32 1D knots are staged as (y, y'') pairs.
 template <typename R, bool MI, bool UT, int GW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bisect(
     const Rep* __restrict__ reps, Mut* __restrict__ mut, double4* __restrict__ beads, const RotBead* __restrict__ rotb,
@@ -262,7 +263,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // the 1D knots, shared by the block's segments
     P4* kn = reinterpret_cast<P4*>(smem);
     int kbytes = l1.n * (int)sizeof(P4);
-    if constexpr (UT) {
+    const bool half = is_fp32<R>() && (UT || l1.uniform);
+    if (half) {
         float2* k2 = reinterpret_cast<float2*>(kn);
         for (int i = threadIdx.x; i < l1.n; i += blockDim.x) k2[i] = make_float2((float)l1.k[i].y, (float)l1.k[i].z);
         kbytes = (l1.n * (int)sizeof(float2) + 15) & ~15;
@@ -424,13 +426,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                     d[U + i][1] = nearest_image(ya - y, bx, 1);
                                     d[U + i][2] = nearest_image(za - z, bx, 2);
                                 }
-                                acc += atom_terms<R, UT, U>(l1, kn, d, U == 1 || jp + G < nat - 1 ? U : 1);
+                                const int ok = U == 1 || jp + G < nat - 1 ? U : 1;
+                                if constexpr (is_fp32<R>() && !UT)
+                                    acc += half ? atom_terms<R, true, U>(l1, kn, d, ok) : atom_terms<R, false, U>(l1, kn, d, ok);
+                                else
+                                    acc += atom_terms<R, UT, U>(l1, kn, d, ok);
                             }
                         };
                         // partners in pairs, so that four look-ups of a lane interleave,
                         // where most lanes have two or more
-                        if (UT && 2 * (nat - 1) > 3 * G) partners(std::integral_constant<int, 2>{});
-                        else partners(std::integral_constant<int, 1>{});
+                        bool two = false;
+                        if constexpr (UT) {
+                            two = 2 * (nat - 1) > 3 * G;
+                            if (two) partners(std::integral_constant<int, 2>{});
+                        }
+                        if (!two) partners(std::integral_constant<int, 1>{});
                     }
                     return acc;
                 };
@@ -1181,8 +1191,14 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
     auto energies = [&](int parity) {  // of the proposals of one parity
         for (int m = emv; m < nmoves; m += MPL > 1 ? nen : nmoves) {
             const int kl = 2 * m + parity + 1;
-            double e = pair_terms<R, UT>(l2, geo + (long long)(kl - 1) * items, eli, lpm, items, na[3 * kl], na[3 * kl + 1],
-                                         na[3 * kl + 2]);
+            // without UT the tables of the launch's chains differ in kind: a chain's own decides
+            auto terms = [&](auto u_c) {
+                return pair_terms<R, decltype(u_c)::value>(l2, geo + (long long)(kl - 1) * items, eli, lpm, items, na[3 * kl],
+                                                           na[3 * kl + 1], na[3 * kl + 2]);
+            };
+            double e;
+            if constexpr (is_fp32<R>() && !UT) e = l2.uniform ? terms(std::true_type{}) : terms(std::false_type{});
+            else e = terms(std::integral_constant<bool, UT>{});
             if constexpr (MPL > 1) {
                 na[3 * kl] = e;
             } else {
