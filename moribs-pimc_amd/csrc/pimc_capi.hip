@@ -962,17 +962,16 @@ static int plan_bisect(pimc_ctx* c, const int want[3]) {
     std::vector<Item> items[3][2];
     for (int k = 0; k < 3; ++k) {
         long long segs = 0;  // of both launches: what the device has to hold
-        size_t knots[2] = {0, 0}, seg_bytes[2] = {0, 0};
+        std::vector<std::pair<size_t, size_t>> need[2];  // LDS of a replica's knots and of one of its segments
         for (const Rep& p : c->rep) {
             if (p.fam || bisect_class(p.natoms) != k) continue;
             segs += c->ref_order ? 1 : p.P / p.S;
-            const int u = uniform_tables(c, p);
-            seg_bytes[u] = std::max(seg_bytes[u], (size_t)bisect_seg_bytes(p.natoms, p.S, rsize));
+            size_t knots = 0;
             if (p.pot1d_id >= 0) {  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
                 const Tab1D& t = c->t1[p.pot1d_id];
-                const size_t b = t.n * (c->fp64 ? sizeof(double4) : (t.uniform ? sizeof(float2) : sizeof(float4)));
-                knots[u] = std::max(knots[u], (b + 15) & ~(size_t)15);
+                knots = t.n * (c->fp64 ? sizeof(double4) : (t.uniform ? sizeof(float2) : sizeof(float4)));
             }
+            need[uniform_tables(c, p)].emplace_back((knots + 15) & ~(size_t)15, bisect_seg_bytes(p.natoms, p.S, rsize));
         }
         for (auto& b : c->bw[k]) b.n = 0;
         if (!segs) continue;
@@ -980,7 +979,11 @@ static int plan_bisect(pimc_ctx* c, const int want[3]) {
         if (gw == 0) gw = bisect_group(k, segs);
         // as many waves per block as share the knots in 64 KB, a single wave when there are few
         // segments for the device's CUs
-        auto lds = [&](int u, int block) { return knots[u] + (size_t)(block / gw) * seg_bytes[u]; };
+        auto lds = [&](int u, int block) {  // a block holds one replica's segments
+            size_t b = 0;
+            for (const auto& n : need[u]) b = std::max(b, n.first + (size_t)(block / gw) * n.second);
+            return b;
+        };
         if (gw < 64 && std::max(lds(0, 64), lds(1, 64)) > 64 * 1024) gw = 64;
         c->bw_gw[k] = gw;
         for (int u = 0; u < 2; ++u) {

@@ -1,0 +1,42 @@
+"""Systems near the LDS limits of a launch: pimc_commit accepts what each replica's own layout fits,
+and the chains are those of the same replicas elsewhere."""
+import numpy as np
+import pytest
+
+import pimc_configs as pc
+import pimc_hip as ph
+import pimc_tables as pt
+
+pytestmark = pytest.mark.gpu
+SEED = 985456376
+
+
+def lattice(n, P, seed):
+    m = int(np.ceil(n ** (1.0 / 3.0)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n] * 3.6
+    return (g.T[:, :, None] + np.random.default_rng(seed).normal(0.0, 0.1, (3, n, P))).reshape(3, -1)
+
+
+def test_a_large_window_beside_a_long_table():
+    """A bisection block holds one replica's segments and knots: 1000 atoms with a short table (87 KB)
+    and 70 atoms with a table of 10000 knots (86 KB) share a size class, though the larger window and
+    the longer table together would not fit."""
+    P, levels = 16, 3
+
+    def run(which):
+        ctx = ph.Context(len(which), seed=SEED)
+        tabs = [ctx.add_pot1d(*pt.lj_table(n=10000)), ctx.add_pot1d(*pt.lj_table(n=500))]
+        for i, (n, t) in enumerate(which):
+            ctx.set_replica(i, 1, [n], [0], [levels], [0.3], [pc.MASS_HE4], P, 0, 2.0, 0.0, pot1d=[tabs[t]], pot2d=[-1])
+        ctx.commit()
+        for i, (n, _) in enumerate(which):
+            ctx.set_state(i, lattice(n, P, i))
+        ctx.run(2)
+        out = ctx.get_state(0)[0], ctx.counters(0)[1]
+        assert ctx.counters(len(which) - 1)[1][0][:2].min() > 0
+        ctx.close()
+        return out
+
+    alone, beside = run([(70, 0)]), run([(70, 0), (1000, 1)])
+    assert np.array_equal(alone[1], beside[1])
+    assert np.abs(alone[0] - beside[0]).max() < 1e-9
