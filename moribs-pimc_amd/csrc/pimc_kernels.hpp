@@ -813,8 +813,9 @@ __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ 
                                                         const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
                                                         unsigned long long* __restrict__ slots, int nslots, Run run) {
     extern __shared__ double smem[];  // the 1D spline knots, then the beads [3][slice][atom]
-    __shared__ double red[2][4];       // two buffers each, for alternate atoms
-    __shared__ double part_sum[2][64];
+    constexpr int NBUF = Staged ? 2 : 1;  // buffers for alternate atoms; unstaged, every atom ends at a barrier
+    __shared__ double red[NBUF][4];
+    __shared__ double part_sum[NBUF][64];
     __shared__ double s_dv;
     __shared__ int s_err;
     const RotPart pt = parts[blockIdx.x];
@@ -856,7 +857,7 @@ __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ 
     };
     if constexpr (Staged) draws(rp.tbegin[ty]);
     for (int ia = 0; ia < rp.tnumb[ty]; ++ia) {
-        const int a = rp.tbegin[ty] + ia;
+        const int a = rp.tbegin[ty] + ia, ib = ia & (NBUF - 1);
         if constexpr (!Staged) draws(a);  // ahead they cost registers, and a full device a resident part
         const double dx = rp.mcstep[ty] * (u53(w0.x, w0.y) - 0.5);
         const double dy = rp.mcstep[ty] * (u53(w0.z, w0.w) - 0.5);
@@ -943,9 +944,9 @@ __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ 
         double partial;
         if constexpr (Staged) {
             acc = wave_sum(acc);
-            if (lane == 0) red[ia & 1][threadIdx.x >> 6] = acc;
+            if (lane == 0) red[ib][threadIdx.x >> 6] = acc;
             lds_barrier();
-            partial = ((red[ia & 1][0] + red[ia & 1][1]) + red[ia & 1][2]) + red[ia & 1][3];
+            partial = ((red[ib][0] + red[ib][1]) + red[ib][2]) + red[ib][3];
         } else {
             partial = block_sum(acc, red[0]);
         }
@@ -974,17 +975,17 @@ __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ 
                     }
                     __builtin_amdgcn_s_sleep(2);
                 }
-                reinterpret_cast<unsigned*>(part_sum[ia & 1])[threadIdx.x] = (unsigned)wv;
+                reinterpret_cast<unsigned*>(part_sum[ib])[threadIdx.x] = (unsigned)wv;
             }
             if constexpr (Staged) lds_barrier();
             else __syncthreads();
             if (s_err) break;  // a part did not arrive: the later atoms' waits would fail as well
             if constexpr (Staged) {
-                deltav = wave_sum(lane < W ? part_sum[ia & 1][lane] : 0.0);
+                deltav = wave_sum(lane < W ? part_sum[ib][lane] : 0.0);
             } else {  // on every wave of a full device it costs more than one lane's turn
                 if (threadIdx.x == 0) {
                     double sum = 0.0;
-                    for (int q = 0; q < W; ++q) sum += part_sum[ia & 1][q];
+                    for (int q = 0; q < W; ++q) sum += part_sum[ib][q];
                     s_dv = sum;
                 }
                 __syncthreads();

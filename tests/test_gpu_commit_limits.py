@@ -40,3 +40,17 @@ def test_a_large_window_beside_a_long_table():
     alone, beside = run([(70, 0)]), run([(70, 0), (1000, 1)])
     assert np.array_equal(alone[1], beside[1])
     assert np.abs(alone[0] - beside[0]).max() < 1e-9
+
+
+def test_the_longest_table_of_a_centroid_part():
+    """10200 FP32 knots are 163200 of a workgroup's 163840 bytes; the rest holds the move's sums."""
+    P, n = 16, 12
+    ctx = ph.Context(1, seed=SEED)
+    t = ctx.add_pot1d(*pt.lj_table(n=10200))
+    ctx.set_replica(0, 1, [n], [0], [2], [0.3], [pc.MASS_HE4], P, 0, 2.0, 0.0, pot1d=[t], pot2d=[-1])
+    ctx.commit()
+    ctx.set_state(0, lattice(n, P, 0))
+    ctx.run(3)
+    total, accepted = ctx.counters(0)
+    assert total[0][0] == 3 * n and 0 < accepted[0][0] <= 3 * n
+    ctx.close()
