@@ -132,6 +132,11 @@ int  pimc_commit(pimc_ctx* ctx);   /* allocates device state after all replicas 
 int  pimc_plan_rotor_parts(int nchains, const int* prot, const int* rot_ratio, const int* natoms, int fp64,
                            int lds_kb, int part_slices_max, int blocks_per_cu, int lds_per_cu, int cus_per_xcd,
                            int* parts_per_chain, int* slices_per_part, long* lds_bytes, char* msg, int len);
+/* Lanes of a bisection segment of a replica of natoms atoms in a context with `segments` segments of
+   its size class (at most 24, at most 64, more atoms), without a device: lanes[0] is what
+   pimc_commit gives it, the others what pimc_autotune also times.  Returns their number, -1 for
+   arguments out of range. */
+int  pimc_plan_bisect_lanes(int natoms, long segments, int lanes[4]);
 /* How pimc_commit splits non-linear rotor chains (MCRotations3D's checkerboard, mc_piqmc.cc:728-
    760) over workgroups, without a device; no counterpart in the reference.  One count W for all
    nchains chains of up to protmax slices with nrot rotors: the largest power of two up to 64 whose
@@ -151,9 +156,9 @@ int  pimc_plan_rotor3d_split(int protmax, int nchains, int nrot, int blocks_per_
                           in all (0, the default: min(1024, half of what the device holds)).  Results do not
                           depend on it: every draw is addressed by (sweep, slice).
      "bisect_lanes_small", "bisect_lanes_medium", "bisect_lanes_large"
-                          lanes (64, 128 or 256) per bisection segment for replicas of at most
-                          24, at most 64 and more atoms; by default chosen from the number of
-                          segments.  Results do not depend on them.
+                          lanes (64, 128 or 256, small also 32) per bisection segment for
+                          replicas of at most 24, at most 64 and more atoms; by default chosen
+                          from the number of segments.  Results do not depend on them.
      "delayed_acceptance" 1: the non-linear rotor move (MCRot3Dstep mc_piqmc.cc:938-1199) runs
                           its test as three Metropolis factors: the density, the surrogate
                           network, then the exact correction (see the surrogate section below);
@@ -189,12 +194,12 @@ int  pimc_get_pass(pimc_ctx* ctx, int replica, unsigned* pass);
 int  pimc_run(pimc_ctx* ctx, int n_passes, int sample_every);
 /* Autotuner of launch shapes (no counterpart in the reference, whose OpenMP loops have no
    tunable shape).  After pimc_commit and the initial state: times each bisection size class
-   at 64, 128 and 256 lanes per segment, the linear-rotor sweep at part LDS budgets of 40,
+   at its lanes per segment and at 64, 128 and 256, the linear-rotor sweep at part LDS budgets of 40,
    52, 64 and 78 KB and the centroid move split into about 256, 512 or 1024 parts, each
    candidate over `passes` passes' launches from the same saved state, and keeps the fastest.  The chains' coordinates, orientations, counters and pass numbers are
    restored, so results are the same as without tuning.  chosen (may be NULL, else 5 entries)
-   receives the lanes of the small, medium and large classes, the rotor budget in KB and the
-   centroid part target. */
+   receives the lanes of the small, medium and large classes (64 for a class without replicas; 32
+   where two segments share a wave), the rotor budget in KB and the centroid part target. */
 int  pimc_autotune(pimc_ctx* ctx, int passes, long* chosen);
 /* samples of one replica, 8 doubles each: K, V, E_rot, E_rot^2 term (ErotSQ), Cv, Cv_trans,
    Cv_rot, Erot_termSQ (mc_main.cc:551-616).  Returns the number copied.  A replica keeps up to

@@ -88,20 +88,6 @@ std::vector<Part> xcd_order(const std::vector<Part>& parts, Work work) {
     return grid;
 }
 
-// bisection size classes of the linear family: lanes per workgroup by atom count
-inline int bisect_class(int natoms) { return natoms <= 24 ? 0 : (natoms <= 64 ? 1 : 2); }
-
-// Lanes of a segment's group in size class k with segs segments in all.  With few segments a chain's
-// atoms in turn are the time, and four waves shorten a move; with many the device is full and one
-// wave a segment wastes least.  Bisection per pass at 256 and 64 lanes: 40 atoms 1.02 and 1.16 ms on
-// 512 segments, 1.28 and 1.24 on 1024; 100 atoms 3.38 and 3.96 ms on 1024, 6.44 and 4.70 on 2048.
-// Up to 24 atoms a wave holds the partners as it is (8 atoms: 0.30 and 0.32 ms on 512), and two
-// segments share one on a full device (0.445 against 0.470 ms on 4096).
-inline int bisect_group(int k, long long segs) {
-    if (k == 0) return segs >= 4096 ? 32 : 64;
-    return segs <= (k == 1 ? 768 : 1280) ? 256 : 64;
-}
-
 template <typename T>
 T* dalloc(size_t n) {
     T* p = nullptr;
@@ -235,7 +221,7 @@ struct pimc_ctx {
         size_t lds = 0;
     };
     BisectLaunch bw[3][2];        // [class][uniform FP32 tables]
-    int bw_opt[3] = {0, 0, 0};    // lanes per segment asked for (64, 128, 256), 0: by load
+    int bw_opt[3] = {0, 0, 0};    // lanes per segment asked for (64, 128, 256; small also 32), 0: by load
     int bw_gw[3] = {64, 64, 64};  // lanes per segment (32: two segments share a wave)
     // proposals of the next bisection launch: the layout of the beads
     double4* d_prop = nullptr;
@@ -699,6 +685,13 @@ int pimc_check_replica(const pimc_replica_desc* d, char* msg, int len) {
     return m.empty() ? 0 : -1;
 }
 
+int pimc_plan_bisect_lanes(int natoms, long segments, int lanes[4]) {
+    if (natoms < 1 || segments < 1 || !lanes) return -1;
+    int n = 0;
+    for (int L : bisect_candidates(bisect_group(bisect_class(natoms), segments))) lanes[n++] = L;
+    return n;
+}
+
 int pimc_plan_rotor3d_split(int protmax, int nchains, int nrot, int blocks_per_cu, int lds_per_cu, int ncu,
                             int cus_per_xcd) {
     if (protmax < 2 || nchains < 1 || nrot < 1 || nrot > 2 || ncu < 1 || cus_per_xcd < 1) return -1;
@@ -751,8 +744,8 @@ int pimc_set_option(pimc_ctx* c, const char* name, long value) {
     static const char* lanes_opt[3] = {"bisect_lanes_small", "bisect_lanes_medium", "bisect_lanes_large"};
     for (int k = 0; k < 3; ++k)
         if (std::strcmp(name, lanes_opt[k]) == 0) {
-            if (value != 64 && value != 128 && value != 256)
-                return fail(c, std::string(name) + " is 64, 128 or 256");
+            if (value != 64 && value != 128 && value != 256 && !(k == 0 && value == 32))
+                return fail(c, std::string(name) + (k == 0 ? " is 32, 64, 128 or 256" : " is 64, 128 or 256"));
             c->bw_opt[k] = (int)value;
             return 0;
         }
@@ -2005,13 +1998,12 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess || copy_all(true)) {
         rc = fail(c, "autotune: event or copy failed");
     } else {
-        static const int lanes[3] = {64, 128, 256};
         int chosen_lanes[3] = {c->bw_gw[0], c->bw_gw[1], c->bw_gw[2]};
         for (int k = 0; k < 3 && rc == 0; ++k) {
             if (c->bw[k][0].n + c->bw[k][1].n == 0) continue;
             int best = chosen_lanes[k];
             double tbest = -1.0;
-            for (int L : lanes) {
+            for (int L : bisect_candidates(best)) {
                 chosen_lanes[k] = L;
                 if (plan_bisect(c, chosen_lanes)) {
                     rc = -1;
@@ -2086,7 +2078,7 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
             *gx = nullptr;
         }
     if (rc == 0 && chosen) {
-        for (int k = 0; k < 3; ++k) chosen[k] = std::max(64, c->bw_gw[k]);
+        for (int k = 0; k < 3; ++k) chosen[k] = c->bw_gw[k];
         chosen[3] = c->rotor_lds_kb;
         chosen[4] = c->centroid_target;
     }

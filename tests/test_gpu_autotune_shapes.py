@@ -1,0 +1,44 @@
+"""Launch shapes of a tuned context: the plan's own are candidates, what is reported is what runs, and
+it can be asked for again."""
+import numpy as np
+import pytest
+
+import pimc_configs as pc
+import pimc_hip as ph
+
+pytestmark = pytest.mark.gpu
+SEED = 985456376
+
+
+def chains(n_he, P, copies, **options):
+    wl = pc.workload("tiny")
+    wl["tables"]["rot"] = [pc.rot_table(0.8, P)]
+    wl["replicas"] = [dict(pc.replica(n_he, P, 0.8, SEED), rotdens=0, pot1d=[0, -1], pot2d=[-1, 0])] * copies
+    ctx = ph.Context(copies, seed=SEED)
+    for k, v in options.items():
+        ctx.set_option(k, v)
+    return pc.load_into_context(ctx, wl)
+
+
+def test_lanes_where_two_segments_share_a_wave():
+    """4096 segments of 9 atoms: the plan's 32 lanes are timed like the others, and the tuned shapes
+    given as options make the same chains."""
+    tuned, plain = chains(8, 64, 512), chains(8, 64, 512)
+    shapes = tuned.autotune(passes=2)
+    assert shapes["bisect_lanes_small"] in ph.plan_bisect_lanes(9, 4096) and 32 in ph.plan_bisect_lanes(9, 4096)
+    asked = chains(8, 64, 512, **{k: v for k, v in shapes.items()})
+    small = chains(8, 64, 512, bisect_lanes_small=32)
+    for c in (tuned, plain, asked, small):
+        c.run(2)
+    for r in (0, 511):
+        for c in (tuned, asked, small):
+            assert np.array_equal(c.counters(r)[1], plain.counters(r)[1])
+            assert all(np.array_equal(a, b) for a, b in zip(c.get_state(r), plain.get_state(r)))
+
+
+def test_other_classes_keep_whole_waves():
+    ctx = ph.Context(1, seed=SEED)
+    for k in ("bisect_lanes_medium", "bisect_lanes_large"):
+        with pytest.raises(ph.PimcError, match="64, 128 or 256"):
+            ctx.set_option(k, 32)
+    ctx.close()

@@ -124,3 +124,14 @@ def test_rotor3d_split_fits_one_xcd():
     # short chains: parts keep at least 16 slices
     assert ph.plan_rotor3d_split(64, 1, 1, blocks_per_cu=2) == 4
     assert ph.plan_rotor3d_split(16, 1, 1, blocks_per_cu=2) == 1
+
+
+@pytest.mark.parametrize("natoms,segments,lanes", [
+    (9, 16, 64), (24, 4095, 64), (9, 4096, 32), (24, 1 << 20, 32),
+    (25, 768, 256), (64, 769, 64), (65, 1280, 256), (101, 1281, 64)])
+def test_the_autotuner_times_the_plan_first(natoms, segments, lanes):
+    """The lanes that pimc_commit gives a bisection segment are among those that pimc_autotune times,
+    so that tuning cannot replace them by slower ones that it had to choose from."""
+    c = ph.plan_bisect_lanes(natoms, segments)
+    assert c[0] == lanes and sorted(set(c)) == sorted(c) and set(c) == {lanes, 64, 128, 256}
+    assert ph.plan_bisect_lanes(0, segments) == [] and ph.plan_bisect_lanes(natoms, 0) == []
