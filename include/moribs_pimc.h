@@ -201,6 +201,11 @@ int  pimc_run(pimc_ctx* ctx, int n_passes, int sample_every);
    receives the lanes of the small, medium and large classes (64 for a class without replicas; 32
    where two segments share a wave), the rotor budget in KB and the centroid part target. */
 int  pimc_autotune(pimc_ctx* ctx, int passes, long* chosen);
+/* A launch shape in force after pimc_commit or pimc_autotune (no counterpart in the reference):
+   "compute_units" of the device, "rotor_blocks" workgroups of the rotor sweep, "rotor_lds_bytes"
+   of dynamic LDS that each of the linear sweep's has, "proposals_beside" whether the next bisection's
+   proposals are formed beside that sweep (1) or between the launches (0). */
+int  pimc_launch_shape(pimc_ctx* ctx, const char* name, long* value);
 /* samples of one replica, 8 doubles each: K, V, E_rot, E_rot^2 term (ErotSQ), Cv, Cv_trans,
    Cv_rot, Erot_termSQ (mc_main.cc:551-616).  Returns the number copied.  A replica keeps up to
    4096 samples between pimc_clear_samples calls; if it took more, the later ones were not

@@ -230,7 +230,7 @@ struct pimc_ctx {
     int path_ring_len = 0;
     hipStream_t side_paths = nullptr;  // the proposals' launch beside the rotor sweep
     hipEvent_t ev_paths[2] = {nullptr, nullptr};
-    bool paths_beside = false;
+    int ncu = 0;  // compute units of the device
     hipStream_t side[5] = {};  // for the bisection launches after the first
     hipEvent_t ev_fork = nullptr, ev_join[5] = {};
     int2* d_rows = nullptr;     // (replica, tile) work of the estimator pair sum
@@ -1345,14 +1345,9 @@ int pimc_commit(pimc_ctx* c) {
         upv(c->d_rot3, rot3.data(), rot3.size() * sizeof(int)) || upv(c->d_rows1, rows1.data(), rows1.size() * sizeof(int2)))
         return fail(c, "upload failed");
     {
-        // the proposals run beside a rotor sweep whose blocks leave half of the CUs free (8.0 against
-        // 8.6 ms per pass on 23 mixed replicas); beside one that fills the device they keep parts
-        // from being resident together, and their neighbours wait (226 against 145 ms on 128 pairs
-        // of water rotors)
         hipDeviceProp_t prop;
         HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
-        const int blocks = c->nparts + (int)rot3.size() + c->nparts3;
-        c->paths_beside = blocks > 0 && blocks <= prop.multiProcessorCount / 2;
+        c->ncu = prop.multiProcessorCount;
     }
     c->nrotreps = (int)rotreps.size();
     c->nrows = (int)rows.size();
@@ -1852,13 +1847,22 @@ void launch_centroid_all(pimc_ctx* c) {
     }
 }
 
+// Whether the proposals run beside the rotor sweep: where its blocks leave half of the CUs free (8.0
+// against 8.6 ms per pass on 23 mixed replicas).  Beside one that fills the device they keep parts
+// from being resident together, and their neighbours wait (226 against 145 ms on 128 pairs of water
+// rotors).  Asked at every launch: the autotuner changes the parts.
+bool proposals_beside(const pimc_ctx* c) {
+    const int blocks = c->nparts + c->nrot3 + c->nparts3;
+    return blocks > 0 && blocks <= c->ncu / 2;
+}
+
 // Rotor sweep of start slice u and, beside it where it leaves CUs free, the proposals of the bisection of start slice u + 1
 // (of n start slices): they read the beads, which the sweep leaves alone.  Returns whether
 // join_paths has to follow before that bisection.
 template <typename R>
 bool launch_rotor_and_paths(pimc_ctx* c, int u, int n) {
     const bool next = u + 1 < n;
-    const bool beside = next && !c->profile && c->paths_beside;
+    const bool beside = next && !c->profile && proposals_beside(c);
     if (beside) {
         (void)hipEventRecord(c->ev_paths[0], c->stream);
         (void)hipStreamWaitEvent(c->side_paths, c->ev_paths[0], 0);
@@ -2083,6 +2087,23 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
         chosen[4] = c->centroid_target;
     }
     return rc;
+}
+
+int pimc_launch_shape(pimc_ctx* c, const char* name, long* value) {
+    if (!c || !name || !value) return fail(c, "pimc_launch_shape: null argument");
+    if (!c->committed) return fail(c, "pimc_commit first");
+    const std::pair<const char*, long> shapes[] = {
+        {"compute_units", c->ncu},
+        {"rotor_blocks", (long)c->nparts + c->nrot3 + c->nparts3},
+        {"rotor_lds_bytes", (long)c->lds_rotor},
+        {"proposals_beside", proposals_beside(c) ? 1 : 0},
+    };
+    for (const auto& s : shapes)
+        if (std::strcmp(name, s.first) == 0) {
+            *value = s.second;
+            return 0;
+        }
+    return fail(c, std::string("unknown launch shape ") + name);
 }
 
 int pimc_synchronize(pimc_ctx* c) {

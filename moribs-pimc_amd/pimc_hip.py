@@ -78,6 +78,7 @@ SIGNATURES = {
     "pimc_get_pass": (_i, [ctypes.c_void_p, _i, ctypes.POINTER(ctypes.c_uint)]),
     "pimc_run": (_i, [ctypes.c_void_p, _i, _i]),
     "pimc_autotune": (_i, [ctypes.c_void_p, _i, ctypes.POINTER(ctypes.c_long)]),
+    "pimc_launch_shape": (_i, [ctypes.c_void_p, ctypes.c_char_p, ctypes.POINTER(ctypes.c_long)]),
     "pimc_get_samples": (_i, [ctypes.c_void_p, _i, _dp, _i]),
     "pimc_clear_samples": (_i, [ctypes.c_void_p]),
     "pimc_get_counters": (_i, [ctypes.c_void_p, _i, _dp, _dp]),
@@ -320,6 +321,12 @@ class Context:
         self._check(self.lib.pimc_autotune(self.h, int(passes), out))
         return dict(bisect_lanes_small=out[0], bisect_lanes_medium=out[1], bisect_lanes_large=out[2],
                     rotor_lds_kb=out[3], centroid_parts=out[4])
+
+    def launch_shape(self, name):
+        """A launch shape in force (pimc_launch_shape)."""
+        v = ctypes.c_long()
+        self._check(self.lib.pimc_launch_shape(self.h, name.encode(), ctypes.byref(v)))
+        return v.value
 
     def samples(self, r, max_samples=1 << 16):
         out = np.empty(8 * max_samples)

@@ -42,3 +42,14 @@ def test_other_classes_keep_whole_waves():
         with pytest.raises(ph.PimcError, match="64, 128 or 256"):
             ctx.set_option(k, 32)
     ctx.close()
+
+
+def test_proposals_follow_the_tuned_parts():
+    """Chains committed with few large rotor parts leave CUs free for the next proposals; the budgets
+    that the tuner times make more parts than that, and the proposals then run between the launches."""
+    ctx = chains(100, 512, 16, rotor_lds_kb=150)
+    cu = ctx.launch_shape("compute_units")
+    assert ctx.launch_shape("rotor_blocks") <= cu // 2 and ctx.launch_shape("proposals_beside") == 1
+    assert ctx.autotune(passes=1)["rotor_lds_kb"] < 150
+    assert ctx.launch_shape("rotor_blocks") > cu // 2 and ctx.launch_shape("proposals_beside") == 0
+    ctx.close()
