@@ -249,7 +249,9 @@ struct pimc_ctx {
     int rotor_lds_kb = 52;          // budget the current parts were planned with
     int rotor_resident = 0;         // parts the device holds at once
     bool rotor_uniform = false;     // the sweep's tables are uniform FP32 ones
-    bool rotor_long = false;        // a part has more than ROTOR_SLICES_MAX slices
+    // parts that leave room for partial sums and knots, parts that do not, parts of more than ROTOR_SLICES_MAX slices
+    enum RotorForm { ROTOR_USUAL, ROTOR_LEAN, ROTOR_LONG } rotor_form = ROTOR_USUAL;
+    int rotor_knots_at = -1;        // of the lean forms: where the launch's LDS has the knots, if it has
     std::vector<int> rot_chains;    // replicas with a linear rotor, heaviest first
     RotPart* d_parts3 = nullptr;     // non-linear chains split by slice range
     unsigned* d_flags3 = nullptr;
@@ -322,9 +324,15 @@ static int fail(pimc_ctx* c, const std::string& m) {
 
 template <typename F>
 static void rotor_kernel(const pimc_ctx* c, F&& f) {  // the linear sweep's instance for this context
-    if (c->fp64) c->rotor_long ? f(k_rotor<double, false, ROTOR_MPL_LONG>) : f(k_rotor<double, false, 1>);
-    else if (c->rotor_long) f(k_rotor<float, false, ROTOR_MPL_LONG>);
-    else c->rotor_uniform ? f(k_rotor<float, true, 1>) : f(k_rotor<float, false, 1>);
+    const auto form = c->rotor_form;
+    if (c->fp64) {
+        if (form == pimc_ctx::ROTOR_LONG) f(k_rotor<double, false, ROTOR_MPL_LONG, true>);
+        else form == pimc_ctx::ROTOR_LEAN ? f(k_rotor<double, false, 1, true>) : f(k_rotor<double, false, 1, false>);
+    } else {
+        if (form == pimc_ctx::ROTOR_LONG) f(k_rotor<float, false, ROTOR_MPL_LONG, true>);
+        else if (form == pimc_ctx::ROTOR_LEAN) f(k_rotor<float, false, 1, true>);
+        else c->rotor_uniform ? f(k_rotor<float, true, 1, false>) : f(k_rotor<float, false, 1, false>);
+    }
 }
 
 namespace {
@@ -807,14 +815,29 @@ static int plan_rotor_parts(pimc_ctx* c, int lds_kb) {
             if (p.k1 - p.k0 > ROTOR_SLICES_MAX) return true;
         return false;
     };
-    c->rotor_long = false;
-    int rc = plan(c->opt_rotor_part_slices > 0 ? c->opt_rotor_part_slices : ROTOR_SLICES_MAX);
+    // each form takes what the one before it cannot: parts that leave no room for the kernel's own LDS,
+    // and parts that have to be long
+    const int most = c->opt_rotor_part_slices > 0 ? c->opt_rotor_part_slices : ROTOR_SLICES_MAX;
+    c->rotor_form = pimc_ctx::ROTOR_USUAL;
+    int rc = plan(most);
+    if (rc) {
+        c->rotor_form = pimc_ctx::ROTOR_LEAN;
+        rc = plan(most);
+    }
     if (rc || too_long()) {
-        c->rotor_long = true;
+        c->rotor_form = pimc_ctx::ROTOR_LONG;
         rc = plan(c->opt_rotor_part_slices);
     }
     if (rc)
         return fail(c, err);
+    c->rotor_knots_at = -1;
+    if (c->rotor_form != pimc_ctx::ROTOR_USUAL) {  // the knots behind the parts, where they cost no resident part
+        const size_t at = (lds_r + 31) & ~(size_t)31, with = at + ROTOR_KNOTS * sizeof(double4);
+        if (with <= ROTOR_LDS_MAX && occupancy(with) == occupancy(lds_r)) {
+            c->rotor_knots_at = (int)(at / sizeof(double));
+            lds_r = with;
+        }
+    }
     const int nflags = (int)parts.size();
     parts = xcd_order(parts, [&](int r) {
         const Rep& p = c->rep[r];
@@ -1784,7 +1807,7 @@ void launch_centroid(pimc_ctx* c, int type) {
 void launch_rotor_parts(pimc_ctx* c, const Run& run) {
     rotor_kernel(c, [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(c->nparts), dim3(256), c->lds_rotor, c->stream, c->d_rep, c->d_mut, c->d_beads,
-                           c->d_rotb, c->tables(), c->d_parts, c->d_flags, c->d_xrec, run);
+                           c->d_rotb, c->tables(), c->d_parts, c->d_flags, c->d_xrec, run, c->rotor_knots_at);
     });
 }
 

@@ -1107,14 +1107,21 @@ constexpr int ROTOR_SLICES_MAX = 256;     // slices of a part where a chain lane
 // slices per chain lane: 2 * 128 * 12 slices are more than LDS holds.
 constexpr int ROTOR_MPL_LONG = 12;
 
-template <typename R, bool UT, int MPL>
+// Lean: LDS for the part alone, for long parts and for those that leave no room for the partial sums
+// and the staged knots (two slices of 1240 partners and more, FP64, two time slices each).  A move's
+// energy lanes are then a power of two within a wave, and its sum takes the place of its proposal's
+// axis; the knots are staged behind the part (at double knots_at of smem) where the launch has
+// room, else read from L2 (knots_at < 0).
+template <typename R, bool UT, int MPL, bool Lean>
 __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut* __restrict__ mut,
                                                const double4* __restrict__ beads, RotBead* __restrict__ rotb,
                                                Tables T, const RotPart* __restrict__ parts,
-                                               unsigned* __restrict__ flags, unsigned long long* __restrict__ xrec, Run run) {
+                                               unsigned* __restrict__ flags, unsigned long long* __restrict__ xrec, Run run,
+                                               int knots_at) {
+    static_assert(Lean || MPL == 1, "long parts are lean");
     extern __shared__ double smem[];
-    __shared__ double pe[2][ROTOR_PARTIALS];
-    __shared__ double4 hk[ROTOR_KNOTS];
+    __shared__ double pe[Lean ? 1 : 2][Lean ? 1 : ROTOR_PARTIALS];
+    __shared__ double4 knots[Lean ? 1 : ROTOR_KNOTS];
     __shared__ unsigned s_acc[2];
     __shared__ int s_err;
     const RotPart pt = parts[blockIdx.x];
@@ -1176,21 +1183,27 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
     const uint32_t pass = mut[r].pass;
     const Lut2D<R> l2 = lut2d<R>(T, rp.pot2d_id);
     const TabRot trt = T.tr[rp.rotdens];
-    for (int i = threadIdx.x; i < trt.n - trt.hot; i += blockDim.x) hk[i] = T.rk[trt.off + trt.hot + i];
+    const double4* hk = T.rk + trt.off + trt.hot;
+    if (!Lean || knots_at >= 0) {
+        double4* to = Lean ? reinterpret_cast<double4*>(smem + knots_at) : knots;
+        for (int i = threadIdx.x; i < trt.n - trt.hot; i += blockDim.x) to[i] = hk[i];
+        hk = to;
+    }
     const unsigned base = __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int nmoves = ns >> 1;                    // of either parity: k0 and ns are even
     const int nchain = nmoves <= 64 ? 64 : 128;    // lanes of the chain waves
     const bool chain = __builtin_amdgcn_readfirstlane((int)threadIdx.x) < nchain;  // a wave's role, scalar
-    // energy lanes: lpm per move, of which each quad or row of 16 leaves one partial sum in pe.  A
-    // long part's lanes take moves in turn and leave the sum in place of the proposal's axis
+    // energy lanes: lpm per move, of which each quad or row of 16 leaves one partial sum in pe
     const int nen = (int)blockDim.x - nchain;
-    int lpm = MPL > 1 ? 1 : nen / nmoves;
-    const int gr = lpm >= 16 ? 16 : (lpm >= 4 ? 4 : 1);
+    int lpm = Lean ? 1 : nen / nmoves;
+    if constexpr (Lean)
+        while (lpm < 64 && 2 * lpm * nmoves <= nen) lpm *= 2;
+    const int gr = Lean ? lpm : (lpm >= 16 ? 16 : (lpm >= 4 ? 4 : 1));
     lpm -= lpm % gr;
     const int npart = lpm / gr;
     const int le = (int)threadIdx.x - nchain, emv = le / lpm, eli = le - emv * lpm;
     auto energies = [&](int parity) {  // of the proposals of one parity
-        for (int m = emv; m < nmoves; m += MPL > 1 ? nen : nmoves) {
+        for (int m = emv; m < nmoves; m += Lean ? nen / lpm : nmoves) {
             const int kl = 2 * m + parity + 1;
             // without UT the tables of the launch's chains differ in kind: a chain's own decides
             auto terms = [&](auto u_c) {
@@ -1200,16 +1213,16 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
             double e;
             if constexpr (is_fp32<R>() && !UT) e = l2.uniform ? terms(std::true_type{}) : terms(std::false_type{});
             else e = terms(std::integral_constant<bool, UT>{});
-            if constexpr (MPL > 1) {
-                na[3 * kl] = e;
+            e = group_sum(e, gr);
+            if constexpr (Lean) {
+                if (eli == 0) na[3 * kl] = e;
             } else {
-                e = group_sum(e, gr);
                 if ((eli & (gr - 1)) == 0) pe[parity][m * npart + eli / gr] = e;
             }
         }
     };
     auto energy_of = [&](int parity, int mv) {  // sum of the partials of a move
-        if constexpr (MPL > 1) return na[3 * (2 * mv + parity + 1)];
+        if constexpr (Lean) return na[3 * (2 * mv + parity + 1)];
         const double* p = &pe[parity][mv * npart];
         double e = p[0];
         if (npart <= 4) {  // read together: one after another they were 0.15 us of a half with three
