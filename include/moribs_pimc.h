@@ -151,7 +151,8 @@ int  pimc_plan_rotor3d_split(int protmax, int nchains, int nrot, int blocks_per_
      "rotor_part_slices"  most rotor slices per workgroup of the rotor sweep (even, >= 2);
                           0 (default) sizes parts from the LDS budget.
      "rotor_lds_kb"       LDS budget of one part of the linear-rotor sweep, 8 to 150 KB (by
-                          default 52, or 78 when those parts are more than the device holds).
+                          default 52, or 78 when those parts are more than the device holds), of
+                          which the kernel keeps 9 for itself; a part's slices get 8 at least.
      "centroid_parts"     about how many workgroups the centroid move's replicas are split into
                           in all (0, the default: min(1024, half of what the device holds)).  Results do not
                           depend on it: every draw is addressed by (sweep, slice).

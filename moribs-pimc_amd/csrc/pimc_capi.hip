@@ -805,9 +805,10 @@ static int plan_rotor_parts(pimc_ctx* c, int lds_kb) {
     size_t lds_r = 0;
     std::string err;
     // parts of at most ROTOR_SLICES_MAX slices, or, where the option asks for more or a chain of those
-    // cannot be resident, as large as they have to be; the budget holds the kernel's own 9 KB too
+    // cannot be resident, as large as they have to be; the budget holds the kernel's own 9 KB too, and
+    // leaves the slices what the smallest budget is
     auto plan = [&](int most) {
-        return plan_linear_rotor(chains, geo_bytes, std::max(1, lds_kb - 9), most, prop.multiProcessorCount / NXCD, occupancy,
+        return plan_linear_rotor(chains, geo_bytes, std::max(8, lds_kb - 9), most, prop.multiProcessorCount / NXCD, occupancy,
                                  parts, lds_r, err);
     };
     auto too_long = [&]() {

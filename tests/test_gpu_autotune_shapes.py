@@ -53,3 +53,12 @@ def test_proposals_follow_the_tuned_parts():
     assert ctx.autotune(passes=1)["rotor_lds_kb"] < 150
     assert ctx.launch_shape("rotor_blocks") > cu // 2 and ctx.launch_shape("proposals_beside") == 0
     ctx.close()
+
+
+@pytest.mark.parametrize("kb,state_kb", [(8, 8), (16, 8), (17, 8), (52, 43), (150, 141)])
+def test_rotor_budget_of_a_part(kb, state_kb):
+    """The budget holds the kernel's own 9 KB, and a part's slices get 8 KB at least."""
+    ctx = chains(40, 128, 1, rotor_lds_kb=kb)
+    want = ph.plan_rotor_parts([128], [1], [41], lds_kb=state_kb)[2]
+    assert ctx.launch_shape("rotor_lds_bytes") == want
+    ctx.close()
