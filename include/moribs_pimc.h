@@ -233,7 +233,9 @@ int  pimc_get_histograms3d(pimc_ctx* ctx, int replica, double* gr3d, double* rel
    (GetRCF mc_estim.cc:1098-1139; the reference adds 1.0 in rows 1..9).  Returns Prot, or 0
    when the replica does not rotate. */
 int  pimc_get_rcf(pimc_ctx* ctx, int replica, double* out, int max_values);
-/* pair evaluations performed and bead moves proposed since creation (all replicas) */
+/* pair evaluations that the moves' tests and the estimators needed, and bead moves proposed, since
+   creation (all replicas).  Terms of a bisection's levels behind its rejection, and of outcomes
+   formed ahead that did not come about, are not counted. */
 int  pimc_get_work(pimc_ctx* ctx, double* pair_evals, double* bead_moves);
 
 /* ---- energies on the current state (batched) ---- */
@@ -260,7 +262,7 @@ int  pimc_estimate(pimc_ctx* ctx, double* out);
    "bisect", "centroid", "rotor", "estimate" */
 int  pimc_kernel_time(pimc_ctx* ctx, const char* family, double* ms, long* launches);
 int  pimc_synchronize(pimc_ctx* ctx);
-/* pair evaluations performed by one kernel family since creation */
+/* pair evaluations of one kernel family since creation, counted as in pimc_get_work */
 int  pimc_family_evals(pimc_ctx* ctx, const char* family, double* evals);
 
 /* ---- surrogate network and delayed acceptance ----

@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const bool has_rotor = rp.lin_atom >= 0;  // then the last atom
     const int nat = has_rotor ? N - 1 : N;    // atoms
     const double tau = rp.tau;
-    unsigned long long evals = 0;
+    unsigned mids = 0;  // midpoints whose terms a move's tests needed: of the levels up to its rejection
     int pb = 0;  // buffer of the next partial sums
     const int tend = run.type_end < rp.ntypes ? run.type_end : rp.ntypes;
 
@@ -467,7 +467,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     pb ^= 1;
                     if ((gl & (G3 - 1)) == 0) pt[m3] = acc;
                     group_sync<GW>();
-                    evals += 14ull * (unsigned)(N - 1);
                     double p[7], t[3];
 #pragma unroll
                     for (int i = 0; i < 7; ++i) p[i] = pt[i];
@@ -476,7 +475,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     // sum over all points up to a level; level acceptance of mc_piqmc.cc:263-273
                     const double c0 = p[0], c1 = (c0 + p[1]) + p[2], c2 = (((c1 + p[3]) + p[4]) + p[5]) + p[6];
                     const double dv0 = c0 * tauh, dv1 = (c1 - 2.0 * c0) * (0.5 * tauh), dv2 = (c2 - 2.0 * c1) * (0.25 * tauh);
-                    alive = (dv0 < 0.0 || dv0 < t[0]) && (dv1 < 0.0 || dv1 < t[1]) && (dv2 < 0.0 || dv2 < t[2]);
+                    const bool a0 = dv0 < 0.0 || dv0 < t[0], a1 = a0 && (dv1 < 0.0 || dv1 < t[1]);
+                    alive = a1 && (dv2 < 0.0 || dv2 < t[2]);
+                    mids += a1 ? 7 : (a0 ? 3 : 1);
                     cum = c2;
                 }
                 for (int l0 = three ? 3 : 0; l0 < L;) {
@@ -516,7 +517,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         pb ^= 1;
                         if ((gl & (Gr - 1)) == 0) pt[gl / Gr] = acc;
                         group_sync<GW>();
-                        evals += 2ull * (unsigned)(nmc * (N - 1));
                         // sum over all points up to a level; level acceptance of mc_piqmc.cc:263-273
                         const int per_m = G / Gr > 0 ? G / Gr : 1, np_all = GW / Gr;
                         for (int level = l0, i = 0; level < l1e; ++level) {
@@ -524,6 +524,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                             const int i1 = l0 > 0 ? np_all : i + (per_m << level);
                             for (; i < i1; ++i) cum += pt[i];
                             const double deltav = (cum - 2.0 * prev) * (tau * (double)(1 << (L - level - 1)));
+                            mids += alive ? 1u << level : 0u;
                             alive = alive && (deltav < 0.0 || deltav < tst[level]);
                         }
                     }
@@ -559,7 +560,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             atomicAdd(&mut[wk.x].accep[ty][1], (unsigned long long)acc_n);
         }
     }
-    if (gl == 0) atomicAdd(&mut[wk.x].pair_evals[0], evals);
+    if (gl == 0) atomicAdd(&mut[wk.x].pair_evals[0], 2ull * mids * (unsigned)(N - 1));
 }
 
 // Non-linear rotors: one workgroup per segment, its window of all atoms' beads and of the rotors'
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
     }
     __syncthreads();
 
-    unsigned long long evals = 0;
+    unsigned mids = 0;  // midpoints whose terms a move's tests needed: of the levels up to its rejection
     int pb = 0;  // buffer of the next level sums
     unsigned long long tot[MAXT] = {0, 0, 0, 0}, acc_n[MAXT] = {0, 0, 0, 0};
     const int tend = run.type_end < rp.ntypes ? run.type_end : rp.ntypes;
@@ -715,7 +716,6 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
 #pragma unroll
                     for (int k = 0; k < 3; ++k) red[pb][tid >> 6][k] = acc[k];
                 lds_barrier();
-                evals += 2ull * (unsigned long long)(nmid * (N - 1));
                 double sum[3];
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {  // at most four waves
@@ -731,6 +731,7 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
                     const double prev = cum;
                     cum += sum[k];
                     const double deltav = (cum - 2.0 * prev) * (rp.tau * (double)(1 << (L - (level + k) - 1)));
+                    mids += accepted ? 1u << (level + k) : 0u;
                     accepted = accepted && (deltav < 0.0 || deltav < tst[level + k]);
                 }
                 level = end;
@@ -767,7 +768,7 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
             atomicAdd(&mut[wk.x].total[ty][1], tot[ty]);
             atomicAdd(&mut[wk.x].accep[ty][1], acc_n[ty]);
         }
-        atomicAdd(&mut[wk.x].pair_evals[0], evals);
+        atomicAdd(&mut[wk.x].pair_evals[0], 2ull * mids * (unsigned)(N - 1));
     }
 }
 
@@ -2252,10 +2253,10 @@ __global__ __launch_bounds__(256, 2) void k_rotor3d_parts(const Rep* __restrict_
         const unsigned long long slices = (unsigned long long)e.nsweep * ns, items_a = (unsigned long long)(rp.RotRatio * rp.nl_atom);
         atomicAdd(&mut[r].total[rp.imtype][2], slices * nrot);
         atomicAdd(&mut[r].accep[rp.imtype][2], sacc);
-        // the atoms' terms of every proposal, the pair terms (two rotors: one per move, and with the
-        // energies ahead the one of both moved), and the current orientations' once per launch
+        // the atoms' terms of every proposal, the pair terms (two rotors: one per move, though with the
+        // energies ahead a third was formed), and the current orientations' once per launch
         const unsigned long long pairs = nrot < 2 ? 0 : (unsigned long long)rp.RotRatio;
-        atomicAdd(&mut[r].pair_evals[2], (slices + ns) * nrot * items_a + (slices * (ahead ? 3 : 2) + ns) * pairs);
+        atomicAdd(&mut[r].pair_evals[2], (slices + ns) * nrot * items_a + (slices * 2 + ns) * pairs);
     }
 }
 
