@@ -1466,6 +1466,17 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
 }
 
 // ------------------------------------------------------------------------- non-linear rotors
+// The axis that MCRot3Dstep keeps of an accepted move (mc_piqmc.cc:938-1199): a frame's third column
+// but for the last bit.  In fixed operations, so that every form of the sweep stores the same bits.
+__device__ __forceinline__ void store_axis(RotBead& b, double phi, double cth) {
+    const double sint = sqrt(fma(-cth, cth, 1.0));
+    double sn, cs;
+    sincos(phi, &sn, &cs);
+    b.nx = sint * cs;
+    b.ny = sint * sn;
+    b.nz = cth;
+}
+
 // MCRotations3D (mc_piqmc.cc:692-779) with MCRot3Dstep (:938-1199): even slices, then odd;
 // at each slice every rotor in turn.  One workgroup per replica and a group of G lanes per
 // slice: the density factors rho(t0,t1), rho(t1,t2) (old) and rho(t0,t1'), rho(t1',t2) (new)
@@ -1589,14 +1600,11 @@ __global__ __launch_bounds__(BLOCK) void k_rotor3d(const Rep* __restrict__ reps,
                     const bool accepted = rd > 1.0 || rd > rand4;
                     if (accepted && gl == 0) {
                         ++nacc;
-                        const double sint = sqrt(1.0 - cost * cost);
                         RotBead b = cur;
                         b.cth = cost;
                         b.phi = phi;
                         b.chi = chi;
-                        b.nx = sint * cos(phi);
-                        b.ny = sint * sin(phi);
-                        b.nz = cost;
+                        store_axis(b, phi, cost);
                         rotb[ik] = b;
                         frames[ik] = gf[nrot];
                         gf[q] = gf[nrot];
@@ -1720,10 +1728,8 @@ __device__ __forceinline__ void rot3d_store(const Rot3dEnv& e, long long i, doub
     b.cth = cth;
     b.chi = chi;
     b.pad0 = 0.0;
-    b.nx = f.m[6];  // the axis is the frame's third column
-    b.ny = f.m[7];
-    b.nz = f.m[8];
     b.pad1 = 0.0;
+    store_axis(b, phi, cth);
     e.rotb[i] = b;
     e.frames[i] = f;
 }
@@ -2544,6 +2550,7 @@ __device__ __forceinline__ void rotor3d_da_short(const Rot3dEnv& e, const RotPar
     ahead(1, 0);
     __syncthreads();
     const int nwords = 2 * nrot * (FRAME_D + 1);
+    unsigned moved = 0;  // bit 2 parity + q: rotor q of the lane's slice (at most one of either parity: c0 is 0) was moved
 #pragma unroll 1
     for (int h = 0; h < 2 * e.nsweep; ++h) {
         const int parity = h & 1, sw = h >> 1;
@@ -2649,7 +2656,7 @@ __device__ __forceinline__ void rotor3d_da_short(const Rot3dEnv& e, const RotPar
                                 fr[q * (ns + 2) + (kl == 1 ? ns + 1 : 0)] = f;
                                 Lk[q * L + (kl == 1 ? ns : 0)] = kl == 1 ? d2 : d3;
                             }
-                            rot3d_store(e, e.at(q, k0 + kl - 1), s.phi, s.cth, s.chi, f);
+                            moved |= 1u << (2 * parity + q);
                         }
                     }
                 }
@@ -2669,6 +2676,13 @@ __device__ __forceinline__ void rotor3d_da_short(const Rot3dEnv& e, const RotPar
         if (sw + 1 < e.nsweep) ahead(parity, sw + 1);
         lds_barrier();
         if (*s_err) break;  // as in rotor3d_ahead
+    }
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+        if (!(moved >> i & 1)) continue;
+        const int kl = 2 * (wv + l * nw) + (i >> 1) + 1, q = i & 1;
+        const Slice& s = sl[q * ns + kl - 1];
+        rot3d_store(e, e.at(q, k0 + kl - 1), s.phi, s.cth, s.chi, fr[q * (ns + 2) + kl]);
     }
 }
 
@@ -2954,14 +2968,11 @@ __device__ __forceinline__ void rotor3d_da_long(const Rot3dEnv& e, const RotPart
                             const double rd2 = exp(-rp.tau * (dve - dvs));
                             if (rd2 > 1.0 || rd2 > rand5) {
                                 ++nacc;
-                                const double sint = sqrt(1.0 - cost * cost);
                                 RotBead b = cur;
                                 b.cth = cost;
                                 b.phi = phi;
                                 b.chi = chi;
-                                b.nx = sint * cos(phi);
-                                b.ny = sint * sin(phi);
-                                b.nz = cost;
+                                store_axis(b, phi, cost);
                                 rotb[ik] = b;
                                 frames[ik] = prop[l];
                                 Lk[q * L + kl - 1] = d2;
