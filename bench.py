@@ -7,9 +7,11 @@ independent replicas (N ~ U{1..100} He around one linear rotor, P in {64,128,256
 T ~ U(0.3, 2) K) in one context.  Prints one JSON line.
 """
 import argparse
+import hashlib
 import json
 import math
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -276,26 +278,37 @@ def cpu_baseline_reference_nl(wl, budget_s=60.0):
                        f"{cores} concurrent processes after parsing the tables; per-pass time from {n1} and {n2} passes")
 
 
-def traffic_per_launch(workload_tag, kernel):
-    """HBM bytes per dispatch of `kernel` from the rocprofv3 FETCH_SIZE/WRITE_SIZE summary in
-    profiles/ (counters scaled by the hbm_copy calibration), or None when not profiled."""
-    path = os.path.join(ROOT, "profiles", f"traffic_{workload_tag}.txt")
+def kernel_sources_id(root=ROOT):
+    """Identifies the device code: the first 16 digits of a hash over its sources without comments
+    and white space."""
+    h = hashlib.sha256()
+    d = os.path.join(root, "moribs-pimc_amd", "csrc")
+    for name in sorted(os.listdir(d)):
+        if name.startswith("pimc_"):
+            with open(os.path.join(d, name)) as f:
+                h.update("".join(re.sub(r"//[^\n]*", "", f.read()).split()).encode())
+    return h.hexdigest()[:16]
+
+
+def traffic_per_launch(workload_tag, family, root=ROOT):
+    """HBM bytes per launch of a kernel family from the rocprofv3 FETCH_SIZE/WRITE_SIZE summary in
+    profiles/ (counters scaled by the hbm_copy calibration), or None when this device code was not
+    profiled: a summary names the sources it was measured with, and counters of other kernels say
+    nothing about the time they would stand beside."""
+    path = os.path.join(root, "profiles", f"traffic_{workload_tag}.txt")
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        for line in f:
-            tok = line.split()
-            if tok and not tok[0].startswith("#") and tok[0] == kernel:
-                return float(tok[-1])
+        lines = f.read().splitlines()
+    if f"# sources {kernel_sources_id(root)}" not in lines:
+        return None
+    for line in lines:
+        tok = line.split()
+        if tok and tok[0] == family + "[launch]":
+            return float(tok[-1])
     return None
 
 
-# the linear family's bisection is one fork-join launch of its size classes; the traffic file
-# holds that launch's bytes as k_bisect<float>[launch]
-KERNEL_NAMES = {"bisect": "k_bisect<float,false>[launch]", "centroid": "k_centroid_parts<float,0,false>",
-                "rotor": "k_rotor<float>", "estimate": "k_est_tiles<float,0,false>"}
-KERNEL_NAMES_NL = {"bisect": "k_bisect_nl<float,false>", "centroid": "k_centroid_parts<float,1,false>",
-                   "rotor": "k_rotor3d_parts<float>", "estimate": "k_est_tiles<float,1,false>"}
 WORKLOAD_TAG = {"c2": "c2_256replicas", "c1": "c1_64he", "c0": "c0_8he", "c3": "c3_asymtop_32h2",
                 "c4": "c4_water2_128replicas"}
 
@@ -526,7 +539,7 @@ def main():
                 "note": "FP32 vector and LDS legs (no matrix contraction on this path); algorithmic FLOPs and "
                         f"operand bytes per pair evaluation ({FLOP_1D:g} FLOP / {BYTES_1D:g} B 1D spline, "
                         f"{FLOP_2D:g} FLOP / {BYTES_2D:g} B 2D bilinear); bound = the leg nearer its peak"}
-    roof["traffic"] = traffic_per_launch(WORKLOAD_TAG[args.workload], (KERNEL_NAMES_NL if nonlinear else KERNEL_NAMES)[dom])
+    roof["traffic"] = traffic_per_launch(WORKLOAD_TAG[args.workload], dom)
     roof["kernel"] = dom
     roof["launch_ms"] = round(launch_s * 1e3, 4)
     out = {
