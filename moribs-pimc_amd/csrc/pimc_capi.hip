@@ -1283,8 +1283,8 @@ int pimc_commit(pimc_ctx* c) {
         if (busy > 1) HIPCHECK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
     }
     // Non-linear chains split by slice range when whole chains would leave CUs idle: as many
-    // parts (powers of two, at least 16 slices each) as the device holds resident at once, since
-    // the parts of a chain wait for one another.  A short chain is one part, a long one that is not
+    // parts (powers of two, at least 16 slices each, 8 with delayed acceptance) as the device holds
+    // resident at once, since the parts of a chain wait for one another.  A short chain is one part, a long one that is not
     // split goes to k_rotor3d; with delayed acceptance every chain runs as parts of k_rotor3d_da.
     if (!rot3.empty()) {
         hipDeviceProp_t prop;

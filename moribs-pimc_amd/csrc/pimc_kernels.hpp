@@ -1,6 +1,6 @@
 // pimc_kernels.hpp -- gfx950 kernels of the sampling hot path.
 //
-//   k_bisect     linear family: a group of 16 to 256 lanes per (replica, imaginary-time segment).
+//   k_bisect     linear family: a group of 32 to 256 lanes per (replica, imaginary-time segment).
 //                All atoms' beads on the segment's inner slices, plus the linear rotor's axis
 //                there, are staged in LDS once and every atom of the selected types is moved in
 //                turn, as MCBisectionMove does (mc_piqmc.cc:194-294).  Segments of one offset
@@ -805,8 +805,8 @@ constexpr unsigned ROT_SPIN_LIMIT = 1u << 22;
 // atoms' chain of sums, exchange and test is then the time, and neither reads nor the stores of an
 // accepted move are waited for in it.  The parts' partials are added across a wave's lanes and the
 // next atom's draws are formed while they travel.  With one lane adding them, beads in memory and
-// barriers that wait for it, a launch over 64 atoms on 64 parts took 495 us, now 350; over 64 atoms
-// of 16 boxes on 8 parts each 269, now 232.
+// barriers that wait for it, a launch over 64 atoms on 64 parts took 495 us, now 345; over 64 atoms
+// of 16 boxes on 8 parts each 269, now 223.
 template <typename R, int FAM, bool MI, bool Staged>
 __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ reps, Mut* __restrict__ mut,
                                                         double4* __restrict__ beads, const RotBead* __restrict__ rotb,
@@ -1995,7 +1995,9 @@ __device__ __forceinline__ void rotor3d_ahead(const Rot3dEnv& e, const RotPart& 
 // instructions (two generator calls, the frame, six arc cosines, an energy) and what it reads: its
 // neighbours' and partner's frames, its angles, and two gathers for its links.  InLds keeps the chain's
 // state in LDS for the launch, which leaves the gathers and positions to memory: of a frame the x and
-// z axes (y is their cross product) and of the angles phi and chi, 72 bytes a rotor and slice with
+// z axes (y is their cross product, which differs from the frame's own in its last bit: a link takes
+// from y the signs of two sines and, within 1e-8 of theta = pi, an arc cosine; energies take x and z,
+// or the proposal's own frame) and of the angles phi and chi, 72 bytes a rotor and slice with
 // the link's density, so that two parts of 512 slices of two rotors share a CU; cos theta is on the
 // lane (at most one move a lane of either parity).  Even and odd slices lie apart: the lanes' accesses
 // then meet no bank twice.

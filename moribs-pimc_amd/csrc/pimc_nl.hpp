@@ -12,8 +12,9 @@ namespace pimc {
 
 constexpr double PI_D = 3.14159265358979323846;
 
-// 1/sqrt(x) for x > 0: the hardware's estimate (2^-23) and one third-order step, within an ulp or
-// so; a square root and a division are four times the instructions.
+// 1/sqrt(x) for x > 0: the hardware's estimate y (2^-23) times the binomial series of 1/sqrt(1 - e),
+// e = 1 - x y^2, to second order: 1 + e/2 + 3 e^2/8, within an ulp or so; a square root and a division
+// are four times the instructions.
 __device__ __forceinline__ double rsqrt_fast(double x) {
     const double y = __builtin_amdgcn_rsq(x);
     const double e = fma(-x * y, y, 1.0);
