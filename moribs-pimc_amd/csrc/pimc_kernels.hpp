@@ -307,7 +307,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const bool has_rotor = rp.lin_atom >= 0;  // then the last atom
     const int nat = has_rotor ? N - 1 : N;    // atoms
     const double tau = rp.tau;
-    unsigned mids = 0;  // midpoints whose terms a move's tests needed: of the levels up to its rejection
+    // Midpoints whose terms a move's tests needed: of the levels up to its rejection.  A wave of one
+    // segment counts them on the scalar unit (on its lanes they were up to 1% of a pass)
+    unsigned mids = 0;
+    auto any = [](bool b) -> bool {
+        if constexpr (GW >= 64) return __builtin_amdgcn_ballot_w64(b) != 0;
+        else return b;
+    };
     int pb = 0;  // buffer of the next partial sums
     const int tend = run.type_end < rp.ntypes ? run.type_end : rp.ntypes;
 
@@ -475,9 +481,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     // sum over all points up to a level; level acceptance of mc_piqmc.cc:263-273
                     const double c0 = p[0], c1 = (c0 + p[1]) + p[2], c2 = (((c1 + p[3]) + p[4]) + p[5]) + p[6];
                     const double dv0 = c0 * tauh, dv1 = (c1 - 2.0 * c0) * (0.5 * tauh), dv2 = (c2 - 2.0 * c1) * (0.25 * tauh);
-                    const bool a0 = dv0 < 0.0 || dv0 < t[0], a1 = a0 && (dv1 < 0.0 || dv1 < t[1]);
-                    alive = a1 && (dv2 < 0.0 || dv2 < t[2]);
-                    mids += a1 ? 7 : (a0 ? 3 : 1);
+                    // without branches: the tests' reads are then under way together
+                    const bool b0 = (dv0 < 0.0) | (dv0 < t[0]), b1 = b0 & ((dv1 < 0.0) | (dv1 < t[1]));
+                    alive = b1 & ((dv2 < 0.0) | (dv2 < t[2]));
+                    mids += 1u + (any(b0) ? 2u : 0u) + (any(b1) ? 4u : 0u);
                     cum = c2;
                 }
                 for (int l0 = three ? 3 : 0; l0 < L;) {
@@ -524,7 +531,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                             const int i1 = l0 > 0 ? np_all : i + (per_m << level);
                             for (; i < i1; ++i) cum += pt[i];
                             const double deltav = (cum - 2.0 * prev) * (tau * (double)(1 << (L - level - 1)));
-                            mids += alive ? 1u << level : 0u;
+                            mids += any(alive) ? 1u << level : 0u;
                             alive = alive && (deltav < 0.0 || deltav < tst[level]);
                         }
                     }
