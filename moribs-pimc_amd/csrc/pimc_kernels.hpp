@@ -33,6 +33,12 @@
 #include "pimc_mlp.hpp"
 #include "pimc_plan.hpp"
 
+// A launch's LDS begins on 16 bytes whatever the kernel's own __shared__ data come to.  Behind an odd
+// number of doubles it would begin 8 bytes off, and every vec4 of knots, beads or frames in it would
+// be read with two instructions or more: on a stretched 1D table k_centroid_parts took 0.31 ms that
+// way on 256 chains of 8 atoms at 128 slices and takes 0.15, 4.34 and 3.09 on 4 chains of 100 at 256.
+#define DYNAMIC_LDS __attribute__((aligned(16)))
+
 namespace pimc {
 
 struct Run {
@@ -131,7 +137,7 @@ __host__ __device__ constexpr int path_batch(int nm, int L) { return 192 > 3 * n
 __global__ __launch_bounds__(256) void k_bisect_paths(const Rep* __restrict__ reps, const Mut* __restrict__ mut,
                                                       const double4* __restrict__ beads, double4* __restrict__ prop,
                                                       const PathItem* __restrict__ items, int ring, Run run) {
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     const int l = threadIdx.x & 63;
     double* gw = smem + (threadIdx.x >> 6) * ring;  // the batch's draws: per pair 3 per midpoint, then one per level
     const PathItem item = items[blockIdx.x * 4 + (threadIdx.x >> 6)];
@@ -250,7 +256,7 @@ template <typename R, bool MI, bool UT, int GW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bisect(
     const Rep* __restrict__ reps, Mut* __restrict__ mut, double4* __restrict__ beads, const RotBead* __restrict__ rotb,
     Tables T, const double4* __restrict__ prop, const int2* __restrict__ work, Run run) {
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     using P4 = vec4_t<R>;
     const int2 wk = work[blockIdx.x];
     const Rep& rp = reps[wk.x];
@@ -587,7 +593,7 @@ __global__ __launch_bounds__(256) void k_bisect_nl(const Rep* __restrict__ reps,
                                                    double4* __restrict__ beads, const RotBead* __restrict__ rotb,
                                                    const Frame* __restrict__ frames, Tables T, Tables3 T3,
                                                    const double4* __restrict__ prop, const int2* __restrict__ work, Run run) {
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     __shared__ double red[2][4][3];  // a pass's level sums per wave, two buffers
     const int2 wk = work[blockIdx.x];
     const Rep& rp = reps[wk.x];
@@ -820,7 +826,7 @@ __global__ __launch_bounds__(256) void k_centroid_parts(const Rep* __restrict__ 
                                                         const Frame* __restrict__ frames, Tables T, Tables3 T3,
                                                         const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
                                                         unsigned long long* __restrict__ slots, int nslots, Run run) {
-    extern __shared__ double smem[];  // the 1D spline knots, then the beads [3][slice][atom]
+    extern __shared__ DYNAMIC_LDS double smem[];  // the 1D spline knots, then the beads [3][slice][atom]
     constexpr int NBUF = Staged ? 2 : 1;  // buffers for alternate atoms; unstaged, every atom ends at a barrier
     __shared__ double red[NBUF][4];
     __shared__ double part_sum[NBUF][64];
@@ -1127,7 +1133,7 @@ __global__ __launch_bounds__(256) void k_rotor(const Rep* __restrict__ reps, Mut
                                                unsigned* __restrict__ flags, unsigned long long* __restrict__ xrec, Run run,
                                                int knots_at) {
     static_assert(Lean || MPL == 1, "long parts are lean");
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     __shared__ double pe[Lean ? 1 : 2][Lean ? 1 : ROTOR_PARTIALS];
     __shared__ double4 knots[Lean ? 1 : ROTOR_KNOTS];
     __shared__ unsigned s_acc[2];
@@ -1501,7 +1507,7 @@ __global__ __launch_bounds__(BLOCK) void k_rotor3d(const Rep* __restrict__ reps,
                                                  const double4* __restrict__ beads, RotBead* __restrict__ rotb,
                                                  Frame* __restrict__ frames, Tables T, Tables3 T3, const int* __restrict__ replist,
                                                  Run run) {
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     __shared__ unsigned long long red_acc[BLOCK / 64];  // one partial per wave
     __shared__ int s_err;
     const int r = replist[blockIdx.x];
@@ -2235,7 +2241,7 @@ __global__ __launch_bounds__(256, 2) void k_rotor3d_parts(const Rep* __restrict_
                                                           Frame* __restrict__ frames, Tables T, Tables3 T3,
                                                           const RotPart* __restrict__ parts, unsigned* __restrict__ flags,
                                                           unsigned long long* __restrict__ pub, int pub_stride, Run run) {
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     __shared__ unsigned long long red_acc[4];
     __shared__ int s_err;
     const RotPart pt = parts[blockIdx.x];
@@ -3160,7 +3166,7 @@ __global__ __launch_bounds__(256) void k_est_tiles(const Rep* __restrict__ reps,
                                                    const RotBead* __restrict__ rotb, const Frame* __restrict__ frames,
                                                    Tables T, Tables3 T3, const int2* __restrict__ tiles,
                                                    unsigned* __restrict__ hist, double2* __restrict__ part) {
-    extern __shared__ double smem[];
+    extern __shared__ DYNAMIC_LDS double smem[];
     __shared__ double red[16];
     __shared__ unsigned g1s[BINSR];
     const int2 tk = tiles[blockIdx.x];
