@@ -132,11 +132,12 @@ int  pimc_commit(pimc_ctx* ctx);   /* allocates device state after all replicas 
 int  pimc_plan_rotor_parts(int nchains, const int* prot, const int* rot_ratio, const int* natoms, int fp64,
                            int lds_kb, int part_slices_max, int blocks_per_cu, int lds_per_cu, int cus_per_xcd,
                            int* parts_per_chain, int* slices_per_part, long* lds_bytes, char* msg, int len);
-/* Lanes of a bisection segment of a replica of natoms atoms in a context with `segments` segments of
-   its size class (at most 24, at most 64, more atoms), without a device: lanes[0] is what
-   pimc_commit gives it, the others what pimc_autotune also times.  Returns their number, -1 for
-   arguments out of range. */
-int  pimc_plan_bisect_lanes(int natoms, long segments, int lanes[4]);
+/* Lanes of a bisection segment of a replica of natoms atoms in a launch of `segments` segments of its
+   size class (at most 24, at most 64, more atoms), without a device: lanes[0] is what pimc_commit
+   gives it, the others what pimc_autotune also times.  A class's replicas on uniform FP32 tables are a
+   launch, the others another; stretched_1d: an FP32 launch with a 1D table of no one spacing.  Returns
+   their number, -1 for arguments out of range. */
+int  pimc_plan_bisect_lanes(int natoms, long segments, int stretched_1d, int lanes[4]);
 /* How pimc_commit splits non-linear rotor chains (MCRotations3D's checkerboard, mc_piqmc.cc:728-
    760) over workgroups, without a device; no counterpart in the reference.  One count W for all
    nchains chains of up to protmax slices with nrot rotors: the largest power of two up to 64 whose
@@ -159,7 +160,7 @@ int  pimc_plan_rotor3d_split(int protmax, int nchains, int nrot, int blocks_per_
      "bisect_lanes_small", "bisect_lanes_medium", "bisect_lanes_large"
                           lanes (64, 128 or 256, small also 32) per bisection segment for
                           replicas of at most 24, at most 64 and more atoms; by default chosen
-                          from the number of segments.  Results do not depend on them.
+                          from a launch's number of segments.  Results do not depend on them.
      "delayed_acceptance" 1: the non-linear rotor move (MCRot3Dstep mc_piqmc.cc:938-1199) runs
                           its test as three Metropolis factors: the density, the surrogate
                           network, then the exact correction (see the surrogate section below);
@@ -194,18 +195,22 @@ int  pimc_get_pass(pimc_ctx* ctx, int replica, unsigned* pass);
    every sample_every passes (0: none).  Pass numbers continue across calls. */
 int  pimc_run(pimc_ctx* ctx, int n_passes, int sample_every);
 /* Autotuner of launch shapes (no counterpart in the reference, whose OpenMP loops have no
-   tunable shape).  After pimc_commit and the initial state: times each bisection size class
-   at its lanes per segment and at 64, 128 and 256, the linear-rotor sweep at part LDS budgets of 40,
-   52, 64 and 78 KB and the centroid move split into about 256, 512 or 1024 parts, each
-   candidate over `passes` passes' launches from the same saved state, and keeps the fastest.  The chains' coordinates, orientations, counters and pass numbers are
-   restored, so results are the same as without tuning.  chosen (may be NULL, else 5 entries)
-   receives the lanes of the small, medium and large classes (64 for a class without replicas; 32
-   where two segments share a wave), the rotor budget in KB and the centroid part target. */
+   tunable shape).  After pimc_commit and the initial state: times each launch of a bisection size
+   class at its lanes per segment and at 64, 128 and 256, the linear-rotor sweep at part LDS budgets
+   of 40, 52, 64 and 78 KB and the centroid move split into about 256, 512 or 1024 parts, each
+   candidate over `passes` passes' launches from the same saved state, and keeps the fastest.  The
+   chains' coordinates, orientations, counters and pass numbers are restored, so results are the same
+   as without tuning.  chosen (may be NULL, else 5 entries) receives the lanes of the small, medium and
+   large classes (64 for a class without replicas; 32 where two segments share a wave; of a class's two
+   launches, replicas on uniform FP32 tables and others, those of the one with more segments), the
+   rotor budget in KB and the centroid part target. */
 int  pimc_autotune(pimc_ctx* ctx, int passes, long* chosen);
 /* A launch shape in force after pimc_commit or pimc_autotune (no counterpart in the reference):
    "compute_units" of the device, "rotor_blocks" workgroups of the rotor sweep, "rotor_lds_bytes"
    of dynamic LDS that each of the linear sweep's has, "proposals_beside" whether the next bisection's
-   proposals are formed beside that sweep (1) or between the launches (0). */
+   proposals are formed beside that sweep (1) or between the launches (0); "bisect_lanes_small",
+   "_medium" and "_large" per bisection segment of the replicas on uniform FP32 tables, with "_general"
+   after them of the others (64 where there are none). */
 int  pimc_launch_shape(pimc_ctx* ctx, const char* name, long* value);
 /* samples of one replica, 8 doubles each: K, V, E_rot, E_rot^2 term (ErotSQ), Cv, Cv_trans,
    Cv_rot, Erot_termSQ (mc_main.cc:551-616).  Returns the number copied.  A replica keeps up to

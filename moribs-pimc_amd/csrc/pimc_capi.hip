@@ -212,17 +212,20 @@ struct pimc_ctx {
     size_t lds_rotor = 0;
     int Smax = 1, Pmax = 1, Nmax = 1, max_types = 1;
     int bisect_block = 64;
-    // linear-family bisection in three size classes (N <= 24, <= 64, larger), each with its own
-    // lanes per segment, and in each the replicas on uniform FP32 tables and the others, with
-    // their own kernel, block and LDS; launched as parallel branches of the pass
+    // linear-family bisection in three size classes (N <= 24, <= 64, larger), and in each the replicas
+    // on uniform FP32 tables and the others, with their own kernel, lanes per segment, block and LDS;
+    // launched as parallel branches of the pass
     struct BisectLaunch {
         int n = 0, off = 0;  // blocks and their place in d_work
+        int gw = 64;         // lanes per segment (32: two segments share a wave)
         int block = 64;      // lanes per block
         size_t lds = 0;
+        long long segs = 0;
     };
-    BisectLaunch bw[3][2];        // [class][uniform FP32 tables]
-    int bw_opt[3] = {0, 0, 0};    // lanes per segment asked for (64, 128, 256; small also 32), 0: by load
-    int bw_gw[3] = {64, 64, 64};  // lanes per segment (32: two segments share a wave)
+    BisectLaunch bw[3][2];      // [class][uniform FP32 tables]
+    int bw_opt[3] = {0, 0, 0};  // lanes per segment asked for (64, 128, 256; small also 32), 0: by load
+    // a class's lanes as they are reported: those of the launch with more segments
+    long bisect_lanes(int k) const { return bw[k][bw[k][1].segs >= bw[k][0].segs].gw; }
     // proposals of the next bisection launch: the layout of the beads
     double4* d_prop = nullptr;
     PathItem* d_paths = nullptr;  // batches of (atom, segment) pairs, grouped by type, four per block
@@ -693,10 +696,10 @@ int pimc_check_replica(const pimc_replica_desc* d, char* msg, int len) {
     return m.empty() ? 0 : -1;
 }
 
-int pimc_plan_bisect_lanes(int natoms, long segments, int lanes[4]) {
+int pimc_plan_bisect_lanes(int natoms, long segments, int stretched_1d, int lanes[4]) {
     if (natoms < 1 || segments < 1 || !lanes) return -1;
     int n = 0;
-    for (int L : bisect_candidates(bisect_group(bisect_class(natoms), segments))) lanes[n++] = L;
+    for (int L : bisect_candidates(bisect_group(bisect_class(natoms), segments, stretched_1d != 0))) lanes[n++] = L;
     return n;
 }
 
@@ -967,59 +970,59 @@ static bool uniform_tables(const pimc_ctx* c, const Rep& p) {
     return !c->fp64 && (p.pot1d_id < 0 || c->t1[p.pot1d_id].uniform) && (p.pot2d_id < 0 || c->t2[p.pot2d_id].uniform);
 }
 
-// The bisection's blocks: per size class the lanes of a segment's group (want[k]: 64, 128 or 256,
-// or 0 for a choice by load), and per launch of a class the block and its LDS, and the (replica,
-// first segment) list.  Called at commit and again by the autotuner.
-static int plan_bisect(pimc_ctx* c, const int want[3]) {
+// The bisection's blocks: per launch of a size class the lanes of a segment's group (want[k][u]: 32, 64,
+// 128 or 256, or 0 for a choice by the launch's load), the block and its LDS, and the (replica, first
+// segment) list.  A launch is planned for its own segments, so that replicas on uniform tables run as
+// they do alone, and a few others among them with many lanes.  Called at commit and by the autotuner.
+static int plan_bisect(pimc_ctx* c, const int (&want)[3][2]) {
     const int rsize = c->fp64 ? 8 : 4;
     struct Item {
         int2 wk;
         long long cost;
     };
     std::vector<Item> items[3][2];
-    for (int k = 0; k < 3; ++k) {
-        long long segs = 0;  // of both launches: what the device has to hold
-        std::vector<std::pair<size_t, size_t>> need[2];  // LDS of a replica's knots and of one of its segments
-        for (const Rep& p : c->rep) {
-            if (p.fam || bisect_class(p.natoms) != k) continue;
-            segs += c->ref_order ? 1 : p.P / p.S;
-            size_t knots = 0;
-            if (p.pot1d_id >= 0) {  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
-                const Tab1D& t = c->t1[p.pot1d_id];
-                knots = t.n * (c->fp64 ? sizeof(double4) : (t.uniform ? sizeof(float2) : sizeof(float4)));
-            }
-            need[uniform_tables(c, p)].emplace_back((knots + 15) & ~(size_t)15, bisect_seg_bytes(p.natoms, p.S, rsize));
-        }
-        for (auto& b : c->bw[k]) b.n = 0;
-        if (!segs) continue;
-        int gw = want[k];
-        if (gw == 0) gw = bisect_group(k, segs);
-        // as many waves per block as share the knots in 64 KB, a single wave when there are few
-        // segments for the device's CUs
-        auto lds = [&](int u, int block) {  // a block holds one replica's segments
-            size_t b = 0;
-            for (const auto& n : need[u]) b = std::max(b, n.first + (size_t)(block / gw) * n.second);
-            return b;
-        };
-        if (gw < 64 && std::max(lds(0, 64), lds(1, 64)) > 64 * 1024) gw = 64;
-        c->bw_gw[k] = gw;
+    for (int k = 0; k < 3; ++k)
         for (int u = 0; u < 2; ++u) {
             pimc_ctx::BisectLaunch& b = c->bw[k][u];
-            b.block = std::max(gw, segs * gw >= 64 * 1024 ? 256 : 64);
-            while (b.block > std::max(gw, 64) && lds(u, b.block) > 64 * 1024) b.block /= 2;
-            b.lds = lds(u, b.block);
+            b = {};
+            std::vector<std::pair<size_t, size_t>> need;  // LDS of a replica's knots and of one of its segments
+            bool stretched = false;
+            auto mine = [&](const Rep& p) { return !p.fam && bisect_class(p.natoms) == k && uniform_tables(c, p) == (u == 1); };
+            for (const Rep& p : c->rep) {
+                if (!mine(p)) continue;
+                b.segs += c->ref_order ? 1 : p.P / p.S;
+                size_t knots = 0;
+                if (p.pot1d_id >= 0) {  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
+                    const Tab1D& t = c->t1[p.pot1d_id];
+                    knots = t.n * (c->fp64 ? sizeof(double4) : (t.uniform ? sizeof(float2) : sizeof(float4)));
+                    stretched |= !c->fp64 && !t.uniform;
+                }
+                need.emplace_back((knots + 15) & ~(size_t)15, bisect_seg_bytes(p.natoms, p.S, rsize));
+            }
+            if (!b.segs) continue;
+            b.gw = want[k][u] ? want[k][u] : bisect_group(k, b.segs, stretched);
+            // as many waves per block as share the knots in 64 KB, a single wave when there are few
+            // segments for the device's CUs
+            auto lds = [&](int block) {  // a block holds one replica's segments
+                size_t m = 0;
+                for (const auto& n : need) m = std::max(m, n.first + (size_t)(block / b.gw) * n.second);
+                return m;
+            };
+            if (b.gw < 64 && lds(64) > 64 * 1024) b.gw = 64;
+            b.block = std::max(b.gw, b.segs * b.gw >= 64 * 1024 ? 256 : 64);
+            while (b.block > std::max(b.gw, 64) && lds(b.block) > 64 * 1024) b.block /= 2;
+            b.lds = lds(b.block);
             if (b.lds > 160 * 1024) return fail(c, "segment window exceeds LDS (too many atoms for this segment size)");
             for (int r = 0; r < c->nrep; ++r) {
                 const Rep& p = c->rep[r];
-                if (p.fam || bisect_class(p.natoms) != k || uniform_tables(c, p) != (u == 1)) continue;
+                if (!mine(p)) continue;
                 const int nseg = c->ref_order ? 1 : p.P / p.S;
-                for (int q = 0; q < nseg; q += b.block / gw)
+                for (int q = 0; q < nseg; q += b.block / b.gw)
                     items[k][u].push_back({make_int2(r, q), (long long)p.natoms * p.natoms * p.S});
             }
             // largest windows first: the longest atom sequences start while the grid fills
             std::stable_sort(items[k][u].begin(), items[k][u].end(), [](const Item& x, const Item& y) { return x.cost > y.cost; });
         }
-    }
     std::vector<int2> work;
     for (int k = 2; k >= 0; --k)
         for (int u = 0; u < 2; ++u) {
@@ -1270,7 +1273,9 @@ int pimc_commit(pimc_ctx* c) {
         return (long long)a.natoms * a.natoms * a.S > (long long)b.natoms * b.natoms * b.S;
     };
     std::stable_sort(work1.begin(), work1.end(), heavier);
-    if (plan_bisect(c, c->bw_opt) || plan_paths(c)) return -1;
+    int lanes[3][2];
+    for (int k = 0; k < 3; ++k) lanes[k][0] = lanes[k][1] = c->bw_opt[k];
+    if (plan_bisect(c, lanes) || plan_paths(c)) return -1;
     {
         int busy = 0;
         for (const auto& cl : c->bw)
@@ -1746,7 +1751,7 @@ void launch_bisect_class(pimc_ctx* c, int k, int uniform, hipStream_t s, const R
     };
     auto group = [&](auto mi_c, auto ut_c) {
         constexpr bool MI = decltype(mi_c)::value, UT = decltype(ut_c)::value;
-        switch (c->bw_gw[k]) {
+        switch (b.gw) {
             case 32: launch(k_bisect<R, MI, UT, 32>); break;
             case 64: launch(k_bisect<R, MI, UT, 64>); break;
             case 128: launch(k_bisect<R, MI, UT, 128>); break;
@@ -2026,13 +2031,16 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess || copy_all(true)) {
         rc = fail(c, "autotune: event or copy failed");
     } else {
-        int chosen_lanes[3] = {c->bw_gw[0], c->bw_gw[1], c->bw_gw[2]};
-        for (int k = 0; k < 3 && rc == 0; ++k) {
-            if (c->bw[k][0].n + c->bw[k][1].n == 0) continue;
-            int best = chosen_lanes[k];
+        int chosen_lanes[3][2];
+        for (int k = 0; k < 3; ++k)
+            for (int v = 0; v < 2; ++v) chosen_lanes[k][v] = c->bw[k][v].gw;
+        for (int kv = 0; kv < 6 && rc == 0; ++kv) {
+            const int k = kv / 2, v = kv % 2;
+            if (c->bw[k][v].n == 0) continue;
+            int best = chosen_lanes[k][v];
             double tbest = -1.0;
             for (int L : bisect_candidates(best)) {
-                chosen_lanes[k] = L;
+                chosen_lanes[k][v] = L;
                 if (plan_bisect(c, chosen_lanes)) {
                     rc = -1;
                     break;
@@ -2040,18 +2048,15 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
                 const double t = timed([&](int u) {
                     const Run run{c->seed, u, c->ref_order ? 1 : 0, 0, c->max_types};
                     launch_paths(c, c->stream, u, 0, PIMC_MAX_TYPES);
-                    for (int v = 0; v < 2; ++v) {
-                        if (!c->bw[k][v].n) continue;
-                        if (c->fp64) launch_bisect_class<double>(c, k, v, c->stream, run);
-                        else launch_bisect_class<float>(c, k, v, c->stream, run);
-                    }
+                    if (c->fp64) launch_bisect_class<double>(c, k, v, c->stream, run);
+                    else launch_bisect_class<float>(c, k, v, c->stream, run);
                 });
                 if (t >= 0.0 && (tbest < 0.0 || t < tbest)) {
                     tbest = t;
                     best = L;
                 }
             }
-            chosen_lanes[k] = best;
+            chosen_lanes[k][v] = best;
         }
         if (rc == 0 && plan_bisect(c, chosen_lanes)) rc = -1;
         if (rc == 0 && !c->rot_chains.empty()) {
@@ -2106,7 +2111,7 @@ int pimc_autotune(pimc_ctx* c, int passes, long* chosen) {
             *gx = nullptr;
         }
     if (rc == 0 && chosen) {
-        for (int k = 0; k < 3; ++k) chosen[k] = c->bw_gw[k];
+        for (int k = 0; k < 3; ++k) chosen[k] = c->bisect_lanes(k);
         chosen[3] = c->rotor_lds_kb;
         chosen[4] = c->centroid_target;
     }
@@ -2121,6 +2126,12 @@ int pimc_launch_shape(pimc_ctx* c, const char* name, long* value) {
         {"rotor_blocks", (long)c->nparts + c->nrot3 + c->nparts3},
         {"rotor_lds_bytes", (long)c->lds_rotor},
         {"proposals_beside", proposals_beside(c) ? 1 : 0},
+        {"bisect_lanes_small", c->bw[0][1].gw},
+        {"bisect_lanes_medium", c->bw[1][1].gw},
+        {"bisect_lanes_large", c->bw[2][1].gw},
+        {"bisect_lanes_small_general", c->bw[0][0].gw},
+        {"bisect_lanes_medium_general", c->bw[1][0].gw},
+        {"bisect_lanes_large_general", c->bw[2][0].gw},
     };
     for (const auto& s : shapes)
         if (std::strcmp(name, s.first) == 0) {

@@ -57,18 +57,24 @@ inline std::string check_replica(const pimc_replica_desc& d) {
 // bisection size classes of the linear family by atom count
 inline int bisect_class(int natoms) { return natoms <= 24 ? 0 : (natoms <= 64 ? 1 : 2); }
 
-// Lanes of a segment's group in size class k with segs segments in all.  With few segments a chain's
+// Lanes of a segment's group in size class k in a launch of segs segments.  With few segments a chain's
 // atoms in turn are the time, and four waves shorten a move; with many the device is full and one
 // wave a segment wastes least.  Bisection per pass at 256 and 64 lanes: 40 atoms 1.02 and 1.16 ms on
 // 512 segments, 1.28 and 1.24 on 1024; 100 atoms 3.38 and 3.96 ms on 1024, 6.44 and 4.70 on 2048.
 // Up to 24 atoms a wave holds the partners as it is (8 atoms: 0.30 and 0.32 ms on 512), and two
 // segments share one on a full device (0.445 against 0.470 ms on 4096).
-inline int bisect_group(int k, long long segs) {
-    if (k == 0) return segs >= 4096 ? 32 : 64;
+// stretched: FP32 1D knots on a grid of no one spacing.  An item's knot is then searched for, a chain of
+// reads that a uniform grid does without, so a move's items go over more lanes: four waves while the
+// device holds all segments at once (1024), two beyond.  At 256, 128 and 64 lanes: 40 atoms 5.6, 7.1
+// and 11.5 ms on 1024 segments, 10.0, 7.4 and 11.5 on 1280; 100 atoms 25.9, 38.7 and 71.5 on 1024,
+// 48.1, 39.8 and 71.4 on 1280, 102, 85.9 and 144 on 4096; 8 atoms at 64 and 32: 0.86 and 1.19 on 4096.
+inline int bisect_group(int k, long long segs, bool stretched) {
+    if (k == 0) return segs >= 4096 && !stretched ? 32 : 64;
+    if (stretched) return segs <= 1024 ? 256 : 128;
     return segs <= (k == 1 ? 768 : 1280) ? 256 : 64;
 }
 
-// Lanes that the autotuner times for a size class: those it has, then the other powers of two that an
+// Lanes that the autotuner times for a launch: those it has, then the other powers of two that an
 // option can ask for.  (32 lanes are a plan's alone: they pay only where it takes them.)
 inline std::vector<int> bisect_candidates(int now) {
     std::vector<int> v{now};

@@ -25,7 +25,7 @@ def stretched_tables():
     return (r, 4.0 * 10.22 * (sr6 * sr6 - sr6)), (rg, cg, rg[1] - rg[0], cg[1] - cg[0], V)
 
 
-def chains(n_he, P, copies, others, npass, **options):
+def chains(n_he, P, copies, others, npass, keep=False, **options):
     """State and counters of `copies` replicas on the workload's uniform tables, beside replicas whose
     1D table, 2D table or both (others: pairs of 0 or 1) are the stretched ones."""
     wl = pc.workload("tiny")
@@ -37,8 +37,19 @@ def chains(n_he, P, copies, others, npass, **options):
     for k, v in options.items():
         ctx.set_option(k, v)
     pc.load_into_context(ctx, wl)
+    if keep:
+        return ctx
     ctx.run(npass)
     out = [(*ctx.get_state(r), *ctx.counters(r)) for r in range(copies)]
+    ctx.close()
+    return out
+
+
+def lanes(n_he, P, copies, others, **options):
+    """Lanes per segment of the launch on uniform tables and of the others' (one size class)."""
+    ctx = chains(n_he, P, copies, others, 0, keep=True, **options)
+    name = "bisect_lanes_" + ("small" if n_he < 24 else "medium" if n_he < 64 else "large")
+    out = ctx.launch_shape(name), ctx.launch_shape(name + "_general")
     ctx.close()
     return out
 
@@ -58,3 +69,14 @@ def test_other_tables_beside_do_not_change_a_chain(n_he, P, copies, npass):
 def test_long_parts_keep_the_arithmetic():
     alone = chains(20, 320, 32, [], 60)
     same(alone, chains(20, 320, 32, [], 60, rotor_part_slices=320, rotor_lds_kb=140))
+
+
+@pytest.mark.parametrize("n_he", [40, 100])
+def test_each_launch_has_the_lanes_of_its_own_load(n_he):
+    """P = 128 at eight slices a segment: 16 segments a chain, 2048 of 128 chains.  Lanes measured on
+    uniform tables made a pass over stretched ones up to 1.4 times as long."""
+    full, few = ph.plan_bisect_lanes(n_he + 1, 2048)[0], ph.plan_bisect_lanes(n_he + 1, 16, stretched_1d=True)[0]
+    assert lanes(n_he, 128, 128, []) == (full, 64)
+    assert lanes(n_he, 128, 128, [(1, 0)]) == (full, few) == (64, 256)
+    assert lanes(n_he, 128, 0, [(1, 1)] * 128) == (64, ph.plan_bisect_lanes(n_he + 1, 2048, stretched_1d=True)[0]) == (64, 128)
+    assert lanes(n_he, 128, 0, [(0, 1)] * 128) == (64, 64)

@@ -135,3 +135,11 @@ def test_the_autotuner_times_the_plan_first(natoms, segments, lanes):
     c = ph.plan_bisect_lanes(natoms, segments)
     assert c[0] == lanes and sorted(set(c)) == sorted(c) and set(c) == {lanes, 64, 128, 256}
     assert ph.plan_bisect_lanes(0, segments) == [] and ph.plan_bisect_lanes(natoms, 0) == []
+
+
+@pytest.mark.parametrize("natoms,segments,lanes", [
+    (9, 16, 64), (24, 1 << 20, 64), (25, 1024, 256), (25, 1025, 128), (64, 4096, 128), (65, 1024, 256), (101, 2048, 128)])
+def test_lanes_where_the_knots_are_searched_for(natoms, segments, lanes):
+    """A stretched 1D table's knots wait on a search, so a segment keeps more lanes on a full device."""
+    c = ph.plan_bisect_lanes(natoms, segments, stretched_1d=True)
+    assert c[0] == lanes and sorted(c) == [64, 128, 256]
