@@ -132,12 +132,13 @@ int  pimc_commit(pimc_ctx* ctx);   /* allocates device state after all replicas 
 int  pimc_plan_rotor_parts(int nchains, const int* prot, const int* rot_ratio, const int* natoms, int fp64,
                            int lds_kb, int part_slices_max, int blocks_per_cu, int lds_per_cu, int cus_per_xcd,
                            int* parts_per_chain, int* slices_per_part, long* lds_bytes, char* msg, int len);
-/* Lanes of a bisection segment of a replica of natoms atoms in a launch of `segments` segments of its
-   size class (at most 24, at most 64, more atoms), without a device: lanes[0] is what pimc_commit
-   gives it, the others what pimc_autotune also times.  A class's replicas on uniform FP32 tables are a
-   launch, the others another; stretched_1d: an FP32 launch with a 1D table of no one spacing.  Returns
-   their number, -1 for arguments out of range. */
-int  pimc_plan_bisect_lanes(int natoms, long segments, int stretched_1d, int lanes[4]);
+/* Lanes of a bisection segment of 2^levels slices of a replica of natoms atoms in a launch of
+   `segments` segments of its size class (at most 24, at most 64, more atoms) on ncu CUs, without a
+   device: lanes[0] is what pimc_commit gives it, the others what pimc_autotune also times.  A class's
+   replicas on uniform FP32 tables are a launch, the others another.  knots: points of the 1D table;
+   stretched_1d: they have no one spacing.  Returns the lanes' number, -1 for arguments out of range. */
+int  pimc_plan_bisect_lanes(int natoms, int levels, int knots, int fp64, int stretched_1d, long segments, int ncu,
+                            int lanes[4]);
 /* How pimc_commit splits non-linear rotor chains (MCRotations3D's checkerboard, mc_piqmc.cc:728-
    760) over workgroups, without a device; no counterpart in the reference.  One count W for all
    nchains chains of up to protmax slices with nrot rotors: the largest power of two up to 64 whose

@@ -696,10 +696,16 @@ int pimc_check_replica(const pimc_replica_desc* d, char* msg, int len) {
     return m.empty() ? 0 : -1;
 }
 
-int pimc_plan_bisect_lanes(int natoms, long segments, int stretched_1d, int lanes[4]) {
-    if (natoms < 1 || segments < 1 || !lanes) return -1;
+int pimc_plan_bisect_lanes(int natoms, int levels, int knots, int fp64, int stretched_1d, long segments, int ncu,
+                           int lanes[4]) {
+    if (natoms < 1 || levels < 1 || levels > 16 || knots < 0 || segments < 1 || ncu < 1 || !lanes) return -1;
+    const int rsize = fp64 ? 8 : 4;
+    const size_t kn = ((size_t)knots * (fp64 || stretched_1d ? 4 * rsize : 2 * rsize) + 15) & ~(size_t)15;
+    auto lds = [&](int block, int gw) {
+        return kn + (size_t)(block / gw) * bisect_seg_bytes(natoms, 1 << levels, rsize);
+    };
     int n = 0;
-    for (int L : bisect_candidates(bisect_group(bisect_class(natoms), segments, stretched_1d != 0))) lanes[n++] = L;
+    for (int L : bisect_candidates(bisect_group(bisect_class(natoms), levels, segments, stretched_1d != 0, ncu, lds))) lanes[n++] = L;
     return n;
 }
 
@@ -987,31 +993,30 @@ static int plan_bisect(pimc_ctx* c, const int (&want)[3][2]) {
             b = {};
             std::vector<std::pair<size_t, size_t>> need;  // LDS of a replica's knots and of one of its segments
             bool stretched = false;
+            int levels = 0;
             auto mine = [&](const Rep& p) { return !p.fam && bisect_class(p.natoms) == k && uniform_tables(c, p) == (u == 1); };
             for (const Rep& p : c->rep) {
                 if (!mine(p)) continue;
                 b.segs += c->ref_order ? 1 : p.P / p.S;
+                levels = std::max(levels, 31 - __builtin_clz(p.S));
                 size_t knots = 0;
                 if (p.pot1d_id >= 0) {  // (y, y'') pairs of uniform FP32 knots, else vec4 knots
                     const Tab1D& t = c->t1[p.pot1d_id];
                     knots = t.n * (c->fp64 ? sizeof(double4) : (t.uniform ? sizeof(float2) : sizeof(float4)));
-                    stretched |= !c->fp64 && !t.uniform;
+                    stretched |= !t.uniform;
                 }
                 need.emplace_back((knots + 15) & ~(size_t)15, bisect_seg_bytes(p.natoms, p.S, rsize));
             }
             if (!b.segs) continue;
-            b.gw = want[k][u] ? want[k][u] : bisect_group(k, b.segs, stretched);
-            // as many waves per block as share the knots in 64 KB, a single wave when there are few
-            // segments for the device's CUs
-            auto lds = [&](int block) {  // a block holds one replica's segments
+            auto lds = [&](int block, int gw) {  // a block holds one replica's segments
                 size_t m = 0;
-                for (const auto& n : need) m = std::max(m, n.first + (size_t)(block / b.gw) * n.second);
+                for (const auto& n : need) m = std::max(m, n.first + (size_t)(block / gw) * n.second);
                 return m;
             };
-            if (b.gw < 64 && lds(64) > 64 * 1024) b.gw = 64;
-            b.block = std::max(b.gw, b.segs * b.gw >= 64 * 1024 ? 256 : 64);
-            while (b.block > std::max(b.gw, 64) && lds(b.block) > 64 * 1024) b.block /= 2;
-            b.lds = lds(b.block);
+            b.gw = want[k][u] ? want[k][u] : bisect_group(k, levels, b.segs, stretched, c->ncu, lds);
+            if (b.gw < 64 && lds(64, b.gw) > 64 * 1024) b.gw = 64;
+            b.block = bisect_block(b.gw, b.segs, lds);
+            b.lds = lds(b.block, b.gw);
             if (b.lds > 160 * 1024) return fail(c, "segment window exceeds LDS (too many atoms for this segment size)");
             for (int r = 0; r < c->nrep; ++r) {
                 const Rep& p = c->rep[r];
@@ -1273,6 +1278,11 @@ int pimc_commit(pimc_ctx* c) {
         return (long long)a.natoms * a.natoms * a.S > (long long)b.natoms * b.natoms * b.S;
     };
     std::stable_sort(work1.begin(), work1.end(), heavier);
+    {
+        hipDeviceProp_t prop;
+        HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
+        c->ncu = prop.multiProcessorCount;
+    }
     int lanes[3][2];
     for (int k = 0; k < 3; ++k) lanes[k][0] = lanes[k][1] = c->bw_opt[k];
     if (plan_bisect(c, lanes) || plan_paths(c)) return -1;
@@ -1373,11 +1383,6 @@ int pimc_commit(pimc_ctx* c) {
     if (upv(c->d_work1, work1.data(), work1.size() * sizeof(int2)) || upv(c->d_all1, all1.data(), all1.size() * sizeof(int)) ||
         upv(c->d_rot3, rot3.data(), rot3.size() * sizeof(int)) || upv(c->d_rows1, rows1.data(), rows1.size() * sizeof(int2)))
         return fail(c, "upload failed");
-    {
-        hipDeviceProp_t prop;
-        HIPCHECK(c, hipGetDeviceProperties(&prop, 0));
-        c->ncu = prop.multiProcessorCount;
-    }
     c->nrotreps = (int)rotreps.size();
     c->nrows = (int)rows.size();
     c->d_rows = dalloc<int2>(rows.size());

@@ -63,15 +63,62 @@ inline int bisect_class(int natoms) { return natoms <= 24 ? 0 : (natoms <= 64 ? 
 // 512 segments, 1.28 and 1.24 on 1024; 100 atoms 3.38 and 3.96 ms on 1024, 6.44 and 4.70 on 2048.
 // Up to 24 atoms a wave holds the partners as it is (8 atoms: 0.30 and 0.32 ms on 512), and two
 // segments share one on a full device (0.445 against 0.470 ms on 4096).
-// stretched: FP32 1D knots on a grid of no one spacing.  An item's knot is then searched for, a chain of
-// reads that a uniform grid does without, so a move's items go over more lanes: four waves while the
-// device holds all segments at once (1024), two beyond.  At 256, 128 and 64 lanes: 40 atoms 5.6, 7.1
-// and 11.5 ms on 1024 segments, 10.0, 7.4 and 11.5 on 1280; 100 atoms 25.9, 38.7 and 71.5 on 1024,
-// 48.1, 39.8 and 71.4 on 1280, 102, 85.9 and 144 on 4096; 8 atoms at 64 and 32: 0.86 and 1.19 on 4096.
-inline int bisect_group(int k, long long segs, bool stretched) {
-    if (k == 0) return segs >= 4096 && !stretched ? 32 : 64;
-    if (stretched) return segs <= 1024 ? 256 : 128;
+inline int bisect_lanes_by_load(int k, long long segs) {
+    if (k == 0) return segs >= 4096 ? 32 : 64;
     return segs <= (k == 1 ? 768 : 1280) ? 256 : 64;
+}
+
+// Lanes of the largest block of gw-lane segments that shares the knots in 64 KB, a single wave when
+// there are few segments for the device's CUs; lds(block, gw) is a block's LDS.
+template <typename Lds>
+int bisect_block(int gw, long long segs, const Lds& lds) {
+    int block = std::max(gw, segs * gw >= 64 * 1024 ? 256 : 64);
+    while (block > std::max(gw, 64) && lds(block, gw) > 64 * 1024) block /= 2;
+    return block;
+}
+
+// How often a device of ncu CUs fills with segs segments of gw lanes: 16 waves (128 registers) and
+// 160 KB a CU.
+template <typename Lds>
+long long bisect_rounds(int gw, long long segs, int ncu, const Lds& lds) {
+    const int block = bisect_block(gw, segs, lds);
+    const long long blocks = std::min<long long>(16 * 64 / block, 160 * 1024 / std::max<size_t>(lds(block, gw), 1));
+    const long long held = std::max(1LL, blocks) * (block / gw) * ncu;
+    return (segs + held - 1) / held;
+}
+
+// Lanes of a segment's group in a launch of segs segments of size class k and up to `levels` levels:
+// those above, but all 256 where the windows' LDS, not the waves, limits the segments that the device
+// holds, and 256 lanes fill it no more often.  Bisection per pass so and with the lanes by load alone:
+// FP32, 100 atoms on 1536 segments of 32 slices 39.7 and 59.6 ms; FP64, 100 atoms on 2048 of 8 14.8
+// and 24.5, of 16 63 and 132, 200 atoms on 1536 of 16 186 and 522.
+// stretched: a 1D table on a grid of no one spacing.  An item's knot is then searched for, a chain of
+// reads that a uniform grid does without.  The time is those chains, so beyond 24 atoms the lanes are
+// those for which the fills of the device, each as long as a segment takes (10, 17 and 29 on 256, 128
+// and 64 lanes), are soonest over.  FP32 on 256, 128 and 64: 40 atoms 5.6, 7.1 and 11.5 ms on 1024
+// segments of 8 slices, 10.0, 7.4 and 11.5 on 1280; 100 atoms 25.9, 38.7 and 71.5 on 1024, 48.1, 39.8
+// and 71.4 on 1280, 102, 85.9 and 144 on 4096, of 4 slices 28.5, 25.3 and 21.3 on 4096; FP64, 100 atoms
+// on 2048 of 8 82, 105 and 155.  Two groups of 128 lanes share a block's barrier, and beyond three
+// levels each waits for the other's passes: 64 atoms on 2048 of 16 61 ms on 256 lanes, 86 on 128.
+// Up to 24 atoms 64 lanes (8 atoms on 4096 segments 0.86 ms, and 1.19 on 32).
+template <typename Lds>
+int bisect_group(int k, int levels, long long segs, bool stretched, int ncu, const Lds& lds) {
+    if (stretched && k > 0) {
+        int best = 256;
+        long long cost = 10 * bisect_rounds(256, segs, ncu, lds);
+        for (const auto& [gw, fill] : {std::pair<int, int>{128, 17}, {64, 29}}) {
+            const long long t = fill * bisect_rounds(gw, segs, ncu, lds);
+            if (t < cost && !(gw == 128 && levels > 3)) {
+                cost = t;
+                best = gw;
+            }
+        }
+        return best;
+    }
+    int gw = stretched ? 64 : bisect_lanes_by_load(k, segs);
+    if (gw < 64 && lds(64, gw) > 64 * 1024) gw = 64;
+    const long long fills = bisect_rounds(gw, segs, ncu, lds);
+    return fills > 1 && bisect_rounds(256, segs, ncu, lds) <= fills ? 256 : gw;
 }
 
 // Lanes that the autotuner times for a launch: those it has, then the other powers of two that an

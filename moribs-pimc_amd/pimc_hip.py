@@ -67,7 +67,7 @@ SIGNATURES = {
     "pimc_commit": (_i, [ctypes.c_void_p]),
     "pimc_check_replica": (_i, [ctypes.POINTER(ReplicaDesc), ctypes.c_char_p, _i]),
     "pimc_set_minimum_image": (_i, [ctypes.c_void_p, _i, _dp]),
-    "pimc_plan_bisect_lanes": (_i, [_i, ctypes.c_long, _i, _ip]),
+    "pimc_plan_bisect_lanes": (_i, [_i, _i, _i, _i, _i, ctypes.c_long, _i, _ip]),
     "pimc_plan_rotor3d_split": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "pimc_plan_rotor_parts": (_i, [_i, _ip, _ip, _ip, _i, _i, _i, _i, _i, _i, _ip, _ip, ctypes.POINTER(ctypes.c_long),
                                    ctypes.c_char_p, _i]),
@@ -150,10 +150,11 @@ def plan_rotor_parts(prot, rot_ratio, natoms, fp64=False, lds_kb=52, part_slices
     return W, ns, lds.value
 
 
-def plan_bisect_lanes(natoms, segments, stretched_1d=False, lib=None):
+def plan_bisect_lanes(natoms, segments, stretched_1d=False, levels=3, knots=500, fp64=False, ncu=256, lib=None):
     """pimc_plan_bisect_lanes: the lanes of a bisection segment, then the autotuner's other candidates."""
     lanes = (ctypes.c_int * 4)()
-    n = (lib or load_library()).pimc_plan_bisect_lanes(int(natoms), int(segments), int(bool(stretched_1d)), lanes)
+    n = (lib or load_library()).pimc_plan_bisect_lanes(int(natoms), int(levels), int(knots), int(bool(fp64)),
+                                                       int(bool(stretched_1d)), int(segments), int(ncu), lanes)
     return list(lanes[:max(n, 0)])
 
 

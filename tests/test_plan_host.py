@@ -137,9 +137,21 @@ def test_the_autotuner_times_the_plan_first(natoms, segments, lanes):
     assert ph.plan_bisect_lanes(0, segments) == [] and ph.plan_bisect_lanes(natoms, 0) == []
 
 
-@pytest.mark.parametrize("natoms,segments,lanes", [
-    (9, 16, 64), (24, 1 << 20, 64), (25, 1024, 256), (25, 1025, 128), (64, 4096, 128), (65, 1024, 256), (101, 2048, 128)])
-def test_lanes_where_the_knots_are_searched_for(natoms, segments, lanes):
-    """A stretched 1D table's knots wait on a search, so a segment keeps more lanes on a full device."""
-    c = ph.plan_bisect_lanes(natoms, segments, stretched_1d=True)
+@pytest.mark.parametrize("natoms,levels,segments,fp64,lanes", [
+    (9, 3, 16, 0, 64), (24, 3, 1 << 20, 0, 64), (25, 3, 1024, 0, 256), (25, 3, 1025, 0, 128), (64, 3, 2048, 0, 128),
+    (41, 2, 4096, 0, 64), (65, 3, 1024, 0, 256), (101, 3, 2048, 0, 128), (101, 3, 4096, 0, 128), (101, 2, 4096, 0, 64),
+    (101, 4, 2048, 0, 256), (101, 3, 2048, 1, 256), (41, 4, 1024, 1, 256), (64, 4, 2048, 0, 256), (201, 3, 3072, 0, 256)])
+def test_lanes_where_the_knots_are_searched_for(natoms, levels, segments, fp64, lanes):
+    """A stretched 1D table's knots wait on a search, so the lanes are those with which the fills of the
+    device (16 waves a CU, and what its LDS holds of the windows) are soonest over."""
+    c = ph.plan_bisect_lanes(natoms, segments, stretched_1d=True, levels=levels, fp64=fp64)
     assert c[0] == lanes and sorted(c) == [64, 128, 256]
+
+
+@pytest.mark.parametrize("natoms,levels,segments,fp64,lanes", [
+    (101, 5, 1536, 0, 256), (101, 3, 2048, 1, 256), (101, 4, 2048, 1, 256), (201, 3, 3072, 1, 256), (65, 4, 2560, 1, 256),
+    (101, 2, 4096, 1, 64), (101, 3, 2048, 0, 64), (101, 3, 1 << 15, 0, 64), (41, 4, 2560, 0, 64), (41, 3, 2048, 1, 64)])
+def test_lanes_where_lds_holds_few_windows(natoms, levels, segments, fp64, lanes):
+    """One wave a segment wastes least on a device full of waves; where the windows' LDS fills it
+    first, four waves a segment fill it no more often and are three times as fast each."""
+    assert ph.plan_bisect_lanes(natoms, segments, levels=levels, fp64=fp64)[0] == lanes
