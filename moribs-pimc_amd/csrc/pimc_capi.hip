@@ -1160,6 +1160,7 @@ int pimc_commit(pimc_ctx* c) {
             if (d.molecule[t] == 1 && (d.pot2d[t] >= (int)c->t2.size() || (n_plain > 0 && d.pot2d[t] < 0)))
                 return fail(c, "linear rotor without a 2D potential table");
         }
+        p.level_passes = bisect_level_passes(p.natoms, S, p.pot1d_id >= 0 && !c->t1[p.pot1d_id].uniform);
         if (p.fam == 1) {
             if (p.pot3d_id >= (int)c->t3.size() || (p.natoms > p.nrot && p.pot3d_id < 0))
                 return fail(c, "non-linear rotor without a 3D potential table");

@@ -43,6 +43,7 @@ struct Rep {
     int h3_off;    // (r, theta, chi) bins around a non-linear rotor, from hist_off; -1 if none
     int hrel_off;  // relative Euler angle bins (theta, phi, chi) of rotor links, from hist_off; -1 if none
     int minimage;  // 1: separations of atom pairs and kinetic links take the nearest periodic image
+    int level_passes;  // 1: the bisection's first three levels are a pass each (bisect_level_passes)
     double lambda[MAXT], mcstep[MAXT];
     double T, beta, tau, rtstep;
     double box[3];  // BoxSize (mc_setup.cc:343-366), used when minimage is set

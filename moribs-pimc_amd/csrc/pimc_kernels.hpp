@@ -341,7 +341,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             nwf[i] = q;
             if (i < L) th[8 * buf + i] = v.w;
         };
-        const bool three = L >= 3;
+        // the first three levels one by one (bisect_level_passes).  The bounds that it implies are for
+        // the compiler: with the flag alone, or with the rule written out here, the loops are 3% slower
+        const bool single = !UT && GW == 256 && !l1.uniform && nat > 64 && rp.level_passes;
+        const bool three = L >= 3 && !single;
         const int m3 = gl / (GW / 8), lv3 = m3 < 7 ? 31 - __clz(m3 + 1) : 0;  // the lane's midpoint of the first three levels
         const int slot3 = m3 < 7 && three ? ((m3 + 1 - (1 << lv3)) << (L - lv3)) + (1 << (L - lv3 - 1)) - 1 : 0;
         const double tauh = tau * (double)(1 << (L - 1));
@@ -495,11 +498,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 }
                 for (int l0 = three ? 3 : 0; l0 < L;) {
                     if (GW >= 64 ? !alive : !__any(alive)) break;
-                    // levels [l0, l1) in this pass: the first three together, then one at a time.
+                    // levels [l0, l1e) in this pass: the first three together, then one at a time.
                     // Terms of levels behind a rejection are a fifth of all on the 256-replica scan
                     // (half on 8 atoms) and cost less than a pass and a reduction per level: 5.5
                     // against 6.2 ms per pass there, 1.31 against 1.55 on a single 64-atom chain
-                    const int l1e = l0 > 0 ? l0 + 1 : (L < 3 ? L : 3);
+                    const int l1e = l0 > 0 || single ? l0 + 1 : (L < 3 ? L : 3);
                     const int m0 = (1 << l0) - 1, nmc = (1 << l1e) - 1 - m0;
                     // lanes per midpoint: the chunk's midpoints rounded up to a power of two
                     const int lgn = l0 > 0 ? l0 : (l1e == 1 ? 0 : l1e);

@@ -121,6 +121,16 @@ int bisect_group(int k, int levels, long long segs, bool stretched, int ncu, con
     return fills > 1 && bisect_rounds(256, segs, ncu, lds) <= fills ? 256 : gw;
 }
 
+// Whether the bisection on 256 lanes tests its first three levels one by one and not in one pass: where
+// a look-up is a search (a stretched 1D table) and the seven midpoints are four searches or more a lane,
+// or three where the moves are longer and their first tests reject more, the searches behind a rejection
+// cost more than the passes saved.  At once and one by one: 90 atoms on 64 segments of 8 slices 15.9 and
+// 17.8 ms, 100 22.7 and 19.7, 300 168 and 122; 64 atoms of 16 slices 26.2 and 31.2, 66 33.7 and 30.4, 100
+// 63.8 and 45.6, of 32 slices 118 and 67.6.
+inline bool bisect_level_passes(int natoms, int slices, bool stretched) {
+    return stretched && natoms > (slices > 8 ? 65 : 98);
+}
+
 // Lanes that the autotuner times for a launch: those it has, then the other powers of two that an
 // option can ask for.  (32 lanes are a plan's alone: they pay only where it takes them.)
 inline std::vector<int> bisect_candidates(int now) {
