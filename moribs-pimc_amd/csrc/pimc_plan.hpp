@@ -91,7 +91,8 @@ long long bisect_rounds(int gw, long long segs, int ncu, const Lds& lds) {
 // those above, but all 256 where the windows' LDS, not the waves, limits the segments that the device
 // holds, and 256 lanes fill it no more often.  Bisection per pass so and with the lanes by load alone:
 // FP32, 100 atoms on 1536 segments of 32 slices 39.7 and 59.6 ms; FP64, 100 atoms on 2048 of 8 14.8
-// and 24.5, of 16 63 and 132, 200 atoms on 1536 of 16 186 and 522.
+// and 24.5, of 16 63 and 132, 200 atoms on 1536 of 16 186 and 522.  Beyond three levels and 24 atoms
+// also where the device fills once: 64 atoms in a box on 1024 of 32 13.1 and 20.1.
 // stretched: a 1D table on a grid of no one spacing.  An item's knot is then searched for, a chain of
 // reads that a uniform grid does without.  The time is those chains, so beyond 24 atoms the lanes are
 // those for which the fills of the device, each as long as a segment takes (10, 17 and 29 on 256, 128
@@ -118,7 +119,7 @@ int bisect_group(int k, int levels, long long segs, bool stretched, int ncu, con
     int gw = stretched ? 64 : bisect_lanes_by_load(k, segs);
     if (gw < 64 && lds(64, gw) > 64 * 1024) gw = 64;
     const long long fills = bisect_rounds(gw, segs, ncu, lds);
-    return fills > 1 && bisect_rounds(256, segs, ncu, lds) <= fills ? 256 : gw;
+    return (fills > 1 || (k > 0 && levels > 3)) && bisect_rounds(256, segs, ncu, lds) <= fills ? 256 : gw;
 }
 
 // Whether the bisection on 256 lanes tests its first three levels one by one and not in one pass: where

@@ -150,7 +150,8 @@ def test_lanes_where_the_knots_are_searched_for(natoms, levels, segments, fp64, 
 
 @pytest.mark.parametrize("natoms,levels,segments,fp64,lanes", [
     (101, 5, 1536, 0, 256), (101, 3, 2048, 1, 256), (101, 4, 2048, 1, 256), (201, 3, 3072, 1, 256), (65, 4, 2560, 1, 256),
-    (101, 2, 4096, 1, 64), (101, 3, 2048, 0, 64), (101, 3, 1 << 15, 0, 64), (41, 4, 2560, 0, 64), (41, 3, 2048, 1, 64)])
+    (101, 2, 4096, 1, 64), (101, 3, 2048, 0, 64), (101, 3, 1 << 15, 0, 64), (41, 4, 2560, 0, 64), (41, 3, 2048, 1, 64),
+    (64, 5, 1024, 0, 256), (41, 4, 1024, 1, 256), (41, 3, 1024, 0, 64), (24, 4, 1024, 0, 64)])
 def test_lanes_where_lds_holds_few_windows(natoms, levels, segments, fp64, lanes):
     """One wave a segment wastes least on a device full of waves; where the windows' LDS fills it
     first, four waves a segment fill it no more often and are three times as fast each."""
