@@ -211,7 +211,8 @@ int  pimc_autotune(pimc_ctx* ctx, int passes, long* chosen);
    of dynamic LDS that each of the linear sweep's has, "proposals_beside" whether the next bisection's
    proposals are formed beside that sweep (1) or between the launches (0); "bisect_lanes_small",
    "_medium" and "_large" per bisection segment of the replicas on uniform FP32 tables, with "_general"
-   after them of the others (64 where there are none). */
+   after them of the others (64 where there are none), "bisect_lanes_non_linear" of those with
+   non-linear rotors. */
 int  pimc_launch_shape(pimc_ctx* ctx, const char* name, long* value);
 /* samples of one replica, 8 doubles each: K, V, E_rot, E_rot^2 term (ErotSQ), Cv, Cv_trans,
    Cv_rot, Erot_termSQ (mc_main.cc:551-616).  Returns the number copied.  A replica keeps up to

@@ -1531,8 +1531,7 @@ int pimc_commit(pimc_ctx* c) {
         c->lds_rot3 = lds_for(c->rot3_block);
         if (!rot3.empty() && c->lds_rot3 > 160 * 1024) return fail(c, "non-linear rotor chain exceeds LDS");
     }
-    // bisection block of the non-linear family: lanes for a pass over three levels of the largest window
-    c->bisect_block = c->Nmax <= 10 ? 64 : (c->Nmax <= 19 ? 128 : 256);
+    c->bisect_block = bisect_nl_lanes(c->Nmax, 31 - __builtin_clz(c->Smax), c->nwork1, c->fp64);
     c->committed = true;
     return 0;
 }
@@ -2132,6 +2131,7 @@ int pimc_launch_shape(pimc_ctx* c, const char* name, long* value) {
         {"rotor_blocks", (long)c->nparts + c->nrot3 + c->nparts3},
         {"rotor_lds_bytes", (long)c->lds_rotor},
         {"proposals_beside", proposals_beside(c) ? 1 : 0},
+        {"bisect_lanes_non_linear", c->bisect_block},
         {"bisect_lanes_small", c->bw[0][1].gw},
         {"bisect_lanes_medium", c->bw[1][1].gw},
         {"bisect_lanes_large", c->bw[2][1].gw},

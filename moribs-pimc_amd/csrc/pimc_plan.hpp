@@ -132,6 +132,22 @@ inline bool bisect_level_passes(int natoms, int slices, bool stretched) {
     return stretched && natoms > (slices > 8 ? 65 : 98);
 }
 
+// Lanes of a non-linear bisection's workgroup, one a segment: a wave or more for a pass over three levels
+// of the largest window, fewer where the device (eight waves a CU) would fill more often than a
+// segment's time is shortened.  FP32, at 256, 128 and 64 lanes: 13 atoms 0.64 and 0.71 ms (128, 64) on
+// 1024 segments, 1.15 and 0.80 on 2048; 25 atoms 0.92, 1.02 and 1.28 on 512, 1.57, 1.09 and 1.31 on 1024,
+// 2.51, 2.05 and 2.57 on 2048; 61 atoms 2.36, 2.85 and 4.13 on 512, 4.25, 3.24 and 4.61 on 1024; 101 on
+// 1024 7.92, 6.36 and 9.73.  FP64 fills by its windows too: 13 atoms 1.76 and 2.02 (128, 64) on 2048; 25
+// atoms 2.16, 1.51 and 1.79 on 1024, 33 3.39, 3.94 and 5.15, and 6.54, 6.12 and 8.27 on 2048, 61 6.57,
+// 8.77 and 12.9 on 1024.  So do windows of more than three levels.
+inline int bisect_nl_lanes(int natoms, int levels, long long segs, bool fp64) {
+    if (natoms <= 10) return 64;
+    if (natoms <= 19) return segs > 1024 && !fp64 ? 64 : 128;
+    if (levels > 3) return 256;
+    if (fp64) return natoms <= 48 && segs > (natoms <= 28 ? 512 : 1024) ? 128 : 256;
+    return segs > 512 ? 128 : 256;
+}
+
 // Lanes that the autotuner times for a launch: those it has, then the other powers of two that an
 // option can ask for.  (32 lanes are a plan's alone: they pay only where it takes them.)
 inline std::vector<int> bisect_candidates(int now) {

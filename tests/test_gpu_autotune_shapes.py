@@ -5,6 +5,8 @@ import pytest
 
 import pimc_configs as pc
 import pimc_hip as ph
+from golden import tables3d
+from test_gpu_nonlinear import nl_workload
 
 pytestmark = pytest.mark.gpu
 SEED = 985456376
@@ -61,4 +63,18 @@ def test_rotor_budget_of_a_part(kb, state_kb):
     ctx = chains(40, 128, 1, rotor_lds_kb=kb)
     want = ph.plan_rotor_parts([128], [1], [41], lds_kb=state_kb)[2]
     assert ctx.launch_shape("rotor_lds_bytes") == want
+    ctx.close()
+
+
+@pytest.mark.parametrize("n_h2,copies,flags,lanes", [
+    (9, 129, 0, 64), (10, 128, 0, 128), (10, 129, 0, 64), (18, 129, 0, 64), (10, 129, ph.FLAG_FP64, 128), (19, 64, 0, 256),
+    (19, 65, 0, 128), (19, 65, ph.FLAG_FP64, 128), (32, 65, ph.FLAG_FP64, 256), (32, 129, ph.FLAG_FP64, 128)])
+def test_lanes_of_a_segment_beside_a_non_linear_rotor(n_h2, copies, flags, lanes):
+    """32 slices at four a segment: eight segments a chain, 1024 of 128 chains."""
+    wl = nl_workload("h2o_h2", tables3d.rot3d(), n_h2=n_h2, P=32, Prot=32)
+    ctx = ph.Context(copies, seed=SEED, flags=flags)
+    pc.load_into_context(ctx, dict(tables=wl["tables"], replicas=wl["replicas"] * copies))
+    assert ctx.launch_shape("bisect_lanes_non_linear") == lanes
+    ctx.run(1)
+    assert ctx.counters(0)[1][0][1] > 0
     ctx.close()
